@@ -529,6 +529,7 @@ struct SysConst {
     float Lh[3], Ll[3];   // box edge as FP32 head + tail (fx_image_c)
     double Ld[3];
     float sqmaxcut;
+    float reach;   // centre distance beyond which no pair term can be non-zero (with a margin for FP32)
     int nt;
 };
 
@@ -556,6 +557,7 @@ struct ChainTab {
     const int* cw;
     const MolP* mol;
     const PP64* pp64;
+    const int* slot;   // slot of a particle, by ID
 };
 
 // EBond::harmonicPotential, paire.h:202-204
@@ -677,14 +679,6 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// The synchronisation of one trial's threads: the block, or (WS) only the
-// calling wave, when the waves of a block evaluate trials of their own.
-template <bool WS>
-__device__ __forceinline__ void tsync() {
-    if constexpr (WS) wave_lds_sync();
-    else __syncthreads();
-}
-
 template <int NW>
 __global__ __launch_bounds__(WAVE * NW) void k_energy_all(Grid g, SysConst sc, const int* __restrict__ starts,
                                                           const uint4* __restrict__ P, const float4* __restrict__ O,
@@ -1066,12 +1060,11 @@ struct MlpConst {
 // state flags (bit 28: old, 29: new), in stencil order.  The first SB threads
 // of the block scan, PA entries each per round; the others only take part in
 // the compaction barriers.  With chain bonds it records the staged index of
-// each bonded partner.  tid is the thread's index among the trial's threads;
-// entries beyond ncap are counted in nn but not stored.
+// each bonded partner.
 template <int NW, int PA>
 __device__ __forceinline__ void scan_stencil(const Stage& S, int k, const uint4 uo, const uint4 un, bool moved,
                                              const SysConst& sc, int bmask, int idk, const TrialScratch& T, int SB,
-                                             bool scanner, int& nn, int& cpar, int ncap, int tid) {
+                                             bool scanner, int& nn, int& cpar, int tid) {
     for (int base = 0; base < S.n; base += PA * SB) {
         int fl[PA], jv[PA];
 #pragma unroll
@@ -1101,33 +1094,27 @@ __device__ __forceinline__ void scan_stencil(const Stage& S, int k, const uint4 
         block_compactK<NW, PA>(fb, nn, T.cnt, cpar, pv);
 #pragma unroll
         for (int h = 0; h < PA; h++)
-            if (fl[h] && pv[h] < ncap) T.nl[pv[h]] = jv[h] | (fl[h] << 28);
+            if (fl[h]) T.nl[pv[h]] = jv[h] | (fl[h] << 28);
     }
 }
 
-// The network's 12 features of expensive-list entry e (moving particle as
-// part1 at the entry's state, the neighbour as part2); false, with zero
-// features, for entries past nx and for pairs of other types (they screen
-// with 0).
-__device__ __forceinline__ bool pair_features(const Stage& S, const TrialScratch& T, int nx, int e, int t,
-                                              const uint4 uo, const uint4 un, const float* mvo, const float* mvn,
-                                              const SysConst& sc, const MlpConst& mc, float* f, int& which) {
+// The network's 12 features of the pair of the moving particle (as part1, at
+// position um with axis dm and patch direction pm) and the staged particle jj
+// at segment distance dseg; false, with zero features, when !valid and for
+// pairs of other types (they screen with 0).
+__device__ __forceinline__ bool pair_features(const Stage& S, bool valid, int jj, float dseg, int t, const uint4 um,
+                                              const V3<float>& dm, const V3<float>& pm, const SysConst& sc,
+                                              const MlpConst& mc, float* f) {
     bool net = false;
-    which = 0;
-    if (e < nx) {
-        int w = T.xl[e];
-        int jj = w & 0x3fffffff;
-        which = (w >> 30) & 1;
+    if (valid) {
         uint4 b = S.u[jj];
         net = t == mc.tnet && (int)b.w == mc.tnet;
         if (net) {
-            V3<float> r = which ? fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll)
-                                : fx_image_c(uo.x, uo.y, uo.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
-            const float* mv = which ? mvn : mvo;
+            V3<float> r = fx_image_c(um.x, um.y, um.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
             float4 ob = S.o[jj];
             float2 qb = S.q[jj];
-            mlp_features(mv_vec(mv, 0), mv_vec(mv, 3), mk<float>(ob.x, ob.y, ob.z), mk<float>(ob.w, qb.x, qb.y), r,
-                         T.xd[e], mc.lsc, mc.rcut, mc.pdis, mc.pswitch, f);
+            mlp_features(dm, pm, mk<float>(ob.x, ob.y, ob.z), mk<float>(ob.w, qb.x, qb.y), r, dseg, mc.lsc, mc.rcut,
+                         mc.pdis, mc.pswitch, f);
         }
     }
     if (!net)
@@ -1145,7 +1132,7 @@ __device__ __forceinline__ bool pair_features(const Stage& S, const TrialScratch
 // bonded partner lies outside the staged stencil is rejected (stage -1): the
 // partner might be moving in another cell of the pass, and the rejection does
 // not depend on the move (the particle stays in its cell).
-template <int DA, int NW, bool WS = false>
+template <int DA, int NW>
 __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint4 uo, const uint4 un,
                                                const float4 oo, const float2 qo, const float4 on, const float2 qn,
                                                const SysConst& sc,
@@ -1154,9 +1141,8 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
                                                const unsigned char* __restrict__ mlp_img,
                                                const MlpConst& mc, const ChainTab& ct, double thr1, double thr2,
                                                const float* hvk, bool translate, double& eo, double& en,
-                                               double& des, int& stage, int ncap, int xcap) {
-    static_assert(!WS || NW == 1, "a wave's own trial is a one-wave trial");
-    const int tid = WS ? lane_id() : (int)threadIdx.x, lane = tid & (WAVE - 1), BS = WAVE * NW;
+                                               double& des, int& stage) {
+    const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1), BS = WAVE * NW;
     int t = uo.w;
     bool moved = (uo.x != un.x) || (uo.y != un.y) || (uo.z != un.z);
     const int idk = S.id[k];
@@ -1189,7 +1175,7 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
         if (lane == 0) mv_store(T.mv + MV_STRIDE, pn);
     }
     if (bmask && tid < 4) T.bp[tid] = -1;
-    if (bmask) tsync<WS>();
+    if (bmask) __syncthreads();
     // phase A: the staged particles inside sqmaxcut at either state -> near
     // list, in stencil order (one barrier per round); all waves scan a
     // translation, the waves but the last one a rotation; a single wave takes
@@ -1197,15 +1183,11 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
     int nn = 0;
     if (NW > 1 && !translate)
         scan_stencil<NW, NW >= 4 ? 3 : 8>(S, k, uo, un, moved, sc, bmask, idk, T, (NW - 1) * WAVE, wv < NW - 1, nn,
-                                         cpar, ncap, tid);
+                                         cpar, tid);
     else
         scan_stencil<NW, NW >= 4 ? 2 : (NW == 1 ? 8 : 4)>(S, k, uo, un, moved, sc, bmask, idk, T, NW * WAVE, true,
-                                                           nn, cpar, ncap, tid);
-    tsync<WS>();
-    if (nn > ncap) {   // a wave's near list is full: the trial cannot be evaluated here
-        stage = -2;
-        return false;
-    }
+                                                           nn, cpar, tid);
+    __syncthreads();
     const V3<float> dnew = translate ? dold : mv_vec(mvn, 0);
     double ao = 0.0, an = 0.0;
     if (bmask) {
@@ -1266,16 +1248,12 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
             }
         }
         int pos = block_compact1<NW>(need, nx, T.cnt, cpar);
-        if (need && pos < xcap) {
+        if (need) {
             T.xl[pos] = jj | (which << 30);
             if constexpr (DA == DA_NET) T.xd[pos] = sqrtf(dseg2);
         }
     }
-    tsync<WS>();
-    if (nx > xcap) {   // the expensive list is full (only with a wave's own bounded lists)
-        stage = -2;
-        return false;
-    }
+    __syncthreads();
     // screens of the delayed acceptance: (1) the exact cheap terms already
     // summed (repulsion, sphere pairs), (2) with DA_NET the network's patch
     // attraction, tiles of 16 pairs on MFMA.  With four waves the network runs
@@ -1303,14 +1281,11 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
             const int wv = tid >> 6;
             for (int t0 = 0; t0 < nx; t0 += MLP_TILE) {   // block-uniform: every wave in every tile
                 float f[MLP_NF];
-                int which = 0;
-                bool net = pair_features(S, T, nx, t0 + (lane & (MLP_TILE - 1)), t, uo, un, mvo, mvn, sc, mc, f,
-                                         which);
-                float out;
-                if constexpr (WS)   // a wave of its own: operands from global memory, as the last wave's screen
-                    out = mlp_tile_g(mlp_img, ml, mlp_slots(f, lane >> 4), lane);
-                else
-                    out = mlp_tile_w<NW>(mr, ml, T.hx, mlp_slots(f, lane >> 4), lane, wv);
+                const int e = t0 + (lane & (MLP_TILE - 1)), xw = e < nx ? T.xl[e] : 0, which = (xw >> 30) & 1;
+                const float* mv = which ? mvn : mvo;
+                bool net = pair_features(S, e < nx, xw & 0x3fffffff, e < nx ? T.xd[e] : 0.0f, t, which ? un : uo,
+                                         mv_vec(mv, 0), mv_vec(mv, 3), sc, mc, f);
+                float out = mlp_tile_w<NW>(mr, ml, T.hx, mlp_slots(f, lane >> 4), lane, wv);
                 if (lane < MLP_TILE && net) {
                     if (which) sn += (double)out; else so += (double)out;
                 }
@@ -1335,8 +1310,10 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
         double so = 0.0, sn = 0.0;
         for (int t0 = 0; t0 < (nx >= mc.minx ? nx : 0); t0 += MLP_TILE) {
             float f[MLP_NF];
-            int which = 0;
-            bool net = pair_features(S, T, nx, t0 + (lane & (MLP_TILE - 1)), t, uo, un, mvo, mvn, sc, mc, f, which);
+            const int e = t0 + (lane & (MLP_TILE - 1)), xw = e < nx ? T.xl[e] : 0, which = (xw >> 30) & 1;
+            const float* mv = which ? mvn : mvo;
+            bool net = pair_features(S, e < nx, xw & 0x3fffffff, e < nx ? T.xd[e] : 0.0f, t, which ? un : uo,
+                                     mv_vec(mv, 0), mv_vec(mv, 3), sc, mc, f);
             float out = mlp_tile_g(mlp_img, ml, mlp_slots(f, lane >> 4), lane);
             if (lane < MLP_TILE && net) {
                 if (which) sn += (double)out; else so += (double)out;
@@ -1346,16 +1323,10 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
         if (lane == 0) *T.netd = ds;
     } else {
     int items = nx * ppmax * 2;
-    // a wave of its own whose items take more than one pass: each lane takes
-    // both sides of its patch pair, one after the other (half the passes, and
-    // the view, set-up and attraction once per patch pair; wave-uniform, and
-    // the same values: each side is the same patch_side call)
-    const bool dual = WS && items > CB;
-    const int nit = dual ? items / 2 : items;
-    for (int base = 0; base < nit; base += CB) {
-        int it = dual ? 2 * (base + tid) : base + tid, which = 0, k1 = 0, k2 = 0, side = it & 1;
-        bool hit = false, hit2 = false, pair_item = false;
-        float x1 = 0.0f, x2 = 0.0f, ev = 0.0f, z1 = 0.0f, z2 = 0.0f;
+    for (int base = 0; base < items; base += CB) {
+        int it = base + tid, which = 0, k1 = 0, k2 = 0, side = it & 1;
+        bool hit = false, pair_item = false;
+        float x1 = 0.0f, x2 = 0.0f, ev = 0.0f;
         const PP32* P2 = pp;
         V3<float> r = mk<float>(0.0f, 0.0f, 0.0f);
         PatchView<float> va, vb;
@@ -1379,7 +1350,6 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
                     va = sw ? vn : vm;
                     vb = sw ? vm : vn;
                     hit = patch_side<float>(*P2, va, vb, r, k1, k2, side, x1, x2);
-                    if (dual) hit2 = patch_side<float>(*P2, va, vb, r, k1, k2, 1, z1, z2);
                     pair_item = true;
                 }
             } else if (mpp == 0 && side == 0) {
@@ -1389,13 +1359,8 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
             }
         }
         // the other side's result (lane ^ 1 holds item it ^ 1: CB is even)
-        float y1 = z1, y2 = z2;
-        int oh = hit2 ? 1 : 0;
-        if (!dual) {
-            y1 = __shfl_xor(x1, 1);
-            y2 = __shfl_xor(x2, 1);
-            oh = __shfl_xor(hit ? 1 : 0, 1);
-        }
+        float y1 = __shfl_xor(x1, 1), y2 = __shfl_xor(x2, 1);
+        int oh = __shfl_xor(hit ? 1 : 0, 1);
         if (pair_item && side == 0 && hit && oh) ev = patch_atr<float>(*P2, va, vb, r, k1, k2, x1, x2, y1, y2);
         if (which) an += (double)ev; else ao += (double)ev;
     }
@@ -1611,8 +1576,7 @@ __device__ __forceinline__ void sweep_cell(int b, const Grid& g, const SysConst&
         int stage;
         const float* hvk = hcache ? hv + (k - S.h0) * MV_STRIDE : nullptr;
         pass = trial_energies<DA, NW>(S, k, uo, un, oo, qo, on, qn, sc, pp, tp, ppmax, T, ml, mr, mlp_img, mc, ct,
-                                      R.thr1,
-                                      R.thr2, hvk, translate, eo, en, des, stage, cap, 2 * cap);
+                                      R.thr1, R.thr2, hvk, translate, eo, en, des, stage);
         if (stage < 0) {   // a chain partner outside the stencil
             n_bond++;
             __syncthreads();
@@ -1695,8 +1659,9 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_pass(Grid g, SysConst sc
 // of states and decisions is the sequential sweep's (only the FP64 sums run
 // in another order, as between the 1- and 4-wave sweeps).
 #define SPEC_W 4
-#define SPEC_LCAP 320   // near-list entries of one wave's trial (a stencil of ~450 has ~60 within maxcut)
-#define SPEC_XCAP 192   // its (pair, state) entries within the attraction's range (typically 10-20)
+#define SPEC_STAGE_BYTES 48   // per staged particle: its record, ID and source index
+#define SPEC_LCAP 320   // candidates of one wave's trial at either state (typically ~20)
+#define SPEC_XCAP 192   // its (pair, state) entries within the attraction's range (typically 5-10)
 
 struct __align__(16) SpecRes {
     uint4 uo, un;    // position at the round's start and proposed
@@ -1713,22 +1678,19 @@ struct __align__(16) SpecRes {
 // scratch blocks, then what the waves share (byte offsets; per-wave fields
 // relative to the wave's block).
 struct SpecLayout {
-    size_t nl, xl, xd, mv, bp, cnt, red, netd, wstride;
+    size_t nl, xl, xd, mv, bp, wstride;
     size_t wbase, sten, misc, res, recs, hv, ml, tab, end;
 };
 __host__ __device__ inline size_t spec_align(size_t x, size_t a) { return (x + a - 1) / a * a; }
-__host__ __device__ inline SpecLayout spec_layout(int cap, int lcap, int xcap, bool net, size_t tab_bytes) {
+__host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_bytes) {
     SpecLayout L;
     L.nl = 0;
-    L.xl = L.nl + 4 * (size_t)lcap;
-    L.xd = L.xl + 4 * (size_t)xcap;
-    L.mv = spec_align(L.xd + (net ? 4 * (size_t)xcap : 0), 16);
+    L.xl = L.nl + 2 * 2 * SPEC_LCAP;
+    L.xd = spec_align(L.xl + 2 * SPEC_XCAP, 4);
+    L.mv = spec_align(L.xd + (net ? 4 * SPEC_XCAP : 0), 16);
     L.bp = L.mv + 4 * 2 * MV_STRIDE;
-    L.cnt = L.bp + 16;
-    L.red = spec_align(L.cnt + 4 * 2 * CNT_HALF, 16);
-    L.netd = L.red + 8 * 16;
-    L.wstride = spec_align(L.netd + 16, 16);
-    L.wbase = spec_align((size_t)cap * (16 + 16 + 8 + 4), 16);   // the stage: u, o, q, id
+    L.wstride = L.bp + 16;
+    L.wbase = spec_align((size_t)cap * SPEC_STAGE_BYTES, 16);
     size_t o = L.wbase + SPEC_W * L.wstride;
     L.sten = o;
     o += 4 * (2 * 125 + 2);
@@ -1812,6 +1774,383 @@ __device__ __forceinline__ void spec_deps_all(const TrialRec* recs, int t, int W
     }
 }
 
+// What the wave that evaluates a speculative trial keeps in LDS.
+struct SpecScratch {
+    uint16_t* nl;   // candidates (staged indices): SPEC_LCAP of the old state, then SPEC_LCAP of the new one
+    uint16_t* xl;   // entries in the attraction's range: staged index, bit 15 the state
+    float* xd;      // segment distance of each entry (network screen)
+    float* mv;      // derived vectors of the old and the new state, MV_STRIDE floats each
+    int* bp;        // staged index of each chain partner
+};
+
+// Squared distance of the point -r (r = segment's centre - point) from the
+// segment of unit axis d and half length h.
+__device__ __forceinline__ float centre_dist2(const V3<float>& d, float h, const V3<float>& r) {
+    float t = -dot(d, r);
+    t = fminf(fmaxf(t, -h), h);
+    V3<float> v = mk<float>(r.x + t * d.x, r.y + t * d.y, r.z + t * d.z);
+    return dot(v, v);
+}
+
+// One trial of the speculative sweep, on one wave: the energies of the moving
+// particle's old and new state, in the three phases of trial_energies (whose
+// contract on eo, en, des and stage it has).  A wave of its own needs no
+// barriers: its lists are stable ballot compactions.
+//   A  per state, the staged particles whose centre lies within reach of the
+//      moving segment (reach2: range + half length, the pair term is 0 beyond
+//      it).  The test on the centre distance alone (sqmaxcut = 1.21 (length +
+//      range)^2) let three times as many through, 62 of 432 staged for
+//      TCHPSC at packing fraction 0.25 against ~20, so that the next phase
+//      took two passes of the wave instead of one.
+//   B  segment distance and repulsion of each (candidate, state)
+//   C  patch terms of the entries in range
+// stage -2: a list is full (more than SPEC_LCAP candidates of a state or
+// SPEC_XCAP entries), the trial cannot be evaluated here.
+template <int DA>
+__device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo, const uint4 un, const float4 oo,
+                                           const float2 qo, const float4 on, const float2 qn, const SysConst& sc,
+                                           const PP32* __restrict__ pp, const TP32* __restrict__ tp, int ppmax,
+                                           const SpecScratch& T, const float* ml,
+                                           const unsigned char* __restrict__ mlp_img, const MlpConst& mc,
+                                           const ChainTab& ct, double thr1, double thr2, const float* hvk,
+                                           bool translate, double& eo, double& en, double& des, int& stage) {
+    const int lane = lane_id(), t = uo.w, idk = S.id[k];
+    const int cwk = ct.cw ? ct.cw[idk] : 0, bmask = cwk & 15;
+    // derived vectors of both states: the old state's from the home cell's
+    // cache when there is one, a translation keeps them
+    const float* mvo = hvk;
+    const float* mvn = T.mv + MV_STRIDE;
+    V3<float> dold;
+    if (hvk) {
+        dold = mv_vec(hvk, 0);
+    } else {
+        DPart<float> po = load_part<float>(oo, qo, t, tp);
+        if (lane == 0) mv_store(T.mv, po);
+        dold = po.dir;
+        mvo = T.mv;
+    }
+    V3<float> dnew = dold;
+    if (translate) {
+        mvn = mvo;
+    } else {
+        DPart<float> pn = load_part<float>(on, qn, t, tp);
+        if (lane == 0) mv_store(T.mv + MV_STRIDE, pn);
+        dnew = pn.dir;
+    }
+    if (bmask) {
+        if (lane < 4) T.bp[lane] = -1;
+        wave_lds_sync();
+    }
+    // phase A, four staged particles per lane per round
+    constexpr int PA = 4;
+    const float hm = tp[t].hl, reach2 = tp[t].reach2;
+    uint16_t* const nl_new = T.nl + SPEC_LCAP;
+    int no = 0, nn = 0;
+    for (int base = 0; base < S.n; base += PA * WAVE) {
+#pragma unroll
+        for (int h = 0; h < PA; h++) {
+            const int j = base + h * WAVE + lane;
+            bool fo = false, fn = false;
+            if (j < S.n && j != k) {
+                uint4 b = S.u[j];
+                V3<float> ro = fx_image_c(uo.x, uo.y, uo.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+                V3<float> rn = ro;
+                if (translate) rn = fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+                fo = centre_dist2(dold, hm, ro) <= reach2;
+                fn = centre_dist2(dnew, hm, rn) <= reach2;
+                if (bmask) {
+                    int bit = cw_bit(S.id[j] - idk);
+                    if (bit >= 0 && ((bmask >> bit) & 1)) T.bp[bit] = j;
+                }
+            }
+            const unsigned long long mo = __ballot(fo), mn = __ballot(fn);
+            if (fo) {
+                int pos = no + wave_prefix(mo);
+                if (pos < SPEC_LCAP) T.nl[pos] = (uint16_t)j;
+            }
+            if (fn) {
+                int pos = nn + wave_prefix(mn);
+                if (pos < SPEC_LCAP) nl_new[pos] = (uint16_t)j;
+            }
+            no += __popcll(mo);
+            nn += __popcll(mn);
+        }
+    }
+    wave_lds_sync();
+    if (no > SPEC_LCAP || nn > SPEC_LCAP) {
+        stage = -2;
+        return false;
+    }
+    double ao = 0.0, an = 0.0;
+    if (bmask) {
+        int found = 0;
+        for (int q = 0; q < 4; q++) found |= (T.bp[q] >= 0 ? 1 : 0) << q;
+        if (found != bmask) {
+            stage = -1;
+            return false;
+        }
+        // lanes 0-3: the old state with partners 0-3, lanes 4-7 the new one
+        int q = lane & 3, which = (lane >> 2) & 1;
+        if (lane < 8 && ((bmask >> q) & 1)) {
+            int j = T.bp[q];
+            uint4 b = S.u[j];
+            float4 ob = S.o[j];
+            float2 qb = S.q[j];
+            const float* mv = which ? mvn : mvo;
+            double eb = bond_energy(ct.mol[cwk >> 8], ct.pp64[t * sc.nt + b.w], cw_rel(q),
+                                    fx_r12(which ? un : uo, b, sc.Ld), unit64(mv[0], mv[1], mv[2]),
+                                    unit64(mv[3], mv[4], mv[5]), unit64(ob.x, ob.y, ob.z), unit64(ob.w, qb.x, qb.y));
+            if (which) an += eb; else ao += eb;
+        }
+    }
+    // phase B
+    int nx = 0;
+    for (int base = 0; base < no + nn; base += WAVE) {
+        const int it = base + lane, which = it >= no ? 1 : 0;
+        int jj = 0;
+        bool need = false;
+        float dseg2 = 0.0f;
+        if (it < no + nn) {
+            jj = which ? nl_new[it - no] : T.nl[it];
+            uint4 b = S.u[jj];
+            V3<float> r = which ? fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll)
+                                : fx_image_c(uo.x, uo.y, uo.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+            // the pair in its canonical order, the higher ID as part1 (the
+            // order of allToAll): the pair term is then one function of the
+            // pair's state whichever particle moves, and the accepted changes
+            // add up to allToAll's differences term by term
+            const bool sw = S.id[jj] > idk;
+            const PP32& P2 = sw ? pp[b.w * sc.nt + t] : pp[t * sc.nt + b.w];
+            if (dot(r, r) <= sc.sqmaxcut) {
+                if (sw) r = mk<float>(-r.x, -r.y, -r.z);
+                float ev = 0.0f;
+                if (P2.kind <= K_SCA && P2.kind >= 0) {
+                    V3<float> dm = which ? dnew : dold, db = normalised(mk<float>(S.o[jj].x, S.o[jj].y, S.o[jj].z));
+                    DPart<float> pa, pb;
+                    pa.dir = sw ? db : dm;
+                    pb.dir = sw ? dm : db;
+                    need = scsc_cheap(P2, pa, pb, r, ev, dseg2);
+                } else if (P2.kind == K_SPH_WCA || P2.kind == K_SPH_TAYLOR) {
+                    ev = sphere_pair(P2, sqrtf(dot(r, r)));
+                } else if (P2.kind != K_NONE) {
+                    need = true;
+                }
+                if (which) an += (double)ev; else ao += (double)ev;
+            }
+        }
+        const unsigned long long m = __ballot(need);
+        if (need) {
+            int pos = nx + wave_prefix(m);
+            if (pos < SPEC_XCAP) {
+                T.xl[pos] = (uint16_t)(jj | (which << 15));
+                if constexpr (DA == DA_NET) T.xd[pos] = sqrtf(dseg2);
+            }
+        }
+        nx += __popcll(m);
+    }
+    wave_lds_sync();
+    if (nx > SPEC_XCAP) {
+        stage = -2;
+        return false;
+    }
+    des = 0.0;
+    stage = 2;
+    if constexpr (DA != DA_OFF) {   // the screens of trial_energies
+        const double rep = wave_sum_dpp(an) - wave_sum_dpp(ao);
+        stage = 0;
+        if (!(rep <= 0.0 || rep < thr1)) return false;
+        des = rep;
+        if constexpr (DA == DA_NET) {
+            stage = 1;
+            if (nx >= mc.minx) {   // the entries of both states, the same for the reverse move
+                double so = 0.0, sn = 0.0;
+                for (int t0 = 0; t0 < nx; t0 += MLP_TILE) {
+                    float f[MLP_NF];
+                    const int e = t0 + (lane & (MLP_TILE - 1)), xw = e < nx ? T.xl[e] : 0, which = xw >> 15;
+                    const float* mv = which ? mvn : mvo;
+                    bool net = pair_features(S, e < nx, xw & 0x7fff, e < nx ? T.xd[e] : 0.0f, t, which ? un : uo,
+                                             mv_vec(mv, 0), mv_vec(mv, 3), sc, mc, f);
+                    float out = mlp_tile_g(mlp_img, ml, mlp_slots(f, lane >> 4), lane);
+                    if (lane < MLP_TILE && net) {
+                        if (which) sn += (double)out; else so += (double)out;
+                    }
+                }
+                const double ds = wave_sum_dpp(sn) - wave_sum_dpp(so);
+                if (!(ds <= 0.0 || ds < thr2)) return false;
+                des = rep + ds;
+            }
+        }
+        // 2: through every screen; 3: past the first, the network not run
+        stage = (DA == DA_NET && nx < mc.minx) ? 3 : 2;
+    }
+    // phase C: (entry, patch pair, side) items, the two wedge intersections of
+    // a patch pair on neighbouring lanes; where they take more than one pass,
+    // each lane takes both sides of its patch pair, one after the other (half
+    // the passes, and the view, set-up and attraction once per patch pair; the
+    // same values: each side is the same patch_side call)
+    const int items = nx * ppmax * 2;
+    const bool dual = items > WAVE;
+    const int nit = dual ? items / 2 : items;
+    for (int base = 0; base < nit; base += WAVE) {
+        int it = dual ? 2 * (base + lane) : base + lane, which = 0, k1 = 0, k2 = 0, side = it & 1;
+        bool hit = false, hit2 = false, pair_item = false;
+        float x1 = 0.0f, x2 = 0.0f, ev = 0.0f, z1 = 0.0f, z2 = 0.0f;
+        const PP32* P2 = pp;
+        V3<float> r = mk<float>(0.0f, 0.0f, 0.0f);
+        PatchView<float> va, vb;
+        if (it < items) {
+            int e = it / (2 * ppmax), mpp = (it - e * 2 * ppmax) >> 1;
+            int w = T.xl[e];
+            int jj = w & 0x7fff;
+            which = w >> 15;
+            uint4 b = S.u[jj];
+            const bool sw = S.id[jj] > idk;   // canonical order, as in phase B
+            P2 = sw ? pp + b.w * sc.nt + t : pp + t * sc.nt + b.w;
+            r = which ? fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll)
+                      : fx_image_c(uo.x, uo.y, uo.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+            if (sw) r = mk<float>(-r.x, -r.y, -r.z);
+            const float* mv = which ? mvn : mvo;
+            if (P2->kind <= K_SCA) {
+                if (mpp < npatch_pairs(*P2)) {
+                    patch_pair_index(*P2, mpp, k1, k2);   // patches of part1 and part2
+                    PatchView<float> vm = mv_view(mv, sw ? k2 : k1),
+                                     vn = load_view<float>(S.o[jj], S.q[jj], b.w, tp, sw ? k1 : k2);
+                    va = sw ? vn : vm;
+                    vb = sw ? vm : vn;
+                    hit = patch_side<float>(*P2, va, vb, r, k1, k2, side, x1, x2);
+                    if (dual) hit2 = patch_side<float>(*P2, va, vb, r, k1, k2, 1, z1, z2);
+                    pair_item = true;
+                }
+            } else if (mpp == 0 && side == 0) {
+                DPart<float> pb = load_part<float>(S.o[jj], S.q[jj], b.w, tp);
+                DPart<float> pm = mv_part(mv, t, tp[t].geotype);
+                ev = sw ? spsc(*P2, pb, pm, r) : spsc(*P2, pm, pb, r);
+            }
+        }
+        // the other side's result (lane ^ 1 holds item it ^ 1)
+        float y1 = z1, y2 = z2;
+        int oh = hit2 ? 1 : 0;
+        if (!dual) {
+            y1 = __shfl_xor(x1, 1);
+            y2 = __shfl_xor(x2, 1);
+            oh = __shfl_xor(hit ? 1 : 0, 1);
+        }
+        if (pair_item && side == 0 && hit && oh) ev = patch_atr<float>(*P2, va, vb, r, k1, k2, x1, x2, y1, y2);
+        if (which) an += (double)ev; else ao += (double)ev;
+    }
+    eo = wave_sum_dpp(ao);
+    en = wave_sum_dpp(an);
+    return true;
+}
+
+// stage_load for the speculative sweep: of the stencil's particles only those
+// that can matter to the home cell are staged, in stencil order: those within
+// sc.reach of the cell's box, where every trial position lies, and chain
+// partners of its particles.  For 65,536 TCHPSC at packing fraction 0.25 that
+// is ~245 of 432, and every trial scans the stage.  Two passes over the
+// stencil (positions, then the records of those kept), so that the records
+// lie packed behind one another.  list: cap source indices at the end of the
+// region, beyond the records (44 cap + 4 cap bytes fit the region).
+template <int NW>
+__device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes, int cap, const Grid& g,
+                            const SysConst& sc, int cx, int cy, int cz, const int* __restrict__ starts,
+                            const uint4* __restrict__ P, const float4* __restrict__ O, const float2* __restrict__ Q,
+                            const int* __restrict__ ID, const ChainTab& ct, int* sten, int* misc) {
+    const int ns = stencil_size(g);
+    int* pre = sten;          // ns+1 prefix of counts
+    int* cst = sten + ns + 1; // cell start per stencil entry
+    const int tid = (int)threadIdx.x;
+    if (tid < WAVE) {
+        const int lane = tid;
+        int home_idx = -1, carry = 0;
+        for (int b = 0; b < ns; b += WAVE) {
+            int i = b + lane, cnt = 0, hm = 0;
+            if (i < ns) {
+                int c = stencil_cell(g, cx, cy, cz, i, hm);
+                int st = starts[c];
+                cnt = starts[c + 1] - st;
+                cst[i] = st;
+            }
+            int v = cnt;   // inclusive wave scan
+            for (int o = 1; o < WAVE; o <<= 1) {
+                int t = __shfl_up(v, o, WAVE);
+                if (lane >= o) v += t;
+            }
+            if (i < ns) pre[i] = carry + v - cnt;
+            unsigned long long hmask = __ballot(i < ns && hm);
+            if (hmask) home_idx = b + __ffsll((long long)hmask) - 1;
+            carry += __shfl(v, WAVE - 1, WAVE);
+        }
+        if (lane == 0) {
+            pre[ns] = carry;
+            misc[0] = home_idx;
+        }
+    }
+    __syncthreads();
+    const int total = pre[ns], home = misc[0], hbeg = pre[home], hend = pre[home + 1];
+    const int gs = cst[home], ge = gs + hend - hbeg;
+    // the home cell's box: centre in fixed point, half edges
+    const int c3[3] = {cx, cy, cz};
+    uint32_t cen[3];
+    float half[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        cen[q] = g.sh[q] + (uint32_t)((((uint64_t)(2 * c3[q] + 1)) << 31) / (uint64_t)g.nc[q]);
+        half[q] = 0.5f * sc.L[q] / (float)g.nc[q];
+    }
+    const float reach2 = sc.reach * sc.reach;
+    int* list = (int*)(region + region_bytes) - cap;
+    int n = 0;
+    for (int base = 0; base < total; base += WAVE * NW) {
+        const int e = base + tid;
+        bool keep = false;
+        int src = 0;
+        if (e < total) {
+            int lo = 0, hi = ns - 1;   // the stencil entry holding element e
+            while (lo < hi) {
+                int mid = (lo + hi + 1) >> 1;
+                if (pre[mid] <= e) lo = mid; else hi = mid - 1;
+            }
+            src = cst[lo] + (e - pre[lo]);
+            const uint4 u = P[src];
+            const V3<float> r = fx_image_c(u.x, u.y, u.z, cen[0], cen[1], cen[2], sc.Lh, sc.Ll);
+            const float dx = fmaxf(fabsf(r.x) - half[0], 0.0f), dy = fmaxf(fabsf(r.y) - half[1], 0.0f),
+                        dz = fmaxf(fabsf(r.z) - half[2], 0.0f);
+            keep = lo == home || dx * dx + dy * dy + dz * dz <= reach2;
+            if (!keep && ct.cw) {
+                const int id = ID[src], w = ct.cw[id];
+                for (int q = 0; q < 4; q++)
+                    if ((w >> q) & 1) {
+                        const int sl = ct.slot[id + cw_rel(q)];
+                        keep |= sl >= gs && sl < ge;
+                    }
+            }
+        }
+        const int pos = block_compact<NW>(keep, n, misc + 4);
+        if (keep && pos < cap) list[pos] = src;
+        if (e == hbeg) misc[1] = pos;
+    }
+    __syncthreads();
+    S.n = n;
+    S.h0 = misc[1];
+    S.h1 = S.h0 + (hend - hbeg);
+    if (n > cap) return false;
+    const int n4 = (n + 3) & ~3;
+    S.u = (uint4*)region;
+    S.o = (float4*)(S.u + n4);
+    S.q = (float2*)(S.o + n4);
+    S.id = (int*)(S.q + n4);
+    for (int i = tid; i < n; i += WAVE * NW) {
+        const int src = list[i];
+        S.u[i] = P[src];
+        S.o[i] = O[src];
+        S.q[i] = Q[src];
+        S.id[i] = ID[src];
+    }
+    __syncthreads();
+    return true;
+}
+
 // LT: the pair and type tables are copied into LDS (systems of up to
 // SWEEP_TABLE_MAXT types).  A compile-time choice, so their loads are LDS
 // loads: chosen at run time, the pointer could be either, and every table
@@ -1821,7 +2160,7 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
                                                 const int* __restrict__ starts, uint4* __restrict__ P,
                                                 float4* __restrict__ O, float2* __restrict__ Q,
                                                 const int* __restrict__ ID, const PP32* __restrict__ pp,
-                                                const TP32* __restrict__ tp, int cap, int lcap, int ppmax,
+                                                const TP32* __restrict__ tp, int cap, int ppmax,
                                                 const int* __restrict__ nonempty,
                                                 const unsigned char* __restrict__ mlp_img, const MlpConst& mc,
                                                 const ChainTab& ct, unsigned long long* __restrict__ stats,
@@ -1833,31 +2172,22 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     int cell = cx + g.nc[0] * (cy + g.nc[1] * cz);
     int nh = starts[cell + 1] - starts[cell];
     if (nh == 0) return;
-    const SpecLayout L = spec_layout(cap, lcap, SPEC_XCAP, NET, 0);
+    const SpecLayout L = spec_layout(cap, NET, 0);
     Stage S;
-    S.u = (uint4*)smem;
-    S.o = (float4*)(S.u + cap);
-    S.q = (float2*)(S.o + cap);
-    S.id = (int*)(S.q + cap);
     const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1), w = tid >> 6;
     unsigned char* wb = smem + L.wbase + (size_t)w * L.wstride;
-    TrialScratch T;
-    T.nl = (int*)(wb + L.nl);
-    T.xl = (int*)(wb + L.xl);
+    SpecScratch T;
+    T.nl = (uint16_t*)(wb + L.nl);
+    T.xl = (uint16_t*)(wb + L.xl);
     T.xd = (float*)(wb + L.xd);
     T.mv = (float*)(wb + L.mv);
     T.bp = (int*)(wb + L.bp);
-    T.cnt = (int*)(wb + L.cnt);
-    T.red = (double*)(wb + L.red);
-    T.hx = nullptr;
-    T.netd = (double*)(wb + L.netd);
     int* sten = (int*)(smem + L.sten);
     int* misc = (int*)(smem + L.misc);
     SpecRes* res = (SpecRes*)(smem + L.res);
     TrialRec* recs = (TrialRec*)(smem + L.recs);
     float* hv = (float*)(smem + L.hv);
-    float* ml = nullptr;
-    MlpRegsW<4> mr;   // not read: a wave's network screen takes its operands from global memory
+    float* ml = nullptr;   // the network's constants (its operands stay in global memory)
     if constexpr (NET) {
         ml = (float*)(smem + L.ml);
         for (int i = tid; i < MLP_C_BYTES / 16; i += WAVE * SPEC_W) ((uint4*)ml)[i] = ((const uint4*)(mlp_img + MLP_C_OFF))[i];
@@ -1871,7 +2201,7 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         pp = ppl;
         tp = tpl;
     }
-    if (!stage_load<SPEC_W>(S, cap, g, cx, cy, cz, starts, P, O, Q, ID, sten)) {
+    if (!stage_reach<SPEC_W>(S, smem, L.wbase, cap, g, sc, cx, cy, cz, starts, P, O, Q, ID, ct, sten, misc)) {
         if (tid == 0) atomicOr(flag, 1);
         return;
     }
@@ -1936,9 +2266,8 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
             } else {
                 double eo, en, des;
                 const float* hvk = hcache ? hv + (k - S.h0) * MV_STRIDE : nullptr;
-                bool pass = trial_energies<DA, 1, true>(S, k, uo, un, oo, qo, on, qn, sc, pp, tp, ppmax, T, ml, mr,
-                                                        mlp_img, mc, ct, R.thr1, R.thr2, hvk, translate, eo, en, des,
-                                                        stage, lcap, SPEC_XCAP);
+                bool pass = spec_trial<DA>(S, k, uo, un, oo, qo, on, qn, sc, pp, tp, ppmax, T, ml, mlp_img, mc, ct,
+                                           R.thr1, R.thr2, hvk, translate, eo, en, des, stage);
                 if (stage == -1) {
                     status = 2;
                 } else if (stage == -2) {
@@ -2049,13 +2378,13 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_spec(Grid g, SysCons
                                                              float4* __restrict__ O, float2* __restrict__ Q,
                                                              const int* __restrict__ ID,
                                                              const PP32* __restrict__ pp,
-                                                             const TP32* __restrict__ tp, int cap, int lcap,
+                                                             const TP32* __restrict__ tp, int cap,
                                                              int ppmax, const int* __restrict__ nonempty,
                                                              const unsigned char* __restrict__ mlp_img, MlpConst mc,
                                                              ChainTab ct, unsigned long long* __restrict__ stats,
                                                              double* __restrict__ de_sum, int* __restrict__ flag) {
     sweep_cell_spec<DA, LT>(xcd_slab_index((int)blockIdx.x, (int)gridDim.x), g, sc, mp, starts, P, O, Q, ID, pp, tp, cap,
-                        lcap, ppmax, nonempty, mlp_img, mc, ct, stats, de_sum, flag);
+                        ppmax, nonempty, mlp_img, mc, ct, stats, de_sum, flag);
 }
 
 // Per-replica parameters of one checkerboard pass of a replica batch.
@@ -2102,7 +2431,7 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_batch_spec(const Rep
                                                                    float2* __restrict__ Q,
                                                                    const int* __restrict__ ID,
                                                                    const PP32* __restrict__ pp,
-                                                                   const TP32* __restrict__ tp, int cap, int lcap,
+                                                                   const TP32* __restrict__ tp, int cap,
                                                                    int ppmax, const int* __restrict__ nonempty,
                                                                    const unsigned char* __restrict__ mlp_img,
                                                                    MlpConst mc, ChainTab ct,
@@ -2116,7 +2445,7 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_batch_spec(const Rep
         if (rp[mid].blk_off <= lb) lo = mid; else hi = mid - 1;
     }
     const RepPass R = rp[lo];
-    sweep_cell_spec<DA, LT>(lb - R.blk_off, R.g, R.sc, R.mp, starts + R.cell_off, P, O, Q, ID, pp, tp, cap, lcap, ppmax,
+    sweep_cell_spec<DA, LT>(lb - R.blk_off, R.g, R.sc, R.mp, starts + R.cell_off, P, O, Q, ID, pp, tp, cap, ppmax,
                         nonempty + R.rep, mlp_img, mc, ct, stats + (size_t)R.rep * STAT_REP * STAT_STRIDE,
                         de_sum + (size_t)R.rep * STAT_REP * STAT_STRIDE, flag);
 }
@@ -3618,6 +3947,7 @@ struct sc_ctx {
     TP32* d_tp32 = nullptr;
     TP64* d_tp64 = nullptr;
     double maxcut = 0, sqmaxcut = 0;
+    double reach = 0;                   // largest centre distance of a non-zero pair term
     double minvol = 1.0;
     // state
     int n = 0;
@@ -3757,6 +4087,7 @@ static ChainTab chain_tab(const sc_ctx* ctx) {
     t.cw = ctx->bonds ? ctx->d_cw : nullptr;
     t.mol = ctx->d_mol;
     t.pp64 = ctx->d_pp64;
+    t.slot = ctx->slot;
     return t;
 }
 
@@ -3896,6 +4227,21 @@ static int upload_tables(sc_ctx* ctx) {
             fill_pair(h64[a * nt + b], p, tr);
         }
     }
+    // the largest centre distance at which a pair term can be non-zero: the
+    // larger range of the type pair, and both half lengths
+    ctx->reach = 0.0;
+    for (int a = 0; a < nt; a++) {
+        double ra = 0.0;   // of centres from a segment of type a
+        for (int b = 0; b < nt; b++) {
+            const PP64& q = h64[a * nt + b];
+            if (q.kind != K_NONE) ra = std::max(ra, std::max({q.rcut, q.rcutwca, q.t_rcut}) + q.hl1);
+        }
+        ctx->reach = std::max(ctx->reach, ra + h64[a * nt + a].hl0);
+        t32[a].hl = (float)h64[a * nt + a].hl0;
+        t32[a].reach2 = (float)(ra * ra * 1.002);
+        t64[a].hl = h64[a * nt + a].hl0;
+        t64[a].reach2 = ra * ra * 1.002;
+    }
     ctx->ppmax = 1;
     for (const PP32& q : h32)
         if (q.kind >= 0 && q.kind <= K_SCA) ctx->ppmax = std::max(ctx->ppmax, npatch_pairs(q));
@@ -3985,6 +4331,7 @@ static SysConst sysconst(const sc_ctx* ctx, const double* box) {
         s.Ll[k] = (float)(box[k] - (double)s.Lh[k]);
     }
     s.sqmaxcut = (float)ctx->sqmaxcut;
+    s.reach = (float)(ctx->reach * 1.001);
     s.nt = ctx->nt;
     return s;
 }
@@ -5578,11 +5925,11 @@ static int sc_sweep_impl(sc_ctx* ctx, int nsweeps, double temper, double transmx
         size_t lds_spec = 0;
         if (spec) {
             size_t tabb = sweep_table_bytes(ctx->nt);
-            long room = (long)SWEEP_LDS_BUDGET - (long)spec_layout(0, SPEC_LCAP, SPEC_XCAP, da, tabb).end - 16;
-            int cmax = room > 0 ? (int)(room / (long)stage_bytes(1)) : 0;
+            long room = (long)SWEEP_LDS_BUDGET - (long)spec_layout(0, da, tabb).end - 16;
+            int cmax = room > 0 ? (int)(room / SPEC_STAGE_BYTES) : 0;
             if (cap_spec > cmax) cap_spec = (cmax / 64) * 64;
             spec = cap_spec >= 64;
-            if (spec) lds_spec = spec_layout(cap_spec, SPEC_LCAP, SPEC_XCAP, da, tabb).end;
+            if (spec) lds_spec = spec_layout(cap_spec, da, tabb).end;
         }
         if (da && (ctx->mlp_type < 0 || ctx->ref2dense[ctx->mlp_type] < 0))
             return fail(ctx, SC_EINVAL, "the network screen needs the network's particle type in the system");
@@ -5652,7 +5999,7 @@ static int sc_sweep_impl(sc_ctx* ctx, int nsweeps, double temper, double transmx
 #define SPEC_PASS_LT(DAM, LT, IMG, MC)                                                                         \
     hipLaunchKernelGGL((k_sweep_spec<DAM, LT>), dim3(nblk), dim3(WAVE * SPEC_W), lds_spec, ctx->stream, g, sc, mp,     \
                        ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32,          \
-                       cap_spec, SPEC_LCAP, ctx->ppmax, ctx->d_nonempty, IMG, MC, chain_tab(ctx), ctx->d_stats,    \
+                       cap_spec, ctx->ppmax, ctx->d_nonempty, IMG, MC, chain_tab(ctx), ctx->d_stats,    \
                        ctx->d_dsum, ctx->d_flag)
             // four waves per cell in every mode (the network screen splits its
             // hidden units, and so its MFMA operands, between the four waves)
@@ -5903,11 +6250,11 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
         size_t lds_spec = 0;
         if (spec) {
             size_t tabb = sweep_table_bytes(ctx->nt);
-            long room = (long)SWEEP_LDS_BUDGET - (long)spec_layout(0, SPEC_LCAP, SPEC_XCAP, false, tabb).end - 16;
-            int cmax = room > 0 ? (int)(room / (long)stage_bytes(1)) : 0;
+            long room = (long)SWEEP_LDS_BUDGET - (long)spec_layout(0, false, tabb).end - 16;
+            int cmax = room > 0 ? (int)(room / SPEC_STAGE_BYTES) : 0;
             if (cap_spec > cmax) cap_spec = (cmax / 64) * 64;
             spec = cap_spec >= 64;
-            if (spec) lds_spec = spec_layout(cap_spec, SPEC_LCAP, SPEC_XCAP, false, tabb).end;
+            if (spec) lds_spec = spec_layout(cap_spec, false, tabb).end;
         }
         size_t fixed = sizeof(float) * 2 * MV_STRIDE + sizeof(int) * (2 * 125 + 2) + SWEEP_SMALL_LDS +
                        sweep_table_bytes(ctx->nt);
@@ -5983,14 +6330,14 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
 #define SWEEP_BATCH(DAM, NWV)                                                                                  \
     SC_LAUNCH((k_sweep_batch<DAM, NWV>), dim3(nblk[ci]), dim3(WAVE * NWV), lds, ctx->stream, rp, R, ctx->starts,     \
               ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, cap, ctx->ppmax,                \
-              ctx->d_rep_nonempty, nullptr, ctx->mlp_c, ChainTab{nullptr, nullptr, ctx->d_pp64}, ctx->d_rep_stats,  \
+              ctx->d_rep_nonempty, nullptr, ctx->mlp_c, ChainTab{nullptr, nullptr, ctx->d_pp64, nullptr}, ctx->d_rep_stats,  \
               ctx->d_rep_dsum, ctx->d_flag)
 #define SPEC_BATCH(DAM)                                                                                        \
     if (spec_lt) SPEC_BATCH_LT(DAM, true); else SPEC_BATCH_LT(DAM, false)
 #define SPEC_BATCH_LT(DAM, LT)                                                                                 \
     SC_LAUNCH((k_sweep_batch_spec<DAM, LT>), dim3(nblk[ci]), dim3(WAVE * SPEC_W), lds_spec, ctx->stream, rp, R,           \
-              ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, cap_spec, SPEC_LCAP,  \
-              ctx->ppmax, ctx->d_rep_nonempty, nullptr, ctx->mlp_c, ChainTab{nullptr, nullptr, ctx->d_pp64},           \
+              ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, cap_spec,  \
+              ctx->ppmax, ctx->d_rep_nonempty, nullptr, ctx->mlp_c, ChainTab{nullptr, nullptr, ctx->d_pp64, nullptr},           \
               ctx->d_rep_stats, ctx->d_rep_dsum, ctx->d_flag)
             int nw = ctx->sweep_nw ? ctx->sweep_nw : 4;
             if (spec) {

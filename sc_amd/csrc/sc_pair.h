@@ -69,6 +69,7 @@ struct PairParamsT {
 template <typename R>
 struct TypeParamsT {
     int geotype, pad;
+    R hl, reach2;   // half length; squared distance of a centre from this type's segment beyond which the pair term is 0
     R pcoshalfi0, psinhalfi0, pcoshalfi2, psinhalfi2;
     R csec, ssec, chcos, chsin;
 };
