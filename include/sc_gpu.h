@@ -218,12 +218,14 @@ int sc_set_block_waves(sc_ctx* ctx, int nw);
  * on = 0 evaluates such systems.  No counterpart in the reference (its loop is
  * sequential). */
 int sc_set_speculation(sc_ctx* ctx, int on);
-/* The sweep keeps the derived vectors (patch sides, second patch, chiral
- * axes: Particle::init, particle.cpp:3-79) of a pass's home-cell particles in
- * LDS, computed once per pass and refreshed on acceptance, for cells of up to
- * `cap` particles (default and maximum 64); larger cells, or cap = 0, derive
- * them at every trial.  Both give the same trajectories; the setting exists
- * so that tests can compare them. */
+/* The sweep keeps derived vectors (patch sides, second patch, chiral axes:
+ * Particle::init, particle.cpp:3-79) in LDS, computed once per pass and
+ * refreshed on acceptance: the speculative sweep those of every staged
+ * particle where they fit beside the stage, else the home cell's; the
+ * sequential sweep the home cell's, for cells of up to 64 particles.  `cap`
+ * (default and maximum 64) below 64 limits that to cells of up to `cap`
+ * particles; larger cells, or cap = 0, derive them at every trial.  All give
+ * the same trajectories; the setting exists so that tests can compare them. */
 int sc_set_home_cache(sc_ctx* ctx, int cap);
 /* Colour passes per sweep of sc_sweep: a sweep visits the first 1/v of its
  * randomly ordered colours (v must divide their number: 8 for 2x2x2), and

@@ -1659,9 +1659,15 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_pass(Grid g, SysConst sc
 // of states and decisions is the sequential sweep's (only the FP64 sums run
 // in another order, as between the 1- and 4-wave sweeps).
 #define SPEC_W 4
-#define SPEC_STAGE_BYTES 48   // per staged particle: its record, ID and source index
+#define SPEC_STAGE_BYTES 48    // per staged particle: its record, ID and source index
+#define SPEC_ROW_BYTES 7168    // beyond that, for rows and chain partners; a stage below its capacity leaves more
 #define SPEC_LCAP 320   // candidates of one wave's trial at either state (typically ~20)
 #define SPEC_XCAP 192   // its (pair, state) entries within the attraction's range (typically 5-10)
+// a staged particle's row of derived vectors: floats, and where its axis and first patch direction lie
+#define VROW 28
+#define VROW_DIR 24
+#define VROW_PD0 3
+#define SPEC_NV 8       // neighbours whose rows a wave derives at once when the stage has none
 
 struct __align__(16) SpecRes {
     uint4 uo, un;    // position at the round's start and proposed
@@ -1678,8 +1684,8 @@ struct __align__(16) SpecRes {
 // scratch blocks, then what the waves share (byte offsets; per-wave fields
 // relative to the wave's block).
 struct SpecLayout {
-    size_t nl, xl, xd, mv, bp, wstride;
-    size_t wbase, sten, misc, res, recs, hv, ml, tab, end;
+    size_t nl, xl, xd, mv, wstride;
+    size_t wbase, sten, misc, res, recs, ml, tab, end;
 };
 __host__ __device__ inline size_t spec_align(size_t x, size_t a) { return (x + a - 1) / a * a; }
 __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_bytes) {
@@ -1688,9 +1694,9 @@ __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_
     L.xl = L.nl + 2 * 2 * SPEC_LCAP;
     L.xd = spec_align(L.xl + 2 * SPEC_XCAP, 4);
     L.mv = spec_align(L.xd + (net ? 4 * SPEC_XCAP : 0), 16);
-    L.bp = L.mv + 4 * 2 * MV_STRIDE;
-    L.wstride = L.bp + 16;
-    L.wbase = spec_align((size_t)cap * SPEC_STAGE_BYTES, 16);
+    L.wstride = L.mv + 4 * 2 * VROW;
+    static_assert(2 * 2 * SPEC_LCAP >= 4 * SPEC_NV * VROW, "neighbour rows over the candidate lists");
+    L.wbase = spec_align((size_t)cap * SPEC_STAGE_BYTES + SPEC_ROW_BYTES, 16);   // the stage and rows
     size_t o = L.wbase + SPEC_W * L.wstride;
     L.sten = o;
     o += 4 * (2 * 125 + 2);
@@ -1700,8 +1706,6 @@ __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_
     o = L.res + SPEC_W * sizeof(SpecRes);
     L.recs = spec_align(o, 16);
     o = L.recs + TRIAL_CHUNK * sizeof(TrialRec);
-    L.hv = spec_align(o, 16);
-    o = L.hv + 4 * (size_t)HCAP * MV_STRIDE;
     L.ml = spec_align(o, 16);
     o = L.ml + (net ? MLP_C_BYTES : 0);
     L.tab = spec_align(o, 16);
@@ -1779,8 +1783,65 @@ struct SpecScratch {
     uint16_t* nl;   // candidates (staged indices): SPEC_LCAP of the old state, then SPEC_LCAP of the new one
     uint16_t* xl;   // entries in the attraction's range: staged index, bit 15 the state
     float* xd;      // segment distance of each entry (network screen)
-    float* mv;      // derived vectors of the old and the new state, MV_STRIDE floats each
-    int* bp;        // staged index of each chain partner
+    float* mv;      // rows of the old and the new state (VROW floats each)
+    float* nv;      // rows of neighbours that have none in the stage (over nl, which is dead by then)
+};
+
+// A particle's derived vectors as the speculative sweep keeps them in LDS:
+// per patch the axis it is attached to, its direction and its two sides (12
+// floats, three 16-byte loads), then the particle's axis as derive leaves it.
+__device__ __forceinline__ void vrow_put(float* row, int k, const PatchView<float>& v) {
+    float4* p = (float4*)(row + 12 * k);
+    p[0] = make_float4(v.ax.x, v.ax.y, v.ax.z, v.pd.x);
+    p[1] = make_float4(v.pd.y, v.pd.z, v.s0.x, v.s0.y);
+    p[2] = make_float4(v.s0.z, v.s1.x, v.s1.y, v.s1.z);
+}
+__device__ __forceinline__ PatchView<float> vrow_view(const float* row, int k) {
+    const float4* p = (const float4*)(row + 12 * k);
+    const float4 a = p[0], b = p[1], c = p[2];
+    PatchView<float> v;
+    v.ax = mk<float>(a.x, a.y, a.z);
+    v.pd = mk<float>(a.w, b.x, b.y);
+    v.s0 = mk<float>(b.z, b.w, c.x);
+    v.s1 = mk<float>(c.y, c.z, c.w);
+    return v;
+}
+// part k (patch k; the axis with k = 0) of a particle's row from its record;
+// the values are derive's
+__device__ __forceinline__ void vrow_derive(float* row, int k, const float4 o, const float2 q, int t,
+                                            const TP32* __restrict__ tp) {
+    vrow_put(row, k, load_view<float>(o, q, t, tp, k));
+    if (k == 0) {
+        const int g = tp[t].geotype;
+        V3<float> d = mk<float>(o.x, o.y, o.z);
+        if (!(g >= 30 || g == G_SCA || g == G_SCN)) d = normalised(d);
+        *(float4*)(row + VROW_DIR) = make_float4(d.x, d.y, d.z, 0.0f);
+    }
+}
+__device__ __forceinline__ V3<float> vrow_dir(const float* row) {
+    const float4 a = *(const float4*)(row + VROW_DIR);
+    return mk<float>(a.x, a.y, a.z);
+}
+// the vectors of a row that a spherocylinder-sphere pair reads
+__device__ __forceinline__ DPart<float> vrow_part(const float* row, int t, int g) {
+    const PatchView<float> a = vrow_view(row, 0), b = vrow_view(row, 1);
+    DPart<float> p;
+    p.dir = vrow_dir(row);
+    p.pd[0] = a.pd; p.pd[1] = b.pd;
+    p.sd[0] = a.s0; p.sd[1] = a.s1; p.sd[2] = b.s0; p.sd[3] = b.s1;
+    p.ax[0] = a.ax; p.ax[1] = b.ax;
+    p.t = t;
+    p.g = g;
+    return p;
+}
+// The rows of the staged particles lo <= j < hi: all of them, the home
+// cell's, or none.  All when they fit beside the stage: then a trial derives
+// nothing but the new state of a rotation, and a patch item is loads.
+struct Rows {
+    float* v;
+    int lo, hi;
+    __device__ __forceinline__ bool has(int j) const { return j >= lo && j < hi; }
+    __device__ __forceinline__ float* row(int j) const { return v + (size_t)(j - lo) * VROW; }
 };
 
 // Squared distance of the point -r (r = segment's centre - point) from the
@@ -1790,6 +1851,28 @@ __device__ __forceinline__ float centre_dist2(const V3<float>& d, float h, const
     t = fminf(fmaxf(t, -h), h);
     V3<float> v = mk<float>(r.x + t * d.x, r.y + t * d.y, r.z + t * d.z);
     return dot(v, v);
+}
+
+// patch_side from the patch rows of part1 and part2 (side 0: particle 2's
+// axis against particle 1's patch region, side 1 the reverse)
+__device__ __forceinline__ bool row_side(const PP32& P, const float* r1, const float* r2, const V3<float>& r, int k1,
+                                         int k2, int side, float& x1, float& x2) {
+    const bool s1 = side != 0;
+    const PatchView<float> a = vrow_view(s1 ? r2 : r1, 0);
+    const float* l = s1 ? r1 : r2;
+    IQ<float> q;
+    q.rcSq = P.rcutSq;
+    q.p1 = a.ax;
+    q.p2 = mk<float>(l[0], l[1], l[2]);
+    q.pdir = a.pd;
+    q.s0 = a.s0;
+    q.s1 = a.s1;
+    q.r = s1 ? mk<float>(r.x * -1.0f, r.y * -1.0f, r.z * -1.0f) : r;
+    q.cossw = P.pcanglsw[s1 ? (k2 ? 3 : 1) : (k1 ? 2 : 0)];
+    q.h1 = s1 ? P.hl1 : P.hl0;
+    q.h2 = s1 ? P.hl0 : P.hl1;
+    const bool c = (P.kind == K_CPSC) || (P.kind == K_MIXED && is_psc(P.g0) == s1);
+    return intersect(q, c, x1, x2);
 }
 
 // One trial of the speculative sweep, on one wave: the energies of the moving
@@ -1812,35 +1895,30 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                                            const PP32* __restrict__ pp, const TP32* __restrict__ tp, int ppmax,
                                            const SpecScratch& T, const float* ml,
                                            const unsigned char* __restrict__ mlp_img, const MlpConst& mc,
-                                           const ChainTab& ct, double thr1, double thr2, const float* hvk,
-                                           bool translate, double& eo, double& en, double& des, int& stage) {
+                                           const ChainTab& ct, double thr1, double thr2, const Rows& rows,
+                                           const int16_t* partner, bool translate, double& eo, double& en,
+                                           double& des, int& stage) {
     const int lane = lane_id(), t = uo.w, idk = S.id[k];
     const int cwk = ct.cw ? ct.cw[idk] : 0, bmask = cwk & 15;
-    // derived vectors of both states: the old state's from the home cell's
-    // cache when there is one, a translation keeps them
-    const float* mvo = hvk;
-    const float* mvn = T.mv + MV_STRIDE;
-    V3<float> dold;
-    if (hvk) {
-        dold = mv_vec(hvk, 0);
-    } else {
-        DPart<float> po = load_part<float>(oo, qo, t, tp);
-        if (lane == 0) mv_store(T.mv, po);
-        dold = po.dir;
-        mvo = T.mv;
+    if (bmask) {   // partner: the staged chain partners of particle k (-1: not staged)
+        int found = 0;
+        for (int q = 0; q < 4; q++) found |= (partner[q] >= 0 ? 1 : 0) << q;
+        if ((found & bmask) != bmask) {
+            stage = -1;
+            return false;
+        }
     }
-    V3<float> dnew = dold;
-    if (translate) {
-        mvn = mvo;
-    } else {
-        DPart<float> pn = load_part<float>(on, qn, t, tp);
-        if (lane == 0) mv_store(T.mv + MV_STRIDE, pn);
-        dnew = pn.dir;
-    }
-    if (bmask) {
-        if (lane < 4) T.bp[lane] = -1;
-        wave_lds_sync();
-    }
+    // rows of both states: the old state's may be there, a translation keeps it
+    const float* mvo = T.mv;
+    const float* mvn = T.mv + VROW;
+    const int npatch = ppmax > 1 ? 2 : 1;
+    const bool had = rows.has(k);
+    if (had) mvo = rows.row(k);
+    else if (lane < npatch) vrow_derive(T.mv, lane, oo, qo, t, tp);
+    if (translate) mvn = mvo;
+    else if (lane < npatch) vrow_derive(T.mv + VROW, lane, on, qn, t, tp);
+    wave_lds_sync();
+    const V3<float> dold = vrow_dir(mvo), dnew = vrow_dir(mvn);
     // phase A, four staged particles per lane per round
     constexpr int PA = 4;
     const float hm = tp[t].hl, reach2 = tp[t].reach2;
@@ -1858,10 +1936,6 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                 if (translate) rn = fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
                 fo = centre_dist2(dold, hm, ro) <= reach2;
                 fn = centre_dist2(dnew, hm, rn) <= reach2;
-                if (bmask) {
-                    int bit = cw_bit(S.id[j] - idk);
-                    if (bit >= 0 && ((bmask >> bit) & 1)) T.bp[bit] = j;
-                }
             }
             const unsigned long long mo = __ballot(fo), mn = __ballot(fn);
             if (fo) {
@@ -1883,23 +1957,19 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     }
     double ao = 0.0, an = 0.0;
     if (bmask) {
-        int found = 0;
-        for (int q = 0; q < 4; q++) found |= (T.bp[q] >= 0 ? 1 : 0) << q;
-        if (found != bmask) {
-            stage = -1;
-            return false;
-        }
         // lanes 0-3: the old state with partners 0-3, lanes 4-7 the new one
         int q = lane & 3, which = (lane >> 2) & 1;
         if (lane < 8 && ((bmask >> q) & 1)) {
-            int j = T.bp[q];
+            int j = partner[q];
             uint4 b = S.u[j];
             float4 ob = S.o[j];
             float2 qb = S.q[j];
             const float* mv = which ? mvn : mvo;
+            const V3<float> d = vrow_dir(mv);
             double eb = bond_energy(ct.mol[cwk >> 8], ct.pp64[t * sc.nt + b.w], cw_rel(q),
-                                    fx_r12(which ? un : uo, b, sc.Ld), unit64(mv[0], mv[1], mv[2]),
-                                    unit64(mv[3], mv[4], mv[5]), unit64(ob.x, ob.y, ob.z), unit64(ob.w, qb.x, qb.y));
+                                    fx_r12(which ? un : uo, b, sc.Ld), unit64(d.x, d.y, d.z),
+                                    unit64(mv[VROW_PD0], mv[VROW_PD0 + 1], mv[VROW_PD0 + 2]),
+                                    unit64(ob.x, ob.y, ob.z), unit64(ob.w, qb.x, qb.y));
             if (which) an += eb; else ao += eb;
         }
     }
@@ -1925,7 +1995,10 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                 if (sw) r = mk<float>(-r.x, -r.y, -r.z);
                 float ev = 0.0f;
                 if (P2.kind <= K_SCA && P2.kind >= 0) {
-                    V3<float> dm = which ? dnew : dold, db = normalised(mk<float>(S.o[jj].x, S.o[jj].y, S.o[jj].z));
+                    V3<float> dm = which ? dnew : dold, db;
+                    if (rows.has(jj)) db = vrow_dir(rows.row(jj));
+                    else db = mk<float>(S.o[jj].x, S.o[jj].y, S.o[jj].z);
+                    if (P2.kind >= K_SCN || !rows.has(jj)) db = normalised(db);
                     DPart<float> pa, pb;
                     pa.dir = sw ? db : dm;
                     pb.dir = sw ? dm : db;
@@ -1969,7 +2042,7 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                     const int e = t0 + (lane & (MLP_TILE - 1)), xw = e < nx ? T.xl[e] : 0, which = xw >> 15;
                     const float* mv = which ? mvn : mvo;
                     bool net = pair_features(S, e < nx, xw & 0x7fff, e < nx ? T.xd[e] : 0.0f, t, which ? un : uo,
-                                             mv_vec(mv, 0), mv_vec(mv, 3), sc, mc, f);
+                                             vrow_dir(mv), mv_vec(mv, VROW_PD0), sc, mc, f);
                     float out = mlp_tile_g(mlp_img, ml, mlp_slots(f, lane >> 4), lane);
                     if (lane < MLP_TILE && net) {
                         if (which) sn += (double)out; else so += (double)out;
@@ -1986,48 +2059,61 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     // phase C: (entry, patch pair, side) items, the two wedge intersections of
     // a patch pair on neighbouring lanes; where they take more than one pass,
     // each lane takes both sides of its patch pair, one after the other (half
-    // the passes, and the view, set-up and attraction once per patch pair; the
-    // same values: each side is the same patch_side call)
-    const int items = nx * ppmax * 2;
-    const bool dual = items > WAVE;
-    const int nit = dual ? items / 2 : items;
-    for (int base = 0; base < nit; base += WAVE) {
-        int it = dual ? 2 * (base + lane) : base + lane, which = 0, k1 = 0, k2 = 0, side = it & 1;
-        bool hit = false, hit2 = false, pair_item = false;
+    // the passes, and the set-up and attraction once per patch pair; the same
+    // values: each side is the same intersect call).  An item's vectors come
+    // from the rows of the mover and of its neighbour: each side picks which
+    // of the two is the region and which the line by pointer.
+    const bool all_rows = rows.hi - rows.lo == S.n;
+    const int psh = ppmax > 2 ? 2 : (ppmax > 1 ? 1 : 0);   // log2 of the patch pairs per entry (1, 2 or 4)
+    const bool dual = all_rows && (nx << (psh + 1)) > WAVE;
+    const int ish = dual ? psh : psh + 1;                  // log2 of the lanes per entry
+    const int eb = all_rows ? WAVE >> ish : min(SPEC_NV, WAVE >> ish);
+    for (int e0 = 0; e0 < nx; e0 += eb) {
+        if (!all_rows) {   // the batch's neighbours' rows
+            wave_lds_sync();
+            const int e = e0 + lane / npatch;
+            if (lane < eb * npatch && e < nx) {
+                const int jj = T.xl[e] & 0x7fff;
+                vrow_derive(T.nv + (e - e0) * VROW, lane % npatch, S.o[jj], S.q[jj], S.u[jj].w, tp);
+            }
+            wave_lds_sync();
+        }
+        const int e = e0 + (lane >> ish), side = dual ? 0 : lane & 1;
+        const int mpp = (dual ? lane : lane >> 1) & ((1 << psh) - 1);
+        int which = 0, k1 = 0, k2 = 0;
+        bool hit = false, hit2 = false, sw = false;
         float x1 = 0.0f, x2 = 0.0f, ev = 0.0f, z1 = 0.0f, z2 = 0.0f;
         const PP32* P2 = pp;
+        const float *r1 = mvo, *r2 = mvo;   // rows of part1 and part2
         V3<float> r = mk<float>(0.0f, 0.0f, 0.0f);
-        PatchView<float> va, vb;
-        if (it < items) {
-            int e = it / (2 * ppmax), mpp = (it - e * 2 * ppmax) >> 1;
-            int w = T.xl[e];
-            int jj = w & 0x7fff;
+        if ((lane >> ish) < eb && e < nx) {
+            const int w = T.xl[e], jj = w & 0x7fff;
             which = w >> 15;
-            uint4 b = S.u[jj];
-            const bool sw = S.id[jj] > idk;   // canonical order, as in phase B
-            P2 = sw ? pp + b.w * sc.nt + t : pp + t * sc.nt + b.w;
-            r = which ? fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll)
-                      : fx_image_c(uo.x, uo.y, uo.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+            const uint4 bu = S.u[jj];
+            sw = S.id[jj] > idk;   // canonical order, as in phase B
+            P2 = sw ? pp + bu.w * sc.nt + t : pp + t * sc.nt + bu.w;
+            r = which ? fx_image_c(un.x, un.y, un.z, bu.x, bu.y, bu.z, sc.Lh, sc.Ll)
+                      : fx_image_c(uo.x, uo.y, uo.z, bu.x, bu.y, bu.z, sc.Lh, sc.Ll);
             if (sw) r = mk<float>(-r.x, -r.y, -r.z);
             const float* mv = which ? mvn : mvo;
+            const float* nv = all_rows ? rows.row(jj) : T.nv + (e - e0) * VROW;
+            r1 = sw ? nv : mv;
+            r2 = sw ? mv : nv;
             if (P2->kind <= K_SCA) {
                 if (mpp < npatch_pairs(*P2)) {
                     patch_pair_index(*P2, mpp, k1, k2);   // patches of part1 and part2
-                    PatchView<float> vm = mv_view(mv, sw ? k2 : k1),
-                                     vn = load_view<float>(S.o[jj], S.q[jj], b.w, tp, sw ? k1 : k2);
-                    va = sw ? vn : vm;
-                    vb = sw ? vm : vn;
-                    hit = patch_side<float>(*P2, va, vb, r, k1, k2, side, x1, x2);
-                    if (dual) hit2 = patch_side<float>(*P2, va, vb, r, k1, k2, 1, z1, z2);
-                    pair_item = true;
+                    r1 += 12 * k1;
+                    r2 += 12 * k2;
+                    hit = row_side(*P2, r1, r2, r, k1, k2, side, x1, x2);
+                    if (dual) hit2 = row_side(*P2, r1, r2, r, k1, k2, 1, z1, z2);
                 }
             } else if (mpp == 0 && side == 0) {
-                DPart<float> pb = load_part<float>(S.o[jj], S.q[jj], b.w, tp);
-                DPart<float> pm = mv_part(mv, t, tp[t].geotype);
+                DPart<float> pb = load_part<float>(S.o[jj], S.q[jj], bu.w, tp);
+                DPart<float> pm = vrow_part(mv, t, tp[t].geotype);
                 ev = sw ? spsc(*P2, pb, pm, r) : spsc(*P2, pm, pb, r);
             }
         }
-        // the other side's result (lane ^ 1 holds item it ^ 1)
+        // the other side's result (lane ^ 1 holds the entry's other side)
         float y1 = z1, y2 = z2;
         int oh = hit2 ? 1 : 0;
         if (!dual) {
@@ -2035,7 +2121,8 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             y2 = __shfl_xor(x2, 1);
             oh = __shfl_xor(hit ? 1 : 0, 1);
         }
-        if (pair_item && side == 0 && hit && oh) ev = patch_atr<float>(*P2, va, vb, r, k1, k2, x1, x2, y1, y2);
+        if (side == 0 && hit && oh)
+            ev = patch_atr<float>(*P2, vrow_view(r1, 0), vrow_view(r2, 0), r, k1, k2, x1, x2, y1, y2);
         if (which) an += (double)ev; else ao += (double)ev;
     }
     eo = wave_sum_dpp(ao);
@@ -2055,7 +2142,8 @@ template <int NW>
 __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes, int cap, const Grid& g,
                             const SysConst& sc, int cx, int cy, int cz, const int* __restrict__ starts,
                             const uint4* __restrict__ P, const float4* __restrict__ O, const float2* __restrict__ Q,
-                            const int* __restrict__ ID, const ChainTab& ct, int* sten, int* misc) {
+                            const int* __restrict__ ID, const ChainTab& ct, int* sten, int* misc, int16_t*& partner,
+                            size_t& used) {
     const int ns = stencil_size(g);
     int* pre = sten;          // ns+1 prefix of counts
     int* cst = sten + ns + 1; // cell start per stencil entry
@@ -2140,12 +2228,28 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
     S.o = (float4*)(S.u + n4);
     S.q = (float2*)(S.o + n4);
     S.id = (int*)(S.q + n4);
+    used = (size_t)n4 * 44;
+    partner = (int16_t*)(region + used);
+    if (ct.cw) {   // the home cell's chain partners: four staged indices per particle
+        used += ((size_t)(hend - hbeg) * 8 + 15) & ~(size_t)15;
+        if (used > region_bytes - 4 * (size_t)cap) return false;   // (not over the list)
+        for (int i = tid; i < 4 * (hend - hbeg); i += WAVE * NW) partner[i] = -1;
+        __syncthreads();
+    }
     for (int i = tid; i < n; i += WAVE * NW) {
-        const int src = list[i];
+        const int src = list[i], id = ID[src];
         S.u[i] = P[src];
         S.o[i] = O[src];
         S.q[i] = Q[src];
-        S.id[i] = ID[src];
+        S.id[i] = id;
+        if (ct.cw) {
+            const int w = ct.cw[id];
+            for (int q = 0; q < 4; q++)   // this particle is partner q ^ 1 (the opposite step) of its partner q
+                if ((w >> q) & 1) {
+                    const int sl = ct.slot[id + cw_rel(q)];
+                    if (sl >= gs && sl < ge) partner[4 * (sl - gs) + (q ^ 1)] = (int16_t)i;
+                }
+        }
     }
     __syncthreads();
     return true;
@@ -2181,12 +2285,11 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     T.xl = (uint16_t*)(wb + L.xl);
     T.xd = (float*)(wb + L.xd);
     T.mv = (float*)(wb + L.mv);
-    T.bp = (int*)(wb + L.bp);
+    T.nv = (float*)T.nl;
     int* sten = (int*)(smem + L.sten);
     int* misc = (int*)(smem + L.misc);
     SpecRes* res = (SpecRes*)(smem + L.res);
     TrialRec* recs = (TrialRec*)(smem + L.recs);
-    float* hv = (float*)(smem + L.hv);
     float* ml = nullptr;   // the network's constants (its operands stay in global memory)
     if constexpr (NET) {
         ml = (float*)(smem + L.ml);
@@ -2201,7 +2304,10 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         pp = ppl;
         tp = tpl;
     }
-    if (!stage_reach<SPEC_W>(S, smem, L.wbase, cap, g, sc, cx, cy, cz, starts, P, O, Q, ID, ct, sten, misc)) {
+    int16_t* partners;
+    size_t used;
+    if (!stage_reach<SPEC_W>(S, smem, L.wbase, cap, g, sc, cx, cy, cz, starts, P, O, Q, ID, ct, sten, misc, partners,
+                             used)) {
         if (tid == 0) atomicOr(flag, 1);
         return;
     }
@@ -2218,10 +2324,25 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         int fl = (int)floorf(mean);
         ntrial = fl + ((u01f(rd.x) < mean - (float)fl) ? 1 : 0);
     }
-    const bool hcache = nh <= min(HCAP, mp.hcap);
-    if (hcache)
-        for (int i = tid; i < nh; i += WAVE * SPEC_W)
-            mv_store(hv + i * MV_STRIDE, load_part<float>(S.o[S.h0 + i], S.q[S.h0 + i], S.u[S.h0 + i].w, tp));
+    // rows of all staged particles, else of the home cell's, where they fit
+    Rows rows;
+    rows.v = (float*)(smem + used);
+    rows.lo = rows.hi = 0;
+    const int fit = (int)((L.wbase - used) / (4 * VROW));
+    if (mp.hcap > 0 && (mp.hcap >= HCAP || nh <= mp.hcap)) {
+        if (S.n <= fit) {
+            rows.hi = S.n;
+        } else if (nh <= fit) {
+            rows.lo = S.h0;
+            rows.hi = S.h1;
+        }
+        const int np = ppmax > 1 ? 2 : 1;
+        for (int i = tid; i < np * (rows.hi - rows.lo); i += WAVE * SPEC_W) {
+            const int j = rows.lo + i / np;
+            vrow_derive(rows.row(j), i % np, S.o[j], S.q[j], S.u[j].w, tp);
+        }
+        __syncthreads();   // (over the stage's source list)
+    }
     // wave 0 keeps the counters of the kept trials (the same on all its lanes)
     unsigned n_tacc = 0, n_ttry = 0, n_racc = 0, n_rtry = 0, n_left = 0, n_s1try = 0, n_s1acc = 0, n_s2try = 0,
              n_s2acc = 0, n_bond = 0;
@@ -2265,9 +2386,9 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
                 status = 1;
             } else {
                 double eo, en, des;
-                const float* hvk = hcache ? hv + (k - S.h0) * MV_STRIDE : nullptr;
                 bool pass = spec_trial<DA>(S, k, uo, un, oo, qo, on, qn, sc, pp, tp, ppmax, T, ml, mlp_img, mc, ct,
-                                           R.thr1, R.thr2, hvk, translate, eo, en, des, stage);
+                                           R.thr1, R.thr2, rows, partners + 4 * (k - S.h0), translate, eo, en, des,
+                                           stage);
                 if (stage == -1) {
                     status = 2;
                 } else if (stage == -2) {
@@ -2344,9 +2465,9 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         }
         __syncthreads();
         const int nfin = misc[0];
-        if (hcache && w < nfin && lane < 27) {   // the derived vectors of a kept, accepted rotation
+        if (w < nfin && lane < VROW) {   // the row of a kept, accepted rotation
             const SpecRes& a = res[w];
-            if (a.acc && !a.translate) hv[(a.k - S.h0) * MV_STRIDE + lane] = T.mv[MV_STRIDE + lane];
+            if (a.acc && !a.translate && rows.has(a.k)) rows.row(a.k)[lane] = T.mv[VROW + lane];
         }
         if (misc[1]) {   // a trial's near list overflowed: stop the cell, report
             if (tid == 0) atomicOr(flag, 16);
