@@ -19,6 +19,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 // Per-expression FMA contraction for the whole file (the pair header's
@@ -1669,23 +1670,28 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_pass(Grid g, SysConst sc
 #define VROW_PD0 3
 #define SPEC_NV 8       // neighbours whose rows a wave derives at once when the stage has none
 
-struct __align__(16) SpecRes {
-    uint4 uo, un;    // position at the round's start and proposed
+// a trial's proposal, for the block's other waves and for its commit
+struct __align__(16) SpecProp {
+    uint4 un;        // proposed position
     float4 on;       // proposed orientation record
     float2 qn;
-    int k, id;       // staged index, particle ID
-    double de;       // E_new - E_old (kept trials that reached the final stage)
-    int status;      // 0 evaluated, 1 left the cell, 2 chain partner outside the stencil, 3 a list full
-    int translate, acc, stage;
-    int dep;         // bit i: the trial depends on the round's trial i, should that one be accepted
+    int k;           // staged index of the particle
+    int pad;
 };
+// a trial's outcome, one word: bit 0 accepted, 1 translation, 2-3 status (0
+// evaluated, 1 left the cell, 2 chain partner outside the stencil, 3 a list
+// full), 4-5 the delayed acceptance's stage, 8-11 bit i: depends on the
+// round's trial i, should that one be accepted
+__device__ __forceinline__ int spec_word(bool acc, bool translate, int status, int stage, int dep) {
+    return (acc ? 1 : 0) | (translate ? 2 : 0) | (status << 2) | ((stage & 3) << 4) | (dep << 8);
+}
 
 // LDS of the speculative sweep: the stage, then SPEC_W per-wave trial
 // scratch blocks, then what the waves share (byte offsets; per-wave fields
 // relative to the wave's block).
 struct SpecLayout {
     size_t nl, xl, xd, mv, wstride;
-    size_t wbase, sten, misc, res, recs, ml, tab, end;
+    size_t wbase, sten, misc, prop, res, recs, ml, tab, end;
 };
 __host__ __device__ inline size_t spec_align(size_t x, size_t a) { return (x + a - 1) / a * a; }
 __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_bytes) {
@@ -1702,8 +1708,9 @@ __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_
     o += 4 * (2 * 125 + 2);
     L.misc = spec_align(o, 16);
     o = L.misc + 4 * 16;
-    L.res = spec_align(o, 16);
-    o = L.res + SPEC_W * sizeof(SpecRes);
+    L.prop = spec_align(o, 16);
+    L.res = L.prop + SPEC_W * sizeof(SpecProp);
+    o = L.res + SPEC_W * sizeof(int);
     L.recs = spec_align(o, 16);
     o = L.recs + TRIAL_CHUNK * sizeof(TrialRec);
     L.ml = spec_align(o, 16);
@@ -1711,71 +1718,6 @@ __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_
     L.tab = spec_align(o, 16);
     L.end = L.tab + tab_bytes;
     return L;
-}
-
-// Can the pair of particles 1 (position u1, orientation record o1, ID id1)
-// and 2 have a non-zero pair term?  The canonical evaluation's own FP32 tests
-// (higher ID as part1): no beyond sqmaxcut (phase A), none for a type pair
-// without a functor, and for spherocylinder pairs none when the segment
-// distance is beyond both the attraction's and the repulsion's range (phase
-// B's scsc_cheap; a relative margin of 1e-5 covers the K_SCA term's
-// square-root test).  Sphere pairs: any pair inside sqmaxcut.
-__device__ __forceinline__ bool pair_active(uint4 u1, float4 o1, int id1, uint4 u2, float4 o2, int id2,
-                                            const SysConst& sc, const PP32* __restrict__ pp) {
-    if (id1 < id2) {
-        uint4 tu = u1; u1 = u2; u2 = tu;
-        float4 to = o1; o1 = o2; o2 = to;
-    }
-    V3<float> r = fx_image_c(u1.x, u1.y, u1.z, u2.x, u2.y, u2.z, sc.Lh, sc.Ll);
-    if (dot(r, r) > sc.sqmaxcut) return false;
-    const PP32& P = pp[u1.w * sc.nt + u2.w];
-    if (P.kind == K_NONE) return false;
-    if (P.kind > K_SCA || P.kind < 0) return true;
-    V3<float> dv = min_dist(normalised(mk<float>(o1.x, o1.y, o1.z)), normalised(mk<float>(o2.x, o2.y, o2.z)), P.hl0,
-                            P.hl1, r);
-    float d2 = dot(dv, dv);
-    return d2 <= fmaxf(P.rcutSq, P.rcutwcaSq) * 1.00001f;
-}
-
-// Every trial's dependences of a round, on one wave (wave 0, whose own trial
-// has none, so the other waves start their trials at once).  Bit i of
-// deps[q]: trial q and the round's earlier trial i would see each other's
-// move: the same particle, chain
-// partners (bond and angle terms reach beyond maxcut), or a pair that can
-// interact in any of their old/new states; the relation is symmetric.  Lanes
-// 4p .. 4p+3 take the p-th pair (q, i) of (1,0) (2,0) (2,1) (3,0) (3,1)
-// (3,2) and its four state combinations.
-__device__ __forceinline__ void spec_deps_all(const TrialRec* recs, int t, int W, const Stage& S, const SysConst& sc,
-                                              const PP32* __restrict__ pp, bool bonded, int* deps) {
-    static_assert(SPEC_W <= 4, "six trial pairs on 24 lanes");
-    const int lane = lane_id(), p = lane >> 2, c = lane & 3;
-    const int q = p < 1 ? 1 : (p < 3 ? 2 : 3), i = p - (q * (q - 1)) / 2;
-    bool d = false;
-    if (p < 6 && q < W) {
-        const TrialRec& Rq = recs[(t + q) & (TRIAL_CHUNK - 1)];
-        const TrialRec& Ra = recs[(t + i) & (TRIAL_CHUNK - 1)];
-        const int k = Rq.k, ka = Ra.k;
-        if (ka == k || (bonded && abs(S.id[ka] - S.id[k]) <= 2)) {
-            d = true;
-        } else {
-            uint4 uo = S.u[k], un, uoa = S.u[ka], una;
-            float4 oo = S.o[k], on, ooa = S.o[ka], ona;
-            float2 qo = S.q[k], qn, qoa = S.q[ka], qna;
-            propose(Rq, uo, oo, qo, un, on, qn);
-            propose(Ra, uoa, ooa, qoa, una, ona, qna);
-            d = pair_active((c & 1) ? una : uoa, (c & 1) ? ona : ooa, S.id[ka], (c & 2) ? un : uo, (c & 2) ? on : oo,
-                            S.id[k], sc, pp);
-        }
-    }
-    const unsigned long long m = __ballot(d);
-#pragma unroll
-    for (int qq = 1; qq < SPEC_W; qq++) {
-        int dep = 0;
-#pragma unroll
-        for (int ii = 0; ii < qq; ii++)
-            if ((m >> (4 * ((qq * (qq - 1)) / 2 + ii))) & 15ull) dep |= 1 << ii;
-        deps[qq] = dep;
-    }
 }
 
 // What the wave that evaluates a speculative trial keeps in LDS.
@@ -1885,7 +1827,8 @@ __device__ __forceinline__ bool row_side(const PP32& P, const float* r1, const f
 //      range)^2) let three times as many through, 62 of 432 staged for
 //      TCHPSC at packing fraction 0.25 against ~20, so that the next phase
 //      took two passes of the wave instead of one.
-//   B  segment distance and repulsion of each (candidate, state)
+//   B  segment distance and repulsion of each (candidate, state); on the lanes
+//      behind them the trial's dependences on the round's earlier trials
 //   C  patch terms of the entries in range
 // stage -2: a list is full (more than SPEC_LCAP candidates of a state or
 // SPEC_XCAP entries), the trial cannot be evaluated here.
@@ -1896,8 +1839,8 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                                            const SpecScratch& T, const float* ml,
                                            const unsigned char* __restrict__ mlp_img, const MlpConst& mc,
                                            const ChainTab& ct, double thr1, double thr2, const Rows& rows,
-                                           const int16_t* partner, bool translate, double& eo, double& en,
-                                           double& des, int& stage) {
+                                           const int16_t* partner, bool translate, const SpecProp* prop, int w,
+                                           double& eo, double& en, double& des, int& stage, int& dep) {
     const int lane = lane_id(), t = uo.w, idk = S.id[k];
     const int cwk = ct.cw ? ct.cw[idk] : 0, bmask = cwk & 15;
     if (bmask) {   // partner: the staged chain partners of particle k (-1: not staged)
@@ -1919,36 +1862,41 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     else if (lane < npatch) vrow_derive(T.mv + VROW, lane, on, qn, t, tp);
     wave_lds_sync();
     const V3<float> dold = vrow_dir(mvo), dnew = vrow_dir(mvn);
-    // phase A, four staged particles per lane per round
-    constexpr int PA = 4;
+    // phase A: the loads of a round's PA staged particles per lane first, then
+    // the tests without branches (a load under a condition waits by itself)
     const float hm = tp[t].hl, reach2 = tp[t].reach2;
     uint16_t* const nl_new = T.nl + SPEC_LCAP;
     int no = 0, nn = 0;
-    for (int base = 0; base < S.n; base += PA * WAVE) {
+    auto scan = [&](int base, auto pa) {
+        constexpr int PA = decltype(pa)::value;
+        uint4 b[PA];
+#pragma unroll
+        for (int h = 0; h < PA; h++) b[h] = S.u[min(base + h * WAVE + lane, S.n - 1)];
+        bool fo[PA], fn[PA];
 #pragma unroll
         for (int h = 0; h < PA; h++) {
             const int j = base + h * WAVE + lane;
-            bool fo = false, fn = false;
-            if (j < S.n && j != k) {
-                uint4 b = S.u[j];
-                V3<float> ro = fx_image_c(uo.x, uo.y, uo.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
-                V3<float> rn = ro;
-                if (translate) rn = fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
-                fo = centre_dist2(dold, hm, ro) <= reach2;
-                fn = centre_dist2(dnew, hm, rn) <= reach2;
-            }
-            const unsigned long long mo = __ballot(fo), mn = __ballot(fn);
-            if (fo) {
-                int pos = no + wave_prefix(mo);
-                if (pos < SPEC_LCAP) T.nl[pos] = (uint16_t)j;
-            }
-            if (fn) {
-                int pos = nn + wave_prefix(mn);
-                if (pos < SPEC_LCAP) nl_new[pos] = (uint16_t)j;
-            }
+            const bool in = j < S.n && j != k;
+            const V3<float> ro = fx_image_c(uo.x, uo.y, uo.z, b[h].x, b[h].y, b[h].z, sc.Lh, sc.Ll);
+            V3<float> rn = ro;
+            if (translate) rn = fx_image_c(un.x, un.y, un.z, b[h].x, b[h].y, b[h].z, sc.Lh, sc.Ll);
+            fo[h] = in & (centre_dist2(dold, hm, ro) <= reach2);
+            fn[h] = in & (centre_dist2(dnew, hm, rn) <= reach2);
+        }
+#pragma unroll
+        for (int h = 0; h < PA; h++) {
+            const int j = base + h * WAVE + lane;
+            const unsigned long long mo = __ballot(fo[h]), mn = __ballot(fn[h]);
+            const int po = no + wave_prefix(mo), pn = nn + wave_prefix(mn);
+            if (fo[h] && po < SPEC_LCAP) T.nl[po] = (uint16_t)j;
+            if (fn[h] && pn < SPEC_LCAP) nl_new[pn] = (uint16_t)j;
             no += __popcll(mo);
             nn += __popcll(mn);
         }
+    };
+    for (int base = 0; base < S.n; base += 4 * WAVE) {
+        if (S.n - base <= 2 * WAVE) scan(base, std::integral_constant<int, 2>());
+        else scan(base, std::integral_constant<int, 4>());
     }
     wave_lds_sync();
     if (no > SPEC_LCAP || nn > SPEC_LCAP) {
@@ -1973,46 +1921,75 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             if (which) an += eb; else ao += eb;
         }
     }
-    // phase B
+    // phase B.  Items: the old state's candidates, the new state's, and 4 w for
+    // the dependences of this trial (the round's w-th) on each earlier one i:
+    // the pair of their particles in any of their old/new states.  Trial i's
+    // particle is then the neighbour, and the trials depend on each other when
+    // the pair can have a non-zero term, by the evaluation's own FP32 tests:
+    // inside sqmaxcut, a type pair with a functor, and for spherocylinders the
+    // segment distance within the attraction's or the repulsion's range (a
+    // relative margin of 1e-5 covers the K_SCA term's square-root test).  The
+    // same particle and chain partners (bond and angle terms reach beyond
+    // maxcut) always depend.
     int nx = 0;
-    for (int base = 0; base < no + nn; base += WAVE) {
-        const int it = base + lane, which = it >= no ? 1 : 0;
+    unsigned long long depm = 0;
+    const int nc = no + nn;
+    for (int base = 0; base < nc + 4 * w; base += WAVE) {
+        const int it = base + lane;
+        const bool cand = it < nc, isdep = !cand && it < nc + 4 * w;
+        const int x = it - nc;
+        const int which = cand ? (it >= no ? 1 : 0) : (x >> 1) & 1;
         int jj = 0;
-        bool need = false;
+        bool need = false, d = false;
         float dseg2 = 0.0f;
-        if (it < no + nn) {
-            jj = which ? nl_new[it - no] : T.nl[it];
+        if (cand || isdep) {
+            const SpecProp& pi = prop[cand ? 0 : x >> 2];
+            jj = cand ? (which ? nl_new[it - no] : T.nl[it]) : pi.k;
             uint4 b = S.u[jj];
+            const int idb = S.id[jj];
+            V3<float> db = rows.has(jj) ? vrow_dir(rows.row(jj)) : mk<float>(S.o[jj].x, S.o[jj].y, S.o[jj].z);
+            bool raw = !rows.has(jj);
+            if (isdep && (x & 1)) {   // trial i's new state
+                b = pi.un;
+                db = mk<float>(pi.on.x, pi.on.y, pi.on.z);
+                raw = true;
+            }
             V3<float> r = which ? fx_image_c(un.x, un.y, un.z, b.x, b.y, b.z, sc.Lh, sc.Ll)
                                 : fx_image_c(uo.x, uo.y, uo.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
             // the pair in its canonical order, the higher ID as part1 (the
             // order of allToAll): the pair term is then one function of the
             // pair's state whichever particle moves, and the accepted changes
             // add up to allToAll's differences term by term
-            const bool sw = S.id[jj] > idk;
+            const bool sw = idb > idk;
             const PP32& P2 = sw ? pp[b.w * sc.nt + t] : pp[t * sc.nt + b.w];
+            const int kind = P2.kind;
+            d = isdep && (idb == idk || (ct.cw && abs(idb - idk) <= 2));
             if (dot(r, r) <= sc.sqmaxcut) {
                 if (sw) r = mk<float>(-r.x, -r.y, -r.z);
                 float ev = 0.0f;
-                if (P2.kind <= K_SCA && P2.kind >= 0) {
-                    V3<float> dm = which ? dnew : dold, db;
-                    if (rows.has(jj)) db = vrow_dir(rows.row(jj));
-                    else db = mk<float>(S.o[jj].x, S.o[jj].y, S.o[jj].z);
-                    if (P2.kind >= K_SCN || !rows.has(jj)) db = normalised(db);
+                if (kind <= K_SCA && kind >= 0) {
+                    V3<float> dm = which ? dnew : dold;
+                    if (kind >= K_SCN && isdep) dm = normalised(dm);
+                    if (kind >= K_SCN || raw) db = normalised(db);
                     DPart<float> pa, pb;
                     pa.dir = sw ? db : dm;
                     pb.dir = sw ? dm : db;
                     need = scsc_cheap(P2, pa, pb, r, ev, dseg2);
-                } else if (P2.kind == K_SPH_WCA || P2.kind == K_SPH_TAYLOR) {
+                    d = d || dseg2 <= fmaxf(P2.rcutSq, P2.rcutwcaSq) * 1.00001f;
+                } else if (kind == K_SPH_WCA || kind == K_SPH_TAYLOR) {
                     ev = sphere_pair(P2, sqrtf(dot(r, r)));
-                } else if (P2.kind != K_NONE) {
+                    d = true;
+                } else if (kind != K_NONE) {
                     need = true;
+                    d = true;
                 }
-                if (which) an += (double)ev; else ao += (double)ev;
+                if (cand) {
+                    if (which) an += (double)ev; else ao += (double)ev;
+                }
             }
         }
-        const unsigned long long m = __ballot(need);
-        if (need) {
+        const unsigned long long m = __ballot(need && cand), md = __ballot(d && isdep);
+        if (need && cand) {
             int pos = nx + wave_prefix(m);
             if (pos < SPEC_XCAP) {
                 T.xl[pos] = (uint16_t)(jj | (which << 15));
@@ -2020,7 +1997,11 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             }
         }
         nx += __popcll(m);
+        const int x0 = nc - base;   // the lane of dependence item 0
+        if (md) depm |= x0 >= 0 ? md >> x0 : md << -x0;
     }
+    dep = 0;
+    for (int i = 0; i < SPEC_W - 1; i++) dep |= ((depm >> (4 * i)) & 15ull) ? 1 << i : 0;
     wave_lds_sync();
     if (nx > SPEC_XCAP) {
         stage = -2;
@@ -2288,7 +2269,8 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     T.nv = (float*)T.nl;
     int* sten = (int*)(smem + L.sten);
     int* misc = (int*)(smem + L.misc);
-    SpecRes* res = (SpecRes*)(smem + L.res);
+    SpecProp* prop = (SpecProp*)(smem + L.prop);
+    int* res = (int*)(smem + L.res);
     TrialRec* recs = (TrialRec*)(smem + L.recs);
     float* ml = nullptr;   // the network's constants (its operands stay in global memory)
     if constexpr (NET) {
@@ -2343,11 +2325,11 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         }
         __syncthreads();   // (over the stage's source list)
     }
-    // wave 0 keeps the counters of the kept trials (the same on all its lanes)
+    // the counters of the kept trials (every wave counts alike); a wave's own
+    // energy changes
     unsigned n_tacc = 0, n_ttry = 0, n_racc = 0, n_rtry = 0, n_left = 0, n_s1try = 0, n_s1acc = 0, n_s2try = 0,
              n_s2acc = 0, n_bond = 0;
     double dsum = 0.0;
-    const bool bonded = ct.cw != nullptr;
     int t = 0, drawn = 0;
     while (t < ntrial) {   // t is block-uniform (from LDS)
         if (t >= drawn) {
@@ -2358,39 +2340,38 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
             __syncthreads();
         }
         const int W = min(SPEC_W, min(ntrial - t, drawn - t));
+        const TrialRec& R = recs[(t + min(w, W - 1)) & (TRIAL_CHUNK - 1)];
+        const int k = R.k;
+        const bool translate = R.translate != 0;
+        const uint4 uo = S.u[k];
+        const float4 oo = S.o[k];
+        const float2 qo = S.q[k];
+        uint4 un;
+        float4 on;
+        float2 qn;
+        propose(R, uo, oo, qo, un, on, qn);
+        if (lane == 0) {
+            SpecProp& p = prop[w];
+            p.un = un;
+            p.on = on;
+            p.qn = qn;
+            p.k = k;
+        }
+        __syncthreads();
+        double de = 0.0;
         if (w < W) {
-            if (w == 0) {   // every trial's dependences, then its own trial
-                int deps[SPEC_W];
-                deps[0] = 0;
-                spec_deps_all(recs, t, W, S, sc, pp, bonded, deps);
-                if (lane == 0) {
-#pragma unroll
-                    for (int q = 0; q < SPEC_W; q++)
-                        if (q < W) res[q].dep = deps[q];
-                }
-            }
-            const TrialRec& R = recs[(t + w) & (TRIAL_CHUNK - 1)];
-            int k = R.k;
-            uint4 uo = S.u[k];
-            float4 oo = S.o[k];
-            float2 qo = S.q[k];
-            bool translate = R.translate != 0;
-            uint4 un;
-            float4 on;
-            float2 qn;
-            propose(R, uo, oo, qo, un, on, qn);
-            int status = 0, stage = 0;
+            int status = 0, stage = 0, dep = 0;
             bool acc = false;
-            double de = 0.0;
             if (translate && cell_of_u(g, un.x, un.y, un.z) != cell) {   // leaving the active cell: rejected
                 status = 1;
+                for (int i = 0; i < w; i++) dep |= prop[i].k == k ? 1 << i : 0;
             } else {
                 double eo, en, des;
                 bool pass = spec_trial<DA>(S, k, uo, un, oo, qo, on, qn, sc, pp, tp, ppmax, T, ml, mlp_img, mc, ct,
-                                           R.thr1, R.thr2, rows, partners + 4 * (k - S.h0), translate, eo, en, des,
-                                           stage);
+                                           R.thr1, R.thr2, rows, partners + 4 * (k - S.h0), translate, prop, w, eo, en,
+                                           des, stage, dep);
                 if (stage == -1) {
-                    status = 2;
+                    status = 2;   // whatever the others do: the partner's cell does not change in a pass
                 } else if (stage == -2) {
                     status = 3;
                 } else if (pass) {
@@ -2400,82 +2381,65 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
                     acc = de2 <= 0.0 || de2 < R.thr;
                 }
             }
-            if (lane == 0) {
-                SpecRes& r = res[w];
-                r.uo = uo;
-                r.un = un;
-                r.on = on;
-                r.qn = qn;
-                r.k = k;
-                r.id = S.id[k];
-                r.de = de;
-                r.status = status;
-                r.translate = translate ? 1 : 0;
-                r.acc = acc ? 1 : 0;
-                r.stage = stage;
-            }
+            if (lane == 0) res[w] = spec_word(acc, translate, status, max(stage, 0), dep);
         }
         __syncthreads();
-        if (w == 0) {
-            // wave 0 takes the round's results, a lane each, in trial order:
-            // kept are the trials before the first that depends on an earlier
-            // accepted one (or overflowed); the counters of the kept trials are
-            // ballot counts; each kept accepted trial commits its own particle
-            // (distinct particles: the same particle is a dependence)
-            const bool valid = lane < W;
-            const SpecRes& a = res[valid ? lane : 0];
-            const int st = valid ? a.status : 0, dep = valid ? a.dep : 0, stg = valid ? a.stage : 0;
-            const bool acc = valid && a.acc, tr = valid && a.translate;
-            const unsigned long long accm = __ballot(acc);
-            const bool depends = valid && (dep & (int)accm & ((1 << lane) - 1)) != 0;
-            const bool full = valid && st == 3;
-            const unsigned long long fullm = __ballot(full);
-            const unsigned long long stopm = __ballot(depends || full);
-            const int first = stopm ? __ffsll((long long)stopm) - 1 : W;
-            const bool kept = valid && lane < first;
-            const bool left = kept && tr && st == 1, bond = kept && !left && st == 2;
-            const bool ev = kept && !left && !bond;   // reached the acceptance decision
-            n_ttry += __popcll(__ballot(kept && tr));
-            n_rtry += __popcll(__ballot(kept && !tr));
-            n_left += __popcll(__ballot(left));
-            n_bond += __popcll(__ballot(bond));
-            if constexpr (DA != DA_OFF) {
-                n_s1try += __popcll(__ballot(ev));
-                n_s1acc += __popcll(__ballot(ev && stg >= 1));
-                if constexpr (DA == DA_NET) {
-                    n_s2try += __popcll(__ballot(ev && (stg == 1 || stg == 2)));   // 3: the network did not run
-                    n_s2acc += __popcll(__ballot(ev && stg == 2));
+        // every wave takes the round's results, in trial order: kept are the
+        // trials before the first that depends on an earlier accepted one (or
+        // overflowed); the wave of a kept accepted trial commits it (distinct
+        // particles: the same particle is a dependence)
+        const int4 rw4 = *(const int4*)res;
+        const int rw[SPEC_W] = {rw4.x, rw4.y, rw4.z, rw4.w};
+        int nfin = 0, accm = 0, full = 0;
+#pragma unroll
+        for (int q = 0; q < SPEC_W; q++) {
+            const int f = __builtin_amdgcn_readfirstlane(rw[q]);
+            const int st = (f >> 2) & 3, stg = (f >> 4) & 3, tr = (f >> 1) & 1, ac = f & 1;
+            if (q < W && nfin == q) {
+                if (st == 3) {
+                    full = 1;   // unless an earlier accepted trial is why
+                }
+                if (((f >> 8) & accm) != 0) full = 0;
+                else if (st != 3) {
+                    nfin = q + 1;
+                    n_ttry += tr;
+                    n_rtry += 1 - tr;
+                    if (st == 1) n_left++;
+                    else if (st == 2) n_bond++;
+                    else {   // reached the acceptance decision
+                        if constexpr (DA != DA_OFF) {
+                            n_s1try++;
+                            n_s1acc += stg >= 1 ? 1 : 0;
+                            if constexpr (DA == DA_NET) {
+                                n_s2try += stg == 1 || stg == 2 ? 1 : 0;   // 3: the network did not run
+                                n_s2acc += stg == 2 ? 1 : 0;
+                            }
+                        }
+                        n_tacc += ac & tr;
+                        n_racc += ac & (1 - tr);
+                        accm |= ac << q;
+                    }
                 }
             }
-            const bool com = ev && acc;
-            n_tacc += __popcll(__ballot(com && tr));
-            n_racc += __popcll(__ballot(com && !tr));
-            if (com) {
-                S.u[a.k] = a.un;
-                S.o[a.k] = a.on;
-                S.q[a.k] = a.qn;
-            }
-            const double dei = com ? a.de : 0.0;
-#pragma unroll
-            for (int q = 0; q < SPEC_W; q++) dsum += __shfl(dei, q, WAVE);   // in trial order
+        }
+        if ((accm >> w) & 1) {
+            dsum += de;
+            const SpecProp& p = prop[w];
             if (lane == 0) {
-                misc[0] = first;
-                misc[1] = (first < W && ((fullm >> first) & 1ull)) ? 1 : 0;
+                S.u[k] = p.un;
+                S.o[k] = p.on;
+                S.q[k] = p.qn;
             }
+            if (!translate && rows.has(k) && lane < VROW) rows.row(k)[lane] = T.mv[VROW + lane];
         }
-        __syncthreads();
-        const int nfin = misc[0];
-        if (w < nfin && lane < VROW) {   // the row of a kept, accepted rotation
-            const SpecRes& a = res[w];
-            if (a.acc && !a.translate && rows.has(a.k)) rows.row(a.k)[lane] = T.mv[VROW + lane];
-        }
-        if (misc[1]) {   // a trial's near list overflowed: stop the cell, report
+        if (full) {   // a trial's list overflowed: stop the cell, report
             if (tid == 0) atomicOr(flag, 16);
             break;
         }
         t += nfin;
         __syncthreads();
     }
+    if (lane == 0) ((double*)sten)[w] = dsum;
     __syncthreads();
     // write the home cell back (same slots it was staged from)
     int gs = starts[cell];
@@ -2489,7 +2453,8 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         const unsigned v[10] = {n_tacc, n_ttry, n_racc, n_rtry, n_left, n_s1acc, n_s1try, n_s2acc, n_s2try, n_bond};
         for (int q = 0; q < 10; q++)
             if (v[q]) atomicAdd(&stats[rep * STAT_STRIDE + q], (unsigned long long)v[q]);
-        atomicAdd(&de_sum[rep * STAT_STRIDE], dsum);
+        const double* ds = (const double*)sten;
+        atomicAdd(&de_sum[rep * STAT_STRIDE], (ds[0] + ds[1]) + (ds[2] + ds[3]));
     }
 }
 
