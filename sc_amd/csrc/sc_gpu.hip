@@ -1795,26 +1795,143 @@ __device__ __forceinline__ float centre_dist2(const V3<float>& d, float h, const
     return dot(v, v);
 }
 
-// patch_side from the patch rows of part1 and part2 (side 0: particle 2's
-// axis against particle 1's patch region, side 1 the reverse)
-__device__ __forceinline__ bool row_side(const PP32& P, const float* r1, const float* r2, const V3<float>& r, int k1,
-                                         int k2, int side, float& x1, float& x2) {
-    const bool s1 = side != 0;
-    const PatchView<float> a = vrow_view(s1 ? r2 : r1, 0);
+// The directional query of patch_side from the patch rows of part1 and part2
+// (side 0: particle 2's axis against particle 1's patch region, side 1 the
+// reverse), with the region's side vector `edge` (0: s0, 1: s1) alone.
+struct RowQuery {
+    V3<float> p1, p2, pdir, s, r;   // region's axis, line's axis, patch direction, side vector, separation
+    float cossw, rcSq, h1, h2;
+    bool cyl;                       // region with flat caps (CPSC)
+};
+__device__ __forceinline__ RowQuery row_query(const PP32& P, const float* r1, const float* r2, const V3<float>& r,
+                                              int k1, int k2, bool s1, int edge) {
+    const float* a = s1 ? r2 : r1;
     const float* l = s1 ? r1 : r2;
-    IQ<float> q;
-    q.rcSq = P.rcutSq;
-    q.p1 = a.ax;
+    const float4 a0 = ((const float4*)a)[0];
+    RowQuery q;
+    q.p1 = mk<float>(a0.x, a0.y, a0.z);
+    q.pdir = mk<float>(a0.w, a[4], a[5]);
+    q.s = mk<float>(a[6 + 3 * edge], a[7 + 3 * edge], a[8 + 3 * edge]);
     q.p2 = mk<float>(l[0], l[1], l[2]);
-    q.pdir = a.pd;
-    q.s0 = a.s0;
-    q.s1 = a.s1;
     q.r = s1 ? mk<float>(r.x * -1.0f, r.y * -1.0f, r.z * -1.0f) : r;
     q.cossw = P.pcanglsw[s1 ? (k2 ? 3 : 1) : (k1 ? 2 : 0)];
+    q.rcSq = P.rcutSq;
     q.h1 = s1 ? P.hl1 : P.hl0;
     q.h2 = s1 ? P.hl0 : P.hl1;
-    const bool c = (P.kind == K_CPSC) || (P.kind == K_MIXED && is_psc(P.g0) == s1);
-    return intersect(q, c, x1, x2);
+    q.cyl = (P.kind == K_CPSC) || (P.kind == K_MIXED && is_psc(P.g0) == s1);
+    return q;
+}
+
+// Lane i of the quad (i = 0..3) on all four lanes.
+template <int I>
+__device__ __forceinline__ float quad_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), I * 0x55, 0xf, 0xf, true));
+}
+
+// intersect() on the four lanes of a quad, its candidates side by side instead
+// of one after the other: the reference's ten candidate points (two bounding
+// planes, two roots on the cylinder, two on each end cap, the two ends of the
+// line) depend on nothing but the query, and its early returns only skip
+// candidates that its list of two would ignore.  Lane roles:
+//   0: plane of s0, root + of the cylinder, end +h2      2: both roots on cap +
+//   1: plane of s1, root - of the cylinder, end -h2      3: both roots on cap -
+// (flat caps have one point each).  Each is intersect's expression for that
+// candidate, so it has intersect's bits; then the quad goes through the ten in
+// the reference's order (0.0 marks an empty place, as there: a candidate at
+// 0.0 is no candidate).  One wave64 pass of ~250 instructions without a
+// branch, where the serial search took ~700 and ~60 branches.  edge must be
+// role & 1.
+__device__ __forceinline__ bool quad_intersect(const RowQuery& q, int role, float& t1, float& t2) {
+    const bool cap = role >= 2;
+    // plane_hit
+    const V3<float> np = cross(q.p1, q.s);
+    const float pa = dot(np, q.p2), ti = dot(np, q.r) / pa;
+    const V3<float> dv = mk<float>(ti * q.p2.x - q.r.x, ti * q.p2.y - q.r.y, ti * q.p2.z - q.r.z);
+    const float c = dot(dv, q.s), d = fabsf(dot(dv, q.p1)) - q.h1;
+    const bool in = q.cyl ? (d <= 0.0f) & (c * c <= q.rcSq) : (((d <= 0.0f) ? c * c : d * d + c * c) <= q.rcSq);
+    const bool pl = !cap & (pa != 0.0f) & !((ti > q.h2) | (ti < -q.h2)) & !(c * q.cossw < 0.0f) & in;
+    // the quadratic of the cylinder (cyl_hits) or of a spherical cap
+    const float sg = role == 3 ? -1.0f : 1.0f;
+    const V3<float> c1 = cross(mk<float>(-1.0f * q.r.x, -1.0f * q.r.y, -1.0f * q.r.z), q.p1), c2 = cross(q.p2, q.p1);
+    const V3<float> vc = mk<float>(sg * q.p1.x * q.h1 - q.r.x, sg * q.p1.y * q.h1 - q.r.y, sg * q.p1.z * q.h1 - q.r.z);
+    const V3<float> u = mk<float>(cap ? vc.x : c1.x, cap ? vc.y : c1.y, cap ? vc.z : c1.z),
+                    w = mk<float>(cap ? q.p2.x : c2.x, cap ? q.p2.y : c2.y, cap ? q.p2.z : c2.z);
+    // (the division stands in a statement of its own: under a condition it can
+    // be hoisted, and then loses the accuracy it is compiled with)
+    const float qa = cap ? 1.0f : dot(c2, c2), qb = 2.0f * dot(u, w), qc = dot(u, u) - q.rcSq,
+                disc = qb * qb - 4.0f * qa * qc, sq = sqrtf(disc), hinv = 0.5f / qa;
+    const float inv = cap ? 0.5f : hinv;
+    const float xp = (-qb + sq) * inv, xm = (-qb - sq) * inv;
+    float x1 = role == 1 ? xm : xp;
+    const float x2 = cap ? xm : (role == 0 ? q.h2 : -q.h2);
+    // the candidate points: inside the region's wedge, and on the right part of the surface
+    auto point = [&](const V3<float>& v, float& a, float& n2) {
+        a = dot(v, q.p1);
+        const V3<float> vec = mk<float>(v.x - q.p1.x * a, v.y - q.p1.y * a, v.z - q.p1.z * a);
+        n2 = dot(vec, vec);
+        return dot(q.pdir, vec) >= q.cossw * sqrtf(n2);
+    };
+    V3<float> v1 = mk<float>(q.p2.x * x1 - q.r.x, q.p2.y * x1 - q.r.y, q.p2.z * x1 - q.r.z);
+    const V3<float> v2 = mk<float>(q.p2.x * x2 - q.r.x, q.p2.y * x2 - q.r.y, q.p2.z * x2 - q.r.z);
+    bool flat = false, on_flat = false;
+    if (q.cyl && cap) {   // a flat cap's point
+        const float a = dot(q.p1, q.p2);
+        const V3<float> o = mk<float>(q.r.x + sg * q.h1 * q.p1.x, q.r.y + sg * q.h1 * q.p1.y,
+                                      q.r.z + sg * q.h1 * q.p1.z);
+        x1 = dot(q.p1, o) / a;
+        v1 = mk<float>(x1 * q.p2.x - o.x, x1 * q.p2.y - o.y, x1 * q.p2.z - o.z);
+        flat = true;
+        on_flat = (a != 0.0f) & !((x1 > q.h2) | (x1 < -q.h2)) & !(dot(v1, v1) > q.rcSq);
+    }
+    float a1, b1, a2, b2;
+    const bool w1 = point(v1, a1, b1), w2 = point(v2, a2, b2);
+    const bool out1 = (a1 >= q.h1) | (a1 <= -q.h1), out2 = (a2 >= q.h1) | (a2 <= -q.h1);
+    const bool on = (disc >= 0.0f) & !((x1 >= q.h2) | (x1 <= -q.h2)) & (out1 == cap) & ((role != 1) | (sq > 0.0f));
+    const bool ok1 = (flat ? on_flat : on) & w1;
+    const float dd = fabsf(a2) - q.h1;
+    const bool end = q.cyl ? (dd <= 0.0f) & (b2 < q.rcSq) : (((dd <= 0.0f) ? b2 : dd * dd + b2) < q.rcSq);
+    const bool ok2 = (cap ? (disc >= 0.0f) & (sq > 0.0f) & !((x2 >= q.h2) | (x2 <= -q.h2)) & out2 & !flat : end) & w2;
+    const float e0 = pl ? ti : 0.0f, e1 = ok1 ? x1 : 0.0f, e2 = ok2 ? x2 : 0.0f;
+    const float cand[10] = {quad_lane<0>(e0), quad_lane<1>(e0), quad_lane<0>(e1), quad_lane<1>(e1), quad_lane<2>(e1),
+                            quad_lane<2>(e2), quad_lane<3>(e1), quad_lane<3>(e2), quad_lane<0>(e2), quad_lane<1>(e2)};
+    t1 = t2 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 10; k++) {   // Ints::add_patch's list
+        const float x = cand[k];
+        const bool none = t1 == 0.0f;
+        t2 = (!none & (t2 == 0.0f) & (x != t1)) ? x : t2;
+        t1 = none ? x : t1;
+    }
+    return t2 != 0.0f;
+}
+
+// Can the query of region axis p1, patch direction pdir and sides s0, s1 be a
+// hit?  False only when it certainly is not: the part of the line x p2 - r,
+// |x| <= h2, inside the two half spaces that bound the region's wedge (their
+// planes hold the axis and one side each) is empty, or stays farther than rcut
+// from the axis.  Every point that the intersection accepts lies in the wedge
+// and within rcut of the axis up to the FP32 error of these products (~1e-6;
+// the half spaces are widened by a hundred times that, rcut^2 by 1e-3), and a
+// pair term needs such a point on both sides.  Wedges of 180 degrees and more
+// (cossw <= 0) are not half-space intersections: always true.  A NaN keeps
+// the item.  Of the patch pairs in range of uniformly oriented TCHPSC 9.7% have both
+// hits and 10.6% pass both tests (without the distance 20%).
+__device__ __forceinline__ bool side_possible(const PatchView<float>& a, const V3<float>& p2, const V3<float>& r,
+                                              float h2, float cossw, float rcSq) {
+    const V3<float> n0 = cross(a.ax, a.s0), n1 = cross(a.ax, a.s1);
+    // inside: b0 - x a0 >= -m and x a1 - b1 >= -m
+    const float a0 = dot(n0, p2), b0 = dot(n0, r) + 1e-4f, a1 = dot(n1, p2), b1 = dot(n1, r) - 1e-4f;
+    const float x0 = b0 * __builtin_amdgcn_rcpf(a0), x1 = b1 * __builtin_amdgcn_rcpf(a1);
+    float lo = -h2, hi = h2;
+    lo = a0 < 0.0f ? fmaxf(lo, x0) : lo;
+    hi = a0 > 0.0f ? fminf(hi, x0) : hi;
+    lo = a1 > 0.0f ? fmaxf(lo, x1) : lo;
+    hi = a1 < 0.0f ? fminf(hi, x1) : hi;
+    // the point of the rest nearest to the axis
+    const V3<float> bp = perp(p2, a.ax), vp = perp(r, a.ax);   // x bp - vp
+    const float x = fminf(fmaxf(dot(vp, bp) * __builtin_amdgcn_rcpf(dot(bp, bp)), lo), hi);
+    const V3<float> w = mk<float>(x * bp.x - vp.x, x * bp.y - vp.y, x * bp.z - vp.z);
+    return !(cossw > 0.01f) | !((lo > hi) | (dot(w, w) > rcSq * 1.001f));
 }
 
 // One trial of the speculative sweep, on one wave: the energies of the moving
@@ -1931,7 +2048,8 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     // relative margin of 1e-5 covers the K_SCA term's square-root test).  The
     // same particle and chain partners (bond and angle terms reach beyond
     // maxcut) always depend.
-    int nx = 0;
+    int nx = 0, nsph = 0;   // entries in range: patch pairs to evaluate, sphere pairs that were
+    double so = 0.0, sn = 0.0;
     unsigned long long depm = 0;
     const int nc = no + nn;
     for (int base = 0; base < nc + 4 * w; base += WAVE) {
@@ -1940,7 +2058,7 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
         const int x = it - nc;
         const int which = cand ? (it >= no ? 1 : 0) : (x >> 1) & 1;
         int jj = 0;
-        bool need = false, d = false;
+        bool need = false, d = false, sphere = false;
         float dseg2 = 0.0f;
         if (cand || isdep) {
             const SpecProp& pi = prop[cand ? 0 : x >> 2];
@@ -1980,8 +2098,16 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                     ev = sphere_pair(P2, sqrtf(dot(r, r)));
                     d = true;
                 } else if (kind != K_NONE) {
-                    need = true;
                     d = true;
+                    if (cand) {   // a sphere and a spherocylinder: its whole term, not a cheap one
+                        const float* mv = which ? mvn : mvo;
+                        DPart<float> pm = vrow_part(mv, t, tp[t].geotype);
+                        DPart<float> pb = rows.has(jj) ? vrow_part(rows.row(jj), b.w, tp[b.w].geotype)
+                                                       : load_part<float>(S.o[jj], S.q[jj], b.w, tp);
+                        const float es = sw ? spsc(P2, pb, pm, r) : spsc(P2, pm, pb, r);
+                        if (which) sn += (double)es; else so += (double)es;
+                        sphere = true;
+                    }
                 }
                 if (cand) {
                     if (which) an += (double)ev; else ao += (double)ev;
@@ -1997,6 +2123,7 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             }
         }
         nx += __popcll(m);
+        nsph += __popcll(__ballot(sphere));
         const int x0 = nc - base;   // the lane of dependence item 0
         if (md) depm |= x0 >= 0 ? md >> x0 : md << -x0;
     }
@@ -2016,8 +2143,8 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
         des = rep;
         if constexpr (DA == DA_NET) {
             stage = 1;
-            if (nx >= mc.minx) {   // the entries of both states, the same for the reverse move
-                double so = 0.0, sn = 0.0;
+            if (nx + nsph >= mc.minx) {   // the entries of both states, the same for the reverse move
+                double no_ = 0.0, nn_ = 0.0;
                 for (int t0 = 0; t0 < nx; t0 += MLP_TILE) {
                     float f[MLP_NF];
                     const int e = t0 + (lane & (MLP_TILE - 1)), xw = e < nx ? T.xl[e] : 0, which = xw >> 15;
@@ -2026,85 +2153,103 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                                              vrow_dir(mv), mv_vec(mv, VROW_PD0), sc, mc, f);
                     float out = mlp_tile_g(mlp_img, ml, mlp_slots(f, lane >> 4), lane);
                     if (lane < MLP_TILE && net) {
-                        if (which) sn += (double)out; else so += (double)out;
+                        if (which) nn_ += (double)out; else no_ += (double)out;
                     }
                 }
-                const double ds = wave_sum_dpp(sn) - wave_sum_dpp(so);
+                const double ds = wave_sum_dpp(nn_) - wave_sum_dpp(no_);
                 if (!(ds <= 0.0 || ds < thr2)) return false;
                 des = rep + ds;
             }
         }
         // 2: through every screen; 3: past the first, the network not run
-        stage = (DA == DA_NET && nx < mc.minx) ? 3 : 2;
+        stage = (DA == DA_NET && nx + nsph < mc.minx) ? 3 : 2;
     }
-    // phase C: (entry, patch pair, side) items, the two wedge intersections of
-    // a patch pair on neighbouring lanes; where they take more than one pass,
-    // each lane takes both sides of its patch pair, one after the other (half
-    // the passes, and the set-up and attraction once per patch pair; the same
-    // values: each side is the same intersect call).  An item's vectors come
-    // from the rows of the mover and of its neighbour: each side picks which
-    // of the two is the region and which the line by pointer.
+    ao += so;
+    an += sn;
+    // phase C: (entry, patch pair) items.  More than eight are first tested for
+    // a possible hit of both wedge intersections, a side per lane
+    // (side_possible: of the ~23 items of a TCHPSC trial at packing fraction
+    // 0.25 about 3 are left); then eight at a time, on eight lanes each: a quad
+    // per wedge intersection, the attraction on the first lane.  An item's
+    // vectors come from the rows of the mover and of its neighbour, region and
+    // line picked by pointer.
     const bool all_rows = rows.hi - rows.lo == S.n;
     const int psh = ppmax > 2 ? 2 : (ppmax > 1 ? 1 : 0);   // log2 of the patch pairs per entry (1, 2 or 4)
-    const bool dual = all_rows && (nx << (psh + 1)) > WAVE;
-    const int ish = dual ? psh : psh + 1;                  // log2 of the lanes per entry
-    const int eb = all_rows ? WAVE >> ish : min(SPEC_NV, WAVE >> ish);
-    for (int e0 = 0; e0 < nx; e0 += eb) {
-        if (!all_rows) {   // the batch's neighbours' rows
-            wave_lds_sync();
-            const int e = e0 + lane / npatch;
-            if (lane < eb * npatch && e < nx) {
-                const int jj = T.xl[e] & 0x7fff;
-                vrow_derive(T.nv + (e - e0) * VROW, lane % npatch, S.o[jj], S.q[jj], S.u[jj].w, tp);
-            }
-            wave_lds_sync();
-        }
-        const int e = e0 + (lane >> ish), side = dual ? 0 : lane & 1;
-        const int mpp = (dual ? lane : lane >> 1) & ((1 << psh) - 1);
-        int which = 0, k1 = 0, k2 = 0;
-        bool hit = false, hit2 = false, sw = false;
-        float x1 = 0.0f, x2 = 0.0f, ev = 0.0f, z1 = 0.0f, z2 = 0.0f;
-        const PP32* P2 = pp;
-        const float *r1 = mvo, *r2 = mvo;   // rows of part1 and part2
-        V3<float> r = mk<float>(0.0f, 0.0f, 0.0f);
-        if ((lane >> ish) < eb && e < nx) {
-            const int w = T.xl[e], jj = w & 0x7fff;
-            which = w >> 15;
-            const uint4 bu = S.u[jj];
-            sw = S.id[jj] > idk;   // canonical order, as in phase B
-            P2 = sw ? pp + bu.w * sc.nt + t : pp + t * sc.nt + bu.w;
-            r = which ? fx_image_c(un.x, un.y, un.z, bu.x, bu.y, bu.z, sc.Lh, sc.Ll)
+    struct Item {
+        const PP32* P;
+        const float *r1, *r2;   // patch rows of part1 and part2
+        V3<float> r;
+        int k1, k2, jj, which;
+        bool sw, patch;
+    };
+    auto item = [&](int it, const float* nrow) {
+        Item I;
+        const int w = T.xl[it >> psh], mpp = it & ((1 << psh) - 1);
+        I.jj = w & 0x7fff;
+        I.which = w >> 15;
+        const uint4 bu = S.u[I.jj];
+        I.sw = S.id[I.jj] > idk;   // canonical order, as in phase B
+        I.P = I.sw ? pp + bu.w * sc.nt + t : pp + t * sc.nt + bu.w;
+        I.r = I.which ? fx_image_c(un.x, un.y, un.z, bu.x, bu.y, bu.z, sc.Lh, sc.Ll)
                       : fx_image_c(uo.x, uo.y, uo.z, bu.x, bu.y, bu.z, sc.Lh, sc.Ll);
-            if (sw) r = mk<float>(-r.x, -r.y, -r.z);
-            const float* mv = which ? mvn : mvo;
-            const float* nv = all_rows ? rows.row(jj) : T.nv + (e - e0) * VROW;
-            r1 = sw ? nv : mv;
-            r2 = sw ? mv : nv;
-            if (P2->kind <= K_SCA) {
-                if (mpp < npatch_pairs(*P2)) {
-                    patch_pair_index(*P2, mpp, k1, k2);   // patches of part1 and part2
-                    r1 += 12 * k1;
-                    r2 += 12 * k2;
-                    hit = row_side(*P2, r1, r2, r, k1, k2, side, x1, x2);
-                    if (dual) hit2 = row_side(*P2, r1, r2, r, k1, k2, 1, z1, z2);
-                }
-            } else if (mpp == 0 && side == 0) {
-                DPart<float> pb = load_part<float>(S.o[jj], S.q[jj], bu.w, tp);
-                DPart<float> pm = vrow_part(mv, t, tp[t].geotype);
-                ev = sw ? spsc(*P2, pb, pm, r) : spsc(*P2, pm, pb, r);
+        if (I.sw) I.r = mk<float>(-I.r.x, -I.r.y, -I.r.z);
+        I.patch = mpp < npatch_pairs(*I.P);
+        patch_pair_index(*I.P, mpp, I.k1, I.k2);   // patches of part1 and part2
+        const float* mv = I.which ? mvn : mvo;
+        const float* nv = all_rows ? rows.row(I.jj) : nrow;
+        I.r1 = (I.sw ? nv : mv) + 12 * I.k1;
+        I.r2 = (I.sw ? mv : nv) + 12 * I.k2;
+        return I;
+    };
+    constexpr int CHUNK = 512;   // items whose survivors the list holds
+    for (int c0 = 0; c0 < nx << psh; c0 += CHUNK) {
+        const int end = min(CHUNK, (nx << psh) - c0);
+        int cnt = end;
+        const bool culled = all_rows && end > 8;
+        if (culled) {
+            cnt = 0;
+            for (int b0 = 0; b0 < end; b0 += WAVE / 2) {
+                const int it = b0 + (lane >> 1), side = lane & 1;
+                const Item I = item(c0 + min(it, end - 1), nullptr);
+                const PatchView<float> a = vrow_view(side ? I.r2 : I.r1, 0);
+                const float* l = side ? I.r1 : I.r2;
+                const V3<float> rs = side ? mk<float>(-I.r.x, -I.r.y, -I.r.z) : I.r;
+                const bool k = side_possible(a, mk<float>(l[0], l[1], l[2]), rs, side ? I.P->hl0 : I.P->hl1,
+                                             I.P->pcanglsw[side ? (I.k2 ? 3 : 1) : (I.k1 ? 2 : 0)], I.P->rcutSq);
+                unsigned long long m = __ballot(k & I.patch & (it < end));
+                m &= (m >> 1) & 0x5555555555555555ull;   // both sides, at the even lane
+                if ((m >> lane) & 1) T.nl[cnt + wave_prefix(m)] = (uint16_t)it;   // (the candidates are done with)
+                cnt += __popcll(m);
             }
+            wave_lds_sync();
         }
-        // the other side's result (lane ^ 1 holds the entry's other side)
-        float y1 = z1, y2 = z2;
-        int oh = hit2 ? 1 : 0;
-        if (!dual) {
-            y1 = __shfl_xor(x1, 1);
-            y2 = __shfl_xor(x2, 1);
-            oh = __shfl_xor(hit ? 1 : 0, 1);
+        for (int b0 = 0; b0 < cnt; b0 += 8) {
+            const int g = b0 + (lane >> 3), role = lane & 3, side = (lane >> 2) & 1;
+            const int it = c0 + (culled ? T.nl[min(g, cnt - 1)] : min(g, cnt - 1));
+            float* nrow = T.nv + (lane >> 3) * VROW;
+            if (!all_rows) {   // the neighbour's patch
+                wave_lds_sync();
+                if ((lane & 7) == 0) {
+                    const Item I = item(it, nrow);
+                    if (I.patch)
+                        vrow_put(nrow, I.sw ? I.k1 : I.k2,
+                                 load_view<float>(S.o[I.jj], S.q[I.jj], S.u[I.jj].w, tp, I.sw ? I.k1 : I.k2));
+                }
+                wave_lds_sync();
+            }
+            const Item I = item(it, nrow);
+            float x1 = 0.0f, x2 = 0.0f, ev = 0.0f;
+            bool hit = false;
+            if (I.patch)
+                hit = quad_intersect(row_query(*I.P, I.r1, I.r2, I.r, I.k1, I.k2, side != 0, role & 1), role, x1, x2);
+            const float y1 = __shfl_xor(x1, 4), y2 = __shfl_xor(x2, 4);   // the other side's
+            const bool both = hit & (__shfl_xor(hit ? 1 : 0, 4) != 0);
+            if ((lane & 7) == 0 && g < cnt) {
+                if (both)
+                    ev = patch_atr<float>(*I.P, vrow_view(I.r1, 0), vrow_view(I.r2, 0), I.r, I.k1, I.k2, x1, x2, y1, y2);
+            }
+            if (I.which) an += (double)ev; else ao += (double)ev;
         }
-        if (side == 0 && hit && oh)
-            ev = patch_atr<float>(*P2, vrow_view(r1, 0), vrow_view(r2, 0), r, k1, k2, x1, x2, y1, y2);
-        if (which) an += (double)ev; else ao += (double)ev;
     }
     eo = wave_sum_dpp(ao);
     en = wave_sum_dpp(an);
