@@ -795,73 +795,6 @@ __global__ __launch_bounds__(1024) void k_reduce(int n, const double* __restrict
     if (t == 0) *out = sh[0];
 }
 
-// --------------------------------------------------------- energy (queries)
-// One wave per query particle: its energy with every particle of the stencil
-// around its cell except those of ID ex_lo..ex_hi (the particle itself, or
-// its whole molecule for mol2others), plus its bonds for oneToAll (not for
-// mol2others, whose connectivity list is empty).  The query state is given
-// explicitly (trial states) or taken from a slot.
-struct Query {
-    uint32_t u[3];
-    int t;
-    float4 o;
-    float2 q;
-    int id;            // the query particle's ID
-    int ex_lo, ex_hi;  // IDs left out
-    int bonds;         // add the bonds with its chain partners
-};
-
-__global__ __launch_bounds__(WAVE) void k_energy_query(int nq, const Query* __restrict__ qs, const int* __restrict__ qslot,
-                                                       Grid g, SysConst sc, const int* __restrict__ starts,
-                                                       const uint4* __restrict__ P, const float4* __restrict__ O,
-                                                       const float2* __restrict__ Q, const int* __restrict__ ID,
-                                                       const PP32* __restrict__ pp, const TP32* __restrict__ tp,
-                                                       ChainTab ct, const int* __restrict__ slot,
-                                                       double* __restrict__ out) {
-    int qi = blockIdx.x;
-    if (qi >= nq) return;
-    int lane = lane_id();
-    Query q;
-    if (qslot) {
-        int s = qslot[qi];
-        uint4 p = P[s];
-        q.u[0] = p.x; q.u[1] = p.y; q.u[2] = p.z; q.t = p.w;
-        q.o = O[s]; q.q = Q[s]; q.id = q.ex_lo = q.ex_hi = ID[s];
-        q.bonds = 1;
-    } else {
-        q = qs[qi];
-    }
-    DPart<float> pa = load_part<float>(q.o, q.q, q.t, tp);
-    int c = cell_of_u(g, q.u[0], q.u[1], q.u[2]);
-    int cx = c % g.nc[0], cy = (c / g.nc[0]) % g.nc[1], cz = c / (g.nc[0] * g.nc[1]);
-    int ns = stencil_size(g);
-    double acc = 0.0;
-    for (int si = 0; si < ns; si++) {
-        int hm;
-        int cc = stencil_cell(g, cx, cy, cz, si, hm);
-        int b = starts[cc], e = starts[cc + 1];
-        for (int k = b + lane; k < e; k += WAVE) {
-            int idk = ID[k];
-            if (idk >= q.ex_lo && idk <= q.ex_hi) continue;
-            uint4 pb4 = P[k];
-            V3<float> r = fx_image_c(q.u[0], q.u[1], q.u[2], pb4.x, pb4.y, pb4.z, sc.Lh, sc.Ll);
-            if (dot(r, r) > sc.sqmaxcut) continue;
-            DPart<float> pb = load_part<float>(O[k], Q[k], pb4.w, tp);
-            // the pair in its canonical order, the higher ID as part1 (allToAll's)
-            if (idk > q.id)
-                acc += pair_energy_d<float>(pp[pb4.w * sc.nt + q.t], pb, pa, mk<float>(-r.x, -r.y, -r.z), sc.sqmaxcut);
-            else
-                acc += pair_energy_d<float>(pp[q.t * sc.nt + pb4.w], pa, pb, r, sc.sqmaxcut);
-        }
-    }
-    // chain partners, wherever they are
-    if (ct.cw && lane == 0 && q.bonds)
-        acc += bonds_global(ct, sc.nt, sc.Ld, q.id, make_uint4(q.u[0], q.u[1], q.u[2], (uint32_t)q.t), q.o, q.q,
-                            15, slot, P, O, Q);
-    double s = wave_sum(acc);
-    if (lane == 0) out[qi] = s;
-}
-
 // ------------------------------------------------------------ pair energies
 // p2p(i, j) with i's connectivity list: the non-bonded functor, plus the bond
 // and angle terms when j is one of i's chain partners
@@ -2254,6 +2187,228 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     eo = wave_sum_dpp(ao);
     en = wave_sum_dpp(an);
     return true;
+}
+
+// --------------------------------------------------------- energy (queries)
+// One query particle per block: its energy with every particle of the stencil
+// around its cell except those of ID ex_lo..ex_hi (the particle itself, or
+// its whole molecule for mol2others), plus its bonds for oneToAll (not for
+// mol2others, whose connectivity list is empty).  The query state is given
+// explicitly (trial states) or taken from a slot.
+struct Query {
+    uint32_t u[3];
+    int t;
+    float4 o;
+    float2 q;
+    int id;            // the query particle's ID
+    int ex_lo, ex_hi;  // IDs left out
+    int bonds;         // add the bonds with its chain partners
+};
+
+// The stencil's particles are flattened over the block's NW waves, PA of them
+// per thread at once, and pass the same stages as a trial of the speculative
+// sweep: centres within reach, then segment distances, then the patch pairs in
+// range, eight lanes each (quad_intersect), behind side_possible where there
+// are more than fit one pass.  Bound by latency: one wave that walked the
+// stencil cell by cell, the whole pair functor inlined per candidate, took
+// 104 us for one query of 1,000 PSC and 720 us for every particle of a 34,000-particle mixture.  NW = 4 for few
+// queries (a host program's single moves); NW = 1 when the queries alone fill
+// the chip.
+constexpr int QRY_LCAP = 1024;   // candidates held before they are evaluated
+template <int NW>
+__global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query* __restrict__ qs,
+                                                            const int* __restrict__ qslot, Grid g, SysConst sc,
+                                                            const int* __restrict__ starts,
+                                                            const uint4* __restrict__ P, const float4* __restrict__ O,
+                                                            const float2* __restrict__ Q, const int* __restrict__ ID,
+                                                            const PP32* __restrict__ pp, const TP32* __restrict__ tp,
+                                                            int ppmax, ChainTab ct, const int* __restrict__ slot,
+                                                            double* __restrict__ out) {
+    constexpr int BS = WAVE * NW, PA = NW == 1 ? 4 : 2;
+    static_assert(PA * BS <= QRY_LCAP / 2, "a scan step fits beside the candidates kept");
+    __shared__ int pre[126], cst[126], list[QRY_LCAP], cnt[2 * CNT_HALF];
+    __shared__ uint4 eu[BS];               // entries in the attraction's range: position and type, ID, row
+    __shared__ int eid[BS];
+    __shared__ __align__(16) float rows[(BS + 1) * VROW];   // row 0: the query
+    __shared__ uint16_t surv[4 * BS];
+    __shared__ double red[NW];
+    const int qi = blockIdx.x;
+    if (qi >= nq) return;
+    const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1);
+    Query q;
+    if (qslot) {
+        int s = qslot[qi];
+        uint4 p = P[s];
+        q.u[0] = p.x; q.u[1] = p.y; q.u[2] = p.z; q.t = p.w;
+        q.o = O[s]; q.q = Q[s]; q.id = q.ex_lo = q.ex_hi = ID[s];
+        q.bonds = 1;
+    } else {
+        q = qs[qi];
+    }
+    const int np = ppmax > 1 ? 2 : 1, psh = ppmax > 2 ? 2 : (ppmax > 1 ? 1 : 0);
+    if (tid < np) vrow_derive(rows, tid, q.o, q.q, q.t, tp);
+    const int c = cell_of_u(g, q.u[0], q.u[1], q.u[2]);
+    const int cx = c % g.nc[0], cy = (c / g.nc[0]) % g.nc[1], cz = c / (g.nc[0] * g.nc[1]);
+    const int ns = stencil_size(g);
+    if (tid < WAVE) {   // prefix of the stencil cells' counts
+        int carry = 0;
+        for (int b = 0; b < ns; b += WAVE) {
+            int i = b + lane, n = 0, hm;
+            if (i < ns) {
+                int cc = stencil_cell(g, cx, cy, cz, i, hm), st = starts[cc];
+                n = starts[cc + 1] - st;
+                cst[i] = st;
+            }
+            int v = n;
+            for (int o = 1; o < WAVE; o <<= 1) {
+                int x = __shfl_up(v, o, WAVE);
+                if (lane >= o) v += x;
+            }
+            if (i < ns) pre[i] = carry + v - n;
+            carry += __shfl(v, WAVE - 1, WAVE);
+        }
+        if (lane == 0) pre[ns] = carry;
+    }
+    __syncthreads();
+    const int total = pre[ns], t = q.t;
+    const V3<float> dq = vrow_dir(rows);
+    const float hq = tp[t].hl, reach2 = tp[t].reach2;
+    double acc = 0.0;
+    int nl = 0, par = 0;
+    for (int base = 0; base < total; base += PA * BS) {
+        int src[PA];
+        bool keep[PA];
+        uint4 u[PA];
+        int id[PA], pos[PA];
+#pragma unroll
+        for (int h = 0; h < PA; h++) {
+            const int e = min(base + h * BS + tid, total - 1);
+            int lo = 0, hi = ns - 1;   // the stencil entry holding element e
+            while (lo < hi) {
+                int mid = (lo + hi + 1) >> 1;
+                if (pre[mid] <= e) lo = mid; else hi = mid - 1;
+            }
+            src[h] = cst[lo] + (e - pre[lo]);
+        }
+#pragma unroll
+        for (int h = 0; h < PA; h++) {
+            u[h] = P[src[h]];
+            id[h] = ID[src[h]];
+        }
+#pragma unroll
+        for (int h = 0; h < PA; h++) {
+            const V3<float> r = fx_image_c(q.u[0], q.u[1], q.u[2], u[h].x, u[h].y, u[h].z, sc.Lh, sc.Ll);
+            keep[h] = (base + h * BS + tid < total) & !((id[h] >= q.ex_lo) & (id[h] <= q.ex_hi)) &
+                      (dot(r, r) <= sc.sqmaxcut) & (centre_dist2(dq, hq, r) <= reach2);
+        }
+        block_compactK<NW, PA>(keep, nl, cnt, par, pos);
+#pragma unroll
+        for (int h = 0; h < PA; h++)
+            if (keep[h]) list[pos[h]] = src[h];
+        if (nl <= QRY_LCAP - PA * BS && base + PA * BS < total) continue;
+        __syncthreads();
+        for (int b = 0; b < nl; b += BS) {
+            bool need = false;
+            uint4 ub = make_uint4(0, 0, 0, 0);
+            float4 ob = make_float4(0, 0, 0, 0);
+            float2 qb = make_float2(0, 0);
+            int ib = 0;
+            if (b + tid < nl) {
+                const int k = list[b + tid];
+                ub = P[k];
+                ob = O[k];
+                qb = Q[k];
+                ib = ID[k];
+                const bool sw = ib > q.id;   // the pair in its canonical order, the higher ID as part1 (allToAll's)
+                const PP32& P2 = sw ? pp[ub.w * sc.nt + t] : pp[t * sc.nt + ub.w];
+                V3<float> r = fx_image_c(q.u[0], q.u[1], q.u[2], ub.x, ub.y, ub.z, sc.Lh, sc.Ll);
+                if (sw) r = mk<float>(-r.x, -r.y, -r.z);
+                if (P2.kind <= K_SCA && P2.kind >= 0) {
+                    V3<float> db = mk<float>(ob.x, ob.y, ob.z);
+                    if (P2.kind < K_SCN) db = normalised(db);   // as derive leaves it
+                    DPart<float> pa, pb;
+                    pa.dir = sw ? db : dq;
+                    pb.dir = sw ? dq : db;
+                    float ev, d2;
+                    need = scsc_cheap(P2, pa, pb, r, ev, d2);
+                    acc += (double)ev;
+                } else if (P2.kind == K_SPH_WCA || P2.kind == K_SPH_TAYLOR) {
+                    acc += (double)sphere_pair(P2, sqrtf(dot(r, r)));
+                } else if (P2.kind != K_NONE) {
+                    DPart<float> pa = load_part<float>(q.o, q.q, t, tp), pb = load_part<float>(ob, qb, ub.w, tp);
+                    acc += (double)(sw ? spsc(P2, pb, pa, r) : spsc(P2, pa, pb, r));
+                }
+            }
+            int ne = 0;
+            const int ep = block_compact<NW>(need, ne, cnt);
+            if (need) {
+                eu[ep] = ub;
+                eid[ep] = ib;
+                for (int k = 0; k < np; k++) vrow_derive(rows + (1 + ep) * VROW, k, ob, qb, ub.w, tp);
+            }
+            __syncthreads();
+            int items = ne << psh;
+            auto patch = [&](int it, int& k1, int& k2, V3<float>& r, const float*& r1, const float*& r2,
+                             bool& ok) -> const PP32* {
+                const int e = it >> psh, mpp = it & ((1 << psh) - 1);
+                const uint4 b4 = eu[e];
+                const bool sw = eid[e] > q.id;
+                const PP32* P2 = sw ? pp + b4.w * sc.nt + t : pp + t * sc.nt + b4.w;
+                r = fx_image_c(q.u[0], q.u[1], q.u[2], b4.x, b4.y, b4.z, sc.Lh, sc.Ll);
+                if (sw) r = mk<float>(-r.x, -r.y, -r.z);
+                ok = mpp < npatch_pairs(*P2);
+                patch_pair_index(*P2, mpp, k1, k2);
+                const int o1 = sw ? 1 + e : 0, o2 = sw ? 0 : 1 + e;
+                r1 = rows + o1 * VROW + 12 * k1;
+                r2 = rows + o2 * VROW + 12 * k2;
+                return P2;
+            };
+            const bool culled = items > BS / 8;
+            if (culled) {
+                int left = 0;
+                for (int b2 = 0; b2 < items; b2 += BS) {
+                    bool k = false;
+                    if (b2 + tid < items) {
+                        int k1, k2;
+                        V3<float> r;
+                        const float *r1, *r2;
+                        bool ok;
+                        const PP32* P2 = patch(b2 + tid, k1, k2, r, r1, r2, ok);
+                        const PatchView<float> va = vrow_view(r1, 0), vb = vrow_view(r2, 0);
+                        k = ok & side_possible(va, vb.ax, r, P2->hl1, P2->pcanglsw[k1 ? 2 : 0], P2->rcutSq) &
+                            side_possible(vb, va.ax, mk<float>(-r.x, -r.y, -r.z), P2->hl0, P2->pcanglsw[k2 ? 3 : 1],
+                                          P2->rcutSq);
+                    }
+                    const int sp = block_compact<NW>(k, left, cnt);
+                    if (k) surv[sp] = (uint16_t)(b2 + tid);
+                }
+                items = left;
+                __syncthreads();
+            }
+            for (int b2 = 0; b2 < items; b2 += BS / 8) {
+                const int gi = b2 + (tid >> 3), role = lane & 3, side = (lane >> 2) & 1, gc = min(gi, items - 1);
+                int k1, k2;
+                V3<float> r;
+                const float *r1, *r2;
+                bool ok;
+                const PP32* P2 = patch(culled ? surv[gc] : gc, k1, k2, r, r1, r2, ok);
+                float x1, x2;
+                const bool hit = quad_intersect(row_query(*P2, r1, r2, r, k1, k2, side != 0, role & 1), role, x1, x2) & ok;
+                const float y1 = __shfl_xor(x1, 4), y2 = __shfl_xor(x2, 4);
+                const bool both = hit & (__shfl_xor(hit ? 1 : 0, 4) != 0);
+                if ((lane & 7) == 0 && gi < items && both)
+                    acc += (double)patch_atr<float>(*P2, vrow_view(r1, 0), vrow_view(r2, 0), r, k1, k2, x1, x2, y1, y2);
+            }
+            __syncthreads();
+        }
+        nl = 0;
+    }
+    // chain partners, wherever they are
+    if (ct.cw && tid == 0 && q.bonds)
+        acc += bonds_global(ct, sc.nt, sc.Ld, q.id, make_uint4(q.u[0], q.u[1], q.u[2], (uint32_t)q.t), q.o, q.q,
+                            15, slot, P, O, Q);
+    const double sum = block_sum<NW>(acc, red);
+    if (tid == 0) out[qi] = sum;
 }
 
 // stage_load for the speculative sweep: of the stencil's particles only those
@@ -5593,9 +5748,15 @@ static int run_queries(sc_ctx* ctx, int nq, const Query* hq, const int* slots_de
     if (hq) HIPCK(hipMemcpyAsync(ctx->d_q, hq, nq * sizeof(Query), hipMemcpyHostToDevice, ctx->stream));
     SysConst sc = sysconst(ctx, ctx->box);
     int c = ctx->cur;
-    hipLaunchKernelGGL(k_energy_query, dim3(nq), dim3(WAVE), 0, ctx->stream, nq, hq ? ctx->d_q : nullptr, slots_dev,
-                       ctx->g, sc, ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32,
-                       chain_tab(ctx), ctx->slot, ctx->d_out);
+    // four waves per query while that leaves a wave slot of the chip to each
+    // (256 CUs x 4 SIMDs x 4 waves of this kernel's registers), else one
+#define QUERY(NWV)                                                                                             \
+    hipLaunchKernelGGL((k_energy_query<NWV>), dim3(nq), dim3(WAVE * NWV), 0, ctx->stream, nq,                    \
+                       hq ? ctx->d_q : nullptr, slots_dev, ctx->g, sc, ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], \
+                       ctx->ID[c], ctx->d_pp32, ctx->d_tp32, ctx->ppmax, chain_tab(ctx), ctx->slot, ctx->d_out)
+    if (nq <= 1024) QUERY(4);
+    else QUERY(1);
+#undef QUERY
     HIPCK(hipGetLastError());
     HIPCK(hipMemcpyAsync(out, ctx->d_out, nq * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPCK(hipStreamSynchronize(ctx->stream));
