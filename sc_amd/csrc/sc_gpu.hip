@@ -653,25 +653,22 @@ __device__ double bonds_global(const ChainTab& ct, int nt, const double* L, int 
 }
 
 // Whole-system bond energy: one thread per ID, its partners of smaller ID
-// (part1 = the larger ID, as TotalEMatrix::allToAll pairs (i, j < i)).
-__global__ void k_bond_all(int n, ChainTab ct, SysConst sc, const int* __restrict__ slot, const uint4* __restrict__ P,
-                           const float4* __restrict__ O, const float2* __restrict__ Q, double* __restrict__ out) {
+// (part1 = the larger ID, as TotalEMatrix::allToAll pairs (i, j < i)); a sum
+// per block of 256 (one value per ID left k_reduce's single block 131,070 of
+// them, 30 us).
+__global__ __launch_bounds__(256) void k_bond_all(int n, ChainTab ct, SysConst sc, const int* __restrict__ slot,
+                                                  const uint4* __restrict__ P, const float4* __restrict__ O,
+                                                  const float2* __restrict__ Q, double* __restrict__ out) {
+    __shared__ double red[4];
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int a = slot[i];
-    out[i] = bonds_global(ct, sc.nt, sc.Ld, i, P[a], O[a], Q[a], 1 | 4, slot, P, O, Q);
+    double e = 0.0;
+    if (i < n) {
+        int a = slot[i];
+        e = bonds_global(ct, sc.nt, sc.Ld, i, P[a], O[a], Q[a], 1 | 4, slot, P, O, Q);
+    }
+    e = block_sum<4>(e, red);
+    if (threadIdx.x == 0) out[blockIdx.x] = e;
 }
-
-// ------------------------------------------------------------ energy (all)
-// One block of NW waves per cell; pairs (i in home cell, j in stencil) with
-// ID_j < ID_i flattened over the block's threads (wave w takes the chunks
-// w, w + NW, ...).  The cheap stage (image, cutoff, segment distance, WCA)
-// runs for every candidate; pairs inside the attraction range are queued in
-// the wave's LDS queue and evaluated 64 at a time so the branch-heavy patch
-// code runs with full lanes.  FP32 pair terms, FP64 accumulation; per-cell
-// partial sums combined in a fixed order.
-#define QCAP 128
-#define ENERGY_NW 4
 
 // the LDS writes of a wave are visible to its own later reads (a wave's LDS
 // operations complete in order; this keeps the compiler from moving them)
@@ -680,106 +677,6 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-template <int NW>
-__global__ __launch_bounds__(WAVE * NW) void k_energy_all(Grid g, SysConst sc, const int* __restrict__ starts,
-                                                          const uint4* __restrict__ P, const float4* __restrict__ O,
-                                                          const float2* __restrict__ Q, const int* __restrict__ ID,
-                                                          const PP32* __restrict__ pp, const TP32* __restrict__ tp,
-                                                          int cap, double* __restrict__ partial, int* __restrict__ flag) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    int cell = blockIdx.x;
-    int cx = cell % g.nc[0], cy = (cell / g.nc[0]) % g.nc[1], cz = cell / (g.nc[0] * g.nc[1]);
-    Stage S;
-    S.u = (uint4*)smem;
-    S.o = (float4*)(S.u + cap);
-    S.q = (float2*)(S.o + cap);
-    S.id = (int*)(S.q + cap);
-    const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1), w = tid >> 6;
-    int* sten = S.id + cap;                              // 2*125+2 ints
-    double* red = (double*)(sten + 2 * 125 + 2);         // NW doubles (8-byte aligned: cap is a multiple of 64)
-    int* queue = (int*)(red + NW) + w * 2 * QCAP;        // this wave's QCAP (hi, j) entries
-    if (starts[cell + 1] == starts[cell]) {
-        if (tid == 0) partial[cell] = 0.0;
-        return;
-    }
-    if (!stage_load<NW>(S, cap, g, cx, cy, cz, starts, P, O, Q, ID, sten)) {
-        if (tid == 0) { atomicOr(flag, 1); partial[cell] = 0.0; }
-        return;
-    }
-    int nh = S.h1 - S.h0, ns = S.n;
-    long total = (long)nh * ns;
-    double acc = 0.0;
-    int qn = 0;   // wave-uniform queue length
-    for (long base = (long)w * WAVE; base < total; base += (long)WAVE * NW) {
-        long pidx = base + lane;
-        bool need = false;
-        int hi_ = 0, j = 0;
-        if (pidx < total) {
-            hi_ = (int)(pidx / ns);
-            j = (int)(pidx - (long)hi_ * ns);
-            int i = S.h0 + hi_;
-            if (S.id[j] < S.id[i]) {
-                uint4 a = S.u[i], b = S.u[j];
-                V3<float> r = fx_image_c(a.x, a.y, a.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
-                float r2 = dot(r, r);
-                if (r2 <= sc.sqmaxcut) {
-                    const PP32& P2 = pp[a.w * sc.nt + b.w];
-                    if (P2.kind <= K_SCA && P2.kind >= 0) {
-                        DPart<float> pa, pb;
-                        pa.dir = mk<float>(S.o[i].x, S.o[i].y, S.o[i].z);
-                        pb.dir = mk<float>(S.o[j].x, S.o[j].y, S.o[j].z);
-                        pa.dir = normalised(pa.dir);
-                        pb.dir = normalised(pb.dir);
-                        float erep, d2;
-                        need = scsc_cheap(P2, pa, pb, r, erep, d2);
-                        acc += (double)erep;
-                    } else if (P2.kind == K_SPH_WCA || P2.kind == K_SPH_TAYLOR) {
-                        acc += (double)sphere_pair(P2, sqrtf(r2));
-                    } else if (P2.kind != K_NONE) {
-                        need = true;   // sphere - spherocylinder: evaluated whole in the queue
-                    }
-                }
-            }
-        }
-        unsigned long long m = __ballot(need);
-        if (need) {
-            int pos = qn + wave_prefix(m);
-            queue[2 * pos] = hi_;
-            queue[2 * pos + 1] = j;
-        }
-        qn += __popcll(m);
-        wave_lds_sync();
-        bool last = base + (long)WAVE * NW >= total;
-        if (qn >= WAVE || (last && qn > 0)) {
-            // drain whole batches of 64 (everything at the end)
-            int take = last ? qn : (qn / WAVE) * WAVE;
-            for (int e0 = 0; e0 < take; e0 += WAVE) {
-                int e = e0 + lane;
-                if (e < take) {
-                    int i = S.h0 + queue[2 * e], jj = queue[2 * e + 1];
-                    uint4 a = S.u[i], b = S.u[jj];
-                    V3<float> r = fx_image_c(a.x, a.y, a.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
-                    const PP32& P2 = pp[a.w * sc.nt + b.w];
-                    DPart<float> pa = load_part<float>(S.o[i], S.q[i], a.w, tp);
-                    DPart<float> pb = load_part<float>(S.o[jj], S.q[jj], b.w, tp);
-                    if (P2.kind <= K_SCA) acc += scsc_attr_d(P2, pa, pb, r);
-                    else acc += (double)spsc(P2, pa, pb, r);
-                }
-            }
-            wave_lds_sync();
-            int rest = qn - take;   // < 64
-            int c0 = 0, c1 = 0;
-            if (lane < rest) { c0 = queue[2 * (take + lane)]; c1 = queue[2 * (take + lane) + 1]; }
-            wave_lds_sync();
-            if (lane < rest) { queue[2 * lane] = c0; queue[2 * lane + 1] = c1; }
-            wave_lds_sync();
-            qn = rest;
-        }
-    }
-    double s = block_sum<NW>(acc, red);
-    if (tid == 0) partial[cell] = s;
-}
-
 // deterministic final reduction of per-cell partial sums
 __global__ __launch_bounds__(1024) void k_reduce(int n, const double* __restrict__ v, double* __restrict__ out) {
     __shared__ double sh[1024];
@@ -2419,12 +2316,14 @@ __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query*
 // stencil (positions, then the records of those kept), so that the records
 // lie packed behind one another.  list: cap source indices at the end of the
 // region, beyond the records (44 cap + 4 cap bytes fit the region).
+// half_stencil: only the home cell and the stencil cells behind it in their
+// order, one of each pair of opposite cells.
 template <int NW>
 __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes, int cap, const Grid& g,
                             const SysConst& sc, int cx, int cy, int cz, const int* __restrict__ starts,
                             const uint4* __restrict__ P, const float4* __restrict__ O, const float2* __restrict__ Q,
                             const int* __restrict__ ID, const ChainTab& ct, int* sten, int* misc, int16_t*& partner,
-                            size_t& used) {
+                            size_t& used, bool half_stencil = false) {
     const int ns = stencil_size(g);
     int* pre = sten;          // ns+1 prefix of counts
     int* cst = sten + ns + 1; // cell start per stencil entry
@@ -2485,7 +2384,7 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
             const V3<float> r = fx_image_c(u.x, u.y, u.z, cen[0], cen[1], cen[2], sc.Lh, sc.Ll);
             const float dx = fmaxf(fabsf(r.x) - half[0], 0.0f), dy = fmaxf(fabsf(r.y) - half[1], 0.0f),
                         dz = fmaxf(fabsf(r.z) - half[2], 0.0f);
-            keep = lo == home || dx * dx + dy * dy + dz * dz <= reach2;
+            keep = lo == home || (dx * dx + dy * dy + dz * dz <= reach2 && !(half_stencil && lo < home));
             if (!keep && ct.cw) {
                 const int id = ID[src], w = ct.cw[id];
                 for (int q = 0; q < 4; q++)
@@ -2834,6 +2733,243 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_batch_spec(const Rep
     sweep_cell_spec<DA, LT>(lb - R.blk_off, R.g, R.sc, R.mp, starts + R.cell_off, P, O, Q, ID, pp, tp, cap, ppmax,
                         nonempty + R.rep, mlp_img, mc, ct, stats + (size_t)R.rep * STAT_REP * STAT_STRIDE,
                         de_sum + (size_t)R.rep * STAT_REP * STAT_STRIDE, flag);
+}
+
+// ------------------------------------------------------------ energy (all)
+// The pairs of one cell, by a block of ENERGY_NW waves: i in the home cell, j
+// in the home cell behind i or in the half of the stencil behind it, so that
+// every pair is met once (on an axis of fewer than 2r + 1 cells, where
+// opposite cells coincide, j in the whole stencil with ID_j < ID_i).  The
+// stages of a speculative trial, on the block: stage_reach, centres of j
+// within reach of i's segment, segment distances and repulsion of those,
+// then the patch pairs in range, eight lanes each, behind side_possible where
+// they are more than one pass.  FP32 pair terms, FP64 accumulation, per-cell
+// partial sums.  The previous kernel took the segment distance of every pair
+// of the full stencil within maxcut as it met them, at 7% of its lanes: 486 us
+// for 65,536 TCHPSC, 660 us for 131,070 chain beads.
+// flag 32: the stage overflowed its estimated capacity (the caller runs it
+// again with `full_cap`, the largest); flag 1: that one did.
+#define ENERGY_NW 4
+#define ENERGY_LCAP 1024
+__device__ __forceinline__ void energy_cell(int cell, const Grid& g, const SysConst& sc, const int* __restrict__ starts,
+                                            const uint4* __restrict__ P, const float4* __restrict__ O,
+                                            const float2* __restrict__ Q, const int* __restrict__ ID,
+                                            const PP32* __restrict__ pp, const TP32* __restrict__ tp, int ppmax,
+                                            int cap, int region_bytes, bool full_cap, double* __restrict__ partial,
+                                            int* __restrict__ flag) {
+    constexpr int NW = ENERGY_NW, BS = WAVE * NW, PA = 2;
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ int sten[2 * 125 + 2], misc[16], cnt[2 * CNT_HALF], list[ENERGY_LCAP], ent[BS];
+    __shared__ uint16_t surv[4 * BS];
+    __shared__ double red[NW];
+    const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1);
+    const int cx = cell % g.nc[0], cy = (cell / g.nc[0]) % g.nc[1], cz = cell / (g.nc[0] * g.nc[1]);
+    if (starts[cell + 1] == starts[cell]) {
+        if (tid == 0) partial[cell] = 0.0;
+        return;
+    }
+    const int w = 2 * g.r + 1;
+    const bool half = g.nc[0] >= w && g.nc[1] >= w && g.nc[2] >= w;
+    Stage S;
+    int16_t* partners;
+    size_t used;
+    if (!stage_reach<NW>(S, smem, (size_t)region_bytes, cap, g, sc, cx, cy, cz, starts, P, O, Q, ID,
+                         ChainTab{nullptr, nullptr, nullptr, nullptr}, sten, misc, partners, used, half)) {
+        if (tid == 0) {
+            atomicOr(flag, full_cap ? 1 : 32);
+            partial[cell] = 0.0;
+        }
+        return;
+    }
+    const int np = ppmax > 1 ? 2 : 1, psh = ppmax > 2 ? 2 : (ppmax > 1 ? 1 : 0);
+    float* rows = (float*)(smem + used);   // of every staged particle, where they fit
+    const bool has_rows = S.n <= (int)(((size_t)region_bytes - used) / (4 * VROW));
+    if (has_rows)
+        for (int i = tid; i < np * S.n; i += BS) {
+            const int j = i / np;
+            vrow_derive(rows + (size_t)j * VROW, i - np * j, S.o[j], S.q[j], S.u[j].w, tp);
+        }
+    __syncthreads();
+    const int nh = S.h1 - S.h0, total = nh * S.n;
+    const uint32_t inv = 0xffffffffu / (uint32_t)S.n + 1u;   // e / S.n = mulhi(e, inv) for e < 2^21 (S.n <= 1408; S.n = 1: inv wraps to 0)
+    double acc = 0.0;
+    int nl = 0, par = 0;
+    for (int base = 0; base < total; base += PA * BS) {
+        bool keep[PA];
+        int pos[PA], pk[PA];
+#pragma unroll
+        for (int h = 0; h < PA; h++) {
+            const int e = min(base + h * BS + tid, total - 1);
+            const int hi = S.n == 1 ? e : (int)__umulhi((uint32_t)e, inv), j = e - hi * S.n, i = S.h0 + hi;
+            const uint4 a = S.u[i], b = S.u[j];
+            const float4 oa = S.o[i];
+            const V3<float> r = fx_image_c(a.x, a.y, a.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+            const bool mine = half ? (j >= S.h1) | (j < S.h0) | (j > i) : S.id[j] < S.id[i];
+            keep[h] = (base + h * BS + tid < total) & mine & (dot(r, r) <= sc.sqmaxcut) &
+                      (centre_dist2(mk<float>(oa.x, oa.y, oa.z), tp[a.w].hl, r) <= tp[a.w].reach2);
+            pk[h] = (i << 16) | j;
+        }
+        block_compactK<NW, PA>(keep, nl, cnt, par, pos);
+#pragma unroll
+        for (int h = 0; h < PA; h++)
+            if (keep[h]) list[pos[h]] = pk[h];
+        if (nl <= ENERGY_LCAP - PA * BS && base + PA * BS < total) continue;
+        __syncthreads();
+        for (int b0 = 0; b0 < nl; b0 += BS) {
+            bool need = false;
+            int pij = 0;
+            if (b0 + tid < nl) {
+                pij = list[b0 + tid];
+                int i = pij >> 16, j = pij & 0xffff;
+                if (S.id[j] > S.id[i]) {   // the canonical order: the higher ID as part1
+                    const int x = i;
+                    i = j;
+                    j = x;
+                    pij = (i << 16) | j;
+                }
+                const uint4 a = S.u[i], b = S.u[j];
+                const PP32& P2 = pp[a.w * sc.nt + b.w];
+                const V3<float> r = fx_image_c(a.x, a.y, a.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+                if (P2.kind <= K_SCA && P2.kind >= 0) {
+                    DPart<float> pa, pb;
+                    pa.dir = normalised(mk<float>(S.o[i].x, S.o[i].y, S.o[i].z));
+                    pb.dir = normalised(mk<float>(S.o[j].x, S.o[j].y, S.o[j].z));
+                    float ev, d2;
+                    need = scsc_cheap(P2, pa, pb, r, ev, d2);
+                    acc += (double)ev;
+                } else if (P2.kind == K_SPH_WCA || P2.kind == K_SPH_TAYLOR) {
+                    acc += (double)sphere_pair(P2, sqrtf(dot(r, r)));
+                } else if (P2.kind != K_NONE) {
+                    DPart<float> pa = load_part<float>(S.o[i], S.q[i], a.w, tp),
+                                 pb = load_part<float>(S.o[j], S.q[j], b.w, tp);
+                    acc += (double)spsc(P2, pa, pb, r);
+                }
+            }
+            int ne = 0;
+            const int ep = block_compact<NW>(need, ne, cnt);
+            if (need) ent[ep] = pij;
+            __syncthreads();
+            int items = ne << psh;
+            auto patch = [&](int it, int& i, int& j, int& k1, int& k2, V3<float>& r, bool& ok) -> const PP32* {
+                const int e = ent[it >> psh], mpp = it & ((1 << psh) - 1);
+                i = e >> 16;
+                j = e & 0xffff;
+                const uint4 a = S.u[i], b = S.u[j];
+                const PP32* P2 = pp + a.w * sc.nt + b.w;
+                r = fx_image_c(a.x, a.y, a.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
+                ok = mpp < npatch_pairs(*P2);
+                patch_pair_index(*P2, mpp, k1, k2);
+                return P2;
+            };
+            if (!has_rows) {   // too crowded for rows: patch pairs derived and searched one per lane
+                for (int it = tid; it < items; it += BS) {
+                    int i, j, k1, k2;
+                    V3<float> r;
+                    bool ok;
+                    const PP32* P2 = patch(it, i, j, k1, k2, r, ok);
+                    if (ok)
+                        acc += (double)patch_pair_v<float>(*P2, load_view<float>(S.o[i], S.q[i], S.u[i].w, tp, k1),
+                                                           load_view<float>(S.o[j], S.q[j], S.u[j].w, tp, k2), r, k1, k2);
+                }
+                items = 0;
+            }
+            const bool culled = items > BS / 8;
+            if (culled) {
+                int left = 0;
+                for (int b2 = 0; b2 < items; b2 += BS) {
+                    bool k = false;
+                    if (b2 + tid < items) {
+                        int i, j, k1, k2;
+                        V3<float> r;
+                        bool ok;
+                        const PP32* P2 = patch(b2 + tid, i, j, k1, k2, r, ok);
+                        const PatchView<float> va = vrow_view(rows + (size_t)i * VROW, k1),
+                                               vb = vrow_view(rows + (size_t)j * VROW, k2);
+                        k = ok & side_possible(va, vb.ax, r, P2->hl1, P2->pcanglsw[k1 ? 2 : 0], P2->rcutSq) &
+                            side_possible(vb, va.ax, mk<float>(-r.x, -r.y, -r.z), P2->hl0, P2->pcanglsw[k2 ? 3 : 1],
+                                          P2->rcutSq);
+                    }
+                    const int sp = block_compact<NW>(k, left, cnt);
+                    if (k) surv[sp] = (uint16_t)(b2 + tid);
+                }
+                items = left;
+                __syncthreads();
+            }
+            for (int b2 = 0; b2 < items; b2 += BS / 8) {
+                const int gi = b2 + (tid >> 3), role = lane & 3, side = (lane >> 2) & 1, gc = min(gi, items - 1);
+                int i, j, k1, k2;
+                V3<float> r;
+                bool ok;
+                const PP32* P2 = patch(culled ? surv[gc] : gc, i, j, k1, k2, r, ok);
+                const float *r1 = rows + (size_t)i * VROW + 12 * k1, *r2 = rows + (size_t)j * VROW + 12 * k2;
+                float x1, x2;
+                const bool hit = quad_intersect(row_query(*P2, r1, r2, r, k1, k2, side != 0, role & 1), role, x1, x2) & ok;
+                const float y1 = __shfl_xor(x1, 4), y2 = __shfl_xor(x2, 4);
+                const bool both = hit & (__shfl_xor(hit ? 1 : 0, 4) != 0);
+                if ((lane & 7) == 0 && gi < items && both)
+                    acc += (double)patch_atr<float>(*P2, vrow_view(r1, 0), vrow_view(r2, 0), r, k1, k2, x1, x2, y1, y2);
+            }
+            __syncthreads();
+        }
+        nl = 0;
+    }
+    const double e = block_sum<NW>(acc, red);
+    if (tid == 0) partial[cell] = e;
+}
+
+__global__ __launch_bounds__(WAVE * ENERGY_NW) void k_energy_all(Grid g, SysConst sc, const int* __restrict__ starts,
+                                                                 const uint4* __restrict__ P,
+                                                                 const float4* __restrict__ O,
+                                                                 const float2* __restrict__ Q,
+                                                                 const int* __restrict__ ID,
+                                                                 const PP32* __restrict__ pp,
+                                                                 const TP32* __restrict__ tp, int ppmax, int cap,
+                                                                 int region_bytes, bool full_cap,
+                                                                 double* __restrict__ partial, int* __restrict__ flag) {
+    energy_cell(xcd_slab_index((int)blockIdx.x, (int)gridDim.x), g, sc, starts, P, O, Q, ID, pp, tp, ppmax, cap,
+                region_bytes, full_cap, partial, flag);
+}
+
+// every cell of every replica of a batch; a block finds its replica by binary
+// search over cell_off
+__global__ __launch_bounds__(WAVE * ENERGY_NW) void k_energy_batch(const RepPass* __restrict__ rp, int nrep,
+                                                                   const int* __restrict__ starts,
+                                                                   const uint4* __restrict__ P,
+                                                                   const float4* __restrict__ O,
+                                                                   const float2* __restrict__ Q,
+                                                                   const int* __restrict__ ID,
+                                                                   const PP32* __restrict__ pp,
+                                                                   const TP32* __restrict__ tp, int ppmax, int cap,
+                                                                   int region_bytes, bool full_cap,
+                                                                   double* __restrict__ partial,
+                                                                   int* __restrict__ flag) {
+    const int b = xcd_slab_index((int)blockIdx.x, (int)gridDim.x);
+    int lo = 0, hi = nrep - 1;
+    while (lo < hi) {
+        int mid = (lo + hi + 1) >> 1;
+        if (rp[mid].cell_off <= b) lo = mid; else hi = mid - 1;
+    }
+    const int off = rp[lo].cell_off;
+    const Grid g = rp[lo].g;
+    const SysConst sc = rp[lo].sc;
+    energy_cell(b - off, g, sc, starts + off, P, O, Q, ID, pp, tp, ppmax, cap, region_bytes, full_cap, partial + off,
+                flag);
+}
+
+// k_reduce per replica of a batch: block r sums its cells' partial sums
+__global__ __launch_bounds__(1024) void k_reduce_batch(const RepPass* __restrict__ rp, int nrep, int ncell,
+                                                       const double* __restrict__ v, double* __restrict__ out) {
+    __shared__ double sh[1024];
+    const int t = threadIdx.x, r = blockIdx.x, b = rp[r].cell_off, e = r + 1 < nrep ? rp[r + 1].cell_off : ncell;
+    double s = 0.0;
+    for (int i = b + t; i < e; i += 1024) s += v[i];
+    sh[t] = s;
+    __syncthreads();
+    for (int o = 512; o > 0; o >>= 1) {
+        if (t < o) sh[t] += sh[t + o];
+        __syncthreads();
+    }
+    if (t == 0) out[r] = sh[0];
 }
 
 // cell list of a replica batch: the cell of every particle in its replica's
@@ -4801,8 +4937,7 @@ static int build_grid_w(sc_ctx* ctx, int r, const uint32_t shift[3], const doubl
 // sweep keeps a block's image under 80 KiB, so two blocks share a CU (the
 // register budget allows two waves per SIMD); a stencil holds at most
 // STAGE_CAP_MAX records (~2.5x the mean of the densest systems built here).
-// The one-wave whole-system energy kernel keeps to ENERGY_CAP_MAX records
-// (~52 KiB), so three of its blocks share a CU.
+// The whole-system energy kernel's largest stage is ENERGY_CAP_MAX records.
 #define SWEEP_LDS_BUDGET 81920
 #define STAGE_CAP_MAX 1408
 #define ENERGY_CAP_MAX 1152
@@ -4835,13 +4970,33 @@ static int stage_cap(const sc_ctx* ctx, const Grid& g, const double* box, int ca
 
 static size_t stage_bytes(int cap) { return (size_t)cap * (16 + 16 + 8 + 4); }
 
-// LDS of k_energy_all: the stage, the stencil scratch, the block sums and one
-// pair queue per wave
-static size_t energy_lds_bytes(int cap) {
-    return stage_bytes(cap) + sizeof(int) * (2 * 125 + 2) + sizeof(double) * ENERGY_NW +
-           sizeof(int) * 2 * QCAP * ENERGY_NW;
+// Stage capacity and dynamic LDS of k_energy_all for a grid: twice the mean
+// number of particles that stage_reach keeps of the half stencil (and rows for
+// 1.25 times), so that four or more blocks share a CU; `full`: the capacity the full stencil may need.
+struct EnergyLds {
+    int cap, bytes;
+};
+static EnergyLds energy_lds(int n, double reach, double minvol, const Grid& g, const double* box, bool full) {
+    const int capmax = stage_cap_n(n, minvol, g, box, ENERGY_CAP_MAX);
+    double a[3], vol = 1.0, cells = 1.0;
+    bool half = true;
+    for (int k = 0; k < 3; k++) {
+        a[k] = box[k] / g.nc[k];
+        vol *= box[k];
+        cells *= std::min(2 * g.r + 1, g.nc[k]);
+        half = half && g.nc[k] >= 2 * g.r + 1;
+    }
+    const double v = a[0] * a[1] * a[2], R = reach;
+    double near = v + 2.0 * R * (a[0] * a[1] + a[1] * a[2] + a[0] * a[2]) + 3.141592653589793 * R * R * (a[0] + a[1] + a[2]) +
+                  4.1887902047863905 * R * R * R;
+    near = std::min(near, cells * v);
+    const double mean = (double)n / vol * (half ? 0.5 * (near + v) : near);
+    EnergyLds L;
+    L.cap = full ? capmax : std::min(capmax, (((int)(2.0 * mean) + 64 + 63) / 64) * 64);
+    const int rows = std::min(L.cap, (int)(1.25 * mean) + 32);
+    L.bytes = std::min(L.cap * SPEC_STAGE_BYTES + rows * 4 * VROW, 55 * 1024);   // 64 KiB with the static part
+    return L;
 }
-
 
 // LDS for the sweep's copy of the parameter tables (with alignment slack)
 static size_t sweep_table_bytes(int nt) {
@@ -4849,12 +5004,17 @@ static size_t sweep_table_bytes(int nt) {
     return (size_t)nt * nt * sizeof(PP32) + (size_t)nt * sizeof(TP32) + 16;
 }
 
-static int check_flag(sc_ctx* ctx, const char* what) {
+// `again` set: the kernel is to be run again with its full stage (flag 32)
+static int check_flag(sc_ctx* ctx, const char* what, bool* again = nullptr) {
     int f = 0;
     HIPCK(hipMemcpyAsync(&f, ctx->d_flag, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIPCK(hipStreamSynchronize(ctx->stream));
     if (f) {
         HIPCK(hipMemset(ctx->d_flag, 0, sizeof(int)));
+        if (again && f == 32) {
+            *again = true;
+            return SC_OK;
+        }
         if (f & 4) return fail(ctx, SC_ECAPACITY, std::string(what) + ": a coarse cell held more than 4096 molecules");
         if (f & 16)
             return fail(ctx, SC_ECAPACITY, std::string(what) + ": more than 320 particles within maxcut, or 192 "
@@ -4910,25 +5070,30 @@ static int energy_all_impl(sc_ctx* ctx, const double* box, double* e) {
     int rc = energy_grid(ctx, box);
     if (rc) return rc;
     const Grid& g = ctx->g;
-    int cap = stage_cap(ctx, g, box, ENERGY_CAP_MAX);
-    size_t lds = energy_lds_bytes(cap);
     if ((rc = ensure_out(ctx, 2))) return rc;
     SysConst sc = sysconst(ctx, box);
     int c = ctx->cur;
-    HIPCK(hipEventRecord(ctx->ev0, ctx->stream));
-    hipLaunchKernelGGL(k_energy_all<ENERGY_NW>, dim3(ctx->ncell), dim3(WAVE * ENERGY_NW), lds, ctx->stream, g, sc, ctx->starts, ctx->P[c],
-                       ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, cap, ctx->partial, ctx->d_flag);
-    HIPCK(hipEventRecord(ctx->ev1, ctx->stream));
-    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, ctx->stream, ctx->ncell, ctx->partial, ctx->d_out);
     double eb[2] = {0.0, 0.0};
-    if (ctx->bonds) {   // chain bonds: FP64 per particle, its partners of smaller ID
-        hipLaunchKernelGGL(k_bond_all, dim3((ctx->n + 255) / 256), dim3(256), 0, ctx->stream, ctx->n, chain_tab(ctx),
-                           sc, ctx->slot, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_bond);
-        hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, ctx->stream, ctx->n, ctx->d_bond, ctx->d_out + 1);
+    for (int pass = 0; pass < 2; pass++) {   // again with the full stage where the estimated one overflowed
+        const EnergyLds L = energy_lds(ctx->n, ctx->reach, ctx->minvol, g, box, pass > 0);
+        HIPCK(hipEventRecord(ctx->ev0, ctx->stream));
+        hipLaunchKernelGGL(k_energy_all, dim3(ctx->ncell), dim3(WAVE * ENERGY_NW), L.bytes, ctx->stream, g, sc,
+                           ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32,
+                           ctx->ppmax, L.cap, L.bytes, pass > 0, ctx->partial, ctx->d_flag);
+        HIPCK(hipEventRecord(ctx->ev1, ctx->stream));
+        hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, ctx->stream, ctx->ncell, ctx->partial, ctx->d_out);
+        if (ctx->bonds) {   // chain bonds: FP64 per particle, its partners of smaller ID
+            hipLaunchKernelGGL(k_bond_all, dim3((ctx->n + 255) / 256), dim3(256), 0, ctx->stream, ctx->n,
+                               chain_tab(ctx), sc, ctx->slot, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_bond);
+            hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, ctx->stream, (ctx->n + 255) / 256, ctx->d_bond,
+                               ctx->d_out + 1);
+        }
+        HIPCK(hipGetLastError());
+        HIPCK(hipMemcpyAsync(eb, ctx->d_out, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        bool again = false;
+        if ((rc = check_flag(ctx, "energy_all", &again))) return rc;
+        if (!again) break;
     }
-    HIPCK(hipGetLastError());
-    HIPCK(hipMemcpyAsync(eb, ctx->d_out, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    if ((rc = check_flag(ctx, "energy_all"))) return rc;
     *e = ctx->bonds ? eb[0] + eb[1] : eb[0];
     float ms = 0;
     HIPCK(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
@@ -6788,7 +6953,8 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
 }
 
 // whole-system energy of every replica (TotalEMatrix::allToAll per replica,
-// totalenergycalculator.h:338-353): one launch per replica over its cells
+// totalenergycalculator.h:338-353): one launch over the cells of all replicas
+// (a launch per replica: 64 x 48 us for 64 replicas of 253,424 particles)
 static int sc_batch_energies_impl(sc_ctx* ctx, double* e) {
     if (!ctx || !e) return SC_EINVAL;
     if (!batch_active(ctx)) return fail(ctx, SC_ESTATE, "no replica batch (sc_batch_set)");
@@ -6796,20 +6962,39 @@ static int sc_batch_energies_impl(sc_ctx* ctx, double* e) {
     int R = ctx->nrep, rc;
     if ((rc = batch_alloc(ctx))) return rc;
     int c = ctx->cur;
-    for (int q = 0; q < R; q++) {
-        const Grid& g = ctx->rep_grid[q].g;
-        double b[3] = {ctx->rep_box[q][0], ctx->rep_box[q][1], ctx->rep_box[q][2]};
-        int cap = stage_cap_n(ctx->rep_n[q], ctx->minvol, g, b, ENERGY_CAP_MAX);
-        size_t lds = energy_lds_bytes(cap);
-        int co = ctx->rep_grid[q].cell_off, nc = ctx->rep_ncell[q];
-        SysConst sc = sysconst(ctx, b);
-        SC_LAUNCH(k_energy_all<ENERGY_NW>, dim3(nc), dim3(WAVE * ENERGY_NW), lds, ctx->stream, g, sc, ctx->starts + co, ctx->P[c], ctx->O[c],
-                  ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, cap, ctx->partial + co, ctx->d_flag);
-        SC_LAUNCH(k_reduce, dim3(1), dim3(1024), 0, ctx->stream, nc, ctx->partial + co, ctx->d_rep_e + q);
+    if (R > ctx->rp_cap) {
+        if ((rc = dalloc(ctx, &ctx->d_rp, R))) return rc;
+        ctx->rp_cap = R;
     }
-    HIPCK(hipGetLastError());
-    HIPCK(hipMemcpyAsync(e, ctx->d_rep_e, R * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    return check_flag(ctx, "batch energies");
+    std::vector<RepPass> hp(R);
+    int ncell = 0;
+    for (int q = 0; q < R; q++) {
+        hp[q].g = ctx->rep_grid[q].g;
+        hp[q].sc = sysconst_box(ctx, ctx->rep_box[q]);
+        hp[q].cell_off = ctx->rep_grid[q].cell_off;
+        ncell = std::max(ncell, ctx->rep_grid[q].cell_off + ctx->rep_ncell[q]);
+    }
+    if ((rc = pin_upload(ctx, ctx->pin_rp, ctx->d_rp, hp.data(), (size_t)R * sizeof(RepPass)))) return rc;
+    for (int pass = 0; pass < 2; pass++) {   // again with the full stage where the estimated one overflowed
+        EnergyLds L = {0, 0};
+        for (int q = 0; q < R; q++) {
+            const double b[3] = {ctx->rep_box[q][0], ctx->rep_box[q][1], ctx->rep_box[q][2]};
+            const EnergyLds l = energy_lds(ctx->rep_n[q], ctx->reach, ctx->minvol, ctx->rep_grid[q].g, b, pass > 0);
+            L.cap = std::max(L.cap, l.cap);
+            L.bytes = std::max(L.bytes, l.bytes);
+        }
+        L.bytes = std::max(L.bytes, L.cap * SPEC_STAGE_BYTES);
+        SC_LAUNCH(k_energy_batch, dim3(ncell), dim3(WAVE * ENERGY_NW), L.bytes, ctx->stream, ctx->d_rp, R, ctx->starts,
+                  ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, ctx->ppmax, L.cap, L.bytes,
+                  pass > 0, ctx->partial, ctx->d_flag);
+        SC_LAUNCH(k_reduce_batch, dim3(R), dim3(1024), 0, ctx->stream, ctx->d_rp, R, ncell, ctx->partial, ctx->d_rep_e);
+        HIPCK(hipGetLastError());
+        HIPCK(hipMemcpyAsync(e, ctx->d_rep_e, R * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+        bool again = false;
+        if ((rc = check_flag(ctx, "batch energies", &again))) return rc;
+        if (!again) break;
+    }
+    return SC_OK;
 }
 
 // One replica-exchange step (MoveCreator::replicaExchangeMove,
