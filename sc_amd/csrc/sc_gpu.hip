@@ -3079,109 +3079,88 @@ __global__ void k_mlp_gen(long ns, uint32_t key0, uint32_t key1, const PP32* __r
 
 // ------------------------------------------------------------- training
 // One training step is two launches.  k_mlp_fwdbwd: each block takes TR_S
-// samples through the forward pass and back, with the weights and every
-// activation in LDS, and writes its share of the gradient (and of the
-// squared error) to its own row of `part`.  k_mlp_reduce_adam sums the rows
-// in a fixed order (the gradient is deterministic) and takes the Adam step.
-// FP32 throughout.  The hidden weight matrices sit in LDS with a row stride
-// of 65 floats, so the backward pass, whose lanes walk down a column, hits
-// 64 different banks.  Eight waves per block (two per SIMD) hide the LDS
-// latency; lane j of wave w owns column j of rows w, w + 8, ...
+// samples through the forward pass and back and writes its share of the
+// gradient (and of the squared error) to its own row of `part`.
+// k_mlp_reduce_adam sums the rows in a fixed order (the gradient is
+// deterministic) and takes the Adam step.  FP32 throughout.
+//
+// Every product of the step is a 16-sample or 16-unit tile of
+// v_mfma_f32_16x16x4_f32 (FP32 operands and accumulation; D[i][j] += sum_k
+// A[i][k] B[k][j], lane l holding A[l%16][l/16], B[l/16][l%16] and
+// D[4 (l/16) + r][l%16]).  Wave (mb, cb) = (w & 1, w >> 1) owns samples
+// 16 mb .. and units 16 cb .. of every layer: its pre-activations stay in
+// registers from the forward pass to the backward one, its columns of the
+// weights come from L2 straight into registers, once.  The order of a
+// product's K index is free as long as both operands share it: with k = 16 (l/16)
+// + step a lane's A values are 16 consecutive floats of an activation row
+// (four 16-byte LDS reads).  The vector version read an LDS operand per
+// multiply-add or two and was bound by that: 22.5 us per step of 4,096 samples.
 #define TR_S 32
 #define TR_NW 8
-#define TR_WS 65
-constexpr int TL_W1 = 0, TL_B1 = TL_W1 + MLP_NF * MLP_NH, TL_W2 = TL_B1 + MLP_NH, TL_B2 = TL_W2 + MLP_NH * TR_WS,
-              TL_W3 = TL_B2 + MLP_NH, TL_B3 = TL_W3 + MLP_NH * TR_WS, TL_W4 = TL_B3 + MLP_NH, TL_B4 = TL_W4 + MLP_NH,
-              TL_X = TL_B4 + 4, TL_Z1 = TL_X + TR_S * MLP_NF, TL_H1 = TL_Z1 + TR_S * MLP_NH,
-              TL_Z2 = TL_H1 + TR_S * MLP_NH, TL_H2 = TL_Z2 + TR_S * MLP_NH, TL_Z3 = TL_H2 + TR_S * MLP_NH,
-              TL_H3 = TL_Z3 + TR_S * MLP_NH, TL_DO = TL_H3 + TR_S * MLP_NH, TL_LS = TL_DO + TR_S,
-              TL_END = TL_LS + TR_NW;
+#define TR_AS 68   // row stride of an activation array: the four lane groups' rows on different banks
+constexpr int TL_X = 0, TL_XS = 20, TL_H1 = TL_X + TR_S * TL_XS, TL_H2 = TL_H1 + TR_S * TR_AS,
+              TL_D3 = TL_H2 + TR_S * TR_AS, TL_D2 = TL_D3 + TR_S * TR_AS, TL_D1 = TL_D2 + TR_S * TR_AS,
+              TL_O = TL_D1 + TR_S * TR_AS, TL_Y = TL_O + 4 * TR_S, TL_DO = TL_Y + TR_S, TL_W4 = TL_DO + TR_S,
+              TL_END = TL_W4 + 2 * MLP_NH;
 constexpr size_t TRAIN_LDS_BYTES = sizeof(float) * TL_END;
 // a block's row of `part`: the gradient, then its sum of squared errors (rows 256-byte aligned)
 constexpr int TR_PART = ((MLP_NPARAM + 1 + 63) / 64) * 64;
-constexpr int TR_ROWS = TR_S / TR_NW;   // sample rows per thread
 
-// z = b + in W (K inputs, W row stride ws), h = SiLU(z), for the block's TR_S
-// x 64 outputs; the inputs of a row are read four at a time (K a multiple
-// of 4, rows 16-byte aligned)
-template <int K>
-__device__ __forceinline__ void tr_dense(const float* in, const float* w, int ws, const float* b, float* z, float* h) {
-    int tid = (int)threadIdx.x, j = tid & 63, s0 = tid >> 6;
-    float acc[TR_ROWS];
-#pragma unroll
-    for (int r = 0; r < TR_ROWS; r++) acc[r] = b[j];
-    for (int k = 0; k < K; k += 4) {
-        float w0 = w[k * ws + j], w1 = w[(k + 1) * ws + j], w2 = w[(k + 2) * ws + j], w3 = w[(k + 3) * ws + j];
-#pragma unroll
-        for (int r = 0; r < TR_ROWS; r++) {
-            float4 x = *(const float4*)&in[(s0 + TR_NW * r) * K + k];
-            acc[r] += x.x * w0 + x.y * w1 + x.z * w2 + x.w * w3;
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < TR_ROWS; r++) {
-        z[(s0 + TR_NW * r) * MLP_NH + j] = acc[r];
-        h[(s0 + TR_NW * r) * MLP_NH + j] = silu(acc[r]);
-    }
+__device__ __forceinline__ floatx4 mfma_f32(float a, float b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// dZprev = (dZ W^T) * SiLU'(Zprev), in place over Zprev; lane k = tid & 63
-__device__ __forceinline__ void tr_back(const float* dz, const float* w, float* zprev) {
-    int tid = (int)threadIdx.x, k = tid & 63, s0 = tid >> 6;
-    float acc[TR_ROWS];
+// the wave's 16 x 16 tile of (16 rows of act, 64 wide) x (its 64 x 16 operand b): two chains of eight
+__device__ __forceinline__ floatx4 tr_tile(const float* act, int mb, int lane, const float* b, floatx4 c) {
+    const float4* a = (const float4*)(act + (16 * mb + (lane & 15)) * TR_AS + 16 * (lane >> 4));
+    floatx4 d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int r = 0; r < TR_ROWS; r++) acc[r] = 0.0f;
-    for (int j = 0; j < MLP_NH; j += 4) {
-        float w0 = w[k * TR_WS + j], w1 = w[k * TR_WS + j + 1], w2 = w[k * TR_WS + j + 2], w3 = w[k * TR_WS + j + 3];
-#pragma unroll
-        for (int r = 0; r < TR_ROWS; r++) {
-            float4 d = *(const float4*)&dz[(s0 + TR_NW * r) * MLP_NH + j];
-            acc[r] += d.x * w0 + d.y * w1 + d.z * w2 + d.w * w3;
-        }
+    for (int q = 0; q < 4; q++) {
+        const float4 v = a[q];
+        c = mfma_f32(v.x, b[4 * q], c);
+        d = mfma_f32(v.y, b[4 * q + 1], d);
+        c = mfma_f32(v.z, b[4 * q + 2], c);
+        d = mfma_f32(v.w, b[4 * q + 3], d);
     }
-#pragma unroll
-    for (int r = 0; r < TR_ROWS; r++) {
-        float& zp = zprev[(s0 + TR_NW * r) * MLP_NH + k];
-        zp = acc[r] * silu_grad(zp);
-    }
+    return c + d;
 }
 
-// gradient block dW[k][j] = sum_s in[s][k] dz[s][j] (K rows) and db[j] =
-// sum_s dz[s][j]: lane j; wave w takes rows w R ... w R + R - 1 (read four
-// at a time) when K is a multiple of 32, else rows w, w + 8, ...
-template <int K>
-__device__ __forceinline__ void tr_grad(const float* in, const float* dz, float* out_w, float* out_b) {
-    int tid = (int)threadIdx.x, j = tid & 63, wv = tid >> 6;
-    constexpr bool blocked = K % (4 * TR_NW) == 0;
-    constexpr int R = blocked ? K / TR_NW : (K + TR_NW - 1) / TR_NW;
-    float acc[R];
+// the wave's tile (samples 16 mb + 4 (l/16) + r, unit 16 cb + l%16) to an activation array
+__device__ __forceinline__ void tr_put(float* act, int mb, int cb, int lane, const floatx4& v) {
 #pragma unroll
-    for (int i = 0; i < R; i++) acc[i] = 0.0f;
-    float bs = 0.0f;
-    for (int s = 0; s < TR_S; s++) {
-        float d = dz[s * MLP_NH + j];
-        bs += d;
-        if constexpr (blocked) {
+    for (int r = 0; r < 4; r++) act[(16 * mb + 4 * (lane >> 4) + r) * TR_AS + 16 * cb + (lane & 15)] = v[r];
+}
+
+// gradient tiles dW[k][j] = sum_s in[s][k] dz[s][j] of rows k in [16 kb, 16 kb + 16) and columns 16 jb .. of `nj`
+// tiles, and with ONES (in = 1) the bias row alone
+template <bool ONES>
+__device__ __forceinline__ floatx4 tr_grad(const float* in, int istride, const float* dz, int kb, int jb, int lane) {
+    floatx4 c = {0.0f, 0.0f, 0.0f, 0.0f}, d = c;
 #pragma unroll
-            for (int i = 0; i < R; i += 4) {
-                float4 x = *(const float4*)&in[s * K + wv * R + i];
-                acc[i] += x.x * d;
-                acc[i + 1] += x.y * d;
-                acc[i + 2] += x.z * d;
-                acc[i + 3] += x.w * d;
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < R; i++)
-                if (wv + TR_NW * i < K) acc[i] += in[s * K + wv + TR_NW * i] * d;
-        }
+    for (int q = 0; q < TR_S / 4; q += 2) {
+        const int s0 = 4 * q + (lane >> 4), s1 = s0 + 4;
+        c = mfma_f32(ONES ? 1.0f : in[s0 * istride + 16 * kb + (lane & 15)], dz[s0 * TR_AS + 16 * jb + (lane & 15)], c);
+        d = mfma_f32(ONES ? 1.0f : in[s1 * istride + 16 * kb + (lane & 15)], dz[s1 * TR_AS + 16 * jb + (lane & 15)], d);
     }
+    return c + d;
+}
+
+// the two 64 x 64 gradient tiles of a wave (row block w >> 1, column blocks 2 (w & 1), + 1) and the bias
+// (waves 0-3, a column block each)
+__device__ __forceinline__ void tr_grad_hidden(const float* in, const float* dz, int w, int lane, float* out_w,
+                                               float* out_b) {
+    const int kb = w >> 1;
 #pragma unroll
-    for (int i = 0; i < R; i++) {
-        int k = blocked ? wv * R + i : wv + TR_NW * i;
-        if (k < K) out_w[k * MLP_NH + j] = acc[i];
+    for (int q = 0; q < 2; q++) {
+        const int jb = 2 * (w & 1) + q;
+        const floatx4 g = tr_grad<false>(in, TR_AS, dz, kb, jb, lane);
+#pragma unroll
+        for (int r = 0; r < 4; r++) out_w[(16 * kb + 4 * (lane >> 4) + r) * MLP_NH + 16 * jb + (lane & 15)] = g[r];
     }
-    if (wv == 0) out_b[j] = bs;
+    if (w < 4) {
+        const floatx4 g = tr_grad<true>(in, TR_AS, dz, 0, w, lane);
+        if (lane < 16) out_b[16 * w + lane] = g[0];
+    }
 }
 
 __device__ __forceinline__ long tr_row(long a, long b, long n, int i) {
@@ -3194,85 +3173,121 @@ __global__ __launch_bounds__(WAVE * TR_NW) void k_mlp_fwdbwd(int B, long n, long
                                                              const float* __restrict__ X, const float* __restrict__ Y,
                                                              const float* __restrict__ W, float* __restrict__ part) {
     extern __shared__ __align__(16) float sm[];
-    constexpr int NT = WAVE * TR_NW;
-    const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = (int)threadIdx.x, lane = tid & 63, w = tid >> 6, mb = w & 1, cb = w >> 1;
+    const int l16 = lane & 15, g = lane >> 4, u = 16 * cb + l16;   // the lane's unit
     const int s0 = blockIdx.x * TR_S, ns = min(TR_S, B - s0);
-    // weights (hidden matrices to the padded stride)
-    for (int i = tid; i < MLP_NF * MLP_NH + MLP_NH; i += NT) sm[TL_W1 + i] = W[MLP_OFF_W1 + i];
-    for (int i = tid; i < MLP_NH * MLP_NH; i += NT) {
-        int k = i >> 6, j = i & 63;
-        sm[TL_W2 + k * TR_WS + j] = W[MLP_OFF_W2 + i];
-        sm[TL_W3 + k * TR_WS + j] = W[MLP_OFF_W3 + i];
-    }
-    if (tid < MLP_NH) {
-        sm[TL_B2 + tid] = W[MLP_OFF_B2 + tid];
-        sm[TL_B3 + tid] = W[MLP_OFF_B3 + tid];
-        sm[TL_W4 + tid] = W[MLP_OFF_W4 + tid];
-    }
-    if (tid == 0) sm[TL_B4] = W[MLP_OFF_B4];
-    // samples (rows past the batch are zero and carry no error)
-    for (int i = tid; i < TR_S * MLP_NF; i += NT) {
-        int s = i / MLP_NF, q = i - s * MLP_NF;
-        sm[TL_X + i] = s < ns ? X[tr_row(a, b, n, s0 + s) * MLP_NF + q] : 0.0f;
-    }
-    __syncthreads();
-    tr_dense<MLP_NF>(sm + TL_X, sm + TL_W1, MLP_NH, sm + TL_B1, sm + TL_Z1, sm + TL_H1);
-    __syncthreads();
-    tr_dense<MLP_NH>(sm + TL_H1, sm + TL_W2, TR_WS, sm + TL_B2, sm + TL_Z2, sm + TL_H2);
-    __syncthreads();
-    tr_dense<MLP_NH>(sm + TL_H2, sm + TL_W3, TR_WS, sm + TL_B3, sm + TL_Z3, sm + TL_H3);
-    __syncthreads();
-    // output layer and error: wave w takes rows w, w + 8, ..., its lanes
-    // split the dot product over the 64 units
-    float l = 0.0f;
-    for (int s = wv; s < TR_S; s += TR_NW) {
-        float o = sm[TL_H3 + s * MLP_NH + lane] * sm[TL_W4 + lane];
-#pragma unroll
-        for (int o2 = 32; o2 >= 1; o2 >>= 1) o += __shfl_xor(o, o2, WAVE);
-        if (lane == 0) {
-            float e = s < ns ? o + sm[TL_B4] - Y[tr_row(a, b, n, s0 + s)] : 0.0f;
-            sm[TL_DO + s] = 2.0f * e / (float)B;
-            l += e * e;
-        }
-    }
-    if (lane == 0) sm[TL_LS + wv] = l;
-    __syncthreads();
-    float* prow = part + (size_t)blockIdx.x * TR_PART;
-    if (tid == 0) {
-        float ls = 0.0f;
-#pragma unroll
-        for (int k = 0; k < TR_NW; k++) ls += sm[TL_LS + k];
-        prow[MLP_NPARAM] = ls;
-    }
-    {   // dZ3 = dOut w4 SiLU'(Z3), in place
-        int j = lane;
-        for (int s = wv; s < TR_S; s += TR_NW) {
-            float& z = sm[TL_Z3 + s * MLP_NH + j];
-            z = sm[TL_DO + s] * sm[TL_W4 + j] * silu_grad(z);
-        }
-    }
-    // gradient of the output layer (wave 0): four independent sums per lane
-    if (wv == 0) {
-        float g[4] = {0.0f, 0.0f, 0.0f, 0.0f}, gb = 0.0f;
-        for (int s = 0; s < TR_S; s += 4) {
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                float d = sm[TL_DO + s + q];
-                g[q] += sm[TL_H3 + (s + q) * MLP_NH + lane] * d;
-                gb += d;
+    // samples (rows past the batch are zero and carry no error); feature 12 is 1: the first layer's bias
+    if (tid < 4 * TR_S) {
+        const int s = tid >> 2, q = tid & 3;
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (s < ns) {
+            const long row = tr_row(a, b, n, s0 + s);
+            if (q < 3) {
+                v = *(const float4*)(X + row * MLP_NF + 4 * q);
+            } else {
+                v.x = 1.0f;
+                sm[TL_Y + s] = Y[row];
             }
         }
-        prow[MLP_OFF_W4 + lane] = (g[0] + g[1]) + (g[2] + g[3]);
-        if (lane == 0) prow[MLP_OFF_B4] = gb;
+        *(float4*)&sm[TL_X + s * TL_XS + 4 * q] = v;
+    }
+    // the wave's operands: its 16 columns of each weight matrix, and for the way
+    // back the same rows' transposes (unit u of the layer below as the column)
+    float w1[4], w2[16], w3[16], t2[16], t3[16];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int k = 4 * g + q;
+        w1[q] = k < MLP_NF ? W[MLP_OFF_W1 + k * MLP_NH + u] : (k == MLP_NF ? W[MLP_OFF_B1 + u] : 0.0f);
+    }
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        w2[q] = W[MLP_OFF_W2 + (16 * g + q) * MLP_NH + u];
+        w3[q] = W[MLP_OFF_W3 + (16 * g + q) * MLP_NH + u];
+        t2[q] = W[MLP_OFF_W2 + u * MLP_NH + 16 * g + q];
+        t3[q] = W[MLP_OFF_W3 + u * MLP_NH + 16 * g + q];
+    }
+    const float b2 = W[MLP_OFF_B2 + u], b3 = W[MLP_OFF_B3 + u], w4 = W[MLP_OFF_W4 + u], b4 = W[MLP_OFF_B4];
+    __syncthreads();
+    floatx4 z1 = {0.0f, 0.0f, 0.0f, 0.0f}, h;
+    {
+        const float4 v = *(const float4*)&sm[TL_X + (16 * mb + l16) * TL_XS + 4 * g];
+        z1 = mfma_f32(v.x, w1[0], z1);
+        z1 = mfma_f32(v.y, w1[1], z1);
+        z1 = mfma_f32(v.z, w1[2], z1);
+        z1 = mfma_f32(v.w, w1[3], z1);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) h[r] = silu(z1[r]);
+    tr_put(sm + TL_H1, mb, cb, lane, h);
+    __syncthreads();
+    const floatx4 z2 = tr_tile(sm + TL_H1, mb, lane, w2, floatx4{b2, b2, b2, b2});
+#pragma unroll
+    for (int r = 0; r < 4; r++) h[r] = silu(z2[r]);
+    tr_put(sm + TL_H2, mb, cb, lane, h);
+    __syncthreads();
+    const floatx4 z3 = tr_tile(sm + TL_H2, mb, lane, w3, floatx4{b3, b3, b3, b3});
+    // output layer: the wave's 16 units' share per sample (a row of 16 lanes), then the four waves'
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        h[r] = silu(z3[r]);
+        float o = h[r] * w4;
+#pragma unroll
+        for (int x = 8; x >= 1; x >>= 1) o += __shfl_xor(o, x, WAVE);
+        if (l16 == 0) sm[TL_O + cb * TR_S + 16 * mb + 4 * g + r] = o;
     }
     __syncthreads();
-    tr_grad<MLP_NH>(sm + TL_H2, sm + TL_Z3, prow + MLP_OFF_W3, prow + MLP_OFF_B3);
-    tr_back(sm + TL_Z3, sm + TL_W3, sm + TL_Z2);   // Z2 <- dZ2
+    float* prow = part + (size_t)blockIdx.x * TR_PART;
+    floatx4 dz;
+    float gw4 = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int s = 16 * mb + 4 * g + r;
+        const float o = (sm[TL_O + s] + sm[TL_O + TR_S + s]) + (sm[TL_O + 2 * TR_S + s] + sm[TL_O + 3 * TR_S + s]);
+        const float e = s < ns ? o + b4 - sm[TL_Y + s] : 0.0f, d = 2.0f * e / (float)B;
+        if (cb == 0 && l16 == 0) sm[TL_DO + s] = e;
+        dz[r] = d * w4 * silu_grad(z3[r]);
+        gw4 += h[r] * d;
+    }
+    gw4 += __shfl_xor(gw4, 16, WAVE);
+    gw4 += __shfl_xor(gw4, 32, WAVE);
+    if (lane < 16) sm[TL_W4 + mb * MLP_NH + u] = gw4;
+    tr_put(sm + TL_D3, mb, cb, lane, dz);
     __syncthreads();
-    tr_grad<MLP_NH>(sm + TL_H1, sm + TL_Z2, prow + MLP_OFF_W2, prow + MLP_OFF_B2);
-    tr_back(sm + TL_Z2, sm + TL_W2, sm + TL_Z1);   // Z1 <- dZ1
+    if (tid < MLP_NH) prow[MLP_OFF_W4 + tid] = sm[TL_W4 + tid] + sm[TL_W4 + MLP_NH + tid];
+    if (w == 1) {   // squared error and the output bias
+        const float e = lane < TR_S ? sm[TL_DO + lane] : 0.0f;
+        float l = e * e, d = 2.0f * e / (float)B;
+#pragma unroll
+        for (int x = 32; x >= 1; x >>= 1) {
+            l += __shfl_xor(l, x, WAVE);
+            d += __shfl_xor(d, x, WAVE);
+        }
+        if (lane == 0) {
+            prow[MLP_NPARAM] = l;
+            prow[MLP_OFF_B4] = d;
+        }
+    }
+    dz = tr_tile(sm + TL_D3, mb, lane, t3, floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+    for (int r = 0; r < 4; r++) dz[r] *= silu_grad(z2[r]);
+    tr_put(sm + TL_D2, mb, cb, lane, dz);
+    tr_grad_hidden(sm + TL_H2, sm + TL_D3, w, lane, prow + MLP_OFF_W3, prow + MLP_OFF_B3);
     __syncthreads();
-    tr_grad<MLP_NF>(sm + TL_X, sm + TL_Z1, prow + MLP_OFF_W1, prow + MLP_OFF_B1);
+    dz = tr_tile(sm + TL_D2, mb, lane, t2, floatx4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+    for (int r = 0; r < 4; r++) dz[r] *= silu_grad(z1[r]);
+    tr_put(sm + TL_D1, mb, cb, lane, dz);
+    tr_grad_hidden(sm + TL_H1, sm + TL_D2, w, lane, prow + MLP_OFF_W2, prow + MLP_OFF_B2);
+    __syncthreads();
+    if (w < 4) {   // the first layer's rows and, at feature 12, its bias: they follow each other in the vector
+        static_assert(MLP_OFF_B1 == MLP_OFF_W1 + MLP_NF * MLP_NH, "bias after the weights");
+        const floatx4 q = tr_grad<false>(sm + TL_X, TL_XS, sm + TL_D1, 0, w, lane);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int k = 4 * g + r;
+            if (k <= MLP_NF) prow[MLP_OFF_W1 + k * MLP_NH + 16 * w + l16] = q[r];
+        }
+    }
 }
 
 // g[p] = sum of the blocks' rows; with lr > 0 also the Adam step; the squared
@@ -3349,17 +3364,70 @@ __global__ void k_mlp_pack(const float* __restrict__ W, unsigned char* __restric
     if (t == 0) { C[192] = W[MLP_OFF_B4]; C[193] = C[194] = C[195] = 0.0f; }
 }
 
-// batched inference: one wave per tile of 16 feature rows; bf16 != 0 uses the
-// MFMA tile (the sweep's path), otherwise the FP32 per-sample forward
+// batched inference in FP32: tiles of TR_S rows on the training step's MFMA
+// forward pass, a block going through the tiles b, b + gridDim.x, ... with its
+// operands in registers.  A row per lane out of private arrays took 210 us for
+// 100,003 rows.
+__global__ __launch_bounds__(WAVE * TR_NW) void k_mlp_forward(int m, const float* __restrict__ X,
+                                                              const float* __restrict__ W, float* __restrict__ out) {
+    __shared__ __align__(16) float x[TR_S * TL_XS], h1[TR_S * TR_AS], h2[TR_S * TR_AS], po[4 * TR_S];
+    const int tid = (int)threadIdx.x, lane = tid & 63, w = tid >> 6, mb = w & 1, cb = w >> 1;
+    const int l16 = lane & 15, g = lane >> 4, u = 16 * cb + l16;
+    float w1[4], w2[16], w3[16];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int k = 4 * g + q;
+        w1[q] = k < MLP_NF ? W[MLP_OFF_W1 + k * MLP_NH + u] : (k == MLP_NF ? W[MLP_OFF_B1 + u] : 0.0f);
+    }
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        w2[q] = W[MLP_OFF_W2 + (16 * g + q) * MLP_NH + u];
+        w3[q] = W[MLP_OFF_W3 + (16 * g + q) * MLP_NH + u];
+    }
+    const float b2 = W[MLP_OFF_B2 + u], b3 = W[MLP_OFF_B3 + u], w4 = W[MLP_OFF_W4 + u], b4 = W[MLP_OFF_B4];
+    for (int s0 = blockIdx.x * TR_S; s0 < m; s0 += gridDim.x * TR_S) {
+        if (tid < 4 * TR_S) {
+            const int s = tid >> 2, q = tid & 3;
+            float4 v = make_float4(q == 3 ? 1.0f : 0.0f, 0.0f, 0.0f, 0.0f);
+            if (q < 3 && s0 + s < m) v = *(const float4*)(X + (size_t)(s0 + s) * MLP_NF + 4 * q);
+            *(float4*)&x[s * TL_XS + 4 * q] = v;
+        }
+        __syncthreads();
+        floatx4 z = {0.0f, 0.0f, 0.0f, 0.0f}, h;
+        const float4 v = *(const float4*)&x[(16 * mb + l16) * TL_XS + 4 * g];
+        z = mfma_f32(v.x, w1[0], z);
+        z = mfma_f32(v.y, w1[1], z);
+        z = mfma_f32(v.z, w1[2], z);
+        z = mfma_f32(v.w, w1[3], z);
+#pragma unroll
+        for (int r = 0; r < 4; r++) h[r] = silu(z[r]);
+        tr_put(h1, mb, cb, lane, h);
+        __syncthreads();
+        z = tr_tile(h1, mb, lane, w2, floatx4{b2, b2, b2, b2});
+#pragma unroll
+        for (int r = 0; r < 4; r++) h[r] = silu(z[r]);
+        tr_put(h2, mb, cb, lane, h);
+        __syncthreads();
+        z = tr_tile(h2, mb, lane, w3, floatx4{b3, b3, b3, b3});
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float o = silu(z[r]) * w4;
+#pragma unroll
+            for (int k = 8; k >= 1; k >>= 1) o += __shfl_xor(o, k, WAVE);
+            if (l16 == 0) po[cb * TR_S + 16 * mb + 4 * g + r] = o;
+        }
+        __syncthreads();
+        if (tid < TR_S && s0 + tid < m)
+            out[s0 + tid] = ((po[tid] + po[TR_S + tid]) + (po[2 * TR_S + tid] + po[3 * TR_S + tid])) + b4;
+    }
+}
+
+// batched inference on the sweep's BF16 MFMA tile: one wave per tile of 16 feature rows
 __global__ __launch_bounds__(WAVE) void k_mlp_infer(int m, const float* __restrict__ X, const unsigned char* __restrict__ img,
-                                                    const float* __restrict__ W, int bf16, float* __restrict__ out) {
+                                                    float* __restrict__ out) {
     extern __shared__ __align__(16) unsigned char smem[];
     int lane = lane_id();
     int row = blockIdx.x * MLP_TILE + (lane & (MLP_TILE - 1));
-    if (!bf16) {
-        if (lane < MLP_TILE && row < m) out[row] = mlp_forward_f32(W, X + (long)row * MLP_NF);
-        return;
-    }
     MlpRegs R;
     float* cst = (float*)smem;
     mlp_setup(img, cst, lane, R);
@@ -7474,19 +7542,15 @@ static int sc_mlp_train_impl(sc_ctx* ctx, int epochs, int batch, double lr, doub
     if (val_rmse) {
         *val_rmse = 0.0;
         if (nval > 0) {
-            std::vector<float> xv((size_t)nval * MLP_NF), yv(nval), ov(nval);
-            HIPCK(hipMemcpy(xv.data(), ctx->tr_x + ntr * MLP_NF, xv.size() * sizeof(float), hipMemcpyDeviceToHost));
-            HIPCK(hipMemcpy(yv.data(), ctx->tr_y + ntr, nval * sizeof(float), hipMemcpyDeviceToHost));
-            float* dx = nullptr;
+            std::vector<float> yv(nval), ov(nval);   // (the rows are on the device)
             float* dout = nullptr;
-            HIPCK(hipMalloc((void**)&dx, xv.size() * sizeof(float)));
             HIPCK(hipMalloc((void**)&dout, nval * sizeof(float)));
-            HIPCK(hipMemcpy(dx, xv.data(), xv.size() * sizeof(float), hipMemcpyHostToDevice));
             SC_LAUNCH(k_mlp_infer, dim3((unsigned)((nval + MLP_TILE - 1) / MLP_TILE)), dim3(WAVE), MLP_LDS_BYTES, ctx->stream,
-                               (int)nval, dx, ctx->mlp_img, ctx->mlp_w, 1, dout);
+                               (int)nval, ctx->tr_x + ntr * MLP_NF, ctx->mlp_img, dout);
             hipError_t e = hipGetLastError();
-            if (e == hipSuccess) e = hipMemcpy(ov.data(), dout, nval * sizeof(float), hipMemcpyDeviceToHost);
-            hipFree(dx);
+            if (e == hipSuccess) e = hipMemcpyAsync(ov.data(), dout, nval * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
+            if (e == hipSuccess) e = hipMemcpyAsync(yv.data(), ctx->tr_y + ntr, nval * sizeof(float), hipMemcpyDeviceToHost, ctx->stream);
+            if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
             hipFree(dout);
             if (e != hipSuccess) return fail(ctx, SC_EHIP, hipGetErrorString(e));
             double ss = 0;
@@ -7512,8 +7576,12 @@ static int sc_mlp_forward_impl(sc_ctx* ctx, int m, const float* x, float* out, i
     if (hipMalloc((void**)&dout, (size_t)m * sizeof(float)) != hipSuccess) { hipFree(dx); return fail(ctx, SC_EHIP, "alloc"); }
     hipError_t e = hipMemcpy(dx, x, (size_t)m * MLP_NF * sizeof(float), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        SC_LAUNCH(k_mlp_infer, dim3((m + MLP_TILE - 1) / MLP_TILE), dim3(WAVE), bf16 ? MLP_LDS_BYTES : 0, ctx->stream, m, dx,
-                           ctx->mlp_img, ctx->mlp_w, bf16, dout);
+        if (bf16)
+            SC_LAUNCH(k_mlp_infer, dim3((m + MLP_TILE - 1) / MLP_TILE), dim3(WAVE), MLP_LDS_BYTES, ctx->stream, m, dx,
+                      ctx->mlp_img, dout);
+        else   // two blocks per CU go through the tiles
+            SC_LAUNCH(k_mlp_forward, dim3(std::min((m + TR_S - 1) / TR_S, 512)), dim3(WAVE * TR_NW), 0, ctx->stream, m,
+                      dx, ctx->mlp_w, dout);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpy(out, dout, (size_t)m * sizeof(float), hipMemcpyDeviceToHost);

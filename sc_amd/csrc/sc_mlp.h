@@ -81,27 +81,6 @@ SC_HD void mlp_features(const V3<float>& adir, const V3<float>& apd, const V3<fl
     f[11] = w;
 }
 
-// FP32 forward of one sample (reference path for tests and training)
-SC_HD float mlp_forward_f32(const float* W, const float* x) {
-    float h1[MLP_NH], h2[MLP_NH];
-    for (int n = 0; n < MLP_NH; n++) {
-        float z = W[MLP_OFF_B1 + n];
-        for (int k = 0; k < MLP_NF; k++) z += x[k] * W[MLP_OFF_W1 + k * MLP_NH + n];
-        h1[n] = silu(z);
-    }
-    for (int n = 0; n < MLP_NH; n++) {
-        float z = W[MLP_OFF_B2 + n];
-        for (int k = 0; k < MLP_NH; k++) z += h1[k] * W[MLP_OFF_W2 + k * MLP_NH + n];
-        h2[n] = silu(z);
-    }
-    float out = W[MLP_OFF_B4];
-    for (int n = 0; n < MLP_NH; n++) {
-        float z = W[MLP_OFF_B3 + n];
-        for (int k = 0; k < MLP_NH; k++) z += h2[k] * W[MLP_OFF_W3 + k * MLP_NH + n];
-        out += silu(z) * W[MLP_OFF_W4 + n];
-    }
-    return out;
-}
 
 // ---------------------------------------------------------------- MFMA tile
 // Inference runs the transposed product H^T = W^T X^T on
