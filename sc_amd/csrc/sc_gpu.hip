@@ -769,6 +769,7 @@ __global__ void k_overlap(int m, const int* __restrict__ pi, const int* __restri
 // ------------------------------------------------------------------- sweep
 struct MoveParams {
     float transmx, rot_half;
+    float fx[3];                 // fixed-point units per unit of length, 2^32 / box edge, correctly rounded
     double temper;
     uint32_t key0, key1;
     uint32_t pass_lo, pass_hi;   // global pass counter
@@ -1213,22 +1214,24 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
 // pass, stream), streams 0 (particle, move kind, translation), 1 (rotation),
 // 2 (final and first-screen uniforms); the second screen's uniform uses
 // stream 2 with the trial's top bit set.
+// home: the home cell's records, the first of them particle h0.
 template <int DA>
-__device__ __forceinline__ TrialRec draw_trial(U4 ctr, int tt, const MoveParams& mp, const Stage& S, int nh,
-                                               const TP32* __restrict__ tp, float Lx, float Ly, float Lz) {
+__device__ __forceinline__ TrialRec draw_trial(U4 ctr, int tt, const MoveParams& mp, const uint4* home, int h0, int nh,
+                                               const TP32* __restrict__ tp) {
     U4 c = ctr;
     c.x = (uint32_t)tt;
     c.w = mp.pass_hi << 2;
     U4 ra = philox(c, mp.key0, mp.key1);
     TrialRec R;
-    R.k = S.h0 + (int)(((uint64_t)ra.x * (uint64_t)nh) >> 32);
-    int g0 = tp[S.u[R.k].w].geotype;
+    const int ik = (int)(((uint64_t)ra.x * (uint64_t)nh) >> 32);
+    R.k = h0 + ik;
+    int g0 = tp[home[ik].w].geotype;
     R.translate = (u01f(ra.y) < 0.5f) || (g0 >= 30);
     if (R.translate) {
         V3<float> d = unit_from(u01f(ra.z), u01f(ra.w));
-        R.w[0] = (int32_t)rintf(d.x * mp.transmx * (4294967296.0f / Lx));
-        R.w[1] = (int32_t)rintf(d.y * mp.transmx * (4294967296.0f / Ly));
-        R.w[2] = (int32_t)rintf(d.z * mp.transmx * (4294967296.0f / Lz));
+        R.w[0] = (int32_t)rintf(d.x * mp.transmx * mp.fx[0]);
+        R.w[1] = (int32_t)rintf(d.y * mp.transmx * mp.fx[1]);
+        R.w[2] = (int32_t)rintf(d.z * mp.transmx * mp.fx[2]);
         R.w[3] = R.w[4] = 0;
     } else {
         c.w = (mp.pass_hi << 2) | 1u;
@@ -1347,7 +1350,6 @@ __device__ __forceinline__ void sweep_cell(int b, const Grid& g, const SysConst&
         if (tid == 0) atomicOr(flag, 1);
         return;
     }
-    const float Lx = sc.L[0], Ly = sc.L[1], Lz = sc.L[2];
     U4 ctr;
     ctr.y = (uint32_t)cell;
     ctr.z = mp.pass_lo;
@@ -1379,7 +1381,7 @@ __device__ __forceinline__ void sweep_cell(int b, const Grid& g, const SysConst&
             __syncthreads();
             int tt = t + tid;
             if (tid < TRIAL_CHUNK && tt < ntrial) {
-                recs[tid] = draw_trial<DA>(ctr, tt, mp, S, nh, tp, Lx, Ly, Lz);
+                recs[tid] = draw_trial<DA>(ctr, tt, mp, S.u + S.h0, S.h0, nh, tp);
             }
             __syncthreads();
         }
@@ -1537,7 +1539,7 @@ __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_
     L.sten = o;
     o += 4 * (2 * 125 + 2);
     L.misc = spec_align(o, 16);
-    o = L.misc + 4 * 16;
+    o = L.misc + 4 * (16 + 2 * CNT_HALF);
     L.prop = spec_align(o, 16);
     L.res = L.prop + SPEC_W * sizeof(SpecProp);
     o = L.res + SPEC_W * sizeof(int);
@@ -2312,9 +2314,9 @@ __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query*
 // that can matter to the home cell are staged, in stencil order: those within
 // sc.reach of the cell's box, where every trial position lies, and chain
 // partners of its particles.  For 65,536 TCHPSC at packing fraction 0.25 that
-// is ~245 of 432, and every trial scans the stage.  Two passes over the
+// is ~245 of 432, and every trial scans the stage.  Two passes over a large
 // stencil (positions, then the records of those kept), so that the records
-// lie packed behind one another.  list: cap source indices at the end of the
+// lie packed behind one another; misc: 16 ints and block_compactK's counts.  list: cap source indices at the end of the
 // region, beyond the records (44 cap + 4 cap bytes fit the region).
 // half_stencil: only the home cell and the stencil cells behind it in their
 // order, one of each pair of opposite cells.
@@ -2367,6 +2369,69 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
         half[q] = 0.5f * sc.L[q] / (float)g.nc[q];
     }
     const float reach2 = sc.reach * sc.reach;
+    // the stencil entry and the source of element e
+    auto source = [&](int e, int& lo) {
+        lo = 0;
+        int hi = ns - 1;
+        while (lo < hi) {
+            int mid = (lo + hi + 1) >> 1;
+            if (pre[mid] <= e) lo = mid; else hi = mid - 1;
+        }
+        return cst[lo] + (e - pre[lo]);
+    };
+    auto near = [&](const uint4 u, int lo) {
+        const V3<float> r = fx_image_c(u.x, u.y, u.z, cen[0], cen[1], cen[2], sc.Lh, sc.Ll);
+        const float dx = fmaxf(fabsf(r.x) - half[0], 0.0f), dy = fmaxf(fabsf(r.y) - half[1], 0.0f),
+                    dz = fmaxf(fabsf(r.z) - half[2], 0.0f);
+        return (lo == home) | ((dx * dx + dy * dy + dz * dz <= reach2) & !(half_stencil & (lo < home)));
+    };
+    const int t4 = (total + 3) & ~3;
+    if (!ct.cw && (size_t)t4 * (44 + 4 * VROW) <= region_bytes && total <= cap) {
+        // room for the whole stencil and its rows: one pass, the records at the
+        // stride of the stencil's count (a second round trip to memory is a
+        // tenth of a pass of a few trials)
+        S.u = (uint4*)region;
+        S.o = (float4*)(S.u + t4);
+        S.q = (float2*)(S.o + t4);
+        S.id = (int*)(S.q + t4);
+        used = (size_t)t4 * 44;
+        partner = nullptr;
+        int n = 0, par = 0;
+        for (int base = 0; base < total; base += 2 * WAVE * NW) {
+            bool keep[2];
+            int pos[2], id[2], lo[2], src[2];
+            uint4 u[2];
+            float4 o[2];
+            float2 q[2];
+#pragma unroll
+            for (int h = 0; h < 2; h++) src[h] = source(min(base + h * WAVE * NW + tid, total - 1), lo[h]);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                u[h] = P[src[h]];
+                o[h] = O[src[h]];
+                q[h] = Q[src[h]];
+                id[h] = ID[src[h]];
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) keep[h] = near(u[h], lo[h]) & (base + h * WAVE * NW + tid < total);
+            block_compactK<NW, 2>(keep, n, misc + 16, par, pos);
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if (keep[h]) {
+                    S.u[pos[h]] = u[h];
+                    S.o[pos[h]] = o[h];
+                    S.q[pos[h]] = q[h];
+                    S.id[pos[h]] = id[h];
+                }
+                if (base + h * WAVE * NW + tid == hbeg) misc[1] = pos[h];
+            }
+        }
+        __syncthreads();
+        S.n = n;
+        S.h0 = misc[1];
+        S.h1 = S.h0 + (hend - hbeg);
+        return true;
+    }
     int* list = (int*)(region + region_bytes) - cap;
     int n = 0;
     for (int base = 0; base < total; base += WAVE * NW) {
@@ -2374,17 +2439,9 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
         bool keep = false;
         int src = 0;
         if (e < total) {
-            int lo = 0, hi = ns - 1;   // the stencil entry holding element e
-            while (lo < hi) {
-                int mid = (lo + hi + 1) >> 1;
-                if (pre[mid] <= e) lo = mid; else hi = mid - 1;
-            }
-            src = cst[lo] + (e - pre[lo]);
-            const uint4 u = P[src];
-            const V3<float> r = fx_image_c(u.x, u.y, u.z, cen[0], cen[1], cen[2], sc.Lh, sc.Ll);
-            const float dx = fmaxf(fabsf(r.x) - half[0], 0.0f), dy = fmaxf(fabsf(r.y) - half[1], 0.0f),
-                        dz = fmaxf(fabsf(r.z) - half[2], 0.0f);
-            keep = lo == home || (dx * dx + dy * dy + dz * dz <= reach2 && !(half_stencil && lo < home));
+            int lo;
+            src = source(e, lo);
+            keep = near(P[src], lo);
             if (!keep && ct.cw) {
                 const int id = ID[src], w = ct.cw[id];
                 for (int q = 0; q < 4; q++)
@@ -2476,6 +2533,26 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         ml = (float*)(smem + L.ml);
         for (int i = tid; i < MLP_C_BYTES / 16; i += WAVE * SPEC_W) ((uint4*)ml)[i] = ((const uint4*)(mlp_img + MLP_C_OFF))[i];
     }
+    U4 ctr;
+    ctr.y = (uint32_t)cell;
+    ctr.z = mp.pass_lo;
+    int ntrial = nh * mp.visit;
+    if (mp.trial_mode == 1) {
+        ctr.x = 0xffffffffu;
+        ctr.w = (mp.pass_hi << 2) | 3u;
+        U4 rd = philox(ctr, mp.key0, mp.key1);
+        float mean = (float)mp.n * (float)mp.visit / (float)max(1, *nonempty);
+        int fl = (int)floorf(mean);
+        ntrial = fl + ((u01f(rd.x) < mean - (float)fl) ? 1 : 0);
+    }
+    // the first trials are drawn on the last wave while the first one finds the
+    // stencil (a cell visited for a few trials is mostly set-up)
+    int drawn = 0;
+    if (ntrial > 0) {
+        if (w == SPEC_W - 1 && lane < min(TRIAL_CHUNK, ntrial))
+            recs[lane] = draw_trial<DA>(ctr, lane, mp, P + starts[cell], 0, nh, tp);
+        drawn = TRIAL_CHUNK;
+    }
     if constexpr (LT) {
         PP32* ppl = (PP32*)(smem + L.tab);
         TP32* tpl = (TP32*)(ppl + sc.nt * sc.nt);
@@ -2491,19 +2568,6 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
                              used)) {
         if (tid == 0) atomicOr(flag, 1);
         return;
-    }
-    const float Lx = sc.L[0], Ly = sc.L[1], Lz = sc.L[2];
-    U4 ctr;
-    ctr.y = (uint32_t)cell;
-    ctr.z = mp.pass_lo;
-    int ntrial = nh * mp.visit;
-    if (mp.trial_mode == 1) {
-        ctr.x = 0xffffffffu;
-        ctr.w = (mp.pass_hi << 2) | 3u;
-        U4 rd = philox(ctr, mp.key0, mp.key1);
-        float mean = (float)mp.n * (float)mp.visit / (float)max(1, *nonempty);
-        int fl = (int)floorf(mean);
-        ntrial = fl + ((u01f(rd.x) < mean - (float)fl) ? 1 : 0);
     }
     // rows of all staged particles, else of the home cell's, where they fit
     Rows rows;
@@ -2529,18 +2593,18 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     unsigned n_tacc = 0, n_ttry = 0, n_racc = 0, n_rtry = 0, n_left = 0, n_s1try = 0, n_s1acc = 0, n_s2try = 0,
              n_s2acc = 0, n_bond = 0;
     double dsum = 0.0;
-    int t = 0, drawn = 0;
+    int t = 0;
     while (t < ntrial) {   // t is block-uniform (from LDS)
         if (t >= drawn) {
             __syncthreads();   // the previous records are no longer read
             int tt = drawn + tid;
-            if (tid < TRIAL_CHUNK && tt < ntrial) recs[tid] = draw_trial<DA>(ctr, tt, mp, S, nh, tp, Lx, Ly, Lz);
+            if (tid < TRIAL_CHUNK && tt < ntrial) recs[tid] = draw_trial<DA>(ctr, tt, mp, S.u + S.h0, 0, nh, tp);
             drawn += TRIAL_CHUNK;
             __syncthreads();
         }
         const int W = min(SPEC_W, min(ntrial - t, drawn - t));
         const TrialRec& R = recs[(t + min(w, W - 1)) & (TRIAL_CHUNK - 1)];
-        const int k = R.k;
+        const int k = S.h0 + R.k;
         const bool translate = R.translate != 0;
         const uint4 uo = S.u[k];
         const float4 oo = S.o[k];
@@ -2759,7 +2823,7 @@ __device__ __forceinline__ void energy_cell(int cell, const Grid& g, const SysCo
                                             int* __restrict__ flag) {
     constexpr int NW = ENERGY_NW, BS = WAVE * NW, PA = 2;
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ int sten[2 * 125 + 2], misc[16], cnt[2 * CNT_HALF], list[ENERGY_LCAP], ent[BS];
+    __shared__ int sten[2 * 125 + 2], misc[16 + 2 * CNT_HALF], cnt[2 * CNT_HALF], list[ENERGY_LCAP], ent[BS];
     __shared__ uint16_t surv[4 * BS];
     __shared__ double red[NW];
     const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1);
@@ -6598,6 +6662,7 @@ static int sc_sweep_impl(sc_ctx* ctx, int nsweeps, double temper, double transmx
             mp.hcap = ctx->home_cache;
             mp.visit = ctx->visit;
             mp.n = ctx->n;
+            for (int k = 0; k < 3; k++) mp.fx[k] = 4294967296.0f / sc.L[k];
             mp.transmx = (float)transmx;
             mp.rot_half = (float)rot_half;
             mp.temper = temper;
@@ -6926,6 +6991,7 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
                 mp.hcap = ctx->home_cache;
                 mp.visit = vfac[q];
                 mp.n = ctx->rep_n[q];
+                for (int k = 0; k < 3; k++) mp.fx[k] = 4294967296.0f / P_.sc.L[k];
                 mp.transmx = (float)transmx;
                 mp.rot_half = (float)rot_half;
                 mp.temper = temper[q];
