@@ -420,6 +420,110 @@ __global__ __launch_bounds__(WAVE * CELL_SORT_CELLS) void k_cell_sort(int ncell,
     }
 }
 
+// The whole cell list of a small system (n <= BUILD_N particles, ncell <=
+// BUILD_CELLS cells) by one block: counts and ranks in LDS, the scan, the
+// order by ID within each cell (a particle's rank is the number of smaller IDs
+// in its cell), and the permuted records.  The general path's two fills and
+// five kernels are bound by their launches: 7 x 4.4 us of device time for
+// 1,000 particles, rebuilt for every sweep and every committed move.
+#define BUILD_N 4096
+#define BUILD_CELLS 8192
+__global__ __launch_bounds__(1024) void k_build_small(int n, int ncell, Grid g, const uint4* __restrict__ Pi,
+                                                      const float4* __restrict__ Oi, const float2* __restrict__ Qi,
+                                                      const int* __restrict__ IDi, uint4* __restrict__ Po,
+                                                      float4* __restrict__ Oo, float2* __restrict__ Qo,
+                                                      int* __restrict__ IDo, int* __restrict__ slot,
+                                                      int* __restrict__ starts, int* __restrict__ maxocc,
+                                                      int* __restrict__ nonempty) {
+    constexpr int NT = 1024, PT = BUILD_N / NT, CT = BUILD_CELLS / NT;
+    __shared__ int cnt[BUILD_CELLS + 1], ids[BUILD_N], wsum[16], wmax[16], wne[16];
+    const int t = (int)threadIdx.x, lane = t & 63, wv = t >> 6;
+    uint4 u[PT];
+    int c[PT], id[PT], r[PT];
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+        const int k = t + NT * q;
+        if (k < n) {
+            u[q] = Pi[k];
+            id[q] = IDi[k];
+        }
+    }
+    for (int i = t; i <= ncell; i += NT) cnt[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PT; q++)
+        if (t + NT * q < n) {
+            c[q] = cell_of_u(g, u[q].x, u[q].y, u[q].z);
+            r[q] = atomicAdd(&cnt[c[q]], 1);
+        }
+    __syncthreads();
+    // exclusive scan of the counts, CT contiguous cells per thread
+    int v[CT], sum = 0, mx = 0, ne = 0;
+#pragma unroll
+    for (int i = 0; i < CT; i++) {
+        v[i] = CT * t + i < ncell ? cnt[CT * t + i] : 0;
+        sum += v[i];
+        mx = max(mx, v[i]);
+        ne += v[i] > 0 ? 1 : 0;
+    }
+    int incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+        int y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+    }
+    for (int o = 32; o >= 1; o >>= 1) {
+        mx = max(mx, __shfl_xor(mx, o, 64));
+        ne += __shfl_xor(ne, o, 64);
+    }
+    if (lane == 63) wsum[wv] = incl;
+    if (lane == 0) {
+        wmax[wv] = mx;
+        wne[wv] = ne;
+    }
+    __syncthreads();
+    int run = incl - sum;
+    for (int k = 0; k < wv; k++) run += wsum[k];
+#pragma unroll
+    for (int i = 0; i < CT; i++) {
+        const int k = CT * t + i;
+        if (k < ncell) {
+            cnt[k] = run;
+            starts[k] = run;
+        }
+        run += v[i];
+    }
+    if (t == 0) {
+        int m = 0, e = 0;
+        for (int k = 0; k < 16; k++) {
+            m = max(m, wmax[k]);
+            e += wne[k];
+        }
+        *maxocc = m;
+        *nonempty = e;
+        starts[ncell] = n;
+        cnt[ncell] = n;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PT; q++)
+        if (t + NT * q < n) ids[cnt[c[q]] + r[q]] = id[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PT; q++) {
+        const int k = t + NT * q;
+        if (k < n) {
+            const int b = cnt[c[q]], e = cnt[c[q] + 1];
+            int pos = b;
+            for (int i = b; i < e; i++) pos += ids[i] < id[q] ? 1 : 0;
+            Po[pos] = u[q];
+            Oo[pos] = Oi[k];
+            Qo[pos] = Qi[k];
+            IDo[pos] = id[q];
+            slot[id[q]] = pos;
+        }
+    }
+}
+
 __global__ void k_permute(int n, const int* __restrict__ src_of_pos, const uint4* __restrict__ Pi,
                           const float4* __restrict__ Oi, const float2* __restrict__ Qi, const int* __restrict__ IDi,
                           uint4* __restrict__ Po, float4* __restrict__ Oo, float2* __restrict__ Qo,
@@ -2093,16 +2197,29 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
 // around its cell except those of ID ex_lo..ex_hi (the particle itself, or
 // its whole molecule for mol2others), plus its bonds for oneToAll (not for
 // mol2others, whose connectivity list is empty).  The query state is given
-// explicitly (trial states) or taken from a slot.
+// explicitly (trial states) or the stored one.  The queries are the array qs,
+// or q1 for all (a single call's query comes with the launch).
 struct Query {
     uint32_t u[3];
-    int t;
+    int t;             // dense type; < 0: the stored state of particle id + query index (id < 0: of that slot)
     float4 o;
     float2 q;
     int id;            // the query particle's ID
-    int ex_lo, ex_hi;  // IDs left out
+    int ex_lo, ex_hi;  // IDs left out (stored states: ex_lo < 0 leaves out the particle itself)
     int bonds;         // add the bonds with its chain partners
 };
+
+// commits of trial states: the records of the queries' particles
+__global__ void k_commit(int nq, const Query* __restrict__ qs, Query q1, const int* __restrict__ slot,
+                         uint4* __restrict__ P, float4* __restrict__ O, float2* __restrict__ Q) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nq) return;
+    const Query q = qs ? qs[i] : q1;
+    const int s = slot[q.id];
+    P[s] = make_uint4(q.u[0], q.u[1], q.u[2], (uint32_t)q.t);
+    O[s] = q.o;
+    Q[s] = q.q;
+}
 
 // The stencil's particles are flattened over the block's NW waves, PA of them
 // per thread at once, and pass the same stages as a trial of the speculative
@@ -2116,13 +2233,13 @@ struct Query {
 constexpr int QRY_LCAP = 1024;   // candidates held before they are evaluated
 template <int NW>
 __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query* __restrict__ qs,
-                                                            const int* __restrict__ qslot, Grid g, SysConst sc,
+                                                            Query q1, Grid g, SysConst sc,
                                                             const int* __restrict__ starts,
                                                             const uint4* __restrict__ P, const float4* __restrict__ O,
                                                             const float2* __restrict__ Q, const int* __restrict__ ID,
                                                             const PP32* __restrict__ pp, const TP32* __restrict__ tp,
                                                             int ppmax, ChainTab ct, const int* __restrict__ slot,
-                                                            double* __restrict__ out) {
+                                                            bool by_id, double* out) {
     constexpr int BS = WAVE * NW, PA = NW == 1 ? 4 : 2;
     static_assert(PA * BS <= QRY_LCAP / 2, "a scan step fits beside the candidates kept");
     __shared__ int pre[126], cst[126], list[QRY_LCAP], cnt[2 * CNT_HALF];
@@ -2134,15 +2251,13 @@ __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query*
     const int qi = blockIdx.x;
     if (qi >= nq) return;
     const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1);
-    Query q;
-    if (qslot) {
-        int s = qslot[qi];
-        uint4 p = P[s];
+    Query q = qs ? qs[qi] : q1;
+    if (q.t < 0) {   // the stored state of particle q.id + qi, or of the particle in slot qi
+        const int s = q.id >= 0 ? slot[q.id + qi] : qi;
+        const uint4 p = P[s];
         q.u[0] = p.x; q.u[1] = p.y; q.u[2] = p.z; q.t = p.w;
-        q.o = O[s]; q.q = Q[s]; q.id = q.ex_lo = q.ex_hi = ID[s];
-        q.bonds = 1;
-    } else {
-        q = qs[qi];
+        q.o = O[s]; q.q = Q[s]; q.id = ID[s];
+        if (q.ex_lo < 0) q.ex_lo = q.ex_hi = q.id;
     }
     const int np = ppmax > 1 ? 2 : 1, psh = ppmax > 2 ? 2 : (ppmax > 1 ? 1 : 0);
     if (tid < np) vrow_derive(rows, tid, q.o, q.q, q.t, tp);
@@ -2307,7 +2422,7 @@ __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query*
         acc += bonds_global(ct, sc.nt, sc.Ld, q.id, make_uint4(q.u[0], q.u[1], q.u[2], (uint32_t)q.t), q.o, q.q,
                             15, slot, P, O, Q);
     const double sum = block_sum<NW>(acc, red);
-    if (tid == 0) out[qi] = sum;
+    if (tid == 0) out[by_id ? q.id : qi] = sum;
 }
 
 // stage_load for the speculative sweep: of the stencil's particles only those
@@ -4584,6 +4699,8 @@ struct PinRing {
     int next = 0;
 };
 
+#define SINGLE_Q 64   // queries whose results the kernel writes to pinned host memory
+
 struct sc_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -4621,7 +4738,6 @@ struct sc_ctx {
     int ncell = 0, ncell_alloc = 0;
     int* starts = nullptr;
     int* counts = nullptr;
-    int* fill = nullptr;
     double* partial = nullptr;
     bool grid_valid = false;
     // scratch
@@ -4635,6 +4751,7 @@ struct sc_ctx {
     unsigned long long* d_stats = nullptr;
     double* d_dsum = nullptr;
     Query* d_q = nullptr;
+    double* h_res = nullptr;            // pinned: the energies of up to SINGLE_Q queries
     int* d_i = nullptr;
     int* d_j = nullptr;
     int ij_cap = 0;
@@ -5039,21 +5156,28 @@ static int build_grid_w(sc_ctx* ctx, int r, const uint32_t shift[3], const doubl
     if (ncell > ctx->ncell_alloc) {
         int rc;
         if ((rc = dalloc(ctx, &ctx->starts, ncell + 1))) return rc;
-        if ((rc = dalloc(ctx, &ctx->counts, ncell))) return rc;
-        if ((rc = dalloc(ctx, &ctx->fill, ncell))) return rc;
+        if ((rc = dalloc(ctx, &ctx->counts, 2 * (size_t)ncell))) return rc;   // counts, then the scatter's fill
         if ((rc = dalloc(ctx, &ctx->partial, ncell))) return rc;
         ctx->ncell_alloc = ncell;
     }
     ctx->g = g;
     ctx->ncell = ncell;
     int n = ctx->n, c = ctx->cur, nb = (n + 255) / 256;
-    HIPCK(hipMemsetAsync(ctx->counts, 0, sizeof(int) * ncell, ctx->stream));
-    HIPCK(hipMemsetAsync(ctx->fill, 0, sizeof(int) * ncell, ctx->stream));
+    if (n > 0 && n <= BUILD_N && ncell <= BUILD_CELLS) {
+        hipLaunchKernelGGL(k_build_small, dim3(1), dim3(1024), 0, ctx->stream, n, ncell, g, ctx->P[c], ctx->O[c],
+                           ctx->Q[c], ctx->ID[c], ctx->P[c ^ 1], ctx->O[c ^ 1], ctx->Q[c ^ 1], ctx->ID[c ^ 1],
+                           ctx->slot, ctx->starts, ctx->d_maxocc, ctx->d_nonempty);
+        HIPCK(hipGetLastError());
+        ctx->cur ^= 1;
+        ctx->grid_valid = true;
+        return SC_OK;
+    }
+    HIPCK(hipMemsetAsync(ctx->counts, 0, 2 * sizeof(int) * (size_t)ncell, ctx->stream));
     if (n > 0) hipLaunchKernelGGL(k_cell_count, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->P[c], g, ctx->cell_tmp, ctx->counts);
     hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, ctx->stream, ncell, ctx->counts, ctx->starts, ctx->d_maxocc,
                        ctx->d_nonempty);
     if (n > 0) {
-        hipLaunchKernelGGL(k_cell_scatter, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->cell_tmp, ctx->starts, ctx->fill, ctx->src_of_pos);
+        hipLaunchKernelGGL(k_cell_scatter, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->cell_tmp, ctx->starts, ctx->counts + ncell, ctx->src_of_pos);
         hipLaunchKernelGGL(k_cell_sort, dim3((ncell + CELL_SORT_CELLS - 1) / CELL_SORT_CELLS), dim3(WAVE * CELL_SORT_CELLS), 0,
                            ctx->stream, ncell, ctx->starts, ctx->src_of_pos, ctx->ID[c]);
         hipLaunchKernelGGL(k_permute, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->src_of_pos, ctx->P[c], ctx->O[c], ctx->Q[c],
@@ -5303,6 +5427,7 @@ static int sc_create_impl(sc_ctx** out, int device) {
     hipEventCreate(&ctx->ev0);
     hipEventCreate(&ctx->ev1);
     if (hipMalloc((void**)&ctx->d_flag, sizeof(int)) != hipSuccess ||
+        hipHostMalloc((void**)&ctx->h_res, SINGLE_Q * sizeof(double)) != hipSuccess ||
         hipMalloc((void**)&ctx->d_maxocc, sizeof(int)) != hipSuccess ||
         hipMalloc((void**)&ctx->d_nonempty, sizeof(int)) != hipSuccess ||
         hipMalloc((void**)&ctx->d_stats, STAT_REP * STAT_STRIDE * sizeof(unsigned long long)) != hipSuccess ||
@@ -5336,7 +5461,7 @@ static void sc_destroy_impl(sc_ctx* ctx) {
     hipStreamSynchronize(ctx->stream);
     void* ptrs[] = {ctx->d_pp32, ctx->d_pp64, ctx->d_tp32, ctx->d_tp64, ctx->P[0], ctx->P[1], ctx->O[0], ctx->O[1],
                     ctx->Q[0], ctx->Q[1], ctx->ID[0], ctx->ID[1], ctx->slot, ctx->cell_tmp, ctx->src_of_pos,
-                    ctx->starts, ctx->counts, ctx->fill, ctx->partial, ctx->d_out, ctx->d_flag, ctx->d_maxocc,
+                    ctx->starts, ctx->counts, ctx->partial, ctx->d_out, ctx->d_flag, ctx->d_maxocc,
                     ctx->d_nonempty, ctx->d_stats, ctx->d_dsum, ctx->d_q, ctx->d_i, ctx->d_j, ctx->mlp_w,
                     ctx->mlp_g, ctx->mlp_m, ctx->mlp_v, ctx->mlp_img, ctx->tr_x, ctx->tr_y, ctx->tr_e, ctx->d_part,
                     ctx->bx, ctx->d_loss, ctx->d_pcount, ctx->d_pi, ctx->d_pj, ctx->d_pe, ctx->d_label, ctx->d_q6,
@@ -5352,6 +5477,7 @@ static void sc_destroy_impl(sc_ctx* ctx) {
             if (r->host[k]) hipHostFree(r->host[k]);
             if (r->ev[k]) hipEventDestroy(r->ev[k]);
         }
+    if (ctx->h_res) hipHostFree(ctx->h_res);
     if (ctx->ev0) hipEventDestroy(ctx->ev0);
     if (ctx->ev1) hipEventDestroy(ctx->ev1);
     if (ctx->stream) hipStreamDestroy(ctx->stream);
@@ -6036,28 +6162,48 @@ int sc_commit_box(sc_ctx* ctx, const double box_new[3]) {
     SC_GUARD(ctx, sc_commit_box_impl(ctx, box_new))
 }
 
-static int run_queries(sc_ctx* ctx, int nq, const Query* hq, const int* slots_dev, double* out) {
+// Energies of nq queries: the array hq, or q1 for all (see Query).  Up to
+// SINGLE_Q results come back through pinned host memory that the kernel writes
+// itself; a host program's single moves are bound by the copies and
+// synchronisations around them.
+static int run_queries(sc_ctx* ctx, int nq, const Query* hq, const Query& q1, double* out, bool by_id = false) {
     int rc;
-    if ((rc = ensure_out(ctx, nq)) || (rc = ensure_ij(ctx, nq))) return rc;
+    const bool pinned = nq <= SINGLE_Q;
+    if (!pinned && (rc = ensure_out(ctx, nq))) return rc;
+    if (hq && (rc = ensure_ij(ctx, nq))) return rc;
     if (!ctx->grid_valid) {
         if ((rc = build_grid(ctx, 2, nullptr, ctx->box))) return rc;
     }
     if (hq) HIPCK(hipMemcpyAsync(ctx->d_q, hq, nq * sizeof(Query), hipMemcpyHostToDevice, ctx->stream));
     SysConst sc = sysconst(ctx, ctx->box);
     int c = ctx->cur;
+    double* res = pinned ? ctx->h_res : ctx->d_out;
     // four waves per query while that leaves a wave slot of the chip to each
     // (256 CUs x 4 SIMDs x 4 waves of this kernel's registers), else one
 #define QUERY(NWV)                                                                                             \
     hipLaunchKernelGGL((k_energy_query<NWV>), dim3(nq), dim3(WAVE * NWV), 0, ctx->stream, nq,                    \
-                       hq ? ctx->d_q : nullptr, slots_dev, ctx->g, sc, ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], \
-                       ctx->ID[c], ctx->d_pp32, ctx->d_tp32, ctx->ppmax, chain_tab(ctx), ctx->slot, ctx->d_out)
+                       hq ? ctx->d_q : nullptr, q1, ctx->g, sc, ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c],        \
+                       ctx->ID[c], ctx->d_pp32, ctx->d_tp32, ctx->ppmax, chain_tab(ctx), ctx->slot, by_id, res)
     if (nq <= 1024) QUERY(4);
     else QUERY(1);
 #undef QUERY
     HIPCK(hipGetLastError());
-    HIPCK(hipMemcpyAsync(out, ctx->d_out, nq * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    if (!pinned) HIPCK(hipMemcpyAsync(out, ctx->d_out, nq * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     HIPCK(hipStreamSynchronize(ctx->stream));
+    if (pinned) std::memcpy(out, ctx->h_res, nq * sizeof(double));
     return SC_OK;
+}
+
+// the stored state of particle id (id < 0: of every slot), leaving out ex_lo..ex_hi (< 0: itself)
+static Query stored_query(int id, int ex_lo, int ex_hi, int bonds) {
+    Query q;
+    std::memset(&q, 0, sizeof(q));
+    q.t = -1;
+    q.id = id;
+    q.ex_lo = ex_lo;
+    q.ex_hi = ex_hi;
+    q.bonds = bonds;
+    return q;
 }
 
 static int sc_energy_one_impl(sc_ctx* ctx, int target, double* e) {
@@ -6065,12 +6211,7 @@ static int sc_energy_one_impl(sc_ctx* ctx, int target, double* e) {
     if (!ctx->have_state) return fail(ctx, SC_ESTATE, "no configuration loaded");
     if (target < 0 || target >= ctx->n) return fail(ctx, SC_EINVAL, "target out of range");
     HIPCK(hipSetDevice(ctx->device));
-    int s = 0;
-    HIPCK(hipMemcpy(&s, ctx->slot + target, sizeof(int), hipMemcpyDeviceToHost));
-    int rc;
-    if ((rc = ensure_ij(ctx, 1))) return rc;
-    HIPCK(hipMemcpy(ctx->d_i, &s, sizeof(int), hipMemcpyHostToDevice));
-    return run_queries(ctx, 1, nullptr, ctx->d_i, e);
+    return run_queries(ctx, 1, nullptr, stored_query(target, -1, -1, 1), e);
 }
 
 int sc_energy_one(sc_ctx* ctx, int target, double* e) {
@@ -6081,19 +6222,8 @@ static int sc_energy_per_particle_impl(sc_ctx* ctx, double* out) {
     if (!ctx || !out) return SC_EINVAL;
     if (!ctx->have_state) return fail(ctx, SC_ESTATE, "no configuration loaded");
     HIPCK(hipSetDevice(ctx->device));
-    int n = ctx->n, rc;
-    if (n == 0) return SC_OK;
-    if ((rc = ensure_ij(ctx, n))) return rc;
-    if (!ctx->grid_valid && (rc = build_grid(ctx, 2, nullptr, ctx->box))) return rc;
-    // queries in slot order (query q = slot q), results mapped back through slot
-    std::vector<int> sl(n), iota(n);
-    for (int k = 0; k < n; k++) iota[k] = k;
-    HIPCK(hipMemcpy(ctx->d_i, iota.data(), n * sizeof(int), hipMemcpyHostToDevice));
-    std::vector<double> bySlot(n);
-    if ((rc = run_queries(ctx, n, nullptr, ctx->d_i, bySlot.data()))) return rc;
-    HIPCK(hipMemcpy(sl.data(), ctx->slot, n * sizeof(int), hipMemcpyDeviceToHost));
-    for (int i = 0; i < n; i++) out[i] = bySlot[sl[i]];
-    return SC_OK;
+    if (ctx->n == 0) return SC_OK;
+    return run_queries(ctx, ctx->n, nullptr, stored_query(-1, -1, -1, 1), out, true);   // slot by slot, to the IDs' places
 }
 
 int sc_energy_per_particle(sc_ctx* ctx, double* out) {
@@ -6129,7 +6259,7 @@ static int sc_energy_one_trial_impl(sc_ctx* ctx, int target, const double pos[3]
     if (target < 0 || target >= ctx->n) return fail(ctx, SC_EINVAL, "target out of range");
     HIPCK(hipSetDevice(ctx->device));
     Query q = make_query(ctx, target, pos, dir, pd0);
-    return run_queries(ctx, 1, &q, nullptr, e);
+    return run_queries(ctx, 1, nullptr, q, e);
 }
 
 int sc_energy_one_trial(sc_ctx* ctx, int target, const double pos[3], const double dir[3], const double pd0[3],
@@ -6143,12 +6273,9 @@ static int sc_commit_particle_impl(sc_ctx* ctx, int target, const double pos[3],
     if (target < 0 || target >= ctx->n) return fail(ctx, SC_EINVAL, "target out of range");
     HIPCK(hipSetDevice(ctx->device));
     Query q = make_query(ctx, target, pos, dir, pd0);
-    int s = 0, c = ctx->cur;
-    HIPCK(hipMemcpy(&s, ctx->slot + target, sizeof(int), hipMemcpyDeviceToHost));
-    uint4 p = make_uint4(q.u[0], q.u[1], q.u[2], (uint32_t)q.t);
-    HIPCK(hipMemcpy(ctx->P[c] + s, &p, sizeof(uint4), hipMemcpyHostToDevice));
-    HIPCK(hipMemcpy(ctx->O[c] + s, &q.o, sizeof(float4), hipMemcpyHostToDevice));
-    HIPCK(hipMemcpy(ctx->Q[c] + s, &q.q, sizeof(float2), hipMemcpyHostToDevice));
+    int c = ctx->cur;
+    hipLaunchKernelGGL(k_commit, dim3(1), dim3(64), 0, ctx->stream, 1, nullptr, q, ctx->slot, ctx->P[c], ctx->O[c], ctx->Q[c]);
+    HIPCK(hipGetLastError());
     ctx->e_valid = false;
     // the particle may have changed cell: rebuild the cell list
     return build_grid(ctx, ctx->grid_valid ? ctx->g.r : 2, nullptr, ctx->box);
@@ -6167,30 +6294,16 @@ static int sc_energy_mol_impl(sc_ctx* ctx, int first, int size, const double* po
     if (!ctx->have_state) return fail(ctx, SC_ESTATE, "no configuration loaded");
     if (first < 0 || first + size > ctx->n) return fail(ctx, SC_EINVAL, "molecule out of range");
     HIPCK(hipSetDevice(ctx->device));
-    std::vector<Query> q(size);
-    if (pos) {
-        for (int a = 0; a < size; a++) q[a] = make_query(ctx, first + a, pos + 3 * a, dir + 3 * a, pd0 + 3 * a);
-    } else {
-        std::vector<int> sl(size);
-        HIPCK(hipMemcpy(sl.data(), ctx->slot + first, size * sizeof(int), hipMemcpyDeviceToHost));
-        int c = ctx->cur;
-        for (int a = 0; a < size; a++) {
-            uint4 p;
-            HIPCK(hipMemcpy(&p, ctx->P[c] + sl[a], sizeof(uint4), hipMemcpyDeviceToHost));
-            HIPCK(hipMemcpy(&q[a].o, ctx->O[c] + sl[a], sizeof(float4), hipMemcpyDeviceToHost));
-            HIPCK(hipMemcpy(&q[a].q, ctx->Q[c] + sl[a], sizeof(float2), hipMemcpyDeviceToHost));
-            q[a].u[0] = p.x; q[a].u[1] = p.y; q[a].u[2] = p.z;
-            q[a].t = (int)p.w;
-            q[a].id = first + a;
-        }
-    }
-    for (int a = 0; a < size; a++) {
-        q[a].ex_lo = first;
-        q[a].ex_hi = first + size - 1;
-        q[a].bonds = 0;
-    }
+    std::vector<Query> q;
     std::vector<double> out(size);
-    int rc = run_queries(ctx, size, q.data(), nullptr, out.data());
+    if (pos)
+        for (int a = 0; a < size; a++) {
+            q.push_back(make_query(ctx, first + a, pos + 3 * a, dir + 3 * a, pd0 + 3 * a));
+            q[a].ex_lo = first;
+            q[a].ex_hi = first + size - 1;
+            q[a].bonds = 0;
+        }
+    int rc = run_queries(ctx, size, pos ? q.data() : nullptr, stored_query(first, first, first + size - 1, 0), out.data());
     if (rc) return rc;
     double s = 0.0;
     for (double v : out) s += v;
@@ -6214,16 +6327,15 @@ static int sc_commit_mol_impl(sc_ctx* ctx, int first, int size, const double* po
     if (!ctx->have_state) return fail(ctx, SC_ESTATE, "no configuration loaded");
     if (first < 0 || first + size > ctx->n) return fail(ctx, SC_EINVAL, "molecule out of range");
     HIPCK(hipSetDevice(ctx->device));
-    std::vector<int> sl(size);
-    HIPCK(hipMemcpy(sl.data(), ctx->slot + first, size * sizeof(int), hipMemcpyDeviceToHost));
-    int c = ctx->cur;
-    for (int a = 0; a < size; a++) {
-        Query q = make_query(ctx, first + a, pos + 3 * a, dir + 3 * a, pd0 + 3 * a);
-        uint4 p = make_uint4(q.u[0], q.u[1], q.u[2], (uint32_t)q.t);
-        HIPCK(hipMemcpy(ctx->P[c] + sl[a], &p, sizeof(uint4), hipMemcpyHostToDevice));
-        HIPCK(hipMemcpy(ctx->O[c] + sl[a], &q.o, sizeof(float4), hipMemcpyHostToDevice));
-        HIPCK(hipMemcpy(ctx->Q[c] + sl[a], &q.q, sizeof(float2), hipMemcpyHostToDevice));
-    }
+    std::vector<Query> q;
+    for (int a = 0; a < size; a++) q.push_back(make_query(ctx, first + a, pos + 3 * a, dir + 3 * a, pd0 + 3 * a));
+    int c = ctx->cur, rc;
+    if ((rc = ensure_ij(ctx, size))) return rc;
+    HIPCK(hipMemcpyAsync(ctx->d_q, q.data(), size * sizeof(Query), hipMemcpyHostToDevice, ctx->stream));
+    HIPCK(hipStreamSynchronize(ctx->stream));   // (q ends here)
+    hipLaunchKernelGGL(k_commit, dim3((size + 63) / 64), dim3(64), 0, ctx->stream, size, ctx->d_q, q[0], ctx->slot,
+                       ctx->P[c], ctx->O[c], ctx->Q[c]);
+    HIPCK(hipGetLastError());
     ctx->e_valid = false;
     return build_grid(ctx, ctx->grid_valid ? ctx->g.r : 2, nullptr, ctx->box);
 }
@@ -6831,21 +6943,20 @@ static int batch_build_grid(sc_ctx* ctx, int r, const std::vector<std::array<uin
     }
     ctx->rep_ncell_total = total;
     if (total > ctx->ncell_alloc) {
-        if ((rc = dalloc(ctx, &ctx->starts, total + 1)) || (rc = dalloc(ctx, &ctx->counts, total)) ||
-            (rc = dalloc(ctx, &ctx->fill, total)) || (rc = dalloc(ctx, &ctx->partial, total)))
+        if ((rc = dalloc(ctx, &ctx->starts, total + 1)) || (rc = dalloc(ctx, &ctx->counts, 2 * (size_t)total)) ||
+            (rc = dalloc(ctx, &ctx->partial, total)))
             return rc;
         ctx->ncell_alloc = total;
     }
     if ((rc = batch_alloc(ctx))) return rc;
     int n = ctx->n, c = ctx->cur, nb = (n + 255) / 256;
     if ((rc = pin_upload(ctx, ctx->pin_rg, ctx->d_rg, ctx->rep_grid.data(), R * sizeof(RepGrid)))) return rc;
-    HIPCK(hipMemsetAsync(ctx->counts, 0, sizeof(int) * total, ctx->stream));
-    HIPCK(hipMemsetAsync(ctx->fill, 0, sizeof(int) * total, ctx->stream));
+    HIPCK(hipMemsetAsync(ctx->counts, 0, 2 * sizeof(int) * (size_t)total, ctx->stream));
     SC_LAUNCH(k_cell_count_batch, dim3(nb), dim3(256), 0, ctx->stream, n, R, ctx->d_rg, ctx->P[c], ctx->ID[c],
               ctx->cell_tmp, ctx->counts);
     SC_LAUNCH(k_scan, dim3(1), dim3(1024), 0, ctx->stream, total, ctx->counts, ctx->starts, ctx->d_maxocc,
               ctx->d_nonempty);
-    SC_LAUNCH(k_cell_scatter, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->cell_tmp, ctx->starts, ctx->fill,
+    SC_LAUNCH(k_cell_scatter, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->cell_tmp, ctx->starts, ctx->counts + total,
               ctx->src_of_pos);
     SC_LAUNCH(k_cell_sort, dim3((total + CELL_SORT_CELLS - 1) / CELL_SORT_CELLS), dim3(WAVE * CELL_SORT_CELLS), 0,
               ctx->stream, total, ctx->starts, ctx->src_of_pos, ctx->ID[c]);
