@@ -798,37 +798,87 @@ __global__ __launch_bounds__(1024) void k_reduce(int n, const double* __restrict
 
 // ------------------------------------------------------------ pair energies
 // p2p(i, j) with i's connectivity list: the non-bonded functor, plus the bond
-// and angle terms when j is one of i's chain partners
+// and angle terms when j is one of i's chain partners.
+// A block takes its threads' pairs in two steps: the cheap stage of each (cutoff,
+// segment distance, repulsion, sphere pairs), which settles most pairs of a
+// list by centre distance, then the rest (in the attraction's range, a sphere
+// with a spherocylinder, bonded) with full waves.  With the whole functor per
+// thread, both particles' derived vectors first, one pair in range made its wave
+// walk all of it: in FP64 147 us for the pairs within maxcut of 24,300 TCHPSC
+// at packing fraction 0.18, 57 us so (FP32, pairs within 2.5: 36 and 31; 512
+// pairs per block of 128 threads: 62 and 59).
+#define PAIRS_NT 256
 template <typename R>
-__global__ void k_pairs(int m, const int* __restrict__ pi, const int* __restrict__ pj, const int* __restrict__ slot,
-                        SysConst sc, const uint4* __restrict__ P, const float4* __restrict__ O,
-                        const float2* __restrict__ Q, const PairParamsT<R>* __restrict__ pp,
-                        const TypeParamsT<R>* __restrict__ tp, R sqmaxcut, ChainTab ct, double* __restrict__ out) {
-    int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= m) return;
-    int a = slot[pi[k]], b = slot[pj[k]];
-    uint4 ua = P[a], ub = P[b];
-    DPart<R> pa = load_part<R>(O[a], Q[a], ua.w, tp);
-    DPart<R> pb = load_part<R>(O[b], Q[b], ub.w, tp);
-    V3<R> r;
-    if (sizeof(R) == 8)
-        r = fx_image<R>(ua.x, ua.y, ua.z, ub.x, ub.y, ub.z, (R)sc.Ld[0], (R)sc.Ld[1], (R)sc.Ld[2]);
-    else {
+__global__ __launch_bounds__(PAIRS_NT) void k_pairs(int m, const int* __restrict__ pi, const int* __restrict__ pj,
+                                                    const int* __restrict__ slot, SysConst sc,
+                                                    const uint4* __restrict__ P, const float4* __restrict__ O,
+                                                    const float2* __restrict__ Q,
+                                                    const PairParamsT<R>* __restrict__ pp,
+                                                    const TypeParamsT<R>* __restrict__ tp, R sqmaxcut, ChainTab ct,
+                                                    double* __restrict__ out) {
+    __shared__ int rest[PAIRS_NT], cnt[PAIRS_NT / WAVE];
+    const int tid = (int)threadIdx.x, k0 = (int)blockIdx.x * PAIRS_NT + tid;
+    auto image = [&](uint4 ua, uint4 ub) {
+        if (sizeof(R) == 8)
+            return fx_image<R>(ua.x, ua.y, ua.z, ub.x, ub.y, ub.z, (R)sc.Ld[0], (R)sc.Ld[1], (R)sc.Ld[2]);
         V3<float> rf = fx_image_c(ua.x, ua.y, ua.z, ub.x, ub.y, ub.z, sc.Lh, sc.Ll);
-        r = mk<R>((R)rf.x, (R)rf.y, (R)rf.z);
+        return mk<R>((R)rf.x, (R)rf.y, (R)rf.z);
+    };
+    int left = 0;
+    bool full = false;
+    if (k0 < m) {
+        const int ia = pi[k0], ib = pj[k0], a = slot[ia], b = slot[ib];
+        const uint4 ua = P[a], ub = P[b];
+        const PairParamsT<R>& P2 = pp[ua.w * sc.nt + ub.w];
+        const V3<R> r = image(ua, ub);
+        R e = R(0);
+        if (ct.cw) {
+            const int bit = cw_bit(ib - ia);
+            full = bit >= 0 && ((ct.cw[ia] >> bit) & 1);
+        }
+        if (!full && !(dot(r, r) > sqmaxcut)) {
+            if (P2.kind >= 0 && P2.kind <= K_SCA) {
+                const float4 oa = O[a], ob = O[b];
+                DPart<R> pa, pb;   // axes as derive leaves them
+                pa.dir = mk<R>((R)oa.x, (R)oa.y, (R)oa.z);
+                pb.dir = mk<R>((R)ob.x, (R)ob.y, (R)ob.z);
+                if (P2.kind < K_SCN) {
+                    pa.dir = normalised(pa.dir);
+                    pb.dir = normalised(pb.dir);
+                }
+                R d2;
+                full = scsc_cheap(P2, pa, pb, r, e, d2);
+            } else if (P2.kind == K_SPH_WCA || P2.kind == K_SPH_TAYLOR) {
+                e = sphere_pair(P2, (R)sqrt(dot(r, r)));
+            } else {
+                full = P2.kind != K_NONE;
+            }
+        }
+        if (!full) out[k0] = (double)e;
     }
-    // FP32: the terms added in FP64, as every FP32 kernel adds them; FP64: the
-    // reference's own order of the sum
-    double e = sizeof(R) == 8 ? (double)pair_energy<R>(pp[ua.w * sc.nt + ub.w], pa, pb, r, sqmaxcut)
-                              : pair_energy_d<R>(pp[ua.w * sc.nt + ub.w], pa, pb, r, sqmaxcut);
-    if (ct.cw) {
-        int bit = cw_bit(pj[k] - pi[k]), cw = ct.cw[pi[k]];
-        if (bit >= 0 && ((cw >> bit) & 1))
-            e += bond_energy(ct.mol[cw >> 8], ct.pp64[ua.w * sc.nt + ub.w], cw_rel(bit), fx_r12(ua, ub, sc.Ld),
-                             unit64(O[a].x, O[a].y, O[a].z), unit64(O[a].w, Q[a].x, Q[a].y),
-                             unit64(O[b].x, O[b].y, O[b].z), unit64(O[b].w, Q[b].x, Q[b].y));
+    const int pos = block_compact<PAIRS_NT / WAVE>(full, left, cnt);
+    if (full) rest[pos] = k0;
+    __syncthreads();
+    if (tid < left) {
+        const int k = rest[tid];
+        int a = slot[pi[k]], b = slot[pj[k]];
+        uint4 ua = P[a], ub = P[b];
+        DPart<R> pa = load_part<R>(O[a], Q[a], ua.w, tp);
+        DPart<R> pb = load_part<R>(O[b], Q[b], ub.w, tp);
+        const V3<R> r = image(ua, ub);
+        // FP32: the terms added in FP64, as every FP32 kernel adds them; FP64: the
+        // reference's own order of the sum
+        double e = sizeof(R) == 8 ? (double)pair_energy<R>(pp[ua.w * sc.nt + ub.w], pa, pb, r, sqmaxcut)
+                                  : pair_energy_d<R>(pp[ua.w * sc.nt + ub.w], pa, pb, r, sqmaxcut);
+        if (ct.cw) {
+            int bit = cw_bit(pj[k] - pi[k]), cw = ct.cw[pi[k]];
+            if (bit >= 0 && ((cw >> bit) & 1))
+                e += bond_energy(ct.mol[cw >> 8], ct.pp64[ua.w * sc.nt + ub.w], cw_rel(bit), fx_r12(ua, ub, sc.Ld),
+                                 unit64(O[a].x, O[a].y, O[a].z), unit64(O[a].w, Q[a].x, Q[a].y),
+                                 unit64(O[b].x, O[b].y, O[b].z), unit64(O[b].w, Q[b].x, Q[b].y));
+        }
+        out[k] = e;
     }
-    out[k] = e;
 }
 
 // ---------------------------------------------------------------- overlaps
@@ -3645,35 +3695,70 @@ __device__ __forceinline__ int axis_offsets(int nc, int* off) {
 // Pairs (ID_i < ID_j) within rc over a cell list with cells >= rc wide: one
 // thread per particle (sorted position), counting (write == nullptr) or
 // writing at its offset.  Within a particle the pairs come in cell-list order.
-__global__ void k_pair_list(int n, const uint4* __restrict__ P, const int* __restrict__ ID, const int* __restrict__ starts,
-                            Grid g, double rc2, double bx, double by, double bz, int* __restrict__ count,
-                            const int* __restrict__ offset, int* __restrict__ pi, int* __restrict__ pj) {
-    int a = blockIdx.x * blockDim.x + threadIdx.x;
+// 32 lanes per particle, a stencil cell each (a thread per particle walked its
+// 27 cells alone: 66 us for 24,300 particles, 19 us so).  Rows by ID: count[i] pairs of
+// particle i with larger IDs; with `offset` the pairs themselves, a row's in
+// any order (k_pair_rank orders them).
+__global__ __launch_bounds__(256) void k_pair_list(int n, const uint4* __restrict__ P, const int* __restrict__ ID,
+                                                   const int* __restrict__ starts, Grid g, double rc2, double bx,
+                                                   double by, double bz, int* __restrict__ count,
+                                                   const int* __restrict__ offset, int* __restrict__ pi,
+                                                   int* __restrict__ pj) {
+    const int a = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 5), l = (int)(threadIdx.x & 31);
     if (a >= n) return;
-    uint4 ua = P[a];
-    int ida = ID[a];
-    int cx = axis_cell(ua.x, g.sh[0], g.nc[0]), cy = axis_cell(ua.y, g.sh[1], g.nc[1]), cz = axis_cell(ua.z, g.sh[2], g.nc[2]);
+    const uint4 ua = P[a];
+    const int ida = ID[a];
+    const int cx = axis_cell(ua.x, g.sh[0], g.nc[0]), cy = axis_cell(ua.y, g.sh[1], g.nc[1]),
+              cz = axis_cell(ua.z, g.sh[2], g.nc[2]);
     int ox[3], oy[3], oz[3];
-    int nx = axis_offsets(g.nc[0], ox), ny = axis_offsets(g.nc[1], oy), nz = axis_offsets(g.nc[2], oz);
-    int k = 0, base = offset ? offset[a] : 0;
-    for (int iz = 0; iz < nz; iz++)
-        for (int iy = 0; iy < ny; iy++)
-            for (int ix = 0; ix < nx; ix++) {
-                int c = ((cx + ox[ix] + g.nc[0]) % g.nc[0]) +
-                        g.nc[0] * (((cy + oy[iy] + g.nc[1]) % g.nc[1]) + g.nc[1] * ((cz + oz[iz] + g.nc[2]) % g.nc[2]));
-                for (int b = starts[c]; b < starts[c + 1]; b++) {
-                    int idb = ID[b];
-                    if (idb <= ida) continue;
-                    if (fx_r2_fp64(ua, P[b], bx, by, bz) <= rc2) {
-                        if (offset) {
-                            pi[base + k] = ida;
-                            pj[base + k] = idb;
-                        }
-                        k++;
-                    }
-                }
-            }
-    if (!offset) count[a] = k;
+    const int nx = axis_offsets(g.nc[0], ox), ny = axis_offsets(g.nc[1], oy), nz = axis_offsets(g.nc[2], oz);
+    int beg = 0, end = 0;
+    if (l < nx * ny * nz) {
+        const int ix = l % nx, iy = (l / nx) % ny, iz = l / (nx * ny);
+        const int c = ((cx + ox[ix] + g.nc[0]) % g.nc[0]) +
+                      g.nc[0] * (((cy + oy[iy] + g.nc[1]) % g.nc[1]) + g.nc[1] * ((cz + oz[iz] + g.nc[2]) % g.nc[2]));
+        beg = starts[c];
+        end = starts[c + 1];
+    }
+    int k = 0;
+    for (int b = beg; b < end; b++) k += ID[b] > ida && fx_r2_fp64(ua, P[b], bx, by, bz) <= rc2 ? 1 : 0;
+    int incl = k;   // prefix over the particle's 32 lanes
+    for (int o = 1; o < 32; o <<= 1) {
+        const int y = __shfl_up(incl, o, 32);
+        if (l >= o) incl += y;
+    }
+    if (!offset) {
+        if (l == 31) count[ida] = incl;
+        return;
+    }
+    int at = offset[ida] + incl - k;
+    for (int b = beg; k > 0 && b < end; b++) {
+        const int idb = ID[b];
+        if (idb > ida && fx_r2_fp64(ua, P[b], bx, by, bz) <= rc2) {
+            pi[at] = ida;
+            pj[at++] = idb;
+            k--;
+        }
+    }
+}
+
+// The interleaved pair list in lexicographic order: row i's partners to the
+// places their rank in the row gives.  32 lanes per row, a rank in as many
+// steps as the row is long: for rows of at most PAIR_RANK_ROW (sorting 390,000
+// keys on the host took longer than the rest of the call; a row of a few
+// hundred costs as much as the host's sort would).
+#define PAIR_RANK_ROW 512
+__global__ __launch_bounds__(256) void k_pair_rank(int n, const int* __restrict__ offset, const int* __restrict__ pj,
+                                                   int2* __restrict__ list) {
+    const int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 5), l = (int)(threadIdx.x & 31);
+    if (i >= n) return;
+    const int b = offset[i], e = offset[i + 1];
+    for (int k = b + l; k < e; k += 32) {
+        const int v = pj[k];
+        int r = b;
+        for (int q = b; q < e; q++) r += pj[q] < v ? 1 : 0;
+        list[r] = make_int2(i, v);
+    }
 }
 
 // Connected components of the graph {pairs with energy <= thr}: hook the
@@ -3734,20 +3819,26 @@ __global__ void k_align_pairs(long m, const int* __restrict__ pi, const int* __r
     out[k] = v;
 }
 
-// Q = sum over particles of u u^T (6 unique components, FP64), per block
-__global__ void k_nematic_q(int n, const float4* __restrict__ O, double* __restrict__ out) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+// Q = sum over particles of u u^T (6 unique components, FP64): per-thread sums
+// over a grid of at most NEMATIC_BLOCKS, one addition per block and component
+// (an addition per wave serialised on six addresses: 30 us for 24,300 particles).
+#define NEMATIC_BLOCKS 64
+__global__ __launch_bounds__(256) void k_nematic_q(int n, const float4* __restrict__ O, double* __restrict__ out) {
+    __shared__ double part[4][6];
     double q[6] = {0, 0, 0, 0, 0, 0};
-    if (i < n) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         float4 o = O[i];
         double x = o.x, y = o.y, z = o.z, inv = 1.0 / sqrt(x * x + y * y + z * z);
         x *= inv; y *= inv; z *= inv;
-        q[0] = x * x; q[1] = y * y; q[2] = z * z; q[3] = x * y; q[4] = x * z; q[5] = y * z;
+        q[0] += x * x; q[1] += y * y; q[2] += z * z; q[3] += x * y; q[4] += x * z; q[5] += y * z;
     }
     for (int c = 0; c < 6; c++) {
         double v = wave_sum(q[c]);
-        if (lane_id() == 0) atomicAdd(&out[c], v);
+        if (lane_id() == 0) part[threadIdx.x >> 6][c] = v;
     }
+    __syncthreads();
+    const int c = (int)threadIdx.x;
+    if (c < 6) atomicAdd(&out[c], (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]));
 }
 
 // ------------------------------------------------------------- chain moves
@@ -5731,7 +5822,7 @@ int sc_build_cells(sc_ctx* ctx, int r, const uint32_t shift[3], int32_t* cell_of
 
 // All pairs within rc on the device: cell list with cells >= rc, count pass,
 // scan, write pass.  Leaves the pairs (IDs, i < j) in d_pi / d_pj.
-static int device_pairs(sc_ctx* ctx, double rc, long* total) {
+static int device_pairs(sc_ctx* ctx, double rc, long* total, bool write = true) {
     int n = ctx->n;
     *total = 0;
     if (n < 2) return SC_OK;
@@ -5746,7 +5837,7 @@ static int device_pairs(sc_ctx* ctx, double rc, long* total) {
             return rc_;
         ctx->pcount_cap = n + 1;
     }
-    int c = ctx->cur, nb = (n + 255) / 256;
+    int c = ctx->cur, nb = (n + 7) / 8;
     const Grid& g = ctx->g;
     double rc2 = rc * rc;
     // counts into d_label (scratch), offsets into d_pcount
@@ -5758,17 +5849,17 @@ static int device_pairs(sc_ctx* ctx, double rc, long* total) {
     HIPCK(hipMemcpyAsync(&tot, ctx->d_pcount + n, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIPCK(hipStreamSynchronize(ctx->stream));
     if (tot < 0) return fail(ctx, SC_ECAPACITY, "more than 2^31 pairs");
+    *total = tot;
+    if (!write || tot == 0) return SC_OK;
     if (tot > ctx->pair_cap) {
         if ((rc_ = dalloc(ctx, &ctx->d_pi, (size_t)tot)) || (rc_ = dalloc(ctx, &ctx->d_pj, (size_t)tot)) ||
             (rc_ = dalloc(ctx, &ctx->d_pe, (size_t)tot)))
             return rc_;
         ctx->pair_cap = tot;
     }
-    if (tot > 0)
-        SC_LAUNCH(k_pair_list, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->P[c], ctx->ID[c], ctx->starts, g, rc2,
-                  ctx->box[0], ctx->box[1], ctx->box[2], (int*)nullptr, (const int*)ctx->d_pcount, ctx->d_pi, ctx->d_pj);
+    SC_LAUNCH(k_pair_list, dim3(nb), dim3(256), 0, ctx->stream, n, ctx->P[c], ctx->ID[c], ctx->starts, g, rc2,
+              ctx->box[0], ctx->box[1], ctx->box[2], (int*)nullptr, (const int*)ctx->d_pcount, ctx->d_pi, ctx->d_pj);
     HIPCK(hipGetLastError());
-    *total = tot;
     return SC_OK;
 }
 
@@ -5776,11 +5867,23 @@ static int sc_neighbor_pairs_impl(sc_ctx* ctx, double rc, int32_t* pairs, long c
     if (!ctx || !count || !(rc > 0)) return SC_EINVAL;
     if (!ctx->have_state) return fail(ctx, SC_ESTATE, "no configuration loaded");
     long tot = 0;
-    int rc_ = device_pairs(ctx, rc, &tot);
+    int rc_ = device_pairs(ctx, rc, &tot, pairs != nullptr);
     if (rc_) return rc_;
     *count = tot;
-    if (!pairs || tot == 0) return SC_OK;
-    // returned in lexicographic (i, j) order
+    const long m = std::min(cap, tot);
+    if (!pairs || m <= 0) return SC_OK;
+    // in lexicographic (i, j) order
+    int row = 0;
+    HIPCK(hipMemcpyAsync(&row, ctx->d_maxocc, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    HIPCK(hipStreamSynchronize(ctx->stream));
+    if (row <= PAIR_RANK_ROW) {
+        int2* list = (int2*)ctx->d_pe;   // no energies of these pairs yet
+        SC_LAUNCH(k_pair_rank, dim3((ctx->n + 7) / 8), dim3(256), 0, ctx->stream, ctx->n, (const int*)ctx->d_pcount,
+                  (const int*)ctx->d_pj, list);
+        HIPCK(hipMemcpyAsync(pairs, list, (size_t)m * sizeof(int2), hipMemcpyDeviceToHost, ctx->stream));
+        HIPCK(hipStreamSynchronize(ctx->stream));
+        return SC_OK;
+    }
     std::vector<int32_t> hi(tot), hj(tot);
     HIPCK(hipMemcpyAsync(hi.data(), ctx->d_pi, tot * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
     HIPCK(hipMemcpyAsync(hj.data(), ctx->d_pj, tot * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -5788,7 +5891,6 @@ static int sc_neighbor_pairs_impl(sc_ctx* ctx, double rc, int32_t* pairs, long c
     std::vector<uint64_t> key(tot);
     for (long k = 0; k < tot; k++) key[k] = ((uint64_t)(uint32_t)hi[k] << 32) | (uint32_t)hj[k];
     std::sort(key.begin(), key.end());
-    long m = std::min(cap, tot);
     for (long k = 0; k < m; k++) {
         pairs[2 * k] = (int32_t)(key[k] >> 32);
         pairs[2 * k + 1] = (int32_t)(key[k] & 0xffffffffu);
@@ -5817,8 +5919,8 @@ static int sc_cluster_labels_impl(sc_ctx* ctx, double threshold, int32_t* labels
     SysConst sc = sysconst(ctx, ctx->box);
     int c = ctx->cur;
     if (m > 0)
-        SC_LAUNCH(k_pairs<double>, dim3((unsigned)((m + 127) / 128)), dim3(128), 0, ctx->stream, (int)m, ctx->d_pi,
-                  ctx->d_pj, ctx->slot, sc, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp64, ctx->d_tp64, ctx->sqmaxcut,
+        SC_LAUNCH(k_pairs<double>, dim3((unsigned)((m + PAIRS_NT - 1) / PAIRS_NT)), dim3(PAIRS_NT), 0, ctx->stream,
+                  (int)m, ctx->d_pi, ctx->d_pj, ctx->slot, sc, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp64, ctx->d_tp64, ctx->sqmaxcut,
                   chain_tab(ctx), ctx->d_pe);
     SC_LAUNCH(k_iota, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, ctx->d_label);
     for (int it = 0; it < 4 * n + 64; it++) {
@@ -5887,7 +5989,7 @@ static int sc_nematic_order_impl(sc_ctx* ctx, double* s2, double director[3]) {
     HIPCK(hipSetDevice(ctx->device));
     if (!ctx->d_q6 && (rc_ = dalloc(ctx, &ctx->d_q6, 6))) return rc_;
     HIPCK(hipMemsetAsync(ctx->d_q6, 0, 6 * sizeof(double), ctx->stream));
-    SC_LAUNCH(k_nematic_q, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, ctx->O[ctx->cur], ctx->d_q6);
+    SC_LAUNCH(k_nematic_q, dim3(std::min((n + 255) / 256, NEMATIC_BLOCKS)), dim3(256), 0, ctx->stream, n, ctx->O[ctx->cur], ctx->d_q6);
     HIPCK(hipGetLastError());
     double q6[6];
     HIPCK(hipMemcpyAsync(q6, ctx->d_q6, sizeof(q6), hipMemcpyDeviceToHost, ctx->stream));
@@ -6002,8 +6104,8 @@ static int sc_write_clusters_impl(sc_ctx* ctx, double threshold, long sweep, cha
     SysConst sc = sysconst(ctx, ctx->box);
     int c = ctx->cur;
     if (m > 0) {
-        SC_LAUNCH(k_pairs<double>, dim3((unsigned)((m + 127) / 128)), dim3(128), 0, ctx->stream, (int)m, ctx->d_pi,
-                  ctx->d_pj, ctx->slot, sc, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp64, ctx->d_tp64, ctx->sqmaxcut,
+        SC_LAUNCH(k_pairs<double>, dim3((unsigned)((m + PAIRS_NT - 1) / PAIRS_NT)), dim3(PAIRS_NT), 0, ctx->stream,
+                  (int)m, ctx->d_pi, ctx->d_pj, ctx->slot, sc, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp64, ctx->d_tp64, ctx->sqmaxcut,
                   chain_tab(ctx), ctx->d_pe);
         HIPCK(hipMemcpyAsync(hi.data(), ctx->d_pi, m * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
         HIPCK(hipMemcpyAsync(hj.data(), ctx->d_pj, m * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -6064,11 +6166,13 @@ static int sc_pair_energies_impl(sc_ctx* ctx, int m, const int32_t* i, const int
     SysConst sc = sysconst(ctx, ctx->box);
     int c = ctx->cur;
     if (fp64)
-        hipLaunchKernelGGL(k_pairs<double>, dim3((m + 127) / 128), dim3(128), 0, ctx->stream, m, ctx->d_i, ctx->d_j,
+        hipLaunchKernelGGL(k_pairs<double>, dim3((m + PAIRS_NT - 1) / PAIRS_NT), dim3(PAIRS_NT), 0, ctx->stream, m,
+                           ctx->d_i, ctx->d_j,
                            ctx->slot, sc, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp64, ctx->d_tp64, ctx->sqmaxcut,
                            chain_tab(ctx), ctx->d_out);
     else
-        hipLaunchKernelGGL(k_pairs<float>, dim3((m + 127) / 128), dim3(128), 0, ctx->stream, m, ctx->d_i, ctx->d_j,
+        hipLaunchKernelGGL(k_pairs<float>, dim3((m + PAIRS_NT - 1) / PAIRS_NT), dim3(PAIRS_NT), 0, ctx->stream, m,
+                           ctx->d_i, ctx->d_j,
                            ctx->slot, sc, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp32, ctx->d_tp32, (float)ctx->sqmaxcut,
                            chain_tab(ctx), ctx->d_out);
     HIPCK(hipGetLastError());
@@ -6107,11 +6211,13 @@ static int sc_pair_energies_noalloc_impl(sc_ctx* ctx, int m, const int32_t* i, c
     SysConst sc = sysconst(ctx, ctx->box);
     int c = ctx->cur;
     if (fp64)
-        hipLaunchKernelGGL(k_pairs<double>, dim3((m + 127) / 128), dim3(128), 0, ctx->stream, m, di, dj, ctx->slot, sc,
+        hipLaunchKernelGGL(k_pairs<double>, dim3((m + PAIRS_NT - 1) / PAIRS_NT), dim3(PAIRS_NT), 0, ctx->stream, m,
+                           di, dj, ctx->slot, sc,
                            ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp64, ctx->d_tp64, ctx->sqmaxcut, chain_tab(ctx),
                            dout);
     else
-        hipLaunchKernelGGL(k_pairs<float>, dim3((m + 127) / 128), dim3(128), 0, ctx->stream, m, di, dj, ctx->slot, sc,
+        hipLaunchKernelGGL(k_pairs<float>, dim3((m + PAIRS_NT - 1) / PAIRS_NT), dim3(PAIRS_NT), 0, ctx->stream, m,
+                           di, dj, ctx->slot, sc,
                            ctx->P[c], ctx->O[c], ctx->Q[c], ctx->d_pp32, ctx->d_tp32, (float)ctx->sqmaxcut,
                            chain_tab(ctx), dout);
     HIPCK(hipGetLastError());
