@@ -20,6 +20,7 @@
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <numeric>
 #include <vector>
 
 // Per-expression FMA contraction for the whole file (the pair header's
@@ -295,49 +296,65 @@ __global__ void k_cell_count(int n, const uint4* __restrict__ P, Grid g, int* __
 }
 
 // exclusive scan of counts[0..ncell) into starts[0..ncell] by one block of
-// 1024 threads, in chunks of 8192 staged through LDS (coalesced loads, each
-// thread scans 8 contiguous entries, wave prefix sums via shuffles); also the
-// maximum occupancy and the number of non-empty cells.
+// 1024 threads, in chunks of 8192: a thread scans 8 contiguous entries in
+// registers (two 16-byte loads and stores), the waves' sums meet in LDS behind
+// one barrier, and the next chunk's entries are on their way meanwhile.  Also
+// the maximum occupancy and the number of non-empty cells.  The chunk's chain
+// of latencies bounds it: 24,300 entries 5.5 us, 15 us with each chunk's loads
+// waited for and LDS between (64 replicas' cells: 20.5 to 6.4 us).
 __global__ __launch_bounds__(1024) void k_scan(int ncell, const int* __restrict__ counts, int* __restrict__ starts,
                                                 int* __restrict__ maxocc, int* __restrict__ nonempty) {
-    __shared__ int tile[8192];
-    __shared__ int wsum[16];
+    __shared__ int wsum[32];
     __shared__ int wmax[16], wne[16];
     int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     int carry = 0, mx = 0, ne = 0;
-    for (int c0 = 0; c0 < ncell; c0 += 8192) {
-        for (int i = 0; i < 8; i++) {
-            int idx = c0 + t + 1024 * i;
-            tile[t + 1024 * i] = idx < ncell ? counts[idx] : 0;
+    auto load = [&](int idx, int* v) {
+        if (idx + 8 <= ncell) {
+            const int4 a = *(const int4*)(counts + idx), b = *(const int4*)(counts + idx + 4);
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+            v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        } else {
+            for (int i = 0; i < 8; i++) v[i] = idx + i < ncell ? counts[idx + i] : 0;
         }
-        __syncthreads();
-        int v[8], sum = 0;
+    };
+    int v[8], nx[8];
+    load(8 * t, nx);
+    for (int c0 = 0, par = 0; c0 < ncell; c0 += 8192, par ^= 16) {
+        const int idx = c0 + 8 * t;
+        int sum = 0;
         for (int i = 0; i < 8; i++) {
-            v[i] = tile[8 * t + i];
+            v[i] = nx[i];
             sum += v[i];
             mx = max(mx, v[i]);
             ne += v[i] > 0 ? 1 : 0;
         }
+        load(idx + 8192, nx);
         int incl = sum;
         for (int o = 1; o < 64; o <<= 1) {
             int y = __shfl_up(incl, o, 64);
             if (lane >= o) incl += y;
         }
-        if (lane == 63) wsum[wv] = incl;
+        if (lane == 63) wsum[par + wv] = incl;
         __syncthreads();
         int wpre = 0, total = 0;
         for (int w = 0; w < 16; w++) {
-            if (w < wv) wpre += wsum[w];
-            total += wsum[w];
+            if (w < wv) wpre += wsum[par + w];
+            total += wsum[par + w];
         }
         int run = carry + wpre + incl - sum;
         for (int i = 0; i < 8; i++) {
-            int idx = c0 + 8 * t + i;
-            if (idx < ncell) starts[idx] = run;
-            run += v[i];
+            const int x = v[i];
+            v[i] = run;
+            run += x;
+        }
+        if (idx + 8 <= ncell) {
+            *(int4*)(starts + idx) = make_int4(v[0], v[1], v[2], v[3]);
+            *(int4*)(starts + idx + 4) = make_int4(v[4], v[5], v[6], v[7]);
+        } else {
+            for (int i = 0; i < 8; i++)
+                if (idx + i < ncell) starts[idx + i] = v[i];
         }
         carry += total;
-        __syncthreads();
     }
     for (int o = 32; o >= 1; o >>= 1) {
         mx = max(mx, __shfl_xor(mx, o, 64));
@@ -2914,7 +2931,12 @@ struct RepPass {
 // One colour pass of every replica of a batch in one launch: the launch's
 // blocks are the replicas' active cells back to back; a block finds its
 // replica by binary search over blk_off (a replica without active cells
-// shares its offset with the next one, and the search takes the last).
+// shares its offset with the next one, and the search takes the last).  The
+// replicas with the longest cells come first, dealt to the XCDs in turn: a
+// small replica's few wide cells run several times as long as the others'
+// (64 replicas of 500-8000 particles in input order, each XCD a contiguous run
+// of them: 1869 us a pass, the end of it a few blocks alone on the chip; so
+// 1518 us).
 template <int DA, int NW>
 __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_batch(const RepPass* __restrict__ rp, int nrep,
                                                       const int* __restrict__ starts, uint4* __restrict__ P,
@@ -2925,7 +2947,7 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_batch(const RepPass* __r
                                                       const unsigned char* __restrict__ mlp_img, MlpConst mc,
                                                       ChainTab ct, unsigned long long* __restrict__ stats,
                                                       double* __restrict__ de_sum, int* __restrict__ flag) {
-    int lb = xcd_slab_index((int)blockIdx.x, (int)gridDim.x);
+    const int lb = (int)blockIdx.x;
     int lo = 0, hi = nrep - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
@@ -2952,7 +2974,7 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_batch_spec(const Rep
                                                                    unsigned long long* __restrict__ stats,
                                                                    double* __restrict__ de_sum,
                                                                    int* __restrict__ flag) {
-    int lb = xcd_slab_index((int)blockIdx.x, (int)gridDim.x);
+    const int lb = (int)blockIdx.x;
     int lo = 0, hi = nrep - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
@@ -7135,7 +7157,7 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
     std::vector<SweepPlan> plans(R);
     std::vector<std::array<uint32_t, 3>> shifts(R);
     std::vector<std::array<int, 27>> vcols(R);
-    std::vector<int> nvis(R), vfac(R);
+    std::vector<int> nvis(R), vfac(R), byload(R);
     long launches = 0;
     HIPCK(hipEventRecord(ctx->ev0, ctx->stream));
     for (int sidx = 0; sidx < nsweeps; sidx++) {
@@ -7186,10 +7208,16 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
             nvis[q] = nv / vfac[q];
             nlaunch = std::max(nlaunch, nvis[q]);
         }
+        // by trials per cell, most first
+        std::iota(byload.begin(), byload.end(), 0);
+        std::stable_sort(byload.begin(), byload.end(), [&](int a, int b) {
+            return (double)ctx->rep_n[a] * vfac[a] * ctx->rep_ncell[b] > (double)ctx->rep_n[b] * vfac[b] * ctx->rep_ncell[a];
+        });
         for (int ci = 0; ci < nlaunch; ci++) {
             int boff = 0;
-            for (int q = 0; q < R; q++) {
-                RepPass& P_ = hp[(size_t)ci * R + q];
+            for (int k_ = 0; k_ < R; k_++) {
+                const int q = byload[k_];
+                RepPass& P_ = hp[(size_t)ci * R + k_];
                 const Grid& g = ctx->rep_grid[q].g;
                 P_.g = g;
                 P_.sc = sysconst_box(ctx, ctx->rep_box[q]);
