@@ -3963,15 +3963,29 @@ __global__ __launch_bounds__(256) void k_chain_anchor(int nchain, const int* __r
     if (v) ccell_id[f + lane] = G.ext2 <= rho2 ? cell : -1;
 }
 
-// the pair functor of a queued pair as a call of its own (its registers are
-// not added to those of the surrounding scan)
+// The pair functor of a queued pair as a call of its own (its registers are
+// not added to those of the surrounding scan), in its canonical order, the
+// higher ID as part1 (allToAll's): the lanes that swap exchange the operands, so
+// a wave walks the functor once (a call per order held it twice, 120 KB of
+// code, and a wave with both orders walked both: the staged pass of 10,001
+// chains 2300 us, 1588 us so).
 __device__ __attribute__((noinline)) double chain_pair(const PP32* __restrict__ pp, const TP32* __restrict__ tp, int nt,
                                                        float sqmaxcut, uint4 ua, float4 oa, float2 qa, uint4 ub,
                                                        float4 ob, float2 qb, V3<float> r, bool sw) {
+    if (sw) {
+        const uint32_t t = ua.w;   // of the records, the functor takes the types
+        ua.w = ub.w;
+        ub.w = t;
+        const float4 o = oa;
+        oa = ob;
+        ob = o;
+        const float2 q = qa;
+        qa = qb;
+        qb = q;
+        r = mk<float>(-r.x, -r.y, -r.z);
+    }
     DPart<float> pa = load_part<float>(oa, qa, ua.w, tp);
     DPart<float> pb = load_part<float>(ob, qb, ub.w, tp);
-    // the pair in its canonical order, the higher ID as part1 (allToAll's)
-    if (sw) return pair_energy_d<float>(pp[ub.w * nt + ua.w], pb, pa, mk<float>(-r.x, -r.y, -r.z), sqmaxcut);
     return pair_energy_d<float>(pp[ua.w * nt + ub.w], pa, pb, r, sqmaxcut);
 }
 
@@ -4354,8 +4368,13 @@ __global__ __launch_bounds__(WAVE * NW) void k_chain_pass(Grid g, Grid gc, SysCo
 // coarse cell (the region its molecules' particles and their neighbours can
 // occupy during the pass), leaving out the particles of molecules that may
 // move in another active cell (they stay beyond maxcut).  The trials then
-// read nothing but LDS; an accepted move updates the staged copy and global
-// memory.  The region is found through the fine cell list (whole cells
+// read nothing but LDS; an accepted move updates the staged copy, and the
+// cell's own particles go back to global memory at the end.  A trial is a
+// chain of latencies (its molecule found and moved in FP64 ~9,000 cycles, the
+// items ~34,000, the decision and commit ~4,000): one wave proposes the next
+// molecule while the others finish this one's items.  10,001 chains of three:
+// 2543 us a pass with every step in turn, 2300 us with that overlap, 1588 us
+// with the functor's single copy (chain_pair) as well.  The region is found through the fine cell list (whole cells
 // overlapping it, filtered by position).  A block whose region holds more
 // than `cap` particles makes no move in this pass (its trials are counted as
 // rejected, and the block in chain_skipped).
@@ -4366,6 +4385,15 @@ __global__ __launch_bounds__(WAVE * NW) void k_chain_pass(Grid g, Grid gc, SysCo
 #define CHAIN_OWN 0x40000000      // stage ID flag: a particle that may move in this pass
 #define CHAIN_IDMASK 0x00ffffff
 
+// ints of the space the staging and the trials share; the trials put 3 ints of
+// alignment, CHAIN_ST_REC bytes of records and 16-bit queues there
+#define CHAIN_ST_REC (CHAIN_MAXM * (4 * 16 + 2 * 8 + 4))
+__host__ __device__ constexpr size_t chain_st_shared(int nw) {
+    return (size_t)nw * (CHAIN_QCAP + 64) > (size_t)2 * CHAIN_ST_RCAP + 1 ? (size_t)nw * (CHAIN_QCAP + 64)
+                                                                          : (size_t)2 * CHAIN_ST_RCAP + 1;
+}
+static_assert(12 + CHAIN_ST_REC + 2 * CHAIN_NW * (CHAIN_QCAP + 64) <= 4 * chain_st_shared(CHAIN_NW),
+              "the trials' records and queues exceed the shared space");
 struct ChainStLayout {
     size_t su, so, sq, red, ints, sid, total;
 };
@@ -4378,9 +4406,10 @@ __host__ __device__ inline ChainStLayout chain_st_layout(int nw, int cap) {
     L.sq = o; o += (size_t)cap * 8;
     L.red = o; o += (size_t)2 * nw * 8;
     // bidx, clist, spre (stage start of each region cell), then the region
-    // prefix (staging) sharing its space with the queues and stencil ranges (trials)
+    // prefix (staging) sharing its space with what the trials need: the second
+    // set of trial records and the waves' queues and stencil ranges
     L.ints = o;
-    size_t shared = std::max((size_t)2 * CHAIN_ST_RCAP + 1, (size_t)nw * (CHAIN_QCAP + 64));
+    size_t shared = chain_st_shared(nw);
     o += sizeof(int) * ((size_t)CHAIN_MAXM + CHAIN_ST_LCAP + CHAIN_ST_OCAP + CHAIN_ST_RCAP + 1 + shared + nw + 4);
     L.sid = o; o += (size_t)cap * 4;
     L.total = o;
@@ -4397,7 +4426,7 @@ __device__ double chain_item_energy_st(uint4 ua, float4 oa, float2 qa, int idk, 
                                        const int* f0,
                                        const int* fn, const int* spre, const int* own, int nown, const SysConst& sc,
                                        const PP32* __restrict__ pp, const TP32* __restrict__ tp, const uint4* su,
-                                       const float4* so, const float2* sq, const int* sid, int* queue, int* spr) {
+                                       const float4* so, const float2* sq, const int* sid, uint16_t* queue, uint16_t* spr) {
     int lane = lane_id();
     int c = cell_of_u(g, ua.x, ua.y, ua.z);
     int cx = c % g.nc[0], cy = (c / g.nc[0]) % g.nc[1], cz = c / (g.nc[0] * g.nc[1]);
@@ -4422,8 +4451,8 @@ __device__ double chain_item_energy_st(uint4 ua, float4 oa, float2 qa, int idk, 
     }
     int total = __shfl(v, WAVE - 1, WAVE), all = total + nown;
     if (lane < 32) {
-        spr[lane] = v - cnt;
-        spr[32 + lane] = beg;
+        spr[lane] = (uint16_t)(v - cnt);
+        spr[32 + lane] = (uint16_t)beg;
     }
     wave_lds_sync();
     double acc = 0.0;
@@ -4459,7 +4488,7 @@ __device__ double chain_item_energy_st(uint4 ua, float4 oa, float2 qa, int idk, 
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             unsigned long long msk = __ballot(need[u]);
-            if (need[u]) queue[qn + wave_prefix(msk)] = si[u];
+            if (need[u]) queue[qn + wave_prefix(msk)] = (uint16_t)si[u];
             qn += __popcll(msk);
         }
         wave_lds_sync();
@@ -4480,7 +4509,7 @@ __device__ double chain_item_energy_st(uint4 ua, float4 oa, float2 qa, int idk, 
             int rest = qn - take;
             int cq = lane < rest ? queue[take + lane] : 0;
             wave_lds_sync();
-            if (lane < rest) queue[lane] = cq;
+            if (lane < rest) queue[lane] = (uint16_t)cq;
             wave_lds_sync();
             qn = rest;
         }
@@ -4504,26 +4533,40 @@ __global__ __launch_bounds__(WAVE * NW) void k_chain_pass_st(Grid g, Grid gc, Sy
                                                              double* __restrict__ de_sum) {
     extern __shared__ __align__(16) unsigned char smem[];
     const ChainStLayout L = chain_st_layout(NW, cap);
-    uint4* Uo = (uint4*)smem;
-    uint4* Un = Uo + CHAIN_MAXM;
-    float4* Oo = (float4*)(Un + CHAIN_MAXM);
-    float4* On = Oo + CHAIN_MAXM;
     uint4* su = (uint4*)(smem + L.su);
     float4* so = (float4*)(smem + L.so);
-    float2* Qo = (float2*)(smem + L.so + (size_t)cap * 16);
-    float2* Qn = Qo + CHAIN_MAXM;
     float2* sq = (float2*)(smem + L.sq);
     double* red = (double*)(smem + L.red);
-    int* bidx = (int*)(smem + L.ints);   // stage index of the trial molecule's particles
-    int* clist = bidx + CHAIN_MAXM;
+    int* clist = (int*)(smem + L.ints) + CHAIN_MAXM;
     int* own = clist + CHAIN_ST_LCAP;    // stage indices of the particles of the cell's movable molecules
     int* spre = own + CHAIN_ST_OCAP;     // stage index of each region cell's first particle (+ the end)
     int* rpre = spre + CHAIN_ST_RCAP + 1; // region cells: prefix of counts, cell starts (staging only)
     int* rbeg = rpre + CHAIN_ST_RCAP + 1;
     const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1), w = tid >> 6;
-    int* queue = rpre + w * (CHAIN_QCAP + 64);   // the same space, once the stage is built
-    int* spr = queue + CHAIN_QCAP;               // this wave's stencil: 32 prefix + 32 starts
-    int* misc = rpre + (2 * CHAIN_ST_RCAP + 1 > NW * (CHAIN_QCAP + 64) ? 2 * CHAIN_ST_RCAP + 1 : NW * (CHAIN_QCAP + 64));
+    // the same space, once the stage is built
+    unsigned char* rec1 = smem + spec_align((size_t)((unsigned char*)rpre - smem), 16);
+    uint16_t* queue = (uint16_t*)(rec1 + CHAIN_ST_REC) + w * (CHAIN_QCAP + 64);
+    uint16_t* spr = queue + CHAIN_QCAP;   // this wave's stencil: 32 prefix + 32 starts
+    int* misc = rpre + chain_st_shared(NW);
+    // the two sets of trial records: the molecule's particles at the old and the
+    // new state and their stage indices
+    struct Rec {
+        uint4 *Uo, *Un;
+        float4 *Oo, *On;
+        float2 *Qo, *Qn;
+        int* bidx;
+    };
+    auto record = [&](int b) {
+        Rec R;
+        R.Uo = b ? (uint4*)rec1 : (uint4*)smem;
+        R.Un = R.Uo + CHAIN_MAXM;
+        R.Oo = (float4*)(R.Un + CHAIN_MAXM);
+        R.On = R.Oo + CHAIN_MAXM;
+        R.Qo = b ? (float2*)(R.On + CHAIN_MAXM) : (float2*)(smem + L.so + (size_t)cap * 16);
+        R.Qn = R.Qo + CHAIN_MAXM;
+        R.bidx = b ? (int*)(R.Qn + CHAIN_MAXM) : (int*)(smem + L.ints);
+        return R;
+    };
     int* sid = (int*)(smem + L.sid);
     int b = blockIdx.x;
     int bx = b % cp.nact[0], by = (b / cp.nact[0]) % cp.nact[1], bz = b / (cp.nact[0] * cp.nact[1]);
@@ -4696,90 +4739,120 @@ __global__ __launch_bounds__(WAVE * NW) void k_chain_pass_st(Grid g, Grid gc, Sy
     int ntrial = (int)floor(mean) + (u01d(rd.x, rd.y) < mean - floor(mean) ? 1 : 0);
     unsigned long long n_dacc = 0, n_dtry = 0, n_racc = 0, n_rtry = 0, n_rej = 0;
     double dsum = 0.0;
+    // Trial t's molecule, its old and its new state, by one wave into record t & 1:
+    // misc[NW + 2 (t & 1)] gets its size and reject code, the next entry its first
+    // particle.
+    auto propose_trial = [&](int t) {
+        const Rec R = record(t & 1);
+        U4 c = ctr;
+        c.x = (uint32_t)t;
+        c.w = cp.pass_hi << 2;
+        const U4 ra = philox(c, cp.key0, cp.key1);
+        const int k = clist[(int)(((uint64_t)ra.x * (uint64_t)total) >> 32)];
+        const int f = cfirst[k], m = csize[k];
+        if (lane < m) R.bidx[lane] = -1;
+        wave_lds_sync();
+        for (int i = lane; i < nown_s; i += WAVE) {   // a movable molecule's particles are all in `own`
+            const int id = sid[own[i]] & CHAIN_IDMASK;
+            if (id >= f && id < f + m) R.bidx[id - f] = own[i];
+        }
+        wave_lds_sync();
+        // a particle outside the region means the molecule is wider than rho
+        const bool miss = __ballot(lane < m && R.bidx[lane] < 0) != 0ull;
+        int rej = 1;
+        if (!miss) {
+            if (lane < m) {
+                const int i = R.bidx[lane];
+                R.Uo[lane] = su[i];
+                R.Oo[lane] = so[i];
+                R.Qo[lane] = sq[i];
+            }
+            wave_lds_sync();
+            rej = chain_trial_state(u01f(ra.y) < 0.5f, ra, c, cp, sc, gc, cell, m, R.Uo, R.Oo, R.Qo, R.Un, R.On, R.Qn,
+                                    vol);
+        }
+        if (lane == 0) {
+            misc[NW + 2 * (t & 1)] = 4 * m + rej;
+            misc[NW + 2 * (t & 1) + 1] = f;
+        }
+    };
     __syncthreads();
-    for (int t = 0; t < ntrial; t++) {
+    for (int t = 0; over && t < ntrial; t++) {   // no move in this pass
         ctr.x = (uint32_t)t;
         ctr.w = cp.pass_hi << 2;
-        U4 ra = philox(ctr, cp.key0, cp.key1);
-        bool disp = u01f(ra.y) < 0.5f;
-        if (disp) n_dtry++; else n_rtry++;
-        if (over) {
-            n_rej++;
-            continue;
-        }
-        int k = clist[(int)(((uint64_t)ra.x * (uint64_t)total) >> 32)];
-        int f = cfirst[k], m = csize[k];
-        if (tid < m) bidx[tid] = -1;
-        __syncthreads();
-        for (int i = tid; i < nown_s; i += WAVE * NW) {   // a movable molecule's particles are all in `own`
-            int id = sid[own[i]] & CHAIN_IDMASK;
-            if (id >= f && id < f + m) bidx[id - f] = own[i];
-        }
-        __syncthreads();
-        if (w == 0) {
-            // a particle outside the region means the molecule is wider than rho
-            bool miss = __ballot(lane < m && bidx[lane] < 0) != 0ull;
-            int rej = 1;
-            if (!miss) {
-                if (lane < m) {
-                    int i = bidx[lane];
-                    Uo[lane] = su[i];
-                    Oo[lane] = so[i];
-                    Qo[lane] = sq[i];
-                }
-                wave_lds_sync();
-                rej = chain_trial_state(disp, ra, ctr, cp, sc, gc, cell, m, Uo, Oo, Qo, Un, On, Qn, vol);
-            }
-            if (lane == 0) misc[NW] = rej;
-        }
-        __syncthreads();
-        if (misc[NW] != 0) {
-            n_rej++;
-            __syncthreads();
-            continue;
-        }
-        ctr.w = (cp.pass_hi << 2) | 2u;
-        U4 rc = philox(ctr, cp.key0, cp.key1);   // the acceptance uniform, drawn ahead of the energies
+        if (u01f(philox(ctr, cp.key0, cp.key1).y) < 0.5f) n_dtry++; else n_rtry++;
+        n_rej++;
+    }
+    // Each turn evaluates trial t while one wave proposes trial t + 1; a turn
+    // without an evaluation (`run` false) only proposes: the first, one after a
+    // rejected proposal, and one that proposes again.
+    int t = -1;
+    bool run = false;
+    while (!over && t < ntrial) {
+        const Rec R = record(t & 1);
+        const int f = misc[NW + 2 * (t & 1) + 1], m = misc[NW + 2 * (t & 1)] >> 2;
         double acc_o = 0.0, acc_n = 0.0;
         // items: (particle, state) for mol2others, then the molecule's own
         // pairs and bonds at each state (waves without a particle item take them)
-        for (int it = w; it < 2 * m + (m > 1 ? 2 : 0); it += NW) {
+        for (int it = run ? w : 2 * m + 2; it < 2 * m + (m > 1 ? 2 : 0); it += NW) {
             if (it >= 2 * m) {
                 bool st = it > 2 * m;
-                double e = chain_intra(f, m, st ? Un : Uo, st ? On : Oo, st ? Qn : Qo, lane, WAVE, sc, pp, tp, ct);
+                double e = chain_intra(f, m, st ? R.Un : R.Uo, st ? R.On : R.Oo, st ? R.Qn : R.Qo, lane, WAVE, sc, pp,
+                                       tp, ct);
                 if (st) acc_n += e; else acc_o += e;
                 continue;
             }
             int a = it >> 1;
             bool st = (it & 1) != 0;
-            uint4 ua = st ? Un[a] : Uo[a];
-            double e = chain_item_energy_st(ua, st ? On[a] : Oo[a], st ? Qn[a] : Qo[a], f + a, f, m, g, f0, fn, spre,
-                                            own,
-                                            nown_s, sc, pp, tp, su, so, sq, sid, queue, spr);
+            uint4 ua = st ? R.Un[a] : R.Uo[a];
+            double e = chain_item_energy_st(ua, st ? R.On[a] : R.Oo[a], st ? R.Qn[a] : R.Qo[a], f + a, f, m, g, f0, fn,
+                                            spre, own, nown_s, sc, pp, tp, su, so, sq, sid, queue, spr);
             if (st) acc_n += e; else acc_o += e;
         }
-
-        double eo, en;
-        int rpar = 0;   // one paired sum per trial, after the previous trial's barrier
-        block_sum2<NW>(acc_o, acc_n, red, rpar, eo, en);
-        double de = en - eo;
-        // moveTry (movecreator.h:175-187) on mol2others before and after
-        bool acc = de <= 0.0 || exp(-de / cp.temper) > u01d(rc.x, rc.y);
-        if (acc) {
-            if (disp) n_dacc++; else n_racc++;
-            dsum += de;
-            if (tid < m) {
-                int i = bidx[tid], s = slot[f + tid];
-                su[i] = Un[tid];
-                so[i] = On[tid];
-                sq[i] = Qn[tid];
-                P[s] = Un[tid];
-                O[s] = On[tid];
-                Q[s] = Qn[tid];
+        // (on the wave with the least to do; it reads the next molecule alone)
+        if (w == NW - 1 && t + 1 < ntrial) propose_trial(t + 1);
+        bool again = false;
+        if (run) {
+            double eo, en;
+            int rpar = 0;   // one paired sum per trial, after the previous trial's barrier
+            block_sum2<NW>(acc_o, acc_n, red, rpar, eo, en);
+            double de = en - eo;
+            ctr.x = (uint32_t)t;
+            ctr.w = cp.pass_hi << 2;
+            const bool disp = u01f(philox(ctr, cp.key0, cp.key1).y) < 0.5f;
+            ctr.w = (cp.pass_hi << 2) | 2u;
+            U4 rc = philox(ctr, cp.key0, cp.key1);
+            // moveTry (movecreator.h:175-187) on mol2others before and after
+            bool acc = de <= 0.0 || exp(-de / cp.temper) > u01d(rc.x, rc.y);
+            if (acc) {
+                if (disp) n_dacc++; else n_racc++;
+                dsum += de;
+                again = t + 1 < ntrial && misc[NW + 2 * ((t + 1) & 1) + 1] == f;   // the next molecule has moved
+                if (tid < m) {
+                    int i = R.bidx[tid];
+                    su[i] = R.Un[tid];
+                    so[i] = R.On[tid];
+                    sq[i] = R.Qn[tid];
+                }
             }
         }
         __syncthreads();
+        run = false;
+        if (again) continue;
+        if (++t >= ntrial) break;
+        ctr.x = (uint32_t)t;
+        ctr.w = cp.pass_hi << 2;
+        if (u01f(philox(ctr, cp.key0, cp.key1).y) < 0.5f) n_dtry++; else n_rtry++;
+        run = (misc[NW + 2 * (t & 1)] & 3) == 0;
+        if (!run) n_rej++;
     }
+    if (!over && n_dacc + n_racc > 0)   // the cell's own particles back to their slots
+        for (int i = tid; i < nown_s; i += WAVE * NW) {
+            const int j = own[i], s = slot[sid[j] & CHAIN_IDMASK];
+            P[s] = su[j];
+            O[s] = so[j];
+            Q[s] = sq[j];
+        }
     int rep = (int)(blockIdx.x & (STAT_REP - 1));
     if (tid < 5) {
         unsigned long long v = tid == 0 ? n_dacc : tid == 1 ? n_dtry : tid == 2 ? n_racc : tid == 3 ? n_rtry : n_rej;
