@@ -209,13 +209,13 @@ int sc_set_block_waves(sc_ctx* ctx, int nw);
  * each of the four waves of an active cell's block evaluates one of the next
  * four trials against the cell's current state; the trials are then kept in
  * order until one depends on an earlier accepted trial of the round (the same
- * particle, the two within maxcut in any of their old/new states, or chain
- * partners), and evaluation resumes from there.  The chain of states and
+ * particle, chain partners, or two whose pair term can be non-zero in any of
+ * their old/new states), and evaluation resumes from there.  The chain of states and
  * decisions is the one-trial-at-a-time sweep's (Updater::simulate's sequence,
  * updater.cpp:206-230, within each cell).  A trial whose moving particle has
- * more than 320 particles within maxcut, or more than 192 (pair, state)
- * entries within the attraction's range, fails the sweep with SC_ECAPACITY;
- * on = 0 evaluates such systems.  No counterpart in the reference (its loop is
+ * more than 320 particles within reach of its terms at either state, or more
+ * than 192 (pair, state) entries within the attraction's range, fails the
+ * sweep with SC_ECAPACITY; on = 0 evaluates such systems.  No counterpart in the reference (its loop is
  * sequential). */
 int sc_set_speculation(sc_ctx* ctx, int on);
 /* The sweep keeps derived vectors (patch sides, second patch, chiral axes:

@@ -1652,15 +1652,14 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_pass(Grid g, SysConst sc
 // The chain of trials of a cell is sequential, and one trial leaves most of
 // a block's lanes idle (its phases hold a few dozen items).  In this variant
 // each of the block's SPEC_W waves evaluates one trial of the next SPEC_W
-// against the cell's current state, all at once; wave 0 then takes the
-// results in trial order and keeps each one unless it depends on an earlier
+// against the cell's current state, all at once; every wave then takes the
+// results in trial order, and each is kept unless it depends on an earlier
 // trial of the round that was accepted (the same particle, chain partners, or
 // two particles whose pair term can be non-zero in any of their old/new
 // states, by the pair code's own cutoff tests), where the round stops: that
 // trial and the later ones are evaluated again in the next round, against the
-// updated state.  A kept
-// trial saw exactly the state it would have seen in sequence, so the chain
-// of states and decisions is the sequential sweep's (only the FP64 sums run
+// updated state.  A kept trial saw exactly the state it would have seen in
+// sequence, so the chain of states and decisions is the sequential sweep's (only the FP64 sums run
 // in another order, as between the 1- and 4-wave sweeps).
 #define SPEC_W 4
 #define SPEC_STAGE_BYTES 48    // per staged particle: its record, ID and source index
@@ -2508,6 +2507,7 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
                             const uint4* __restrict__ P, const float4* __restrict__ O, const float2* __restrict__ Q,
                             const int* __restrict__ ID, const ChainTab& ct, int* sten, int* misc, int16_t*& partner,
                             size_t& used, bool half_stencil = false) {
+    static_assert(NW > 1, "the home cell's box is the second wave's");
     const int ns = stencil_size(g);
     int* pre = sten;          // ns+1 prefix of counts
     int* cst = sten + ns + 1; // cell start per stencil entry
@@ -2537,18 +2537,29 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
             pre[ns] = carry;
             misc[0] = home_idx;
         }
+    } else if (tid < WAVE + 3) {   // meanwhile the home cell's box: centre in fixed point, half edges; a lane per axis
+        const int q = tid - WAVE;
+        const int c = q == 0 ? cx : q == 1 ? cy : cz, nc = q == 0 ? g.nc[0] : q == 1 ? g.nc[1] : g.nc[2];
+        const uint32_t sh = q == 0 ? g.sh[0] : q == 1 ? g.sh[1] : g.sh[2];
+        const float L = q == 0 ? sc.L[0] : q == 1 ? sc.L[1] : sc.L[2];
+        misc[4 + q] = (int)(sh + (uint32_t)((((uint64_t)(2 * c + 1)) << 31) / (uint64_t)nc));
+        misc[8 + q] = __float_as_int(0.5f * L / (float)nc);
     }
     __syncthreads();
     const int total = pre[ns], home = misc[0], hbeg = pre[home], hend = pre[home + 1];
     const int gs = cst[home], ge = gs + hend - hbeg;
-    // the home cell's box: centre in fixed point, half edges
-    const int c3[3] = {cx, cy, cz};
+    if (hbeg == hend) {   // nothing to move: nothing staged
+        S.n = S.h0 = S.h1 = 0;
+        used = 0;
+        partner = nullptr;
+        return true;
+    }
     uint32_t cen[3];
     float half[3];
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        cen[q] = g.sh[q] + (uint32_t)((((uint64_t)(2 * c3[q] + 1)) << 31) / (uint64_t)g.nc[q]);
-        half[q] = 0.5f * sc.L[q] / (float)g.nc[q];
+        cen[q] = (uint32_t)misc[4 + q];
+        half[q] = __int_as_float(misc[8 + q]);
     }
     const float reach2 = sc.reach * sc.reach;
     // the stencil entry and the source of element e
@@ -2693,8 +2704,7 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     int ax = b % mp.nact[0], ay = (b / mp.nact[0]) % mp.nact[1], az = b / (mp.nact[0] * mp.nact[1]);
     int cx = mp.ox + mp.p * ax, cy = mp.oy + mp.p * ay, cz = mp.oz + mp.p * az;
     int cell = cx + g.nc[0] * (cy + g.nc[1] * cz);
-    int nh = starts[cell + 1] - starts[cell];
-    if (nh == 0) return;
+    const int nh = starts[cell + 1] - starts[cell];   // (first used where the first wave is past its own loads)
     const SpecLayout L = spec_layout(cap, NET, 0);
     Stage S;
     const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1), w = tid >> 6;
@@ -2729,18 +2739,22 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     }
     // the first trials are drawn on the last wave while the first one finds the
     // stencil (a cell visited for a few trials is mostly set-up)
-    int drawn = 0;
-    if (ntrial > 0) {
-        if (w == SPEC_W - 1 && lane < min(TRIAL_CHUNK, ntrial))
+    int drawn = TRIAL_CHUNK;
+    if (w == SPEC_W - 1) {
+        if (nh > 0 && lane < min(TRIAL_CHUNK, ntrial))
             recs[lane] = draw_trial<DA>(ctr, lane, mp, P + starts[cell], 0, nh, tp);
-        drawn = TRIAL_CHUNK;
     }
     if constexpr (LT) {
         PP32* ppl = (PP32*)(smem + L.tab);
         TP32* tpl = (TP32*)(ppl + sc.nt * sc.nt);
         const int w4 = (int)(sizeof(PP32) / 4), t4 = (int)(sizeof(TP32) / 4);
-        for (int e = tid; e < sc.nt * sc.nt * w4; e += WAVE * SPEC_W) ((int*)ppl)[e] = ((const int*)pp)[e];
-        for (int e = tid; e < sc.nt * t4; e += WAVE * SPEC_W) ((int*)tpl)[e] = ((const int*)tp)[e];
+        // by the waves that neither find the stencil nor draw: a copy by the whole
+        // block before the stencil was a round trip to memory of its own (1,000
+        // PSC, ten sweeps of 27 launches: 6.51 ms, 6.26 so)
+        if (w > 0 && w < SPEC_W - 1) {
+            for (int e = tid - WAVE; e < sc.nt * sc.nt * w4; e += WAVE * (SPEC_W - 2)) ((int*)ppl)[e] = ((const int*)pp)[e];
+            for (int e = tid - WAVE; e < sc.nt * t4; e += WAVE * (SPEC_W - 2)) ((int*)tpl)[e] = ((const int*)tp)[e];
+        }
         pp = ppl;
         tp = tpl;
     }
@@ -2751,6 +2765,7 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         if (tid == 0) atomicOr(flag, 1);
         return;
     }
+    if (nh == 0) return;
     // rows of all staged particles, else of the home cell's, where they fit
     Rows rows;
     rows.v = (float*)(smem + used);
@@ -5459,7 +5474,7 @@ static int check_flag(sc_ctx* ctx, const char* what, bool* again = nullptr) {
         }
         if (f & 4) return fail(ctx, SC_ECAPACITY, std::string(what) + ": a coarse cell held more than 4096 molecules");
         if (f & 16)
-            return fail(ctx, SC_ECAPACITY, std::string(what) + ": more than 320 particles within maxcut, or 192 "
+            return fail(ctx, SC_ECAPACITY, std::string(what) + ": more than 320 particles within reach, or 192 "
                                                                "(pair, state) entries within the attraction's range, "
                                                                "of a moving particle (the speculative sweep's lists); "
                                                                "sc_set_speculation(ctx, 0) evaluates such systems");
