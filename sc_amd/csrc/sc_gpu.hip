@@ -3982,8 +3982,8 @@ __global__ __launch_bounds__(256) void k_chain_anchor(int nchain, const int* __r
 // not added to those of the surrounding scan), in its canonical order, the
 // higher ID as part1 (allToAll's): the lanes that swap exchange the operands, so
 // a wave walks the functor once (a call per order held it twice, 120 KB of
-// code, and a wave with both orders walked both: the staged pass of 10,001
-// chains 2300 us, 1588 us so).
+// code, and a wave with both orders walked both: four NPT steps of
+// 10,001 chains 14.0 ms, 13.3 ms so).
 __device__ __attribute__((noinline)) double chain_pair(const PP32* __restrict__ pp, const TP32* __restrict__ tp, int nt,
                                                        float sqmaxcut, uint4 ua, float4 oa, float2 qa, uint4 ub,
                                                        float4 ob, float2 qb, V3<float> r, bool sw) {
@@ -4388,8 +4388,9 @@ __global__ __launch_bounds__(WAVE * NW) void k_chain_pass(Grid g, Grid gc, SysCo
 // chain of latencies (its molecule found and moved in FP64 ~9,000 cycles, the
 // items ~34,000, the decision and commit ~4,000): one wave proposes the next
 // molecule while the others finish this one's items.  10,001 chains of three:
-// 2543 us a pass with every step in turn, 2300 us with that overlap, 1588 us
-// with the functor's single copy (chain_pair) as well.  The region is found through the fine cell list (whole cells
+// 2543 us a pass with every step in turn, 1590-1830 us with that and the
+// functor's single copy (chain_pair); four NPT steps of them 16.9 ms, 14.0 with
+// the overlap alone, 13.3 with both.  The region is found through the fine cell list (whole cells
 // overlapping it, filtered by position).  A block whose region holds more
 // than `cap` particles makes no move in this pass (its trials are counted as
 // rejected, and the block in chain_skipped).

@@ -81,7 +81,6 @@ SC_HD void mlp_features(const V3<float>& adir, const V3<float>& apd, const V3<fl
     f[11] = w;
 }
 
-
 // ---------------------------------------------------------------- MFMA tile
 // Inference runs the transposed product H^T = W^T X^T on
 // v_mfma_f32_16x16x32_bf16 (D[i][j] = sum_k A[i][k] B[k][j], 16x16 output,
