@@ -2497,10 +2497,13 @@ __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query*
 // partners of its particles.  For 65,536 TCHPSC at packing fraction 0.25 that
 // is ~245 of 432, and every trial scans the stage.  Two passes over a large
 // stencil (positions, then the records of those kept), so that the records
-// lie packed behind one another; misc: 16 ints and block_compactK's counts.  list: cap source indices at the end of the
-// region, beyond the records (44 cap + 4 cap bytes fit the region).
-// half_stencil: only the home cell and the stencil cells behind it in their
-// order, one of each pair of opposite cells.
+// lie packed behind one another.  misc: 16 ints (home entry, home start, cell
+// centre and half edges) and the compaction counts of either path behind them:
+// the waves read the centre after the first barrier, and a wave that has no
+// particle to load writes its count before the next one.
+// list: cap source indices at the end of the region, beyond the records (44
+// cap + 4 cap bytes fit the region).  half_stencil: only the home cell and the
+// stencil cells behind it in their order, one of each pair of opposite cells.
 template <int NW>
 __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes, int cap, const Grid& g,
                             const SysConst& sc, int cx, int cy, int cz, const int* __restrict__ starts,
@@ -2644,7 +2647,7 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
                     }
             }
         }
-        const int pos = block_compact<NW>(keep, n, misc + 4);
+        const int pos = block_compact<NW>(keep, n, misc + 16);
         if (keep && pos < cap) list[pos] = src;
         if (e == hbeg) misc[1] = pos;
     }

@@ -1,0 +1,66 @@
+"""Faults that were found in the kernels and mended, each with the case that showed it, through the C ABI.
+
+Tolerances as where the kernels' sizes are tested: trajectories bit for bit; a whole-system energy within 1e-5 of
+the sum of the particles' |E| + 2e-4 kT, a particle's energy within 1e-5 |E| + 2e-4 kT of the FP64 oracle.
+"""
+import numpy as np
+import pytest
+
+import sc_amd
+from sc_amd import workloads as W
+import pyoracle as po
+
+pytestmark = pytest.mark.gpu
+ROT_HALF = 20.0 / 180 * np.pi / 4
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def psc_state(g, n, eta, seed, box=None):
+    """n PSC at random without overlap; the oracle's topology and the device's own state"""
+    top = W.top_init([W.TYPES["psc"]], [n])
+    types = np.ones(n, np.int32)
+    box = np.full(3, (n * W.particle_volume(1.0, 3.0) / eta) ** (1.0 / 3.0)) if box is None else np.asarray(box, float)
+    g.load_topology(top)
+    pos, d, q = g.generate_rsa(types, box, seed)
+    g.set_config(box, pos, d, q, types)
+    b, p, dd, qq = g.get_config()
+    return po.Topo(top), po.State(b, p, dd, qq, types)
+
+
+@pytest.mark.parametrize("eta,r", [(0.01, 1), (0.02, 1), (0.02, 2), (0.04, 1)])
+def test_chain_sweep_of_sparse_stencils(eta, r):
+    """A stage copied in two passes, from stencils of fewer particles than the block has lanes: waves without a
+    particle of their own must not write over the cell's centre that the others still read (the compaction counts
+    lay in the same LDS words).  The one-trial-at-a-time trajectory bit for bit."""
+    say("case: chain sweep, eta %.2f, r %d" % (eta, r))
+    box, pos, d, q, t = W.chain_lattice(300, eta, 11)
+    out = []
+    for nw in (0, 1):
+        with sc_amd.GpuSystem(0) as g:
+            g.load_topology(W.chain_topology(300))
+            g.set_config(box, pos, d, q, t)
+            g.set_block_waves(nw)
+            s = g.sweep(20, 1.1, 0.3, ROT_HALF, r=r, seed=23, counter=0)
+            out.append((s, g.get_config()))
+    (s1, c1), (s2, c2) = out
+    say("accepted %d / %d" % (s1["trans_acc"] + s1["rot_acc"], s1["trans_try"] + s1["rot_try"]))
+    assert s1["trans_acc"] + s1["rot_acc"] > 0
+    for k in ("trans_acc", "trans_try", "rot_acc", "rot_try", "left_cell", "bond_rejected"):
+        assert s1[k] == s2[k], k
+    for a, b in zip(c1, c2):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("n,eta", [(150, 0.05), (1000, 0.20), (3000, 0.20)])
+def test_whole_system_energy_of_two_pass_stages(n, eta):
+    """the same words under the whole-system energy: stencils of one to a few waves of particles"""
+    say("case: whole-system energy, %d PSC at eta %.2f" % (n, eta))
+    with sc_amd.GpuSystem(0) as g:
+        tp, st = psc_state(g, n, eta, n)
+        e, want = g.allToAll(), po.energy_all(tp, st, use_cells=True)
+        size = np.abs(po.energy_one_each(tp, st, np.arange(n))).sum()
+        say("gpu %.8f oracle %.8f" % (e, want))
+        assert abs(e - want) <= 1e-5 * size + 2e-4
