@@ -6382,6 +6382,18 @@ int sc_commit_box(sc_ctx* ctx, const double box_new[3]) {
     SC_GUARD(ctx, sc_commit_box_impl(ctx, box_new))
 }
 
+// Does the grid's stencil hold every partner of a pair term in box `box`?  A
+// pair list's grid has cells of its own width, and a grid made for a larger
+// trial box too many.  (The cutoff's own margin covers the rounding of a cell
+// count that divides the edge.)
+static bool grid_covers(const sc_ctx* ctx, const double* box) {
+    if (!ctx->grid_valid) return false;
+    const Grid& g = ctx->g;
+    for (int k = 0; k < 3; k++)
+        if (g.nc[k] > 2 * g.r + 1 && g.r * box[k] * (1.0 + 1e-9) < ctx->maxcut * g.nc[k]) return false;
+    return true;
+}
+
 // Energies of nq queries: the array hq, or q1 for all (see Query).  Up to
 // SINGLE_Q results come back through pinned host memory that the kernel writes
 // itself; a host program's single moves are bound by the copies and
@@ -6391,9 +6403,7 @@ static int run_queries(sc_ctx* ctx, int nq, const Query* hq, const Query& q1, do
     const bool pinned = nq <= SINGLE_Q;
     if (!pinned && (rc = ensure_out(ctx, nq))) return rc;
     if (hq && (rc = ensure_ij(ctx, nq))) return rc;
-    if (!ctx->grid_valid) {
-        if ((rc = build_grid(ctx, 2, nullptr, ctx->box))) return rc;
-    }
+    if (!grid_covers(ctx, ctx->box) && (rc = build_grid(ctx, 2, nullptr, ctx->box))) return rc;
     if (hq) HIPCK(hipMemcpyAsync(ctx->d_q, hq, nq * sizeof(Query), hipMemcpyHostToDevice, ctx->stream));
     SysConst sc = sysconst(ctx, ctx->box);
     int c = ctx->cur;

@@ -64,3 +64,29 @@ def test_whole_system_energy_of_two_pass_stages(n, eta):
         size = np.abs(po.energy_one_each(tp, st, np.arange(n))).sum()
         say("gpu %.8f oracle %.8f" % (e, want))
         assert abs(e - want) <= 1e-5 * size + 2e-4
+
+
+@pytest.mark.parametrize("before", ["pair list", "pair list below the cells' width", "alignment order", "trial box"])
+def test_particle_energies_after_another_grid(before):
+    """Energies of single particles search the cell list that is there: not one with narrower cells, as a pair list
+    of a short range and a larger trial box leave it."""
+    say("case: particle energies after a", before)
+    n = 3000
+    with sc_amd.GpuSystem(0) as g:
+        tp, st = psc_state(g, n, 0.2, 21)
+        if before == "pair list":
+            g.neighbor_pairs(2.5)
+        elif before == "pair list below the cells' width":
+            g.neighbor_pairs(0.5)
+        elif before == "alignment order":
+            g.alignment_order()
+        else:
+            g.allToAllTrial(2.0 * st.box)
+        one = g.oneToAll(7)
+        trial = g.oneToAllTrial(7, st.pos[7], st.dir[7], st.pd0[7])
+        mol = g.mol2others(7, 1)
+        e, want = g.energy_per_particle(), po.energy_one_each(tp, st, np.arange(n))
+        say("max error %.2e; particle 7: %.8f, oracle %.8f" % (np.abs(e - want).max(), one, want[7]))
+        assert np.all(np.abs(e - want) <= 1e-5 * np.abs(want) + 2e-4)
+        for v in (one, trial, mol):
+            assert abs(v - want[7]) <= 1e-5 * abs(want[7]) + 2e-4
