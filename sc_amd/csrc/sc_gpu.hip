@@ -1950,7 +1950,7 @@ __device__ __forceinline__ bool side_possible(const PatchView<float>& a, const V
 //      behind them the trial's dependences on the round's earlier trials
 //   C  patch terms of the entries in range
 // stage -2: a list is full (more than SPEC_LCAP candidates of a state or
-// SPEC_XCAP entries), the trial cannot be evaluated here.
+// SPEC_XCAP entries), the trial cannot be evaluated here (dep holds).
 template <int DA>
 __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo, const uint4 un, const float4 oo,
                                            const float2 qo, const float4 on, const float2 qn, const SysConst& sc,
@@ -2019,6 +2019,9 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     }
     wave_lds_sync();
     if (no > SPEC_LCAP || nn > SPEC_LCAP) {
+        // (the candidates are counted at more than a pair term's range, so any
+        // accepted move before this one may be why)
+        dep = (1 << w) - 1;
         stage = -2;
         return false;
     }

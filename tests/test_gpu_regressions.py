@@ -90,3 +90,37 @@ def test_particle_energies_after_another_grid(before):
         assert np.all(np.abs(e - want) <= 1e-5 * np.abs(want) + 2e-4)
         for v in (one, trial, mol):
             assert abs(v - want[7]) <= 1e-5 * abs(want[7]) + 2e-4
+
+
+def crowded_ball(g):
+    """320 small spheres in a ball, a sphere beside it that has them all within reach (as many as a trial's list
+    holds), and one more at the end of that sphere's reach"""
+    k = np.stack(np.meshgrid(*[np.arange(7)] * 3, indexing="ij"), -1).reshape(-1, 3)[:320]
+    pos = np.concatenate([(k - 3) * 0.35, [[3.0, 0.0, 0.0], [8.003, 0.0, 0.0]]]) + 8.0
+    n = len(pos)
+    g.load_topology(W.top_init(["S 1 SPA 1.0 0.3 4.5 0.5"], [n]))
+    g.set_config(np.full(3, 24.0), pos / 24.0, np.tile([0.0, 0.0, 1.0], (n, 1)), np.tile([1.0, 0.0, 0.0], (n, 1)),
+                 np.ones(n, np.int32))
+
+
+def test_full_list_of_a_trial_behind_an_accepted_one():
+    """A speculative trial whose list is full because of where an earlier accepted trial of its round stood is
+    evaluated again, not reported: at these seeds the far sphere leaves the reach before the near one's trial."""
+    for seed in (94, 149, 176, 461):
+        say("case: the last candidate has left, seed %d" % seed)
+        out = []
+        for nw in (0, 1):
+            with sc_amd.GpuSystem(0) as g:
+                crowded_ball(g)
+                g.set_block_waves(nw)
+                s = g.sweep(1, 1000.0, 0.05, 0.1, r=1, seed=seed, counter=0)
+                out.append((s["trans_acc"], s["trans_try"], g.get_config()))
+        assert out[0][:2] == out[1][:2] and out[0][0] > 0
+        for a, b in zip(out[0][2], out[1][2]):
+            np.testing.assert_array_equal(a, b)
+    for seed in (0, 1):
+        say("case: the list is full in sequence too, seed %d" % seed)
+        with sc_amd.GpuSystem(0) as g:
+            crowded_ball(g)
+            with pytest.raises(sc_amd.SCError, match="320 particles"):
+                g.sweep(1, 1000.0, 0.05, 0.1, r=1, seed=seed, counter=0)
