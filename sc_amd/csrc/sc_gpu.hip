@@ -1789,7 +1789,8 @@ struct Rows {
 };
 
 // Squared distance of the point -r (r = segment's centre - point) from the
-// segment of unit axis d and half length h.
+// segment of unit axis d and half length h; NaN for an axis that is (a test
+// for what is out of reach must keep it).
 __device__ __forceinline__ float centre_dist2(const V3<float>& d, float h, const V3<float>& r) {
     float t = -dot(d, r);
     t = fminf(fmaxf(t, -h), h);
@@ -1983,7 +1984,12 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     const V3<float> dold = vrow_dir(mvo), dnew = vrow_dir(mvn);
     // phase A: the loads of a round's PA staged particles per lane first, then
     // the tests without branches (a load under a condition waits by itself)
-    const float hm = tp[t].hl, reach2 = tp[t].reach2;
+    const float hm = tp[t].hl;
+    // (an axis that is no number reaches whatever lies within the cutoff: the
+    // pair terms decide, of spheres a value, of rods NaN)
+    const bool nan_o = !(dot(dold, dold) < 4.0f), nan_n = !(dot(dnew, dnew) < 4.0f);
+    const V3<float> zero = mk<float>(0.0f, 0.0f, 0.0f), axo = nan_o ? zero : dold, axn = nan_n ? zero : dnew;
+    const float reach2o = nan_o ? sc.sqmaxcut : tp[t].reach2, reach2n = nan_n ? sc.sqmaxcut : tp[t].reach2;
     uint16_t* const nl_new = T.nl + SPEC_LCAP;
     int no = 0, nn = 0;
     auto scan = [&](int base, auto pa) {
@@ -1999,8 +2005,8 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             const V3<float> ro = fx_image_c(uo.x, uo.y, uo.z, b[h].x, b[h].y, b[h].z, sc.Lh, sc.Ll);
             V3<float> rn = ro;
             if (translate) rn = fx_image_c(un.x, un.y, un.z, b[h].x, b[h].y, b[h].z, sc.Lh, sc.Ll);
-            fo[h] = in & (centre_dist2(dold, hm, ro) <= reach2);
-            fn[h] = in & (centre_dist2(dnew, hm, rn) <= reach2);
+            fo[h] = in & (centre_dist2(axo, hm, ro) <= reach2o);
+            fn[h] = in & (centre_dist2(axn, hm, rn) <= reach2n);
         }
 #pragma unroll
         for (int h = 0; h < PA; h++) {
@@ -2382,7 +2388,7 @@ __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query*
         for (int h = 0; h < PA; h++) {
             const V3<float> r = fx_image_c(q.u[0], q.u[1], q.u[2], u[h].x, u[h].y, u[h].z, sc.Lh, sc.Ll);
             keep[h] = (base + h * BS + tid < total) & !((id[h] >= q.ex_lo) & (id[h] <= q.ex_hi)) &
-                      (dot(r, r) <= sc.sqmaxcut) & (centre_dist2(dq, hq, r) <= reach2);
+                      (dot(r, r) <= sc.sqmaxcut) & !(centre_dist2(dq, hq, r) > reach2);
         }
         block_compactK<NW, PA>(keep, nl, cnt, par, pos);
 #pragma unroll
@@ -3078,7 +3084,7 @@ __device__ __forceinline__ void energy_cell(int cell, const Grid& g, const SysCo
             const V3<float> r = fx_image_c(a.x, a.y, a.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
             const bool mine = half ? (j >= S.h1) | (j < S.h0) | (j > i) : S.id[j] < S.id[i];
             keep[h] = (base + h * BS + tid < total) & mine & (dot(r, r) <= sc.sqmaxcut) &
-                      (centre_dist2(mk<float>(oa.x, oa.y, oa.z), tp[a.w].hl, r) <= tp[a.w].reach2);
+                      !(centre_dist2(mk<float>(oa.x, oa.y, oa.z), tp[a.w].hl, r) > tp[a.w].reach2);
             pk[h] = (i << 16) | j;
         }
         block_compactK<NW, PA>(keep, nl, cnt, par, pos);

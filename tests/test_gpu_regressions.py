@@ -124,3 +124,56 @@ def test_full_list_of_a_trial_behind_an_accepted_one():
             crowded_ball(g)
             with pytest.raises(sc_amd.SCError, match="320 particles"):
                 g.sweep(1, 1000.0, 0.05, 0.1, r=1, seed=seed, counter=0)
+
+
+def with_nan_axis(g, line, n, box, seed, k=5):
+    """n particles at random, the axis of particle k no number; (positions, axes, patch directions)"""
+    rng = np.random.default_rng(seed)
+    top, types = W.top_init([line], [n]), np.ones(n, np.int32)
+    g.load_topology(top)
+    pos, d, q = g.generate_rsa(types, np.full(3, box), seed)
+    bad = d.copy()
+    bad[k] = np.nan
+    g.set_config(np.full(3, box), pos, bad, q, types)
+    return pos, d, q
+
+
+def test_axis_that_is_no_number():
+    """A rod with a NaN axis has NaN energies with what lies within the cutoff; a sphere's axis does not matter."""
+    say("case: rods")
+    rod = W.TYPES["psc"]
+    with sc_amd.GpuSystem(0) as g:
+        pos, d, q = with_nan_axis(g, rod, 600, 22.0, 3)
+        assert np.isnan(g.allToAll()) and np.isnan(g.oneToAll(5))
+        g.set_config(np.full(3, 22.0), pos, d, q, np.ones(600, np.int32))
+        assert np.isfinite(g.allToAll()) and np.isnan(g.oneToAllTrial(9, pos[9], np.full(3, np.nan), q[9]))
+    say("case: spheres")
+    with sc_amd.GpuSystem(0) as g:
+        pos, d, q = with_nan_axis(g, "S 1 SPA 1.0 1.0 1.0 0.2", 600, 10.0, 4)
+        e, each = g.allToAll(), g.energy_per_particle()
+        g.set_config(np.full(3, 10.0), pos, d, q, np.ones(600, np.int32))
+        assert each[5] != 0.0
+        np.testing.assert_array_equal(each, g.energy_per_particle())
+        assert e == g.allToAll()
+
+
+def test_sweep_with_an_axis_that_is_no_number():
+    """A rod of NaN axis with others in its cutoff never moves (its energy differences are NaN); a sphere's moves
+    are those of the one-trial-at-a-time trajectory."""
+    say("case: sweep of rods")
+    with sc_amd.GpuSystem(0) as g:
+        with_nan_axis(g, W.TYPES["psc"], 600, 22.0, 6)
+        u = g.fixed_positions()
+        s = g.sweep(10, 1.0, 0.2, ROT_HALF, r=1, seed=2, counter=0)
+        assert s["trans_acc"] > 0
+        np.testing.assert_array_equal(g.fixed_positions()[5], u[5])
+    say("case: sweep of spheres")
+    out = []
+    for nw in (0, 1):
+        with sc_amd.GpuSystem(0) as g:
+            with_nan_axis(g, "S 1 SPA 1.0 1.0 1.0 0.2", 600, 10.0, 6)
+            g.set_block_waves(nw)
+            s = g.sweep(10, 1.0, 0.2, ROT_HALF, r=1, seed=2, counter=0)
+            out.append((s, g.fixed_positions()))
+    assert out[0][0]["trans_acc"] == out[1][0]["trans_acc"] > 0
+    np.testing.assert_array_equal(out[0][1], out[1][1])
