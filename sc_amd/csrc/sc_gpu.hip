@@ -1662,8 +1662,7 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_pass(Grid g, SysConst sc
 // sequence, so the chain of states and decisions is the sequential sweep's (only the FP64 sums run
 // in another order, as between the 1- and 4-wave sweeps).
 #define SPEC_W 4
-#define SPEC_STAGE_BYTES 48    // per staged particle: its record, ID and source index
-#define SPEC_ROW_BYTES 7168    // beyond that, for rows and chain partners; a stage below its capacity leaves more
+#define SPEC_STAGE_BYTES 48    // per staged particle: its record, ID and source index (the rest: rows, chain partners)
 #define SPEC_LCAP 320   // candidates of one wave's trial at either state (typically ~20)
 #define SPEC_XCAP 192   // its (pair, state) entries within the attraction's range (typically 5-10)
 // a staged particle's row of derived vectors: floats, and where its axis and first patch direction lie
@@ -1688,15 +1687,16 @@ __device__ __forceinline__ int spec_word(bool acc, bool translate, int status, i
     return (acc ? 1 : 0) | (translate ? 2 : 0) | (status << 2) | ((stage & 3) << 4) | (dep << 8);
 }
 
-// LDS of the speculative sweep: the stage, then SPEC_W per-wave trial
-// scratch blocks, then what the waves share (byte offsets; per-wave fields
-// relative to the wave's block).
+// LDS of the speculative sweep: a region of `region` bytes (a multiple of 16)
+// for the stage and its rows, then SPEC_W per-wave trial scratch blocks, then
+// what the waves share (byte offsets; per-wave fields relative to the wave's
+// block).
 struct SpecLayout {
     size_t nl, xl, xd, mv, wstride;
     size_t wbase, sten, misc, prop, res, recs, ml, tab, end;
 };
 __host__ __device__ inline size_t spec_align(size_t x, size_t a) { return (x + a - 1) / a * a; }
-__host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_bytes) {
+__host__ __device__ inline SpecLayout spec_layout(size_t region, bool net, size_t tab_bytes) {
     SpecLayout L;
     L.nl = 0;
     L.xl = L.nl + 2 * 2 * SPEC_LCAP;
@@ -1704,7 +1704,7 @@ __host__ __device__ inline SpecLayout spec_layout(int cap, bool net, size_t tab_
     L.mv = spec_align(L.xd + (net ? 4 * SPEC_XCAP : 0), 16);
     L.wstride = L.mv + 4 * 2 * VROW;
     static_assert(2 * 2 * SPEC_LCAP >= 4 * SPEC_NV * VROW, "neighbour rows over the candidate lists");
-    L.wbase = spec_align((size_t)cap * SPEC_STAGE_BYTES + SPEC_ROW_BYTES, 16);   // the stage and rows
+    L.wbase = region;
     size_t o = L.wbase + SPEC_W * L.wstride;
     L.sten = o;
     o += 4 * (2 * 125 + 2);
@@ -1965,6 +1965,16 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     const int cwk = ct.cw ? ct.cw[idk] : 0, bmask = cwk & 15;
     if (bmask) {   // partner: the staged chain partners of particle k (-1: not staged)
         int found = 0;
+        if (!partner) {   // a stage without room for them: found among the staged (in the entries' list, empty yet)
+            if (lane < 4) T.xl[lane] = 0xffff;
+            wave_lds_sync();
+            for (int j = lane; j < S.n; j += WAVE) {
+                const int q = cw_bit(S.id[j] - idk);
+                if (q >= 0) T.xl[q] = (uint16_t)j;
+            }
+            wave_lds_sync();
+            partner = (const int16_t*)T.xl;
+        }
         for (int q = 0; q < 4; q++) found |= (partner[q] >= 0 ? 1 : 0) << q;
         if ((found & bmask) != bmask) {
             stage = -1;
@@ -2671,10 +2681,12 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
     S.q = (float2*)(S.o + n4);
     S.id = (int*)(S.q + n4);
     used = (size_t)n4 * 44;
-    partner = (int16_t*)(region + used);
-    if (ct.cw) {   // the home cell's chain partners: four staged indices per particle
-        used += ((size_t)(hend - hbeg) * 8 + 15) & ~(size_t)15;
-        if (used > region_bytes - 4 * (size_t)cap) return false;   // (not over the list)
+    partner = nullptr;
+    const size_t pbytes = ((size_t)(hend - hbeg) * 8 + 15) & ~(size_t)15;
+    if (ct.cw && used + pbytes <= region_bytes - 4 * (size_t)cap) {   // (not over the list)
+        // the home cell's chain partners: four staged indices per particle
+        partner = (int16_t*)(region + used);
+        used += pbytes;
         for (int i = tid; i < 4 * (hend - hbeg); i += WAVE * NW) partner[i] = -1;
         __syncthreads();
     }
@@ -2684,7 +2696,7 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
         S.o[i] = O[src];
         S.q[i] = Q[src];
         S.id[i] = id;
-        if (ct.cw) {
+        if (partner) {
             const int w = ct.cw[id];
             for (int q = 0; q < 4; q++)   // this particle is partner q ^ 1 (the opposite step) of its partner q
                 if ((w >> q) & 1) {
@@ -2706,7 +2718,7 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
                                                 const int* __restrict__ starts, uint4* __restrict__ P,
                                                 float4* __restrict__ O, float2* __restrict__ Q,
                                                 const int* __restrict__ ID, const PP32* __restrict__ pp,
-                                                const TP32* __restrict__ tp, int cap, int ppmax,
+                                                const TP32* __restrict__ tp, int region, int ppmax,
                                                 const int* __restrict__ nonempty,
                                                 const unsigned char* __restrict__ mlp_img, const MlpConst& mc,
                                                 const ChainTab& ct, unsigned long long* __restrict__ stats,
@@ -2717,7 +2729,7 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     int cx = mp.ox + mp.p * ax, cy = mp.oy + mp.p * ay, cz = mp.oz + mp.p * az;
     int cell = cx + g.nc[0] * (cy + g.nc[1] * cz);
     const int nh = starts[cell + 1] - starts[cell];   // (first used where the first wave is past its own loads)
-    const SpecLayout L = spec_layout(cap, NET, 0);
+    const SpecLayout L = spec_layout(region, NET, 0);
     Stage S;
     const int tid = (int)threadIdx.x, lane = tid & (WAVE - 1), w = tid >> 6;
     unsigned char* wb = smem + L.wbase + (size_t)w * L.wstride;
@@ -2772,7 +2784,7 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
     }
     int16_t* partners;
     size_t used;
-    if (!stage_reach<SPEC_W>(S, smem, L.wbase, cap, g, sc, cx, cy, cz, starts, P, O, Q, ID, ct, sten, misc, partners,
+    if (!stage_reach<SPEC_W>(S, smem, L.wbase, region / SPEC_STAGE_BYTES, g, sc, cx, cy, cz, starts, P, O, Q, ID, ct, sten, misc, partners,
                              used)) {
         if (tid == 0) atomicOr(flag, 1);
         return;
@@ -2839,9 +2851,9 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
                 for (int i = 0; i < w; i++) dep |= prop[i].k == k ? 1 << i : 0;
             } else {
                 double eo, en, des;
+                const int16_t* pk = partners ? partners + 4 * (k - S.h0) : nullptr;
                 bool pass = spec_trial<DA>(S, k, uo, un, oo, qo, on, qn, sc, pp, tp, ppmax, T, ml, mlp_img, mc, ct,
-                                           R.thr1, R.thr2, rows, partners + 4 * (k - S.h0), translate, prop, w, eo, en,
-                                           des, stage, dep);
+                                           R.thr1, R.thr2, rows, pk, translate, prop, w, eo, en, des, stage, dep);
                 if (stage == -1) {
                     status = 2;   // whatever the others do: the partner's cell does not change in a pass
                 } else if (stage == -2) {
@@ -2936,12 +2948,12 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_spec(Grid g, SysCons
                                                              float4* __restrict__ O, float2* __restrict__ Q,
                                                              const int* __restrict__ ID,
                                                              const PP32* __restrict__ pp,
-                                                             const TP32* __restrict__ tp, int cap,
+                                                             const TP32* __restrict__ tp, int region,
                                                              int ppmax, const int* __restrict__ nonempty,
                                                              const unsigned char* __restrict__ mlp_img, MlpConst mc,
                                                              ChainTab ct, unsigned long long* __restrict__ stats,
                                                              double* __restrict__ de_sum, int* __restrict__ flag) {
-    sweep_cell_spec<DA, LT>(xcd_slab_index((int)blockIdx.x, (int)gridDim.x), g, sc, mp, starts, P, O, Q, ID, pp, tp, cap,
+    sweep_cell_spec<DA, LT>(xcd_slab_index((int)blockIdx.x, (int)gridDim.x), g, sc, mp, starts, P, O, Q, ID, pp, tp, region,
                         ppmax, nonempty, mlp_img, mc, ct, stats, de_sum, flag);
 }
 
@@ -2994,7 +3006,7 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_batch_spec(const Rep
                                                                    float2* __restrict__ Q,
                                                                    const int* __restrict__ ID,
                                                                    const PP32* __restrict__ pp,
-                                                                   const TP32* __restrict__ tp, int cap,
+                                                                   const TP32* __restrict__ tp, int region,
                                                                    int ppmax, const int* __restrict__ nonempty,
                                                                    const unsigned char* __restrict__ mlp_img,
                                                                    MlpConst mc, ChainTab ct,
@@ -3008,7 +3020,7 @@ __global__ __launch_bounds__(WAVE * SPEC_W, 2) void k_sweep_batch_spec(const Rep
         if (rp[mid].blk_off <= lb) lo = mid; else hi = mid - 1;
     }
     const RepPass R = rp[lo];
-    sweep_cell_spec<DA, LT>(lb - R.blk_off, R.g, R.sc, R.mp, starts + R.cell_off, P, O, Q, ID, pp, tp, cap, ppmax,
+    sweep_cell_spec<DA, LT>(lb - R.blk_off, R.g, R.sc, R.mp, starts + R.cell_off, P, O, Q, ID, pp, tp, region, ppmax,
                         nonempty + R.rep, mlp_img, mc, ct, stats + (size_t)R.rep * STAT_REP * STAT_STRIDE,
                         de_sum + (size_t)R.rep * STAT_REP * STAT_STRIDE, flag);
 }
@@ -5474,6 +5486,24 @@ static size_t sweep_table_bytes(int nt) {
     return (size_t)nt * nt * sizeof(PP32) + (size_t)nt * sizeof(TP32) + 16;
 }
 
+// LDS of the speculative sweep: all that a block may have.  Its registers let
+// two blocks share a CU whatever their LDS, and what the stage leaves holds
+// rows: with no more than an estimated stage's room, 200 TCHPSC in a box of
+// two cells an axis had rows for the home cell alone (three sweeps 3249 us,
+// 1766 us so).  One type's 68,624 bytes hold up to 1,429 staged particles, 439
+// with their rows.
+struct SpecLds {
+    int region;
+    size_t bytes;
+};
+static SpecLds spec_lds(bool net, int nt) {
+    const size_t tabb = sweep_table_bytes(nt), fixed = spec_layout(0, net, tabb).end;
+    SpecLds l;
+    l.region = (int)((SWEEP_LDS_BUDGET - fixed) / 16 * 16);
+    l.bytes = spec_layout(l.region, net, tabb).end;
+    return l;
+}
+
 // `again` set: the kernel is to be run again with its full stage (flag 32)
 static int check_flag(sc_ctx* ctx, const char* what, bool* again = nullptr) {
     int f = 0;
@@ -6961,16 +6991,7 @@ static int sc_sweep_impl(sc_ctx* ctx, int nsweeps, double temper, double transmx
         // the speculative variant: the stage that fits beside SPEC_W trials' lists
         bool spec = ctx->spec && ctx->sweep_nw == 0;
         const bool spec_lt = sweep_table_bytes(ctx->nt) > 0;   // the tables fit in LDS beside the stage
-        int cap_spec = cap;
-        size_t lds_spec = 0;
-        if (spec) {
-            size_t tabb = sweep_table_bytes(ctx->nt);
-            long room = (long)SWEEP_LDS_BUDGET - (long)spec_layout(0, da, tabb).end - 16;
-            int cmax = room > 0 ? (int)(room / SPEC_STAGE_BYTES) : 0;
-            if (cap_spec > cmax) cap_spec = (cmax / 64) * 64;
-            spec = cap_spec >= 64;
-            if (spec) lds_spec = spec_layout(cap_spec, da, tabb).end;
-        }
+        const SpecLds ls = spec_lds(da, ctx->nt);
         if (da && (ctx->mlp_type < 0 || ctx->ref2dense[ctx->mlp_type] < 0))
             return fail(ctx, SC_EINVAL, "the network screen needs the network's particle type in the system");
         MlpConst mlpc = ctx->mlp_c;
@@ -7038,9 +7059,9 @@ static int sc_sweep_impl(sc_ctx* ctx, int nsweeps, double temper, double transmx
 #define SPEC_PASS(DAM, IMG, MC)                                                                                \
     if (spec_lt) SPEC_PASS_LT(DAM, true, IMG, MC); else SPEC_PASS_LT(DAM, false, IMG, MC)
 #define SPEC_PASS_LT(DAM, LT, IMG, MC)                                                                         \
-    hipLaunchKernelGGL((k_sweep_spec<DAM, LT>), dim3(nblk), dim3(WAVE * SPEC_W), lds_spec, ctx->stream, g, sc, mp,     \
+    hipLaunchKernelGGL((k_sweep_spec<DAM, LT>), dim3(nblk), dim3(WAVE * SPEC_W), ls.bytes, ctx->stream, g, sc, mp,     \
                        ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32,          \
-                       cap_spec, ctx->ppmax, ctx->d_nonempty, IMG, MC, chain_tab(ctx), ctx->d_stats,    \
+                       ls.region, ctx->ppmax, ctx->d_nonempty, IMG, MC, chain_tab(ctx), ctx->d_stats,    \
                        ctx->d_dsum, ctx->d_flag)
             // four waves per cell in every mode (the network screen splits its
             // hidden units, and so its MFMA operands, between the four waves)
@@ -7286,16 +7307,7 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
         // the speculative variant (block waves 0): the stage beside SPEC_W trials' lists
         bool spec = ctx->spec && ctx->sweep_nw == 0;
         const bool spec_lt = sweep_table_bytes(ctx->nt) > 0;   // the tables fit in LDS beside the stage
-        int cap_spec = cap;
-        size_t lds_spec = 0;
-        if (spec) {
-            size_t tabb = sweep_table_bytes(ctx->nt);
-            long room = (long)SWEEP_LDS_BUDGET - (long)spec_layout(0, false, tabb).end - 16;
-            int cmax = room > 0 ? (int)(room / SPEC_STAGE_BYTES) : 0;
-            if (cap_spec > cmax) cap_spec = (cmax / 64) * 64;
-            spec = cap_spec >= 64;
-            if (spec) lds_spec = spec_layout(cap_spec, false, tabb).end;
-        }
+        const SpecLds ls = spec_lds(false, ctx->nt);
         size_t fixed = sizeof(float) * 2 * MV_STRIDE + sizeof(int) * (2 * 125 + 2) + SWEEP_SMALL_LDS +
                        sweep_table_bytes(ctx->nt);
         size_t per = stage_bytes(1) + sizeof(int) * 3;
@@ -7382,8 +7394,8 @@ static int sc_batch_sweep_impl(sc_ctx* ctx, int nsweeps, const double* temper, d
 #define SPEC_BATCH(DAM)                                                                                        \
     if (spec_lt) SPEC_BATCH_LT(DAM, true); else SPEC_BATCH_LT(DAM, false)
 #define SPEC_BATCH_LT(DAM, LT)                                                                                 \
-    SC_LAUNCH((k_sweep_batch_spec<DAM, LT>), dim3(nblk[ci]), dim3(WAVE * SPEC_W), lds_spec, ctx->stream, rp, R,           \
-              ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, cap_spec,  \
+    SC_LAUNCH((k_sweep_batch_spec<DAM, LT>), dim3(nblk[ci]), dim3(WAVE * SPEC_W), ls.bytes, ctx->stream, rp, R,           \
+              ctx->starts, ctx->P[c], ctx->O[c], ctx->Q[c], ctx->ID[c], ctx->d_pp32, ctx->d_tp32, ls.region,  \
               ctx->ppmax, ctx->d_rep_nonempty, nullptr, ctx->mlp_c, ChainTab{nullptr, nullptr, ctx->d_pp64, nullptr},           \
               ctx->d_rep_stats, ctx->d_rep_dsum, ctx->d_flag)
             int nw = ctx->sweep_nw ? ctx->sweep_nw : 4;

@@ -177,3 +177,49 @@ def test_sweep_with_an_axis_that_is_no_number():
             out.append((s, g.fixed_positions()))
     assert out[0][0]["trans_acc"] == out[1][0]["trans_acc"] > 0
     np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
+def crowded_cell(g):
+    """1,280 rods of two types within 28 sigma of a box of 240"""
+    types = np.repeat([1, 2], 640).astype(np.int32)
+    g.load_topology(W.top_init([W.TYPES["psc"], W.TYPES["cpsc"]], [640, 640]))
+    pos, d, q = g.generate_rsa(types, np.full(3, 28.0), 8)
+    g.set_config(np.full(3, 240.0), pos * 28.0 / 240.0 + 0.3, d, q, types)
+    g.set_max_active_cells(1)
+
+
+def test_sweep_of_a_crowded_cell():
+    """as many rods in one cell as a stage of records alone holds: the rows and the source list beside them are no
+    reason to refuse it"""
+    say("case: 1280 rods in one cell")
+    with sc_amd.GpuSystem(0) as g:
+        crowded_cell(g)
+        e0 = 0.5 * g.energy_per_particle().sum()
+        s = g.sweep(10, 1.0, 0.3, ROT_HALF, r=1, seed=3, counter=0)
+        e1 = 0.5 * g.energy_per_particle().sum()
+        say("accepted %d / %d" % (s["trans_acc"] + s["rot_acc"], s["trans_try"] + s["rot_try"]))
+        assert s["trans_try"] + s["rot_try"] == 12800 and s["trans_acc"] + s["rot_acc"] > 0
+        assert abs(e1 - e0 - s["energy_change"]) <= 1e-8 * max(abs(e0), abs(e1), 1.0)
+
+
+def test_chain_sweep_of_a_crowded_cell():
+    """402 chains in one cell: the table of their partners does not fit beside the stage, and the
+    one-trial-at-a-time trajectory comes out all the same."""
+    say("case: 402 chains in one cell")
+    small, pos, d, q, t = W.chain_lattice(402, 0.2, 5)
+    out = []
+    for nw in (0, 1):
+        with sc_amd.GpuSystem(0) as g:
+            g.load_topology(W.chain_topology(402))
+            g.set_config(np.full(3, 120.0), pos * small / 120.0 + 0.35, d, q, t)
+            g.set_max_active_cells(1)
+            g.set_block_waves(nw)
+            s = g.sweep(10, 1.1, 0.3, ROT_HALF, r=1, seed=29, counter=0)
+            out.append((s, g.get_config()))
+    (s1, c1), (s2, c2) = out
+    say("accepted %d / %d" % (s1["trans_acc"] + s1["rot_acc"], s1["trans_try"] + s1["rot_try"]))
+    assert s1["trans_acc"] + s1["rot_acc"] > 0
+    for k in ("trans_acc", "trans_try", "rot_acc", "rot_try", "left_cell", "bond_rejected"):
+        assert s1[k] == s2[k], k
+    for a, b in zip(c1, c2):
+        np.testing.assert_array_equal(a, b)
