@@ -1669,7 +1669,7 @@ __global__ __launch_bounds__(WAVE * NW, 2) void k_sweep_pass(Grid g, SysConst sc
 #define VROW 28
 #define VROW_DIR 24
 #define VROW_PD0 3
-#define SPEC_NV 8       // neighbours whose rows a wave derives at once when the stage has none
+#define SPEC_NV 16      // neighbours' patches whose vectors a wave derives at once when the stage has no rows
 
 // a trial's proposal, for the block's other waves and for its commit
 struct __align__(16) SpecProp {
@@ -1703,7 +1703,8 @@ __host__ __device__ inline SpecLayout spec_layout(size_t region, bool net, size_
     L.xd = spec_align(L.xl + 2 * SPEC_XCAP, 4);
     L.mv = spec_align(L.xd + (net ? 4 * SPEC_XCAP : 0), 16);
     L.wstride = L.mv + 4 * 2 * VROW;
-    static_assert(2 * 2 * SPEC_LCAP >= 4 * SPEC_NV * VROW, "neighbour rows over the candidate lists");
+    static_assert(2 * 2 * SPEC_LCAP >= 4 * 12 * SPEC_NV + 2 * 4 * SPEC_NV,
+                  "neighbours' patches and a chunk's survivors over the candidates");
     L.wbase = region;
     size_t o = L.wbase + SPEC_W * L.wstride;
     L.sten = o;
@@ -1728,7 +1729,7 @@ struct SpecScratch {
     uint16_t* xl;   // entries in the attraction's range: staged index, bit 15 the state
     float* xd;      // segment distance of each entry (network screen)
     float* mv;      // rows of the old and the new state (VROW floats each)
-    float* nv;      // rows of neighbours that have none in the stage (over nl, which is dead by then)
+    float* nv;      // patches of neighbours that have no row in the stage (over nl, which is dead by then)
 };
 
 // A particle's derived vectors as the speculative sweep keeps them in LDS:
@@ -2203,7 +2204,8 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
         int k1, k2, jj, which;
         bool sw, patch;
     };
-    auto item = [&](int it, const float* nrow) {
+    int c0 = 0;   // the first item of the chunk
+    auto item = [&](int it) {
         Item I;
         const int w = T.xl[it >> psh], mpp = it & ((1 << psh) - 1);
         I.jj = w & 0x7fff;
@@ -2217,21 +2219,36 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
         I.patch = mpp < npatch_pairs(*I.P);
         patch_pair_index(*I.P, mpp, I.k1, I.k2);   // patches of part1 and part2
         const float* mv = I.which ? mvn : mvo;
-        const float* nv = all_rows ? rows.row(I.jj) : nrow;
+        const float* nv = all_rows ? rows.row(I.jj) : T.nv + ((it - c0) >> psh) * 12 * npatch;
         I.r1 = (I.sw ? nv : mv) + 12 * I.k1;
         I.r2 = (I.sw ? mv : nv) + 12 * I.k2;
         return I;
     };
-    constexpr int CHUNK = 512;   // items whose survivors the list holds
-    for (int c0 = 0; c0 < nx << psh; c0 += CHUNK) {
-        const int end = min(CHUNK, (nx << psh) - c0);
+    // A chunk: as many items as the list of survivors holds, or (a stage without
+    // everyone's rows) those of SPEC_NV neighbours' patches, whose vectors are
+    // derived first, a lane each.  Derived for eight items at a time, on a lane of
+    // eight, and without the test, a sweep of 700 TCHPSC at packing fraction 0.4
+    // in a box of two cells an axis took 6.1 ms, 3.2 ms so (3.5 with whole
+    // searches, one per lane).
+    uint16_t* const surv = all_rows ? T.nl : T.nl + 2 * 12 * SPEC_NV;
+    const int chunk = all_rows ? 512 : (SPEC_NV / npatch) << psh;
+    for (; c0 < nx << psh; c0 += chunk) {
+        const int end = min(chunk, (nx << psh) - c0);
         int cnt = end;
-        const bool culled = all_rows && end > 8;
+        if (!all_rows) {
+            wave_lds_sync();
+            if (lane < (end >> psh) * npatch) {
+                const int kk = npatch > 1 ? lane & 1 : 0, jj = T.xl[(c0 >> psh) + (npatch > 1 ? lane >> 1 : lane)] & 0x7fff;
+                vrow_put(T.nv + 12 * (lane - kk), kk, load_view<float>(S.o[jj], S.q[jj], S.u[jj].w, tp, kk));
+            }
+            wave_lds_sync();
+        }
+        const bool culled = end > 8;
         if (culled) {
             cnt = 0;
             for (int b0 = 0; b0 < end; b0 += WAVE / 2) {
                 const int it = b0 + (lane >> 1), side = lane & 1;
-                const Item I = item(c0 + min(it, end - 1), nullptr);
+                const Item I = item(c0 + min(it, end - 1));
                 const PatchView<float> a = vrow_view(side ? I.r2 : I.r1, 0);
                 const float* l = side ? I.r1 : I.r2;
                 const V3<float> rs = side ? mk<float>(-I.r.x, -I.r.y, -I.r.z) : I.r;
@@ -2239,26 +2256,15 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                                              I.P->pcanglsw[side ? (I.k2 ? 3 : 1) : (I.k1 ? 2 : 0)], I.P->rcutSq);
                 unsigned long long m = __ballot(k & I.patch & (it < end));
                 m &= (m >> 1) & 0x5555555555555555ull;   // both sides, at the even lane
-                if ((m >> lane) & 1) T.nl[cnt + wave_prefix(m)] = (uint16_t)it;   // (the candidates are done with)
+                if ((m >> lane) & 1) surv[cnt + wave_prefix(m)] = (uint16_t)it;   // (the candidates are done with)
                 cnt += __popcll(m);
             }
             wave_lds_sync();
         }
         for (int b0 = 0; b0 < cnt; b0 += 8) {
             const int g = b0 + (lane >> 3), role = lane & 3, side = (lane >> 2) & 1;
-            const int it = c0 + (culled ? T.nl[min(g, cnt - 1)] : min(g, cnt - 1));
-            float* nrow = T.nv + (lane >> 3) * VROW;
-            if (!all_rows) {   // the neighbour's patch
-                wave_lds_sync();
-                if ((lane & 7) == 0) {
-                    const Item I = item(it, nrow);
-                    if (I.patch)
-                        vrow_put(nrow, I.sw ? I.k1 : I.k2,
-                                 load_view<float>(S.o[I.jj], S.q[I.jj], S.u[I.jj].w, tp, I.sw ? I.k1 : I.k2));
-                }
-                wave_lds_sync();
-            }
-            const Item I = item(it, nrow);
+            const int it = c0 + (culled ? surv[min(g, cnt - 1)] : min(g, cnt - 1));
+            const Item I = item(it);
             float x1 = 0.0f, x2 = 0.0f, ev = 0.0f;
             bool hit = false;
             if (I.patch)

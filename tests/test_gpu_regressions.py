@@ -223,3 +223,33 @@ def test_chain_sweep_of_a_crowded_cell():
         assert s1[k] == s2[k], k
     for a, b in zip(c1, c2):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("key,cap", [("psc", 0), ("psc", 4), ("tchpsc", 0), ("tchpsc", 4)])
+def test_sweep_without_rows(key, cap):
+    """Patch terms of neighbours whose vectors the stage does not hold, derived a chunk of entries at a time (16 of one
+    patch, 8 of two): the one-trial-at-a-time trajectory bit for bit in a dense system, entries beyond one chunk."""
+    say("case: sweep of %s without rows, home cache %d" % (key, cap))
+    n, ty, length = 800, {"psc": 1, "tchpsc": 3}[key], {"psc": 3.0, "tchpsc": 4.0}[key]
+    start = np.full(3, (n * W.particle_volume(1.0, length) / 0.13) ** (1.0 / 3.0))
+    box = start * (0.13 / 0.38) ** (1.0 / 3.0)
+    out = []
+    for nw in (0, 1):
+        with sc_amd.GpuSystem(0) as g:
+            g.load_topology(W.top_init([W.TYPES[key]], [n]))
+            pos, d, q = g.generate_rsa(np.full(n, ty, np.int32), start, 12)
+            g.set_config(start, pos, d, q, np.full(n, ty, np.int32))
+            for k in range(1, 9):
+                g.update_box(start * (box / start) ** (k / 8.0))
+                g.sweep(5, 0.3, 0.3, ROT_HALF, r=1, seed=4, counter=10 * k)
+            g.set_block_waves(nw)
+            g.set_home_cache(cap)
+            s = g.sweep(10, 0.3, 0.2, ROT_HALF, r=1, seed=7, counter=1000)
+            out.append((s, g.get_config()))
+    (s1, c1), (s2, c2) = out
+    say("accepted %d / %d" % (s1["trans_acc"] + s1["rot_acc"], s1["trans_try"] + s1["rot_try"]))
+    assert s1["trans_acc"] + s1["rot_acc"] > 0
+    for k in ("trans_acc", "trans_try", "rot_acc", "rot_try", "left_cell"):
+        assert s1[k] == s2[k], k
+    for a, b in zip(c1, c2):
+        np.testing.assert_array_equal(a, b)
