@@ -5014,7 +5014,7 @@ struct sc_ctx {
     double* d_loss = nullptr;
     int da_mode = DA_OFF;              // delayed-acceptance mode of sc_sweep
     // pair lists, clusters, order parameter
-    int* d_pcount = nullptr;            // per sorted particle: pair count, then offsets (n + 1)
+    int* d_pcount = nullptr;            // per ID: where its row of the pair list begins (n + 1)
     int pcount_cap = 0;
     int* d_pi = nullptr;
     int* d_pj = nullptr;
@@ -5045,8 +5045,7 @@ struct sc_ctx {
     bool molecules = false;             // some molecule has more than one particle
     int* d_cw = nullptr;                // chain word per ID
     MolP* d_mol = nullptr;              // per molecule type
-    double* d_bond = nullptr;           // per-ID bond energies (n)
-    int bond_cap = 0;
+    double* d_bond = nullptr;           // bond energies, a sum per 256 IDs
     // whole-system energy carried from move to move (the counterpart of
     // TotalEMatrix::allToAll, which sums the cached pair energies): set by a
     // full evaluation, advanced by the sweeps' accepted dE, dropped when the
@@ -5316,7 +5315,7 @@ static int upload_chains(sc_ctx* ctx) {
     }
     int rc;
     if ((rc = dalloc(ctx, &ctx->d_cw, cw.size())) || (rc = dalloc(ctx, &ctx->d_mol, mp.size())) ||
-        (rc = dalloc(ctx, &ctx->d_bond, cw.size())))
+        (rc = dalloc(ctx, &ctx->d_bond, (cw.size() + 255) / 256)))
         return rc;
     HIPCK(hipMemcpy(ctx->d_cw, cw.data(), cw.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCK(hipMemcpy(ctx->d_mol, mp.data(), mp.size() * sizeof(MolP), hipMemcpyHostToDevice));

@@ -155,20 +155,6 @@ __device__ __forceinline__ void mlp_setup_w(const unsigned char* __restrict__ im
 __device__ __forceinline__ void mlp_setup(const unsigned char* __restrict__ img, float* lds, int lane, MlpRegs& R) {
     mlp_setup_w<4>(img, lds, lane, 0, R);
 }
-// this lane's operands of all four unit blocks from the packed image in
-// global memory (the constants stay where mlp_setup put them)
-__device__ __forceinline__ void mlp_load_ops(const unsigned char* __restrict__ img, int lane, MlpRegs& R) {
-    const bf16x8* a1 = (const bf16x8*)(img + MLP_A1_OFF);
-    const bf16x8* a2 = (const bf16x8*)(img + MLP_A2_OFF);
-    const bf16x8* a3 = (const bf16x8*)(img + MLP_A3_OFF);
-#pragma unroll
-    for (int b = 0; b < 4; b++) R.a1[b] = a1[b * 64 + lane];
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        R.a2[q] = a2[q * 64 + lane];
-        R.a3[q] = a3[q * 64 + lane];
-    }
-}
 
 // SiLU for inference: hardware exp2 and reciprocal
 __device__ __forceinline__ float silu_fast(float z) {
