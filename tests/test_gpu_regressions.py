@@ -253,3 +253,25 @@ def test_sweep_without_rows(key, cap):
         assert s1[k] == s2[k], k
     for a, b in zip(c1, c2):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("nchains", [30, 250])
+def test_chain_moves_proposed_beside_a_move(nchains):
+    """Few molecules per coarse cell and 27 visits: the molecule proposed beside a move is often the one that moves,
+    and is proposed again.  Staged passes, moves of both kinds accepted, no cell left out; every accepted energy
+    change was taken from the state that the move found (a stale proposal breaks the sum)."""
+    say("case: proposals beside moves, %d chains" % nchains)
+    with sc_amd.GpuSystem(0) as g:
+        box, pos, d, q, t = W.chain_lattice(nchains, 0.2 if nchains > 100 else 0.01, 4)
+        g.load_topology(W.chain_topology(nchains))
+        g.set_config(box, pos, d, q, t)
+        g.set_trial_mode(1)
+        g.set_chain_moves(0.3, 0.5, 0.2)
+        g.set_chain_visit_factor(27)
+        e0 = g.allToAll()
+        s = g.sweep(20, 1.0, 0.3, ROT_HALF, r=1, seed=9, counter=0)
+        e1 = g.allToAll()
+        say({k: v for k, v in s.items() if k.startswith("chain")})
+        assert g.chain_pass_info()[1] and s["chain_cells_skipped"] == 0
+        assert s["chain_disp_acc"] > 0 and s["chain_rot_acc"] > 0
+        assert abs(e1 - e0 - s["energy_change"]) <= 1e-8 * max(abs(e0), abs(e1), 1.0)
