@@ -1952,7 +1952,7 @@ __device__ __forceinline__ bool side_possible(const PatchView<float>& a, const V
 //      behind them the trial's dependences on the round's earlier trials
 //   C  patch terms of the entries in range
 // stage -2: a list is full (more than SPEC_LCAP candidates of a state or
-// SPEC_XCAP entries), the trial cannot be evaluated here (dep holds).
+// SPEC_XCAP entries), the trial cannot be evaluated here.
 template <int DA>
 __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo, const uint4 un, const float4 oo,
                                            const float2 qo, const float4 on, const float2 qn, const SysConst& sc,
@@ -1995,15 +1995,10 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     const V3<float> dold = vrow_dir(mvo), dnew = vrow_dir(mvn);
     // phase A: the loads of a round's PA staged particles per lane first, then
     // the tests without branches (a load under a condition waits by itself)
-    const float hm = tp[t].hl;
-    // (an axis that is no number reaches whatever lies within the cutoff: the
-    // pair terms decide, of spheres a value, of rods NaN)
-    const bool nan_o = !(dot(dold, dold) < 4.0f), nan_n = !(dot(dnew, dnew) < 4.0f);
-    const V3<float> zero = mk<float>(0.0f, 0.0f, 0.0f), axo = nan_o ? zero : dold, axn = nan_n ? zero : dnew;
-    const float reach2o = nan_o ? sc.sqmaxcut : tp[t].reach2, reach2n = nan_n ? sc.sqmaxcut : tp[t].reach2;
+    const float hm = tp[t].hl, reach2 = tp[t].reach2;
     uint16_t* const nl_new = T.nl + SPEC_LCAP;
     int no = 0, nn = 0;
-    auto scan = [&](int base, auto pa) {
+    auto scan = [&](int base, auto pa, auto by_cutoff) {
         constexpr int PA = decltype(pa)::value;
         uint4 b[PA];
 #pragma unroll
@@ -2016,8 +2011,13 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             const V3<float> ro = fx_image_c(uo.x, uo.y, uo.z, b[h].x, b[h].y, b[h].z, sc.Lh, sc.Ll);
             V3<float> rn = ro;
             if (translate) rn = fx_image_c(un.x, un.y, un.z, b[h].x, b[h].y, b[h].z, sc.Lh, sc.Ll);
-            fo[h] = in & (centre_dist2(axo, hm, ro) <= reach2o);
-            fn[h] = in & (centre_dist2(axn, hm, rn) <= reach2n);
+            if constexpr (decltype(by_cutoff)::value) {
+                fo[h] = in & (dot(ro, ro) <= sc.sqmaxcut);
+                fn[h] = in & (dot(rn, rn) <= sc.sqmaxcut);
+            } else {
+                fo[h] = in & (centre_dist2(dold, hm, ro) <= reach2);
+                fn[h] = in & (centre_dist2(dnew, hm, rn) <= reach2);
+            }
         }
 #pragma unroll
         for (int h = 0; h < PA; h++) {
@@ -2030,15 +2030,19 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             nn += __popcll(mn);
         }
     };
-    for (int base = 0; base < S.n; base += 4 * WAVE) {
-        if (S.n - base <= 2 * WAVE) scan(base, std::integral_constant<int, 2>());
-        else scan(base, std::integral_constant<int, 4>());
+    if (__ballot(dold.x != dold.x)) {
+        // an axis that is no number: whatever lies within the cutoff is a
+        // candidate, and the pair terms decide (of spheres a value, of rods NaN)
+        for (int base = 0; base < S.n; base += 2 * WAVE)
+            scan(base, std::integral_constant<int, 2>(), std::true_type());
+    } else {
+        for (int base = 0; base < S.n; base += 4 * WAVE) {
+            if (S.n - base <= 2 * WAVE) scan(base, std::integral_constant<int, 2>(), std::false_type());
+            else scan(base, std::integral_constant<int, 4>(), std::false_type());
+        }
     }
     wave_lds_sync();
     if (no > SPEC_LCAP || nn > SPEC_LCAP) {
-        // (the candidates are counted at more than a pair term's range, so any
-        // accepted move before this one may be why)
-        dep = (1 << w) - 1;
         stage = -2;
         return false;
     }
@@ -2204,10 +2208,13 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
         int k1, k2, jj, which;
         bool sw, patch;
     };
-    int c0 = 0;   // the first item of the chunk
-    auto item = [&](int it) {
+    // the patches beside the mover's: a row per staged particle, or one per entry of the chunk
+    const float* const nvb = all_rows ? rows.v : T.nv;
+    const int nvs = all_rows ? VROW : 12 * npatch;
+    int e0 = 0;   // the first entry of the chunk
+    auto item = [&](int it) {   // (of the chunk)
         Item I;
-        const int w = T.xl[it >> psh], mpp = it & ((1 << psh) - 1);
+        const int e = it >> psh, w = T.xl[e0 + e], mpp = it & ((1 << psh) - 1);
         I.jj = w & 0x7fff;
         I.which = w >> 15;
         const uint4 bu = S.u[I.jj];
@@ -2219,7 +2226,7 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
         I.patch = mpp < npatch_pairs(*I.P);
         patch_pair_index(*I.P, mpp, I.k1, I.k2);   // patches of part1 and part2
         const float* mv = I.which ? mvn : mvo;
-        const float* nv = all_rows ? rows.row(I.jj) : T.nv + ((it - c0) >> psh) * 12 * npatch;
+        const float* nv = nvb + (all_rows ? I.jj : e) * nvs;
         I.r1 = (I.sw ? nv : mv) + 12 * I.k1;
         I.r2 = (I.sw ? mv : nv) + 12 * I.k2;
         return I;
@@ -2231,14 +2238,14 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
     // in a box of two cells an axis took 6.1 ms, 3.2 ms so (3.5 with whole
     // searches, one per lane).
     uint16_t* const surv = all_rows ? T.nl : T.nl + 2 * 12 * SPEC_NV;
-    const int chunk = all_rows ? 512 : (SPEC_NV / npatch) << psh;
-    for (; c0 < nx << psh; c0 += chunk) {
-        const int end = min(chunk, (nx << psh) - c0);
+    const int chunk = all_rows ? 512 >> psh : SPEC_NV / npatch;   // entries
+    for (; e0 < nx; e0 += chunk) {
+        const int end = min(chunk, nx - e0) << psh;
         int cnt = end;
         if (!all_rows) {
             wave_lds_sync();
             if (lane < (end >> psh) * npatch) {
-                const int kk = npatch > 1 ? lane & 1 : 0, jj = T.xl[(c0 >> psh) + (npatch > 1 ? lane >> 1 : lane)] & 0x7fff;
+                const int kk = npatch > 1 ? lane & 1 : 0, jj = T.xl[e0 + (npatch > 1 ? lane >> 1 : lane)] & 0x7fff;
                 vrow_put(T.nv + 12 * (lane - kk), kk, load_view<float>(S.o[jj], S.q[jj], S.u[jj].w, tp, kk));
             }
             wave_lds_sync();
@@ -2248,7 +2255,7 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             cnt = 0;
             for (int b0 = 0; b0 < end; b0 += WAVE / 2) {
                 const int it = b0 + (lane >> 1), side = lane & 1;
-                const Item I = item(c0 + min(it, end - 1));
+                const Item I = item(min(it, end - 1));
                 const PatchView<float> a = vrow_view(side ? I.r2 : I.r1, 0);
                 const float* l = side ? I.r1 : I.r2;
                 const V3<float> rs = side ? mk<float>(-I.r.x, -I.r.y, -I.r.z) : I.r;
@@ -2263,8 +2270,7 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
         }
         for (int b0 = 0; b0 < cnt; b0 += 8) {
             const int g = b0 + (lane >> 3), role = lane & 3, side = (lane >> 2) & 1;
-            const int it = c0 + (culled ? surv[min(g, cnt - 1)] : min(g, cnt - 1));
-            const Item I = item(it);
+            const Item I = item(culled ? surv[min(g, cnt - 1)] : min(g, cnt - 1));
             float x1 = 0.0f, x2 = 0.0f, ev = 0.0f;
             bool hit = false;
             if (I.patch)
@@ -2886,11 +2892,9 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
             const int f = __builtin_amdgcn_readfirstlane(rw[q]);
             const int st = (f >> 2) & 3, stg = (f >> 4) & 3, tr = (f >> 1) & 1, ac = f & 1;
             if (q < W && nfin == q) {
-                if (st == 3) {
-                    full = 1;   // unless an earlier accepted trial is why
-                }
-                if (((f >> 8) & accm) != 0) full = 0;
-                else if (st != 3) {
+                if (st == 3) {   // (behind an accepted trial, which may be why: evaluated again)
+                    full = accm == 0;
+                } else if (((f >> 8) & accm) == 0) {
                     nfin = q + 1;
                     n_ttry += tr;
                     n_rtry += 1 - tr;
