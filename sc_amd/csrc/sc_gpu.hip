@@ -2522,6 +2522,9 @@ __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query*
     if (tid == 0) out[by_id ? q.id : qi] = sum;
 }
 
+typedef float vec4f __attribute__((ext_vector_type(4)));
+typedef float vec2f __attribute__((ext_vector_type(2)));
+
 // stage_load for the speculative sweep: of the stencil's particles only those
 // that can matter to the home cell are staged, in stencil order: those within
 // sc.reach of the cell's box, where every trial position lies, and chain
@@ -2572,10 +2575,15 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
             misc[0] = home_idx;
         }
     } else if (tid < WAVE + 3) {   // meanwhile the home cell's box: centre in fixed point, half edges; a lane per axis
+        // (values chosen, not places: a choice between the structures' members
+        // puts the structures on every lane's stack)
         const int q = tid - WAVE;
-        const int c = q == 0 ? cx : q == 1 ? cy : cz, nc = q == 0 ? g.nc[0] : q == 1 ? g.nc[1] : g.nc[2];
-        const uint32_t sh = q == 0 ? g.sh[0] : q == 1 ? g.sh[1] : g.sh[2];
-        const float L = q == 0 ? sc.L[0] : q == 1 ? sc.L[1] : sc.L[2];
+        const int n0 = g.nc[0], n1 = g.nc[1], n2 = g.nc[2];
+        const uint32_t h0 = g.sh[0], h1 = g.sh[1], h2 = g.sh[2];
+        const float l0 = sc.L[0], l1 = sc.L[1], l2 = sc.L[2];
+        const int c = q == 0 ? cx : q == 1 ? cy : cz, nc = q == 0 ? +n0 : q == 1 ? +n1 : +n2;
+        const uint32_t sh = q == 0 ? +h0 : q == 1 ? +h1 : +h2;
+        const float L = q == 0 ? +l0 : q == 1 ? +l1 : +l2;
         misc[4 + q] = (int)(sh + (uint32_t)((((uint64_t)(2 * c + 1)) << 31) / (uint64_t)nc));
         misc[8 + q] = __float_as_int(0.5f * L / (float)nc);
     }
@@ -2628,15 +2636,15 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
             bool keep[2];
             int pos[2], id[2], lo[2], src[2];
             uint4 u[2];
-            float4 o[2];
-            float2 q[2];
+            vec4f o[2];   // (arrays of the float4 class are kept on the stack)
+            vec2f q[2];
 #pragma unroll
             for (int h = 0; h < 2; h++) src[h] = source(min(base + h * WAVE * NW + tid, total - 1), lo[h]);
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 u[h] = P[src[h]];
-                o[h] = O[src[h]];
-                q[h] = Q[src[h]];
+                o[h] = *(const vec4f*)(O + src[h]);
+                q[h] = *(const vec2f*)(Q + src[h]);
                 id[h] = ID[src[h]];
             }
 #pragma unroll
@@ -2646,8 +2654,8 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
             for (int h = 0; h < 2; h++) {
                 if (keep[h]) {
                     S.u[pos[h]] = u[h];
-                    S.o[pos[h]] = o[h];
-                    S.q[pos[h]] = q[h];
+                    *(vec4f*)(S.o + pos[h]) = o[h];
+                    *(vec2f*)(S.q + pos[h]) = q[h];
                     S.id[pos[h]] = id[h];
                 }
                 if (base + h * WAVE * NW + tid == hbeg) misc[1] = pos[h];
