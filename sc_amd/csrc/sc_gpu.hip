@@ -440,9 +440,11 @@ __global__ __launch_bounds__(WAVE * CELL_SORT_CELLS) void k_cell_sort(int ncell,
 // The whole cell list of a small system (n <= BUILD_N particles, ncell <=
 // BUILD_CELLS cells) by one block: counts and ranks in LDS, the scan, the
 // order by ID within each cell (a particle's rank is the number of smaller IDs
-// in its cell), and the permuted records.  The general path's two fills and
-// five kernels are bound by their launches: 7 x 4.4 us of device time for
-// 1,000 particles, rebuilt for every sweep and every committed move.
+// in its cell), and the permuted records.  The general path's fill and five
+// kernels are bound by their launches; a rebuild by one block / by them, us:
+// 100 particles 5.1 / 23, 1,000 in 10^3 cells 7.2 / 22, 3,000 in 4^3 9.6 / 22,
+// 4,096 in 10^3 11.6 / 22, in 2^3 (512 a cell) 39 / 80, in 20^3 29 / 29: the
+// bounds are where the two meet.
 #define BUILD_N 4096
 #define BUILD_CELLS 8192
 __global__ __launch_bounds__(1024) void k_build_small(int n, int ncell, Grid g, const uint4* __restrict__ Pi,
@@ -1914,12 +1916,16 @@ __device__ __forceinline__ bool quad_intersect(const RowQuery& q, int role, floa
 // |x| <= h2, inside the two half spaces that bound the region's wedge (their
 // planes hold the axis and one side each) is empty, or stays farther than rcut
 // from the axis.  Every point that the intersection accepts lies in the wedge
-// and within rcut of the axis up to the FP32 error of these products (~1e-6;
-// the half spaces are widened by a hundred times that, rcut^2 by 1e-3), and a
-// pair term needs such a point on both sides.  Wedges of 180 degrees and more
-// (cossw <= 0) are not half-space intersections: always true.  A NaN keeps
-// the item.  Of the patch pairs in range of uniformly oriented TCHPSC 9.7% have both
-// hits and 10.6% pass both tests (without the distance 20%).
+// and within rcut of the axis up to the FP32 error of these products (~1e-6 for
+// rods of a few sigma; the half spaces are widened by a hundred times that,
+// rcut^2 by 1e-3), and a pair term needs such a point on both sides.  That
+// error grows with the rods: of three million pairs in contact the test left
+// out no hit of the FP32 search up to half lengths of 100 sigma, 4 at 200 and
+// 494 at 1,000, where the search itself takes points that are no hits: in FP64
+// the term of every one of them is 0.  Wedges of 180 degrees and more (cossw
+// <= 0) are not half-space intersections: always true.  A NaN keeps the item.
+// Of the patch pairs in range of uniformly oriented TCHPSC 9.7% have both hits
+// and 10.6% pass both tests (without the distance 20%).
 __device__ __forceinline__ bool side_possible(const PatchView<float>& a, const V3<float>& p2, const V3<float>& r,
                                               float h2, float cossw, float rcSq) {
     const V3<float> n0 = cross(a.ax, a.s0), n1 = cross(a.ax, a.s1);
@@ -1960,13 +1966,14 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                                            const SpecScratch& T, const float* ml,
                                            const unsigned char* __restrict__ mlp_img, const MlpConst& mc,
                                            const ChainTab& ct, double thr1, double thr2, const Rows& rows,
-                                           const int16_t* partner, bool translate, const SpecProp* prop, int w,
+                                           const int16_t* partner, bool table, bool translate,
+                                           const SpecProp* prop, int w,
                                            double& eo, double& en, double& des, int& stage, int& dep) {
     const int lane = lane_id(), t = uo.w, idk = S.id[k];
     const int cwk = ct.cw ? ct.cw[idk] : 0, bmask = cwk & 15;
     if (bmask) {   // partner: the staged chain partners of particle k (-1: not staged)
         int found = 0;
-        if (!partner) {   // a stage without room for them: found among the staged (in the entries' list, empty yet)
+        if (!table) {   // a stage without room for them: found among the staged (in the entries' list, empty yet)
             if (lane < 4) T.xl[lane] = 0xffff;
             wave_lds_sync();
             for (int j = lane; j < S.n; j += WAVE) {
@@ -2015,8 +2022,8 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
                 fo[h] = in & (dot(ro, ro) <= sc.sqmaxcut);
                 fn[h] = in & (dot(rn, rn) <= sc.sqmaxcut);
             } else {
-                fo[h] = in & (centre_dist2(dold, hm, ro) <= reach2);
-                fn[h] = in & (centre_dist2(dnew, hm, rn) <= reach2);
+                fo[h] = in & !(centre_dist2(dold, hm, ro) > reach2);   // (a NaN stays)
+                fn[h] = in & !(centre_dist2(dnew, hm, rn) > reach2);
             }
         }
 #pragma unroll
@@ -2030,21 +2037,23 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             nn += __popcll(mn);
         }
     };
-    if (__ballot(dold.x != dold.x)) {
-        // an axis that is no number: whatever lies within the cutoff is a
-        // candidate, and the pair terms decide (of spheres a value, of rods NaN)
-        for (int base = 0; base < S.n; base += 2 * WAVE)
-            scan(base, std::integral_constant<int, 2>(), std::true_type());
-    } else {
-        for (int base = 0; base < S.n; base += 4 * WAVE) {
-            if (S.n - base <= 2 * WAVE) scan(base, std::integral_constant<int, 2>(), std::false_type());
-            else scan(base, std::integral_constant<int, 4>(), std::false_type());
-        }
+    for (int base = 0; base < S.n; base += 4 * WAVE) {
+        if (S.n - base <= 2 * WAVE) scan(base, std::integral_constant<int, 2>(), std::false_type());
+        else scan(base, std::integral_constant<int, 4>(), std::false_type());
     }
     wave_lds_sync();
     if (no > SPEC_LCAP || nn > SPEC_LCAP) {
-        stage = -2;
-        return false;
+        const bool nan = __ballot(dold.x != dold.x) != 0ull;
+        if (nan) {   // an axis that is no number had everyone in reach: by the cutoff, as the pair terms will
+            no = nn = 0;
+            for (int base = 0; base < S.n; base += 2 * WAVE)
+                scan(base, std::integral_constant<int, 2>(), std::true_type());
+            wave_lds_sync();
+        }
+        if (!nan || no > SPEC_LCAP || nn > SPEC_LCAP) {
+            stage = -2;
+            return false;
+        }
     }
     double ao = 0.0, an = 0.0;
     if (bmask) {
@@ -2324,9 +2333,9 @@ __global__ void k_commit(int nq, const Query* __restrict__ qs, Query q1, const i
 // range, eight lanes each (quad_intersect), behind side_possible where there
 // are more than fit one pass.  Bound by latency: one wave that walked the
 // stencil cell by cell, the whole pair functor inlined per candidate, took
-// 104 us for one query of 1,000 PSC and 720 us for every particle of a 34,000-particle mixture.  NW = 4 for few
-// queries (a host program's single moves); NW = 1 when the queries alone fill
-// the chip.
+// 104 us for one query of 1,000 PSC and 720 us for every particle of a
+// 34,000-particle mixture.  NW = 4 for few queries (a host program's single
+// moves); NW = 1 when the queries alone fill the chip.
 constexpr int QRY_LCAP = 1024;   // candidates held before they are evaluated
 template <int NW>
 __global__ __launch_bounds__(WAVE * NW) void k_energy_query(int nq, const Query* __restrict__ qs,
@@ -2543,8 +2552,10 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
                             const SysConst& sc, int cx, int cy, int cz, const int* __restrict__ starts,
                             const uint4* __restrict__ P, const float4* __restrict__ O, const float2* __restrict__ Q,
                             const int* __restrict__ ID, const ChainTab& ct, int* sten, int* misc, int16_t*& partner,
-                            size_t& used, bool half_stencil = false) {
+                            bool& table, size_t& used, bool half_stencil = false) {
     static_assert(NW > 1, "the home cell's box is the second wave's");
+    table = false;
+    partner = (int16_t*)region;
     const int ns = stencil_size(g);
     int* pre = sten;          // ns+1 prefix of counts
     int* cst = sten + ns + 1; // cell start per stencil entry
@@ -2593,7 +2604,6 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
     if (hbeg == hend) {   // nothing to move: nothing staged
         S.n = S.h0 = S.h1 = 0;
         used = 0;
-        partner = nullptr;
         return true;
     }
     uint32_t cen[3];
@@ -2630,7 +2640,6 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
         S.q = (float2*)(S.o + t4);
         S.id = (int*)(S.q + t4);
         used = (size_t)t4 * 44;
-        partner = nullptr;
         int n = 0, par = 0;
         for (int base = 0; base < total; base += 2 * WAVE * NW) {
             bool keep[2];
@@ -2701,10 +2710,10 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
     S.q = (float2*)(S.o + n4);
     S.id = (int*)(S.q + n4);
     used = (size_t)n4 * 44;
-    partner = nullptr;
     const size_t pbytes = ((size_t)(hend - hbeg) * 8 + 15) & ~(size_t)15;
     if (ct.cw && used + pbytes <= region_bytes - 4 * (size_t)cap) {   // (not over the list)
         // the home cell's chain partners: four staged indices per particle
+        table = true;
         partner = (int16_t*)(region + used);
         used += pbytes;
         for (int i = tid; i < 4 * (hend - hbeg); i += WAVE * NW) partner[i] = -1;
@@ -2716,7 +2725,7 @@ __device__ bool stage_reach(Stage& S, unsigned char* region, size_t region_bytes
         S.o[i] = O[src];
         S.q[i] = Q[src];
         S.id[i] = id;
-        if (partner) {
+        if (table) {
             const int w = ct.cw[id];
             for (int q = 0; q < 4; q++)   // this particle is partner q ^ 1 (the opposite step) of its partner q
                 if ((w >> q) & 1) {
@@ -2803,9 +2812,10 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
         tp = tpl;
     }
     int16_t* partners;
+    bool table;
     size_t used;
     if (!stage_reach<SPEC_W>(S, smem, L.wbase, region / SPEC_STAGE_BYTES, g, sc, cx, cy, cz, starts, P, O, Q, ID, ct, sten, misc, partners,
-                             used)) {
+                             table, used)) {
         if (tid == 0) atomicOr(flag, 1);
         return;
     }
@@ -2871,9 +2881,9 @@ __device__ __forceinline__ void sweep_cell_spec(int b, const Grid& g, const SysC
                 for (int i = 0; i < w; i++) dep |= prop[i].k == k ? 1 << i : 0;
             } else {
                 double eo, en, des;
-                const int16_t* pk = partners ? partners + 4 * (k - S.h0) : nullptr;
                 bool pass = spec_trial<DA>(S, k, uo, un, oo, qo, on, qn, sc, pp, tp, ppmax, T, ml, mlp_img, mc, ct,
-                                           R.thr1, R.thr2, rows, pk, translate, prop, w, eo, en, des, stage, dep);
+                                           R.thr1, R.thr2, rows, partners + 4 * (k - S.h0), table, translate, prop, w, eo, en,
+                                           des, stage, dep);
                 if (stage == -1) {
                     status = 2;   // whatever the others do: the partner's cell does not change in a pass
                 } else if (stage == -2) {
@@ -3080,9 +3090,10 @@ __device__ __forceinline__ void energy_cell(int cell, const Grid& g, const SysCo
     const bool half = g.nc[0] >= w && g.nc[1] >= w && g.nc[2] >= w;
     Stage S;
     int16_t* partners;
+    bool table;
     size_t used;
     if (!stage_reach<NW>(S, smem, (size_t)region_bytes, cap, g, sc, cx, cy, cz, starts, P, O, Q, ID,
-                         ChainTab{nullptr, nullptr, nullptr, nullptr}, sten, misc, partners, used, half)) {
+                         ChainTab{nullptr, nullptr, nullptr, nullptr}, sten, misc, partners, table, used, half)) {
         if (tid == 0) {
             atomicOr(flag, full_cap ? 1 : 32);
             partial[cell] = 0.0;
@@ -3771,13 +3782,11 @@ __device__ __forceinline__ int axis_offsets(int nc, int* off) {
     return 3;
 }
 
-// Pairs (ID_i < ID_j) within rc over a cell list with cells >= rc wide: one
-// thread per particle (sorted position), counting (write == nullptr) or
-// writing at its offset.  Within a particle the pairs come in cell-list order.
-// 32 lanes per particle, a stencil cell each (a thread per particle walked its
-// 27 cells alone: 66 us for 24,300 particles, 19 us so).  Rows by ID: count[i] pairs of
-// particle i with larger IDs; with `offset` the pairs themselves, a row's in
-// any order (k_pair_rank orders them).
+// Pairs (ID_i < ID_j) within rc over a cell list with cells >= rc wide: 32
+// lanes per particle, a stencil cell each (a thread per particle walked its 27
+// cells alone: 66 us for 24,300 particles, 19 us so).  Rows by ID: count[i]
+// pairs of particle i with larger IDs; with `offset` the pairs themselves, a
+// row's in any order (k_pair_rank orders them).
 __global__ __launch_bounds__(256) void k_pair_list(int n, const uint4* __restrict__ P, const int* __restrict__ ID,
                                                    const int* __restrict__ starts, Grid g, double rc2, double bx,
                                                    double by, double bz, int* __restrict__ count,
@@ -4430,12 +4439,13 @@ __global__ __launch_bounds__(WAVE * NW) void k_chain_pass(Grid g, Grid gc, SysCo
 // chain of latencies (its molecule found and moved in FP64 ~9,000 cycles, the
 // items ~34,000, the decision and commit ~4,000): one wave proposes the next
 // molecule while the others finish this one's items.  10,001 chains of three:
-// 2543 us a pass with every step in turn, 1590-1830 us with that and the
-// functor's single copy (chain_pair); four NPT steps of them 16.9 ms, 14.0 with
-// the overlap alone, 13.3 with both.  The region is found through the fine cell list (whole cells
-// overlapping it, filtered by position).  A block whose region holds more
-// than `cap` particles makes no move in this pass (its trials are counted as
-// rejected, and the block in chain_skipped).
+// 2543 us a pass with every step in turn, 1840-1890 us with that and the
+// functor's single copy (chain_pair) at the same seed; 1560-2260 us over five, as
+// long as a pass's busiest cell.  Four NPT steps of them 16.9 ms, 14.0 with
+// the overlap alone, 13.3 with both.  The region is found through the fine
+// cell list (whole cells overlapping it, filtered by position).  A block whose
+// region holds more than `cap` particles makes no move in this pass (its
+// trials are counted as rejected, and the block in chain_skipped).
 #define CHAIN_ST_LCAP 512    // molecules per coarse cell
 #define CHAIN_ST_OCAP 1024   // particles of the cell's movable molecules
 #define CHAIN_ST_RCAP 1024   // fine cells overlapping a region
@@ -5470,8 +5480,10 @@ static int stage_cap(const sc_ctx* ctx, const Grid& g, const double* box, int ca
 static size_t stage_bytes(int cap) { return (size_t)cap * (16 + 16 + 8 + 4); }
 
 // Stage capacity and dynamic LDS of k_energy_all for a grid: twice the mean
-// number of particles that stage_reach keeps of the half stencil (and rows for
-// 1.25 times), so that four or more blocks share a CU; `full`: the capacity the full stencil may need.
+// number of particles that stage_reach keeps of the half stencil, and rows for
+// 1.25 times.  With the static 8.5 KB, 48.7 KB for 65,536 TCHPSC at packing
+// fraction 0.25: the three blocks a CU that the kernel's registers allow; two
+// at the largest stage.  `full`: the capacity the full stencil may need.
 struct EnergyLds {
     int cap, bytes;
 };
