@@ -95,6 +95,22 @@ template <typename R> SC_HD V3<R> normalised(V3<R> a) {
     if (t != R(0)) { t = R(1) / t; a.x *= t; a.y *= t; a.z *= t; }
     return a;
 }
+// FP32 on the device: the hardware's square root and reciprocal by name.  Left
+// to the compiler, the operators are these (about 1 ulp) except where it moves
+// one out of a loop or a condition: there it drops the note on its accuracy and
+// rounds correctly, so that the same vector would differ in the last place
+// between kernels.
+SC_HD V3<float> normalised(V3<float> a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float t = __builtin_amdgcn_sqrtf(a.x * a.x + a.y * a.y + a.z * a.z);
+    if (t != 0.0f) { t = __builtin_amdgcn_rcpf(t); a.x *= t; a.y *= t; a.z *= t; }
+    return a;
+#else
+    float t = sqrtf(a.x * a.x + a.y * a.y + a.z * a.z);
+    if (t != 0.0f) { t = 1.0f / t; a.x *= t; a.y *= t; a.z *= t; }
+    return a;
+#endif
+}
 // quaternion rotation by (c, s*ax) -- Vector::rotate, Vector.h:138-160
 template <typename R> SC_HD V3<R> qrot(const V3<R>& v, const V3<R>& ax, R c, R s) {
     R qx = ax.x * s, qy = ax.y * s, qz = ax.z * s;

@@ -275,3 +275,40 @@ def test_chain_moves_proposed_beside_a_move(nchains):
         assert g.chain_pass_info()[1] and s["chain_cells_skipped"] == 0
         assert s["chain_disp_acc"] > 0 and s["chain_rot_acc"] > 0
         assert abs(e1 - e0 - s["energy_change"]) <= 1e-8 * max(abs(e0), abs(e1), 1.0)
+
+
+SPECIES = {"psc": (W.TYPES["psc"], 1, 3.0), "cpsc": (W.TYPES["cpsc"], 2, 3.0), "tchpsc": (W.TYPES["tchpsc"], 3, 4.0),
+           "tcpsc": ("D 4 TCPSC 1.0 1.0 1.0 0.2 80.0 5.0 3.0 0.0 120.0 70.0 5.0", 4, 3.0),
+           "spa": ("S 6 SPA 1.0 1.0 1.0 0.2", 6, 0.0)}
+
+
+@pytest.mark.parametrize("keys", [("psc",), ("cpsc",), ("tchpsc",), ("tcpsc",), ("tchpsc", "spa"), ("psc", "cpsc", "tchpsc")])
+def test_one_value_of_a_pair_in_queries_and_lists(keys):
+    """A pair has one FP32 value wherever it is priced: a particle's energy is the sum of its pairs' energies, the
+    whole system's the sum of all, but for the order of FP64 sums.  (The queries normalised their neighbours' axes
+    with a correctly rounded root where the other kernels have the hardware's: 1e-7 to 1e-6 kT off.)"""
+    say("case: pair values of", *keys)
+    m = 1800 // len(keys)
+    types = np.concatenate([np.full(m, SPECIES[k][1], np.int32) for k in keys])
+    vol = sum(m * W.particle_volume(1.0, SPECIES[k][2]) for k in keys)
+    start = np.full(3, (vol / 0.12) ** (1.0 / 3.0))
+    with sc_amd.GpuSystem(0) as g:
+        g.load_topology(W.top_init([SPECIES[k][0] for k in keys], [m] * len(keys)))
+        pos, d, q = g.generate_rsa(types, start, 3)
+        g.set_config(start, pos, d, q, types)
+        for k in range(1, 7):
+            g.update_box(start * (0.12 / 0.28) ** (k / 18.0))
+            g.sweep(4, 1.0, 0.3, ROT_HALF, r=1, seed=4, counter=10 * k)
+        p = g.neighbor_pairs(g.maxcut)
+        e = g.p2p(p[:, 1], p[:, 0])
+        each = np.zeros(len(types))
+        np.add.at(each, p[:, 0], e)
+        np.add.at(each, p[:, 1], e)
+        got = g.energy_per_particle()
+        say("largest difference %.2e kT" % np.abs(got - each).max())
+        size = np.zeros(len(types))
+        np.add.at(size, p[:, 0], np.abs(e))
+        np.add.at(size, p[:, 1], np.abs(e))
+        assert np.all(np.abs(got - each) <= 1e-12 * (1.0 + size))
+        assert abs(g.oneToAll(5) - each[5]) <= 1e-12 * (1.0 + size[5])
+        assert abs(g.allToAll() - e.sum()) <= 1e-12 * (1.0 + np.abs(e).sum())
