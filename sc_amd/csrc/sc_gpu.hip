@@ -1013,7 +1013,7 @@ __device__ __forceinline__ DPart<float> mv_part(const float* mv, int t, int g) {
 struct TrialScratch {
     int* nl;     // near list, cap entries
     int* xl;     // expensive list, 2*cap entries
-    float* xd;   // segment distance of each expensive entry, 2*cap
+    float* xd;   // squared segment distance of each expensive entry, 2*cap
     float* mv;   // 2 * MV_STRIDE floats
     int* bp;     // staged index of each chain partner (4 ints)
     int* cnt;    // block compaction counts (2 CNT_HALF ints)
@@ -1105,9 +1105,9 @@ __device__ __forceinline__ void scan_stencil(const Stage& S, int k, const uint4 
 
 // The network's 12 features of the pair of the moving particle (as part1, at
 // position um with axis dm and patch direction pm) and the staged particle jj
-// at segment distance dseg; false, with zero features, when !valid and for
-// pairs of other types (they screen with 0).
-__device__ __forceinline__ bool pair_features(const Stage& S, bool valid, int jj, float dseg, int t, const uint4 um,
+// at squared segment distance dseg2; false, with zero features, when !valid and
+// for pairs of other types (they screen with 0).
+__device__ __forceinline__ bool pair_features(const Stage& S, bool valid, int jj, float dseg2, int t, const uint4 um,
                                               const V3<float>& dm, const V3<float>& pm, const SysConst& sc,
                                               const MlpConst& mc, float* f) {
     bool net = false;
@@ -1118,8 +1118,11 @@ __device__ __forceinline__ bool pair_features(const Stage& S, bool valid, int jj
             V3<float> r = fx_image_c(um.x, um.y, um.z, b.x, b.y, b.z, sc.Lh, sc.Ll);
             float4 ob = S.o[jj];
             float2 qb = S.q[jj];
-            mlp_features(dm, pm, mk<float>(ob.x, ob.y, ob.z), mk<float>(ob.w, qb.x, qb.y), r, dseg, mc.lsc, mc.rcut,
-                         mc.pdis, mc.pswitch, f);
+            // (the root rounded correctly by way of FP64: an FP32 one is that or
+            // the hardware's, by where the compiler leaves it, and the sweep's
+            // variants are to screen alike)
+            mlp_features(dm, pm, mk<float>(ob.x, ob.y, ob.z), mk<float>(ob.w, qb.x, qb.y), r,
+                         (float)sqrt((double)dseg2), mc.lsc, mc.rcut, mc.pdis, mc.pswitch, f);
         }
     }
     if (!net)
@@ -1255,7 +1258,7 @@ __device__ __forceinline__ bool trial_energies(const Stage& S, int k, const uint
         int pos = block_compact1<NW>(need, nx, T.cnt, cpar);
         if (need) {
             T.xl[pos] = jj | (which << 30);
-            if constexpr (DA == DA_NET) T.xd[pos] = sqrtf(dseg2);
+            if constexpr (DA == DA_NET) T.xd[pos] = dseg2;
         }
     }
     __syncthreads();
@@ -1729,7 +1732,7 @@ __host__ __device__ inline SpecLayout spec_layout(size_t region, bool net, size_
 struct SpecScratch {
     uint16_t* nl;   // candidates (staged indices): SPEC_LCAP of the old state, then SPEC_LCAP of the new one
     uint16_t* xl;   // entries in the attraction's range: staged index, bit 15 the state
-    float* xd;      // segment distance of each entry (network screen)
+    float* xd;      // squared segment distance of each entry (network screen)
     float* mv;      // rows of the old and the new state (VROW floats each)
     float* nv;      // patches of neighbours that have no row in the stage (over nl, which is dead by then)
 };
@@ -2154,7 +2157,7 @@ __device__ __forceinline__ bool spec_trial(const Stage& S, int k, const uint4 uo
             int pos = nx + wave_prefix(m);
             if (pos < SPEC_XCAP) {
                 T.xl[pos] = (uint16_t)(jj | (which << 15));
-                if constexpr (DA == DA_NET) T.xd[pos] = sqrtf(dseg2);
+                if constexpr (DA == DA_NET) T.xd[pos] = dseg2;
             }
         }
         nx += __popcll(m);

@@ -312,3 +312,41 @@ def test_one_value_of_a_pair_in_queries_and_lists(keys):
         assert np.all(np.abs(got - each) <= 1e-12 * (1.0 + size))
         assert abs(g.oneToAll(5) - each[5]) <= 1e-12 * (1.0 + size[5])
         assert abs(g.allToAll() - e.sum()) <= 1e-12 * (1.0 + np.abs(e).sum())
+
+
+def test_network_screen_of_the_sweeps_variants():
+    """The speculative sweep with the network screen is the one-trial-at-a-time sweep: every trial past the first
+    screen goes to the network, so a feature an ulp off in one of them would show as another decision."""
+    say("case: network screen, 32,768 TCHPSC, speculative and four waves a trial")
+    n = 32768
+    types = np.full(n, 3, np.int32)
+    start = np.full(3, (n * W.particle_volume(1.0, 4.0) / 0.13) ** (1.0 / 3.0))
+    rng = np.random.default_rng(5)
+    w = None
+    out = []
+    for nw in (0, 4):
+        with sc_amd.GpuSystem(0) as g:
+            g.load_topology(W.top_init([W.TYPES["tchpsc"]], [n]))
+            pos, d, q = g.generate_rsa(types, start, 6)
+            g.set_config(start, pos, d, q, types)
+            for k in range(1, 7):
+                g.update_box(start * (0.13 / 0.25) ** (k / 18.0))
+                g.sweep(4, 1.0, 0.3, ROT_HALF, r=1, seed=4, counter=10 * k)
+            g.mlp_init(3, seed=2)
+            if w is None:
+                w = g.mlp_get_weights()
+                w[-65:-1] = 3.0 * rng.normal(size=64)
+            g.mlp_set_weights(w)
+            g.set_surrogate(1)
+            g.set_network_min_entries(0)
+            g.set_trial_mode(1)
+            g.set_visit_factor(8)
+            g.set_block_waves(nw)
+            s = g.sweep(400, 1.0, 0.3, ROT_HALF, r=1, seed=8, counter=1000)
+            out.append((s, g.fixed_positions()))
+    (s1, u1), (s2, u2) = out
+    say("screened %d, passed %d and %d" % (s1["stage2_try"], s1["stage2_acc"], s2["stage2_acc"]))
+    assert s1["stage2_try"] > 10 ** 6
+    for k in ("stage1_acc", "stage2_try", "stage2_acc", "trans_acc", "rot_acc"):
+        assert s1[k] == s2[k], k
+    np.testing.assert_array_equal(u1, u2)
